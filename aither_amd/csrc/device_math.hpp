@@ -534,6 +534,82 @@ __device__ __forceinline__ void RoeOffDiag(const GasT<double> &g, const double W
   }
 }
 
+// ---------------------------------------------------------------------------
+// Several quotients by one divisor: the reciprocal y is refined once by two
+// Newton steps (one in FP32), then each quotient takes one product and one
+// (two) residual corrections (Markstein, "Computation of elementary functions
+// on the IBM RISC System/6000 processor", 1990), and div_fixup settles signs
+// of zeros, infinities and NaN.  These are the operations of the compiler's
+// division without its scaling of operands near the ends of the exponent
+// range, so a quotient is that of operator/ bit for bit while divisor,
+// numerator residual (numerator 2^-53) and quotient are normal numbers; below
+// that it may be off by a few units of the smallest denormal.  A division by
+// operator/ is eleven operations, four of them in a row through one condition
+// register; four by one divisor are 17 here.
+template <typename T>
+struct Divisor {
+  T d, y;
+};
+__device__ __forceinline__ Divisor<double> MakeDivisor(double d) {
+  double y = __builtin_amdgcn_rcp(d);
+  y = fma(y, fma(-d, y, 1.0), y);
+  y = fma(y, fma(-d, y, 1.0), y);
+  return {d, y};
+}
+__device__ __forceinline__ Divisor<float> MakeDivisor(float d) {
+  const float y = __builtin_amdgcn_rcpf(d);
+  return {d, fmaf(fmaf(-d, y, 1.0f), y, y)};
+}
+__device__ __forceinline__ double Quot(double n, const Divisor<double> &v) {
+  const double q = n * v.y;
+  return __builtin_amdgcn_div_fixup(fma(fma(-v.d, q, n), v.y, q), v.d, n);
+}
+__device__ __forceinline__ float Quot(float n, const Divisor<float> &v) {
+  float q = n * v.y;
+  q = fmaf(fmaf(-v.d, q, n), v.y, q);
+  return __builtin_amdgcn_div_fixupf(fmaf(fmaf(-v.d, q, n), v.y, q), v.d, n);
+}
+// sqrt for x = 0 or x >= 2^-760: the Goldschmidt iteration of sqrt() without
+// its scaling of small arguments (inf and NaN pass through)
+__device__ __forceinline__ double SqrtInRange(double x) {
+  const double y = __builtin_amdgcn_rsq(x);
+  double g = x * y, h = 0.5 * y;
+  const double r = fma(-h, g, 0.5);
+  g = fma(g, r, g);
+  h = fma(h, r, h);
+  g = fma(fma(-g, g, x), h, g);
+  g = fma(fma(-g, g, x), h, g);
+  return (x == 0.0 || __builtin_isinf(x)) ? x : g;
+}
+// ConsToPrim and the Enthalpy of its result in one, with the same operations
+// on the same values; `byCvs` is the divisor cvs
+__device__ __forceinline__ void ConsToPrimH(const GasT<double> &g, const Divisor<double> &byCvs, const double U[5],
+                                            double W[5], double &H) {
+#pragma clang fp contract(off)
+  const Divisor<double> byRho = MakeDivisor(U[0]);
+  const double rhoR = U[0] * g.R;
+  const Divisor<double> byRhoR = MakeDivisor(rhoR);
+  W[0] = U[0];
+  W[1] = Quot(U[1], byRho);
+  W[2] = Quot(U[2], byRho);
+  W[3] = Quot(U[3], byRho);
+  const double en = Quot(U[4], byRho);
+  const double vel = SqrtInRange((W[1] * W[1] + W[2] * W[2]) + W[3] * W[3]);
+  const double ke = 0.5 * vel * vel;
+  W[4] = rhoR * Quot(en - ke, byCvs);
+  H = g.cps * Quot(W[4], byRhoR) + ke;
+}
+// PhysFlux of a state whose enthalpy is known
+__device__ __forceinline__ void PhysFluxH(const double W[5], double H, double nx, double ny, double nz, double F[5]) {
+  const double vn = (W[1] * nx + W[2] * ny) + W[3] * nz;
+  const double rvn = W[0] * vn;
+  F[0] = rvn;
+  F[1] = rvn * W[1] + W[4] * nx;
+  F[2] = rvn * W[2] + W[4] * ny;
+  F[3] = rvn * W[3] + W[4] * nz;
+  F[4] = rvn * H;
+}
+
 // F(prim(cons(W) + du)) - F(W), the flux change the off-diagonal products
 // take, with every term a product of the increments and the base state, so
 // that nothing cancels: rho' = rho + drho, v' = v + dv with
@@ -546,26 +622,54 @@ __device__ __forceinline__ void RoeOffDiag(const GasT<double> &g, const double W
 // of the state once the iteration converges, and F(U + du) - F(U) formed in
 // FP32 would round it away.  (The FP64 operator forms both fluxes, as the
 // reference's RusanovScalarOffDiagonal does.)
+// the part of the change that no face enters: velocities and pressure after
+// the update and their increments
+template <typename T>
+struct StateChange {
+  T dr, dux, duy, duz, u1, v1, w1, dp;
+};
+template <typename T>
+__device__ __forceinline__ StateChange<T> ChangeOf(const GasT<T> &g, const T W[5], const T du[5]) {
+  const T rho = W[0], u = W[1], v = W[2], w = W[3];
+  const Divisor<T> by = MakeDivisor(rho + du[0]);
+  StateChange<T> c;
+  c.dr = du[0];
+  c.dux = Quot(du[1] - u * c.dr, by);
+  c.duy = Quot(du[2] - v * c.dr, by);
+  c.duz = Quot(du[3] - w * c.dr, by);
+  c.u1 = u + c.dux;
+  c.v1 = v + c.duy;
+  c.w1 = w + c.duz;
+  const T q1 = (c.u1 * c.u1 + c.v1 * c.v1) + c.w1 * c.w1;
+  const T dq = (c.dux * (T(2) * u + c.dux) + c.duy * (T(2) * v + c.duy)) + c.duz * (T(2) * w + c.duz);
+  c.dp = (g.gamma - T(1)) * (du[4] - T(0.5) * (c.dr * q1 + rho * dq));
+  return c;
+}
+// the base state's part: rho E + p
+template <typename T>
+__device__ __forceinline__ T EnergyPlusP(const GasT<T> &g, const T W[5]) {
+  const T rE = W[4] / (g.gamma - T(1)) + T(0.5) * W[0] * ((W[1] * W[1] + W[2] * W[2]) + W[3] * W[3]);
+  return rE + W[4];
+}
+// dF through a face of unit normal n; vn = v.n of the base state, rEp its
+// EnergyPlusP
+template <typename T>
+__device__ __forceinline__ void ChangeThrough(const StateChange<T> &c, T rho, T dE, T vn, T rEp, T nx, T ny, T nz,
+                                              T dF[5]) {
+  const T dvn = (c.dux * nx + c.duy * ny) + c.duz * nz, vn1 = vn + dvn;
+  const T dm = rho * dvn + c.dr * vn1;
+  const T rvn = rho * vn;
+  dF[0] = dm;
+  dF[1] = dm * c.u1 + rvn * c.dux + c.dp * nx;
+  dF[2] = dm * c.v1 + rvn * c.duy + c.dp * ny;
+  dF[3] = dm * c.w1 + rvn * c.duz + c.dp * nz;
+  dF[4] = rEp * dvn + (dE + c.dp) * vn1;
+}
 template <typename T>
 __device__ __forceinline__ void DeltaFlux(const GasT<T> &g, const T W[5], const T du[5], T nx, T ny, T nz,
                                           T dF[5]) {
-  const T rho = W[0], u = W[1], v = W[2], w = W[3], p = W[4];
-  const T gm1 = g.gamma - T(1);
-  const T dr = du[0], r1 = rho + dr;
-  const T dux = (du[1] - u * dr) / r1, duy = (du[2] - v * dr) / r1, duz = (du[3] - w * dr) / r1;
-  const T u1 = u + dux, v1 = v + duy, w1 = w + duz;
-  const T q1 = (u1 * u1 + v1 * v1) + w1 * w1;
-  const T dq = (dux * (T(2) * u + dux) + duy * (T(2) * v + duy)) + duz * (T(2) * w + duz);
-  const T dp = gm1 * (du[4] - T(0.5) * (dr * q1 + rho * dq));
-  const T vn = (u * nx + v * ny) + w * nz, dvn = (dux * nx + duy * ny) + duz * nz, vn1 = vn + dvn;
-  const T dm = rho * dvn + dr * vn1;
-  const T rE = p / gm1 + T(0.5) * rho * ((u * u + v * v) + w * w);
-  const T rvn = rho * vn;
-  dF[0] = dm;
-  dF[1] = dm * u1 + rvn * dux + dp * nx;
-  dF[2] = dm * v1 + rvn * duy + dp * ny;
-  dF[3] = dm * w1 + rvn * duz + dp * nz;
-  dF[4] = (rE + p) * dvn + (du[4] + dp) * vn1;
+  const T vn = (W[1] * nx + W[2] * ny) + W[3] * nz;
+  ChangeThrough(ChangeOf(g, W, du), W[0], du[4], vn, EnergyPlusP(g, W), nx, ny, nz, dF);
 }
 
 // RusanovScalarOffDiagonal for the inviscid equations
@@ -581,10 +685,13 @@ __device__ __forceinline__ void ScalarOffDiag(const GasT<T> &g, const T Wnb[5], 
   if constexpr (sizeof(T) == 4) {
     DeltaFlux(g, Wnb, du, nx, ny, nz, dF);
   } else {
-    T Wu[5], Fo[5], Fn[5];
-    UpdatePrim(g, Wnb, du, Wu);
+    T U[5], Wu[5], Fo[5], Fn[5], H;
+    PrimToCons(g, Wnb, U);
+#pragma unroll
+    for (int e = 0; e < 5; ++e) U[e] = U[e] + du[e];
+    ConsToPrimH(g, MakeDivisor(g.cvs), U, Wu, H);
     PhysFlux(g, Wnb, nx, ny, nz, Fo);
-    PhysFlux(g, Wu, nx, ny, nz, Fn);
+    PhysFluxH(Wu, H, nx, ny, nz, Fn);
 #pragma unroll
     for (int e = 0; e < 5; ++e) dF[e] = Fn[e] - Fo[e];
   }

@@ -45,7 +45,16 @@ struct DevBlock {
   float ATH_GLOBAL *x32;            // 5 * ncell (FP32 operator)
   double ATH_GLOBAL *xold;          // 5 * ncell, DP-LUR Jacobi copy
   float ATH_GLOBAL *xold32;
-  double ATH_GLOBAL *rhs;           // 5 * ncell, LU-SGS right-hand side (pencil sweep)
+  double ATH_GLOBAL *rhs;           // 5 * ncell, right-hand side of the row-parallel block sweep
+  // scalar LU-SGS: the pencil sweep's inputs in the order the sweep takes
+  // them.  Pencils run along axis pl, pa x pb of them along the axes pl + 1
+  // and pl + 2 (mod 3), pns steps stored for each; record (pencil, step) holds
+  // its values 64 lanes at a time (KPencilFaces, KPencilPrep, KPencilOther)
+  int pl, pa, pb, pns;
+  double ATH_GLOBAL *skF;  // face data, both sides
+  double ATH_GLOBAL *skS;  // state, right-hand side, D^-1 (and viscosity)
+  double ATH_GLOBAL *skX;  // forward du (operator precision)
+  double ATH_GLOBAL *skO;  // other-side sums of a full sweep (operator precision), null with one sweep
   // block matrix solvers: main diagonal after AddDiagonalTerms, 25 * ncell,
   // entry (r, c) of cell p at (5 r + c) ncell + p; its inverse in the
   // tile-blocked layout of TileBase (the sweep's 8 x 8 x 4 tiles: one tile's
@@ -2816,75 +2825,89 @@ __global__ void __launch_bounds__(kPThreads) KBlockSweepRows(const DevBlock *__r
 }
 
 // ---------------------------------------------------------------------------
-// Pencil-wavefront LU-SGS sweep.
+// Pencil-wavefront LU-SGS sweep (scalar operator).
 //
-// The block is cut into kPW x kPW columns ("pencils") that run the full k
-// extent.  One workgroup of five waves owns a pencil; lane l of every wave
-// stands for column (li, lj) = (l % kPW, l / kPW).  At pencil step s the lanes
-// update the cells of local hyperplane li + lj + k = s (forward; mirrored for
-// the backward sweep), so a pencil walks nk + 2 kPW - 2 steps:
+// The block is cut into kPW x kPW columns ("pencils") that run the whole
+// extent of its longest axis C; A = C + 1 and B = C + 2 (mod 3) are the axes
+// of the cut.  One workgroup owns a pencil; lane l of its compute wave stands
+// for the column (la, lb) = (l % kPW, l / kPW).  At pencil step s the lanes
+// update the cells of the local hyperplane la + lb + c = s (forward; mirrored
+// in the backward pass, whose step s is the forward step ns - 1 - s), so a
+// pencil of full width walks nc + 2 kPW - 2 steps.  The longest axis gives
+// the fewest column handoffs and the fewest idle steps.
 //
-//  * waves 0, 1, 2 evaluate the dependency-side off-diagonal product of the
-//    i, j and k neighbour (and, when the sweep also needs it, the other side's
-//    product from the previous sweep's du);
-//  * wave 3 sums the products in the order of ImplicitLower/ImplicitUpper,
-//    writes du and publishes the pencil's progress;
-//  * wave 4 loads the right-hand side and D^-1 and stages them in LDS.
+// What bounds it is the dependency chain of na + nb + nc - 2 hyperplanes, not
+// memory or arithmetic, so the kernel is laid out to make one step of that
+// chain short:
 //
-// Everything that does not depend on this sweep's du (neighbour states, face
-// vectors, right-hand side, D^-1, du across a pencil face) is loaded two
-// steps ahead into registers, so the step-to-step chain is LDS, barriers and
-// arithmetic.  In-pencil neighbours come from LDS (the previous step's du).
-// The neighbour across a pencil face comes from global memory once that
-// pencil's progress counter covers it; the i- and j-neighbour pencils run at
-// least kPW steps ahead, so a 64^3 block's dependency chain stays at the
-// 3*64-2 hyperplanes of HyperplaneReorder plus 14 pencil handoffs.
+//  * A cell's products are formed by the cell itself.  The off-diagonal
+//    product that a cell's neighbour adds (RusanovScalarOffDiagonal,
+//    src/fluxJacobian.cpp:122-162) takes this cell's state and du and the
+//    shared face only.  The lane that has just formed du therefore forms its
+//    three outgoing products (three faces) with one U + du -> primitive
+//    conversion and one enthalpy, where the neighbours together would do it
+//    three times; it hands products, not du, to the next step.  One wave does
+//    a whole step and needs no other wave's result of the same step.
+//  * The inputs lie in the order the sweep takes them (DevBlock::skS, skF):
+//    step by step, 64 lanes of one value contiguous, so that a stager's loads
+//    are whole lines.  In the natural layout the 64 cells of a hyperplane lie
+//    in different lines and each load fetches 64 of them.
+//  * Products cross a pencil face as self-validating messages: the receiving
+//    pencil polls the eight lanes' values themselves (every slot holds the
+//    all-ones pattern until its value arrives), which saves the wait for the
+//    stores' completion, the progress flag and the acquire.  The two
+//    directions have slots of their own, and each pass empties the other's.
 //
-// Progress: wave 3 stores du with agent-coherent stores, waits for them to
-// complete, then stores the step count with an agent-scope store.  A consumer reads the
-// count with agent-scope loads and issues its loads of that du only after it
-// has seen a count that covers them; those loads are agent-scope (coherent)
-// loads, so no acquire fence (which would drain the prefetch loads in flight)
-// is needed on the consumer side.
+// Waves of a workgroup: the compute wave; a halo wave that polls the next
+// step's messages into an LDS ring (or reads the connection terms on a block
+// face); a send wave that stores the messages of the step just done; and
+// kStagers waves that form, up to kPenSlots steps ahead, everything of the
+// products that does not depend on du (U, F(W), the normal, half the face
+// area, the spectral radius term) in LDS slots.  They synchronise through
+// step counters in LDS, each with one writer.
 //
 // Pencils are taken from an atomic ticket in pencil-hyperplane order, so a
 // pencil only ever waits on pencils whose workgroups are already running: no
-// co-residency assumption.  Every wait is bounded.  Two divergent regions with
-// the same condition are always separated by a barrier, so the compiler cannot
-// merge them across the loop's back edge.
+// co-residency assumption.  The ticket counts on from launch to launch
+// (every launch takes exactly nent of them).  Every wait is bounded.
+//
+// Measured per pass on a 64^3 block, against a sweep that handed du from an
+// owner wave to three neighbour waves and published progress counts: FP64 785
+// -> 184 us, FP32 790 -> 166 us.  A step takes 0.80 us (0.47 us of it
+// the compute wave's arithmetic, the rest its LDS and store instructions,
+// which hold the wave's issue for 13-29 cycles each), a handoff 1.6 us more
+// than its step.  Three compute waves, one per outgoing product, took 0.82 us
+// a step (the exchange between them costs what the arithmetic saves).
 constexpr int kPW = 8;
 constexpr int kPenLanes = kPW * kPW;
-
-
-// one block's view of a pencil sweep
-struct PencilCtl {
-  int *prog;          // per pencil of the block: steps completed in the current sweep
-  int *err;           // bit 1: a dependency wait exceeded the spin limit
-  int pa, pb;         // pencil grid of the block
-  void *sinkv;        // per pencil 5 x 64 operator words: stores of idle lanes
-};
+constexpr int kStagers = 4;
+constexpr int kPenSlots = kStagers;
+constexpr int kPenWaves = 3 + kStagers;
+constexpr int kProdRing = 4;   // steps of products kept in LDS for the send wave (a power of two)
+constexpr int kHaloRing = 8;   // steps of halo products in LDS
+constexpr int kMsg = 5 * kPW;  // values of one message
+constexpr int kPenS = 11;      // per-relax values of a cell: W, right-hand side, D^-1 (and viscosity)
+constexpr int kPenF = 12;      // values of a cell's three faces on one side: unit normal, area (and centre distance)
+constexpr int kLdsSpinLimit = 1 << 24;
+static_assert(kHaloRing * kPW == kPenLanes, "halo ring layout");
 
 // the pencils of every block in one launch: entry t = (a, b, block, first
-// pencil of the block), ordered by pencil hyperplane a + b, then block, then
-// b, a.  A pencil depends only on pencils of its own block one hyperplane
-// lower (forward; higher in the backward pass, which takes the entries in
-// reverse), all of which hold earlier tickets.
+// message step of the block), ordered by pencil hyperplane a + b, then block,
+// then b, a.  A pencil depends only on pencils of its own block one
+// hyperplane lower (forward; higher in the backward pass, which takes the
+// entries in reverse), all of which hold earlier tickets.
 struct PencilGroup {
-  int *ticket;          // reset to 0 before each sweep
-  int *prog;            // per pencil of every block
-  int *err;
+  unsigned long long *ticket;
+  int *err;             // bit 1: a dependency wait exceeded the spin limit
   const int4 *entries;
   int nent;             // pencils of all blocks
-  void *sinkv;          // 5 x 64 operator words per pencil
+  void *msg[2];         // of the forward and backward passes: per pencil 2 faces x pns steps x kMsg
+                        // operator words, all ones when empty
   const DevBlock *blocks;
 };
 
-__global__ void __launch_bounds__(256) KPencilPrologue(PencilGroup s) {
-  if (threadIdx.x == 0) *s.ticket = 0;
-  for (int q = threadIdx.x; q < s.nent; q += blockDim.x) s.prog[q] = 0;
-}
-
-// pencil width (cells) in i or j
+__device__ __forceinline__ int AxisN(const DevBlock &b, int d) { return d == 0 ? b.ni : (d == 1 ? b.nj : b.nk); }
+// pencil width (cells) along a cut axis of n cells
 __device__ __forceinline__ int PenWidth(int n, int a) { return min(kPW, n - a * kPW); }
 
 template <typename T>
@@ -2892,100 +2915,183 @@ __device__ __forceinline__ T CoherentLoad(const T *p) {
   return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
-// spin until pencil `id` has completed `need` steps; uniform across the wave
-__device__ __forceinline__ void PencilSpin(const PencilCtl &s, int id, int need, int &known) {
-  long spins = 0;
-  while (known < need) {
-    known = __builtin_amdgcn_readfirstlane(CoherentLoad(&s.prog[id]));
-    if (known >= need) break;
-    if ((++spins & 255) == 0 && (__builtin_amdgcn_readfirstlane(CoherentLoad(s.err)) & 2)) break;
-    if (spins > kSpinLimit) {
-      __hip_atomic_fetch_or(s.err, 2, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-      break;
-    }
-    __builtin_amdgcn_s_sleep(1);
-  }
+// the empty message slot: all bits one, a NaN that no product is stored as
+__device__ __forceinline__ bool IsEmpty(double v) { return __double_as_longlong(v) == -1LL; }
+__device__ __forceinline__ bool IsEmpty(float v) { return __float_as_int(v) == -1; }
+// Arithmetic passes on the payload of a NaN it is given and makes no all-ones
+// one of its own, so it is enough that no input of a product holds one.
+template <typename T>
+__device__ __forceinline__ T NotEmpty(T v) {
+  return IsEmpty(v) ? T(__builtin_nan("")) : v;
+}
+template <typename T>
+__device__ __forceinline__ T EmptySlot();
+template <>
+__device__ __forceinline__ double EmptySlot<double>() { return __longlong_as_double(-1LL); }
+template <>
+__device__ __forceinline__ float EmptySlot<float>() { return __int_as_float(-1); }
+
+// record (pid, s, lane) of the sweep-ordered arrays and its cell
+struct PenCell {
+  bool active;
+  int i, j, k;
+};
+__device__ __forceinline__ PenCell PencilCell(const DevBlock &b, int pid, int s, int lane) {
+  const int a = pid % b.pa, bb = pid / b.pa;
+  const int na = AxisN(b, (b.pl + 1) % 3), nb = AxisN(b, (b.pl + 2) % 3), nc = AxisN(b, b.pl);
+  const int la = lane % kPW, lb = lane / kPW, c = s - la - lb;
+  PenCell r;
+  r.active = la < PenWidth(na, a) && lb < PenWidth(nb, bb) && c >= 0 && c < nc;
+  Map3(b.pl, c, a * kPW + la, bb * kPW + lb, r.i, r.j, r.k);
+  return r;
 }
 
-// per-lane geometry of a pencil
-struct PenLane {
-  int i, j, li, lj, wi, wj, off, nsteps;
-  bool col;
-  // k of the lane's cell at step s, or -1 when the lane is idle
-  __device__ __forceinline__ int K(int s, int nk, bool fwd) const {
-    const int kk = s - off;
-    if (!col || kk < 0 || kk >= nk) return -1;
-    return fwd ? kk : nk - 1 - kk;
+// The face data of every pencil record, laid out once per case: side 0 the
+// lower faces (what the backward pass's products cross), side 1 the upper
+// ones (forward), axes in the order A, B, C.  Records of idle lanes, which the
+// sweep reads and whose results it drops, start from zeros.
+__global__ void __launch_bounds__(256) KPencilFaces(const DevBlock b, int visc) {
+  const long t = (long)blockIdx.x * blockDim.x + threadIdx.x;
+  const int lane = (int)(t % kPenLanes);
+  const long rec = t / kPenLanes, nrec = (long)b.pa * b.pb * b.pns;
+  if (rec >= nrec) return;
+  const PenCell c = PencilCell(b, (int)(rec / b.pns), (int)(rec % b.pns), lane);
+  const int nF = kPenF + (visc ? 3 : 0), nS = kPenS + (visc ? 1 : 0);
+  if (!c.active) {
+    for (int q = 0; q < nF; ++q)
+      b.skF[(rec * nF + q) * kPenLanes + lane] = b.skF[((nrec + rec) * nF + q) * kPenLanes + lane] = 0.0;
+    for (int q = 0; q < nS; ++q) b.skS[(rec * nS + q) * kPenLanes + lane] = 0.0;
+    for (int q = 0; q < 5; ++q) {
+      b.skX[(rec * 5 + q) * kPenLanes + lane] = 0.0;
+      if (b.skO) b.skO[(rec * 5 + q) * kPenLanes + lane] = 0.0;
+    }
+    return;
   }
-};
+  for (int side = 0; side < 2; ++side)
+    for (int q = 0; q < 3; ++q) {
+      const int d = (b.pl + 1 + q) % 3;
+      const long f = FaceIdx(b, d, c.i + (side && d == 0), c.j + (side && d == 1), c.k + (side && d == 2));
+      const double4 a = (d == 0 ? b.fa[0] : (d == 1 ? b.fa[1] : b.fa[2]))[f];
+      double *o = b.skF + ((side * nrec + rec) * nF + 4 * q) * kPenLanes + lane;
+      o[0] = a.x;
+      o[kPenLanes] = a.y;
+      o[2 * kPenLanes] = a.z;
+      o[3 * kPenLanes] = a.w;
+      if (visc)
+        b.skF[((side * nrec + rec) * nF + kPenF + q) * kPenLanes + lane] =
+            (d == 0 ? b.c2c[0] : (d == 1 ? b.c2c[1] : b.c2c[2]))[f];
+    }
+}
 
-// The right-hand side b of every cell, computed before the pencil sweeps
-// (it depends only on data the sweeps do not modify)
-__global__ void __launch_bounds__(256) KLusgsRhs(BlockMap M, Params P) {
+// The inputs of a relax in sweep order: the state, the right-hand side
+// (which the sweeps do not change), D^-1 and, with the viscous terms, the
+// viscosity of every cell
+template <typename T>
+__global__ void __launch_bounds__(256) KPencilPrep(BlockMap M, Params P) {
   const Unit U = MapUnit(M);
   const DevBlock &b = *U.b;
-  const long p = (long)U.local * blockDim.x + threadIdx.x;
-  if (p >= b.ncell) return;
-  const int i = (int)(p % b.ni), j = (int)((p / b.ni) % b.nj), k = (int)(p / ((long)b.ni * b.nj));
+  const long t = (long)U.local * blockDim.x + threadIdx.x;
+  const int lane = (int)(t % kPenLanes);
+  const long rec = t / kPenLanes;
+  if (rec >= (long)b.pa * b.pb * b.pns) return;
+  const PenCell q = PencilCell(b, (int)(rec / b.pns), (int)(rec % b.pns), lane);
+  if (!q.active) return;
+  const long p = (long)q.i + (long)q.j * b.ni + (long)q.k * b.ni * b.nj, c = PadIdx(b, q.i, q.j, q.k);
+  const int nS = kPenS + (P.visc.on ? 1 : 0);
+  double *o = b.skS + rec * nS * kPenLanes + lane;
   double rb[5];
-  Rhs(b, P, p, PadIdx(b, i, j, k), rb);
+  Rhs(b, P, p, c, rb);
 #pragma unroll
-  for (int e = 0; e < 5; ++e) b.rhs[e * b.ncell + p] = rb[e];
+  for (int e = 0; e < 5; ++e) {
+    o[e * kPenLanes] = b.W[e * b.npad + c];
+    o[(5 + e) * kPenLanes] = rb[e];
+  }
+  o[10 * kPenLanes] = double(OpBuf<T>::Ainv(b)[p]);
+  if (P.visc.on) o[kPenS * kPenLanes] = b.mu[c];
 }
 
-// ---- decoupled waves of the pencil sweep.
-//
-// A pencil's workgroup has eight waves that run their own loops and
-// synchronise through step counters in LDS (no workgroup barrier in the
-// loop), so a wave that waits on global memory holds up only the waves that
-// need its result:
-//
-//  * waves 4-7 (stagers): stager j prepares every step s = j mod 4 into LDS
-//    slot j.  It loads, for each lane, the three dependency-side neighbours
-//    and computes everything of their off-diagonal products that does not
-//    depend on this sweep's du (conservative state U, flux F(W), the face
-//    normal, half the face area, the spectral radius term), the du across the
-//    i and j pencil faces (after the neighbour pencil's progress covers it),
-//    the right-hand side (or the cell's forward du) and D^-1, and in the
-//    two-sided sweep the whole other-side sum.  It waits only for the slot to
-//    be released (the owner finished step s-4) and for the neighbour pencils.
-//  * waves 0-2 (neighbours): wave d finishes the dependency-side product of
-//    direction d: U + du, primitive state, flux, and the Rusanov combination
-//    (the operations of RusanovScalarOffDiagonal, in the same order).
-//  * wave 3 (owner): sums the products in the order of ImplicitLower /
-//    ImplicitUpper, forms du, passes it to the neighbour waves through LDS,
-//    stores it (agent-coherent), and every kPubEvery steps waits for its
-//    stores and publishes the pencil's progress.
-//
-// Counters are monotone; each has one writer and is written with a
-// workgroup-scope release after the data it covers, read with an acquire.
-// Every wait is bounded (an exceeded bound sets err bit 1 and stops waiting).
-constexpr int kStagers = 4;
-constexpr int kPenWaves = 4 + kStagers;
-constexpr int kPubEvery = 2;
-constexpr long kLdsSpinLimit = 1L << 24;
+// A full sweep's other-side sums (OffDiagSum over the upper neighbours in a
+// forward pass, the lower ones in a backward pass), formed before the pass:
+// none of the du they read is written by the pass before the cell itself is
+// updated, so the values are those the sweep would form in place.
+template <typename T, bool FWD>
+__global__ void __launch_bounds__(256) KPencilOther(BlockMap M, Params P) {
+  const Unit U = MapUnit(M);
+  const DevBlock &b = *U.b;
+  const long t = (long)U.local * blockDim.x + threadIdx.x;
+  const int lane = (int)(t % kPenLanes);
+  const long rec = t / kPenLanes;
+  if (rec >= (long)b.pa * b.pb * b.pns) return;
+  const PenCell q = PencilCell(b, (int)(rec / b.pns), (int)(rec % b.pns), lane);
+  if (!q.active) return;
+  T O[5];
+  OffDiagSum<T>(b, Cast<T>(P.gas), P.visc, OpBuf<T>::X(b), q.i, q.j, q.k, FWD, O);
+  T *o = (T *)b.skO + rec * 5 * kPenLanes + lane;
+#pragma unroll
+  for (int e = 0; e < 5; ++e) o[e * kPenLanes] = O[e];
+}
 
+// Values in LDS go 16 bytes a lane: a 16-byte read takes 13 cycles of the
+// LDS pipe for a wave, two 8-byte reads 33.  Value q of a lane's record is
+// v[q % kVecN] of its vector q / kVecN.
+template <typename T>
+struct alignas(16) LdsVec {
+  T v[16 / sizeof(T)];
+};
+template <typename T>
+constexpr int kVecN = 16 / (int)sizeof(T);
+template <typename T>
+constexpr int Vecs(int n) { return (n + kVecN<T> - 1) / kVecN<T>; }
+
+// everything of one step that does not depend on this sweep's du.  Early:
+// right-hand side or the cell's forward du (5), D^-1, state
+// (5: conservative, or primitive for the FP32 operator's flux change), the
+// other-side sum of a full sweep (5).  Late, for the face of each axis A, B,
+// C: unit normal (3), 0.5 |A|, the spectral radius term, then FP64: F(W)
+// through the face (5), FP32: v.n there and rho E + p.
+template <typename T, bool FULL>
+constexpr int kEarly = FULL ? 16 : 11;
+template <typename T>
+constexpr int kLate = sizeof(T) == 8 ? 10 : 7;
 template <typename T, bool FULL>
 struct PenSlot {
-  T U[3][5][kPenLanes];   // neighbour conservative state
-  T Fo[3][5][kPenLanes];  // neighbour flux through the face
-  T n[3][3][kPenLanes];   // face unit normal
-  T half[3][kPenLanes];   // 0.5 |A|
-  T lam[3][kPenLanes];    // 0.5 |A| (|v.n| + c) of the neighbour
-  T halo[2][5][kPenLanes];  // du across the i and j pencil faces
-  double v5[5][kPenLanes];  // right-hand side, or the cell's forward du
-  T ainv[kPenLanes];
-  T O[FULL ? 5 : 1][kPenLanes];  // other-side sum (two-sided sweep)
+  LdsVec<T> early[Vecs<T>(kEarly<T, FULL>)][kPenLanes];
+  LdsVec<T> late[3][Vecs<T>(kLate<T>)][kPenLanes];
 };
+// n values of a lane from / to its vectors
+template <typename T, int N>
+__device__ __forceinline__ void LdsGet(const LdsVec<T> *p, T *v) {
+#pragma unroll
+  for (int q = 0; q < Vecs<T>(N); ++q) {
+    const LdsVec<T> w = p[q * kPenLanes];
+#pragma unroll
+    for (int r = 0; r < kVecN<T>; ++r)
+      if (q * kVecN<T> + r < N) v[q * kVecN<T> + r] = w.v[r];
+  }
+}
+template <typename T, int N>
+__device__ __forceinline__ void LdsPut(LdsVec<T> *p, const T *v) {
+#pragma unroll
+  for (int q = 0; q < Vecs<T>(N); ++q) {
+    LdsVec<T> w;
+#pragma unroll
+    for (int r = 0; r < kVecN<T>; ++r) w.v[r] = q * kVecN<T> + r < N ? v[q * kVecN<T> + r] : T(0);
+    p[q * kPenLanes] = w;
+  }
+}
 
 template <typename T, bool FULL>
 struct PenShared {
-  PenSlot<T, FULL> slot[kStagers];
-  T sX[5][kPenLanes];     // du of the owner's last step
-  T sO[3][5][kPenLanes];  // dependency-side products of the current step
-  int stageReady[kStagers];  // slot j holds step stageReady[j] - 1
-  int oReady[3];             // wave d has written sO for oReady[d] steps
-  int xReady;                // the owner has finished xReady steps
+  PenSlot<T, FULL> slot[kPenSlots];
+  // the products across axes A and B: of the last kProdRing steps, a lane
+  // each, and those that enter through the pencil's faces: entry q of step s
+  // in column kPW (s mod kHaloRing) + q
+  LdsVec<T> prod[kProdRing][2][Vecs<T>(5)][kPenLanes];
+  LdsVec<T> halo[2][Vecs<T>(5)][kPenLanes];
+  int stageReady[kPenSlots];  // slot j holds step stageReady[j] - 1
+  int haloReady;              // steps whose halo products are in the ring
+  int xReady;                 // steps the compute wave has finished
+  int sentReady;              // steps whose outgoing products have been sent
   int ticket;
 };
 
@@ -2994,303 +3100,392 @@ __device__ __forceinline__ int LdsLoad(const int *p) {
 }
 // publish a step counter for the whole wave: the wave barrier is a
 // convergent point the compiler cannot duplicate into a lane-divergent
-// branch, the release fence waits for every lane's earlier LDS and global
-// writes, and then one lane stores the count
+// branch, the release fence waits for every lane's earlier LDS writes, and
+// then one lane stores the count
 __device__ __forceinline__ void LdsStore(int *p, int v) {
   __builtin_amdgcn_wave_barrier();
   __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
   if (__lane_id() == 0) __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
 }
-// wait until an LDS counter reaches `need`; uniform across the wave
+// a counter read without waiting for it, to be tested later (an acquire fence
+// comes between the test and the reads of what it covers)
+__device__ __forceinline__ int LdsPeek(const int *p) {
+  return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+}
+// store a counter that covers only this wave's LDS reads whose values have
+// been used: nothing of other waves is released by it, so no wait is needed
+__device__ __forceinline__ void LdsPost(int *p, int v) {
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  if (__lane_id() == 0) __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+}
+// wait until an LDS counter reaches `need`; uniform across the wave.  Waves
+// that run ahead sleep between polls (polls take LDS cycles from the compute
+// wave); the compute wave does not.
+template <int SLEEP = 8>
 __device__ __forceinline__ void LdsWait(const int *p, int need, int *err) {
-  long spins = 0;
+  int spins = 0;
   while (__builtin_amdgcn_readfirstlane(LdsLoad(p)) < need) {
     if (++spins > kLdsSpinLimit) {
       __hip_atomic_fetch_or(err, 2, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
       break;
     }
-    __builtin_amdgcn_s_sleep(1);
+    if (SLEEP) __builtin_amdgcn_s_sleep(SLEEP);
   }
 }
 
-__device__ __forceinline__ int Clamp(int v, int n) { return v < 0 ? 0 : (v >= n ? n - 1 : v); }
+// a workgroup's pencil
+struct Pencil {
+  int a, b;             // position in the pencil grid
+  int pid;              // number within the block
+  int wa, wb, nc, ns;   // widths, length, steps
+  long rec;             // first record of the pencil
+  long nrec;            // records of the block
+};
 
-__device__ __forceinline__ bool InBlock(const DevBlock &b, int i, int j, int k) {
-  return i >= 0 && j >= 0 && k >= 0 && i < b.ni && j < b.nj && k < b.nk;
-}
-
-// Lane divergence and the step counters.  A counter is stored after data
-// written by every lane of the wave.  If the counter store sat in a
-// lane-divergent region, the compiler could duplicate it into both sides of
-// a branch and run the idle lanes' copy first, publishing the counter before
-// the active lanes have written.  Two things prevent that: LdsStore joins
-// the wave at a wave barrier and fences before a single lane stores the
-// counter, and everything from a wave's loads to its counter store is
-// straight-line code (idle lanes and absent neighbours compute on clamped,
-// valid addresses, their results are selected away, and their stores go to
-// a per-pencil sink).
-
-// stager: prepare step st into `sl`
+// one step's slot from the sweep-ordered inputs
 template <typename T, bool FWD, bool FULL>
-__device__ __forceinline__ void PenStage(const DevBlock &b, const Params &P, const PencilCtl &s,
-                                         PenSlot<T, FULL> &sl, const PenLane &L, int lane, int st,
-                                         const int nbId[2], const int nbW[2], const int nbTotal[2], int known[2]) {
-  const int sgn = FWD ? -1 : 1;
+__device__ __forceinline__ void PenStage(const DevBlock &b, const Params &P, const Pencil &pen,
+                                         PenSlot<T, FULL> &sl, int lane, int st, const int *xReady, int *err) {
   const GasT<T> g = Cast<T>(P.gas);
-  const T *x = OpBuf<T>::X(b);
-  // the du across the i and j pencil faces must be published first (uniform)
-  bool fresh = false;
+  const long rec = pen.rec + (FWD ? st : pen.ns - 1 - st);
+  const int nS = kPenS + (P.visc.on ? 1 : 0), nF = kPenF + (P.visc.on ? 3 : 0);
+  const double *S = b.skS + rec * nS * kPenLanes + lane;
+  const double *F = b.skF + ((FWD ? pen.nrec : 0) + rec) * nF * kPenLanes + lane;
+  // every load before the wait for the slot
+  T W[5], fa[12], early[kEarly<T, FULL>];
 #pragma unroll
-  for (int h = 0; h < 2; ++h) {
-    const int need = min(st + nbW[h], nbTotal[h]);
-    if (nbId[h] >= 0 && known[h] < need) {
-      PencilSpin(s, nbId[h], need, known[h]);
-      fresh = true;
+  for (int e = 0; e < 5; ++e) W[e] = T(S[e * kPenLanes]);
+#pragma unroll
+  for (int q = 0; q < 12; ++q) fa[q] = T(F[q * kPenLanes]);
+  if (FWD || FULL) {
+#pragma unroll
+    for (int e = 0; e < 5; ++e) early[e] = T(S[(5 + e) * kPenLanes]);
+  } else {
+    const T *X = (const T *)b.skX + rec * 5 * kPenLanes + lane;
+#pragma unroll
+    for (int e = 0; e < 5; ++e) early[e] = X[e * kPenLanes];
+  }
+  early[5] = T(S[10 * kPenLanes]);
+  if constexpr (FULL) {
+    const T *o = (const T *)b.skO + rec * 5 * kPenLanes + lane;
+#pragma unroll
+    for (int e = 0; e < 5; ++e) early[11 + e] = o[e * kPenLanes];
+  }
+  T mu = T(0), dist[3] = {T(1), T(1), T(1)};
+  if (P.visc.on) {
+    mu = T(S[kPenS * kPenLanes]);
+#pragma unroll
+    for (int q = 0; q < 3; ++q) dist[q] = T(F[(kPenF + q) * kPenLanes]);
+  }
+  // (NotEmpty: no product may look like an empty message slot)
+#pragma unroll
+  for (int e = 0; e < 5; ++e) W[e] = NotEmpty(W[e]);
+#pragma unroll
+  for (int e = 0; e < kEarly<T, FULL>; ++e)
+    if (e < 6 || e >= 11) early[e] = NotEmpty(early[e]);
+  T late[3][kLate<T>];
+  if constexpr (sizeof(T) == 8) {
+    PrimToCons(g, W, &early[6]);
+  } else {
+#pragma unroll
+    for (int e = 0; e < 5; ++e) early[6 + e] = W[e];
+  }
+#pragma unroll
+  for (int q = 0; q < 3; ++q) {
+    const T nx = fa[4 * q], ny = fa[4 * q + 1], nz = fa[4 * q + 2], mag = fa[4 * q + 3];
+    T lam = T(0.5) * mag * (fabs((W[1] * nx + W[2] * ny) + W[3] * nz) + SoS(g, W[0], W[4]));
+    if (P.visc.on) lam += ViscFaceSR<T>(g, W, mag, dist[q], mu, P.visc);
+    late[q][0] = nx;
+    late[q][1] = ny;
+    late[q][2] = nz;
+    late[q][3] = T(0.5) * mag;
+    late[q][4] = lam;
+    if constexpr (sizeof(T) == 8) {
+      PhysFlux(g, W, nx, ny, nz, &late[q][5]);
+    } else {
+      late[q][5] = (W[1] * nx + W[2] * ny) + W[3] * nz;
+      late[q][6] = EnergyPlusP(g, W);
     }
   }
-  if (fresh) __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
-  const int k = L.K(st, b.nk, FWD);
-  const int i = Clamp(L.i, b.ni), j = Clamp(L.j, b.nj), kc = k < 0 ? 0 : k;
-  const long p = (long)i + (long)j * b.ni + (long)kc * b.ni * b.nj;
+  // the slot is free once the compute wave has finished step st - kPenSlots
+  LdsWait(xReady, st - kPenSlots + 1, err);
+  LdsPut<T, kEarly<T, FULL>>(&sl.early[0][lane], early);
 #pragma unroll
-  for (int d = 0; d < 3; ++d) {
-    const int ci = Clamp(i + (d == 0 ? sgn : 0), b.ni), cj = Clamp(j + (d == 1 ? sgn : 0), b.nj),
-              ck = Clamp(kc + (d == 2 ? sgn : 0), b.nk);
-    const long fq = FWD ? FaceIdx(b, d, i, j, kc) : FaceIdx(b, d, ci, cj, ck);
-    const double4 a = b.fa[d][fq];
-    const long c = PadIdx(b, ci, cj, ck);
-    T W[5], U[5], Fo[5];
-#pragma unroll
-    for (int e = 0; e < 5; ++e) W[e] = T(b.W[e * b.npad + c]);
-    const T nx = T(a.x), ny = T(a.y), nz = T(a.z), mag = T(a.w);
-    if constexpr (sizeof(T) == 4) {
-      // the FP32 operator's flux change is formed from the primitive state
-      // (DeltaFlux): the slot of U carries W
-#pragma unroll
-      for (int e = 0; e < 5; ++e) {
-        U[e] = W[e];
-        Fo[e] = T(0);
-      }
-    } else {
-      PrimToCons(g, W, U);
-      PhysFlux(g, W, nx, ny, nz, Fo);
-    }
-    const T half = T(0.5) * mag;
-    T lam = T(0.5) * mag * (fabs((W[1] * nx + W[2] * ny) + W[3] * nz) + SoS(g, W[0], W[4]));
-    if (P.visc.on) lam += ViscFaceSR<T>(g, W, mag, T(b.c2c[d][fq]), T(b.mu[c]), P.visc);
-    // a neighbour outside the block: the slot of Fo carries the connection
-    // term instead (zero off connections), selected by the neighbour wave
-    const bool outside = !InBlock(b, i + (d == 0 ? sgn : 0), j + (d == 1 ? sgn : 0), kc + (d == 2 ? sgn : 0));
-    T bv[5] = {T(0), T(0), T(0), T(0), T(0)};
+  for (int q = 0; q < 3; ++q) LdsPut<T, kLate<T>>(&sl.late[q][0][lane], late[q]);
+}
+
+// The compute wave.  A wave issues one instruction in 4.6 cycles whatever it
+// depends on, so a step costs its instruction count plus what it waits for,
+// and it is ordered so that it waits for nothing: each value of the next step
+// is read from LDS as soon as this step has used the last one, between the
+// arithmetic; the counters are read well before they are tested; the products
+// across B and A go into LDS (where the next step's lanes and the send wave
+// take them) before the one across C, which stays in the lane's registers, is
+// formed.
+template <typename T, bool FWD, bool FULL, int C>
+__device__ __forceinline__ void PenCompute(const DevBlock &b, const Params &P, const Pencil &pen,
+                                           PenShared<T, FULL> &sh, int lane, int store, bool sends, int *err) {
+  constexpr int sgn = FWD ? -1 : 1;  // direction of the dependency neighbours
+  constexpr int V5 = Vecs<T>(5);
+  const GasT<T> g = Cast<T>(P.gas);
+  const auto byCvs = MakeDivisor(g.cvs);
+  const int ns = pen.ns, nc = pen.nc;
+  const int la = lane % kPW, lb = lane / kPW;
+  const bool col = la < pen.wa && lb < pen.wb;
+  const int off = FWD ? la + lb : (pen.wa - 1 - la) + (pen.wb - 1 - lb);
+  const bool firstA = FWD ? la == 0 : la == pen.wa - 1, firstB = FWD ? lb == 0 : lb == pen.wb - 1;
+  // where the lane's incoming products lie: the neighbour lane's of the step
+  // before, or the halo ring's
+  const int nlA = min(max(lane + sgn, 0), kPenLanes - 1), nlB = min(max(lane + sgn * kPW, 0), kPenLanes - 1);
+  const LdsVec<T> *const inA = firstA ? &sh.halo[0][0][lb] : &sh.prod[0][0][0][nlA];
+  const LdsVec<T> *const inB = firstB ? &sh.halo[1][0][la] : &sh.prod[0][1][0][nlB];
+  constexpr int kProdStep = 2 * V5 * kPenLanes;  // vectors of one step of the product ring
+  const int gA = pen.a * kPW + la, gB = pen.b * kPW + lb;
+  // the first cell of a lane takes the connection term across C (zero off
+  // connections)
+  T oC[5];
+  {
     const T *bt = OpBuf<T>::Bt(b);
-    if (bt) {
-      const long q = BtSlot(b, d, FWD ? 0 : 1, i, j, kc);
+    int i, j, k;
+    Map3(C, FWD ? 0 : nc - 1, gA, gB, i, j, k);
+    const bool conn = bt && col;
+    const long q = conn ? BtSlot(b, C, FWD ? 0 : 1, i, j, k) : 0;
 #pragma unroll
-      for (int e = 0; e < 5; ++e) bv[e] = bt[e * b.nbf + q];
-    }
+    for (int e = 0; e < 5; ++e) oC[e] = conn ? NotEmpty(bt[e * b.nbf + q]) : T(0);
+  }
+  // du in the natural layout: a lane's cells follow each other along C
+  T *const x = OpBuf<T>::X(b);
+  int i0, j0, k0;
+  Map3(C, FWD ? -off : nc - 1 + off, gA, gB, i0, j0, k0);
+  const int sC = -sgn * (C == 0 ? 1 : (C == 1 ? b.ni : b.ni * b.nj));
+  int p = i0 + j0 * b.ni + k0 * b.ni * b.nj;  // cell of step st (of the active steps)
+  T *Xs = (T *)b.skX + pen.rec * 5 * kPenLanes + lane;
+  T xA[5], xB[5], early[kEarly<T, FULL>], late[3][kLate<T>];
+  int next = 1;  // slot of the next step
+  LdsWait<0>(&sh.stageReady[0], 1, err);
+  LdsWait<0>(&sh.haloReady, 1, err);
+  int stage = LdsPeek(&sh.stageReady[next]), halo, sent;
+  LdsGet<T, kEarly<T, FULL>>(&sh.slot[0].early[0][lane], early);
+  LdsGet<T, 5>(inA, xA);
+  LdsGet<T, 5>(inB, xB);
+#pragma unroll
+  for (int q = 0; q < 2; ++q) LdsGet<T, kLate<T>>(&sh.slot[0].late[q][0][lane], late[q]);
+  const PenSlot<T, FULL> *cur = &sh.slot[0];
+  for (int st = 0; st < ns; ++st) {
+    const bool more = st + 1 < ns;
+    __builtin_amdgcn_sched_barrier(0);
+    LdsGet<T, kLate<T>>(&cur->late[2][0][lane], late[2]);
+    // the dependency-side sum in the order of ImplicitLower / ImplicitUpper
+    // (i, j, k); products of absent neighbours are +0 and leave it unchanged
+    // (it starts at +0 and is never -0)
+    T xn[5], Un[5], W0[5];
 #pragma unroll
     for (int e = 0; e < 5; ++e) {
-      sl.U[d][e][lane] = U[e];
-      sl.Fo[d][e][lane] = outside ? bv[e] : Fo[e];
+      const T o0 = C == 2 ? xA[e] : (C == 0 ? oC[e] : xB[e]), o1 = C == 2 ? xB[e] : (C == 0 ? xA[e] : oC[e]),
+              o2 = C == 2 ? oC[e] : (C == 0 ? xB[e] : xA[e]);
+      const T D = ((T(0) + o0) + o1) + o2, v = early[e], ainv = early[5];
+      if constexpr (FULL) xn[e] = FWD ? (v + (D - early[11 + e])) * ainv : ((v + early[11 + e]) - D) * ainv;
+      else xn[e] = FWD ? (v + D) * ainv : v - D * ainv;
+      W0[e] = early[6 + e];
+      Un[e] = W0[e] + xn[e];
     }
-    sl.n[d][0][lane] = nx;
-    sl.n[d][1][lane] = ny;
-    sl.n[d][2][lane] = nz;
-    sl.half[d][lane] = half;
-    sl.lam[d][lane] = lam;
-    if (d < 2) {
-      // du of the neighbour; used only across the pencil face
-      const long q = (long)ci + (long)cj * b.ni + (long)ck * b.ni * b.nj;
+    __builtin_amdgcn_sched_barrier(0);
+    if (more && __builtin_amdgcn_readfirstlane(stage) < st + 2) LdsWait<0>(&sh.stageReady[next], st + 2, err);
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    const PenSlot<T, FULL> &sl = sh.slot[next];
+    LdsGet<T, kEarly<T, FULL>>(&sl.early[0][lane], early);
+    next = next + 1 == kPenSlots ? 0 : next + 1;
+    stage = LdsPeek(&sh.stageReady[next]);
+    sent = LdsPeek(&sh.sentReady);
+    // the updated state
+    T Wu[5], H = T(0);
+    StateChange<T> ch;
+    if constexpr (sizeof(T) == 8) ConsToPrimH(g, byCvs, Un, Wu, H);
+    else ch = ChangeOf(g, W0, xn);
+    // the outgoing product across axis q
+    auto product = [&](int q, T o[5]) {
+      if constexpr (sizeof(T) == 8) {
+        PhysFluxH(Wu, H, late[q][0], late[q][1], late[q][2], o);
 #pragma unroll
-      for (int e = 0; e < 5; ++e) sl.halo[d][e][lane] = x[e * b.ncell + q];
-    }
-  }
-#pragma unroll
-  for (int e = 0; e < 5; ++e) sl.v5[e][lane] = (FWD || FULL) ? b.rhs[e * b.ncell + p] : double(x[e * b.ncell + p]);
-  sl.ainv[lane] = OpBuf<T>::Ainv(b)[p];
-  if (FULL) {
-    // other side from the previous sweep's du, as in OffDiagSum (a missing
-    // neighbour adds +0, which leaves the sum unchanged: it starts at +0 and
-    // a sum of finite terms reached from +0 is never -0)
-    T O[5] = {T(0), T(0), T(0), T(0), T(0)};
-#pragma unroll
-    for (int d = 0; d < 3; ++d) {
-      const int hi = i - (d == 0 ? sgn : 0), hj = j - (d == 1 ? sgn : 0), hk = kc - (d == 2 ? sgn : 0);
-      const bool ok = k >= 0 && InBlock(b, hi, hj, hk);
-      const int ui = Clamp(hi, b.ni), uj = Clamp(hj, b.nj), uk = Clamp(hk, b.nk);
-      const long fq = FWD ? FaceIdx(b, d, ui, uj, uk) : FaceIdx(b, d, i, j, kc);
-      const double4 a = b.fa[d][fq];
-      const long c = PadIdx(b, ui, uj, uk);
-      const long q = (long)ui + (long)uj * b.ni + (long)uk * b.ni * b.nj;
-      double Wn[5];
-      T dn[5], u[5];
+        for (int e = 0; e < 5; ++e) o[e] = o[e] - late[q][5 + e];
+      } else {
+        ChangeThrough(ch, W0[0], xn[4], late[q][5], late[q][6], late[q][0], late[q][1], late[q][2], o);
+      }
 #pragma unroll
       for (int e = 0; e < 5; ++e) {
-        Wn[e] = b.W[e * b.npad + c];
-        dn[e] = x[e * b.ncell + q];
+        const T fc = late[q][3] * o[e];
+        o[e] = FWD ? fc + xn[e] * late[q][4] : fc - xn[e] * late[q][4];
       }
-      if (P.visc.on) NbOffDiag<T>(g, Wn, dn, a, !FWD, u, &P.visc, b.c2c[d][fq], b.mu[c]);
-      else NbOffDiag<T>(g, Wn, dn, a, !FWD, u);
-      T bv[5] = {T(0), T(0), T(0), T(0), T(0)};
-      const T *bt = OpBuf<T>::Bt(b);
-      if (bt) {
-        const long qb = BtSlot(b, d, FWD ? 1 : 0, i, j, kc);
+    };
+    // the product ring's place is free once its products have been sent
+    if (sends && __builtin_amdgcn_readfirstlane(sent) < st + 1 - kProdRing)
+      LdsWait<0>(&sh.sentReady, st + 1 - kProdRing, err);
+    LdsVec<T> *const out = &sh.prod[st & (kProdRing - 1)][0][0][lane];
+    T o[5];
+    product(1, o);
+    LdsPut<T, 5>(out + V5 * kPenLanes, o);
+    __builtin_amdgcn_sched_barrier(0);
+    halo = LdsPeek(&sh.haloReady);
+    LdsGet<T, kLate<T>>(&sl.late[1][0][lane], late[1]);
+    product(0, o);
+    LdsPut<T, 5>(out, o);
+    // this step's slot (read in the step before) and ring columns are free,
+    // and its products are in LDS (a wave's LDS operations complete in order)
+    LdsPost(&sh.xReady, st + 1);
+    __builtin_amdgcn_sched_barrier(0);
+    if (more && __builtin_amdgcn_readfirstlane(halo) < st + 2) LdsWait<0>(&sh.haloReady, st + 2, err);
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    const int ro = kPW * ((st + 1) % kHaloRing), po = kProdStep * (st & (kProdRing - 1));
+    LdsGet<T, 5>(inB + (firstB ? ro : po), xB);
+    LdsGet<T, 5>(inA + (firstA ? ro : po), xA);
+    LdsGet<T, kLate<T>>(&sl.late[0][0][lane], late[0]);
+    cur = &sl;
+    const int kk = st - off;
+    if (col && kk >= 0 && kk < nc) {
+      product(2, oC);
+      if (store & 1) {
 #pragma unroll
-        for (int e = 0; e < 5; ++e) bv[e] = bt[e * b.nbf + qb];
+        for (int e = 0; e < 5; ++e) x[e * b.ncell + p] = xn[e];
       }
-#pragma unroll
-      for (int e = 0; e < 5; ++e) O[e] += ok ? u[e] : bv[e];
     }
+    if (FWD && !FULL && (store & 2)) {
 #pragma unroll
-    for (int e = 0; e < 5; ++e) sl.O[FULL ? e : 0][lane] = O[e];
+      for (int e = 0; e < 5; ++e) Xs[e * kPenLanes] = xn[e];
+    }
+    p += sC;
+    Xs += 5 * kPenLanes;
   }
 }
 
+// `store`: bit 0 du in the natural layout, bit 1 in sweep order (a forward
+// pass whose backward pass reads it)
 template <typename T, bool FWD, bool FULL>
-__global__ void __launch_bounds__(kPenWaves * kPenLanes) KLusgsPencil(PencilGroup G, Params P) {
+__global__ void __launch_bounds__(kPenWaves * kPenLanes) KLusgsPencil(PencilGroup G, Params P, int store) {
   __shared__ PenShared<T, FULL> sh;
-  const int tid = threadIdx.x, wave = tid / kPenLanes, lane = tid % kPenLanes;
-  if (tid == 0) sh.ticket = __hip_atomic_fetch_add(G.ticket, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-  if (tid < kStagers) sh.stageReady[tid] = 0;
-  if (tid < 3) sh.oReady[tid] = 0;
-  if (tid == 0) sh.xReady = 0;
+  const int tid = threadIdx.x, lane = tid % kPenLanes;
+  const int wave = __builtin_amdgcn_readfirstlane(tid / kPenLanes);
+  if (tid == 0) {
+    sh.ticket = (int)(__hip_atomic_fetch_add(G.ticket, 1ULL, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) %
+                      (unsigned long long)G.nent);
+    sh.haloReady = 0;
+    sh.xReady = 0;
+    sh.sentReady = 0;
+  }
+  if (tid < kPenSlots) sh.stageReady[tid] = 0;
   __syncthreads();
   const int t = __builtin_amdgcn_readfirstlane(sh.ticket);
-  if (t >= G.nent) return;
   const int4 ent = G.entries[FWD ? t : G.nent - 1 - t];
   const DevBlock b = G.blocks[ent.z];
-  PencilCtl s;
-  s.prog = G.prog + ent.w;
-  s.err = G.err;
-  s.pa = (b.ni + kPW - 1) / kPW;
-  s.pb = (b.nj + kPW - 1) / kPW;
-  s.sinkv = static_cast<T *>(G.sinkv) + (size_t)ent.w * 5 * kPenLanes;
-  const int2 pc = make_int2(ent.x, ent.y);
-  PenLane L;
-  L.li = lane % kPW;
-  L.lj = lane / kPW;
-  L.wi = PenWidth(b.ni, pc.x);
-  L.wj = PenWidth(b.nj, pc.y);
-  L.nsteps = L.wi + L.wj + b.nk - 2;
-  L.i = pc.x * kPW + L.li;
-  L.j = pc.y * kPW + L.lj;
-  L.col = L.li < L.wi && L.lj < L.wj;
-  L.off = FWD ? L.li + L.lj : (L.wi - 1 - L.li) + (L.wj - 1 - L.lj);
-  const int pid = pc.x + s.pa * pc.y;
-  const int sgn = FWD ? -1 : 1;
-  const int ns = L.nsteps;
+  const int C = b.pl, A = (C + 1) % 3, B = (C + 2) % 3;
+  const int na = AxisN(b, A), nb = AxisN(b, B);
+  Pencil pen;
+  pen.a = ent.x;
+  pen.b = ent.y;
+  pen.pid = pen.a + b.pa * pen.b;
+  pen.wa = PenWidth(na, pen.a);
+  pen.wb = PenWidth(nb, pen.b);
+  pen.nc = AxisN(b, C);
+  pen.ns = pen.wa + pen.wb + pen.nc - 2;
+  pen.rec = (long)pen.pid * b.pns;
+  pen.nrec = (long)b.pa * b.pb * b.pns;
+  const int sgn = FWD ? -1 : 1;  // direction of the dependency neighbours
+  const int ns = pen.ns, nc = pen.nc;
+  const T *bt = OpBuf<T>::Bt(b);
+  // messages of pencil (pa, pb) of this block through its face f (0 A, 1 B)
+  T *const msg0 = (T *)G.msg[FWD ? 0 : 1] + (long)ent.w * kMsg;
+  auto messages = [&](int pa, int pb, int f) { return msg0 + ((long)(pa + b.pa * pb) * 2 + f) * b.pns * kMsg; };
 
-  if (wave >= 4) {
-    // ---- stager j: steps j, j+4, ...
-    const int jst = wave - 4;
-    int nbId[2], nbW[2], nbTotal[2], known[2] = {0, 0};
-#pragma unroll
-    for (int h = 0; h < 2; ++h) {
-      const int na = pc.x + (h == 0 ? sgn : 0), nb = pc.y + (h == 1 ? sgn : 0);
-      nbId[h] = -1;
-      nbW[h] = nbTotal[h] = 0;
-      if (na >= 0 && nb >= 0 && na < s.pa && nb < s.pb) {
-        nbId[h] = na + s.pa * nb;
-        const int nwi = PenWidth(b.ni, na), nwj = PenWidth(b.nj, nb);
-        nbW[h] = h == 0 ? nwi : nwj;
-        nbTotal[h] = nwi + nwj + b.nk - 2;
-      }
-    }
-    for (int st = jst; st < ns; st += kStagers) {
-      // the slot is free once the owner has finished step st - kStagers
-      LdsWait(&sh.xReady, st - kStagers + 1, s.err);
-      PenStage<T, FWD, FULL>(b, P, s, sh.slot[jst], L, lane, st, nbId, nbW, nbTotal, known);
-      LdsStore(&sh.stageReady[jst], st + 1);
-    }
-  } else if (wave < 3) {
-    // ---- neighbour wave d
-    const int d = wave;
-    const GasT<T> g = Cast<T>(P.gas);
-    // in-pencil neighbour lane (clamped: lanes across the pencil face read a
-    // valid slot and use the staged du instead)
-    const int nl = min(max(lane + sgn * (d == 0 ? 1 : (d == 1 ? kPW : 0)), 0), kPenLanes - 1);
-    const bool cross = (d == 0 && (FWD ? L.li == 0 : L.li == L.wi - 1)) ||
-                       (d == 1 && (FWD ? L.lj == 0 : L.lj == L.wj - 1));
+  const int da = pen.a - sgn, db = pen.b - sgn;  // the pencils downstream
+  const bool toA = da >= 0 && da < b.pa, toB = db >= 0 && db < b.pb;
+  if (wave == 0) {
+    // ---- compute wave
+    __builtin_amdgcn_s_setprio(3);
+    const bool sends = toA || toB;
+    if (C == 0) PenCompute<T, FWD, FULL, 0>(b, P, pen, sh, lane, store, sends, G.err);
+    else if (C == 1) PenCompute<T, FWD, FULL, 1>(b, P, pen, sh, lane, store, sends, G.err);
+    else PenCompute<T, FWD, FULL, 2>(b, P, pen, sh, lane, store, sends, G.err);
+  } else if (wave == 2) {
+    // ---- send wave: lane = (value e, entry q), as in the halo wave
+    if (!toA && !toB) return;
+    const int e = lane / kPW, q = lane % kPW;
+    // the columns whose products leave the pencil
+    const int cA = (FWD ? pen.wa - 1 : 0) + kPW * q, cB = q + kPW * (FWD ? pen.wb - 1 : 0);
+    const int offA = FWD ? pen.wa - 1 + q : pen.wa - 1 + pen.wb - 1 - q,
+              offB = FWD ? q + pen.wb - 1 : pen.wa - 1 - q + pen.wb - 1;
+    const bool useA = toA && e < 5 && q < pen.wb, useB = toB && e < 5 && q < pen.wa;
+    T *const mA = toA ? messages(da, pen.b, 0) + e * kPW + q - (long)(pen.wa - 1) * kMsg : nullptr;
+    T *const mB = toB ? messages(pen.a, db, 1) + e * kPW + q - (long)(pen.wb - 1) * kMsg : nullptr;
+    const int ev = e < 5 ? e / kVecN<T> : 0, er = e % kVecN<T>;
     for (int st = 0; st < ns; ++st) {
-      const PenSlot<T, FULL> &sl = sh.slot[st % kStagers];
-      LdsWait(&sh.stageReady[st % kStagers], st + 1, s.err);
-      LdsWait(&sh.xReady, st, s.err);
-      const int k = L.K(st, b.nk, FWD);
-      const bool dep = k >= 0 && InBlock(b, L.i + (d == 0 ? sgn : 0), L.j + (d == 1 ? sgn : 0), k + (d == 2 ? sgn : 0));
-      T du[5], U[5], Wu[5], Fn[5];
+      LdsWait<1>(&sh.xReady, st + 1, G.err);
+      const T vA = sh.prod[st & (kProdRing - 1)][0][ev][cA].v[er], vB = sh.prod[st & (kProdRing - 1)][1][ev][cB].v[er];
+      // (no wait for the stores of the steps before)
+      asm volatile("" ::"v"(vA), "v"(vB));
+      LdsPost(&sh.sentReady, st + 1);
+      const int kA = st - offA, kB = st - offB;
+      if (useA && kA >= 0 && kA < nc) StoreCoherent(mA + (long)st * kMsg, vA);
+      if (useB && kB >= 0 && kB < nc) StoreCoherent(mB + (long)st * kMsg, vB);
+    }
+  } else if (wave == 1) {
+    // ---- halo wave: lane = (value e, entry q); entry q of face A is the
+    // row lb = q, of face B the row la = q
+    const int e = lane / kPW, q = lane % kPW;
+    const int ua = pen.a + sgn, ub = pen.b + sgn;  // the pencils upstream
+    const bool from[2] = {ua >= 0 && ua < b.pa, ub >= 0 && ub < b.pb};
+    const int w[2] = {pen.wb, pen.wa};
+    const T *in[2];
+    int off[2];
+    bool use[2];
 #pragma unroll
-      for (int e = 0; e < 5; ++e) {
-        const T hx = sl.halo[d < 2 ? d : 0][e][lane], px = sh.sX[e][nl];
-        du[e] = cross ? hx : px;
-        U[e] = sl.U[d][e][lane] + du[e];
-      }
-      if constexpr (sizeof(T) == 4) {
-        // flux change from the staged primitive state (DeltaFlux)
-        T Wn[5];
+    for (int f = 0; f < 2; ++f) {
+      in[f] = messages(pen.a, pen.b, f) + min(lane, kMsg - 1);
+      off[f] = FWD ? q : w[f] - 1 - q;
+      use[f] = e < 5 && q < w[f];
+    }
+    bool dead = false;
+    for (int st = 0; st < ns; ++st) {
+      LdsWait<1>(&sh.xReady, st + 1 - kHaloRing, G.err);
+      T v[2];
+      for (int spins = 0;;) {
+        bool empty = false;
 #pragma unroll
-        for (int e = 0; e < 5; ++e) Wn[e] = sl.U[d][e][lane];
-        DeltaFlux(g, Wn, du, sl.n[d][0][lane], sl.n[d][1][lane], sl.n[d][2][lane], Fn);
-      } else {
-        // UpdatePrim + PhysFlux of the updated state + the Rusanov terms
-        ConsToPrim(g, U, Wu);
-        PhysFlux(g, Wu, sl.n[d][0][lane], sl.n[d][1][lane], sl.n[d][2][lane], Fn);
+        for (int f = 0; f < 2; ++f) {
+          v[f] = from[f] ? CoherentLoad(in[f]) : T(0);
+          empty |= use[f] && (unsigned)(st - off[f]) < (unsigned)nc && IsEmpty(v[f]);
+        }
+        if (dead || !__any(empty)) break;
+        if (((++spins & 255) == 0 && (__builtin_amdgcn_readfirstlane(CoherentLoad(G.err)) & 2)) || spins > kSpinLimit) {
+          // a wait of this launch has timed out: stop waiting at all
+          __hip_atomic_fetch_or(G.err, 2, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+          dead = true;
+        }
       }
-      const T half = sl.half[d][lane], lam = sl.lam[d][lane];
-      // a neighbour outside the block contributes the staged connection
-      // term (zero off connections); idle steps contribute zero
-      const bool outside = k >= 0 && !dep;
 #pragma unroll
-      for (int e = 0; e < 5; ++e) {
-        const T fc = half * (sizeof(T) == 4 ? Fn[e] : Fn[e] - sl.Fo[d][e][lane]);
-        const T o = FWD ? fc + du[e] * lam : fc - du[e] * lam;
-        sh.sO[d][e][lane] = dep ? o : (outside ? sl.Fo[d][e][lane] : T(0));
+      for (int f = 0; f < 2; ++f) {
+        const int kk = st - off[f];
+        if (bt && !from[f] && use[f] && kk >= 0 && kk < nc) {
+          // on a block face: the connection term (zero off connections)
+          int i, j, k;
+          const int edgeA = FWD ? 0 : na - 1, edgeB = FWD ? 0 : nb - 1;
+          Map3(C, FWD ? kk : nc - 1 - kk, f == 0 ? edgeA : pen.a * kPW + q, f == 0 ? pen.b * kPW + q : edgeB, i, j, k);
+          v[f] = NotEmpty(bt[e * b.nbf + BtSlot(b, f == 0 ? A : B, FWD ? 0 : 1, i, j, k)]);
+        }
+        if (e < 5) sh.halo[f][e / kVecN<T>][kPW * (st % kHaloRing) + q].v[e % kVecN<T>] = v[f];
+        in[f] += kMsg;
       }
-      LdsStore(&sh.oReady[d], st + 1);
+      LdsPost(&sh.haloReady, st + 1);
     }
   } else {
-    // ---- owner
-    T *x = OpBuf<T>::X(b);
-    T *sink = static_cast<T *>(s.sinkv) + (size_t)pid * 5 * kPenLanes;
-    for (int st = 0; st < ns; ++st) {
-      const PenSlot<T, FULL> &sl = sh.slot[st % kStagers];
-      LdsWait(&sh.oReady[0], st + 1, s.err);
-      LdsWait(&sh.oReady[1], st + 1, s.err);
-      LdsWait(&sh.oReady[2], st + 1, s.err);
-      const int k = L.K(st, b.nk, FWD);
-      const T ainv = sl.ainv[lane];
-      // products of absent neighbours are +0 and leave D unchanged (D starts
-      // at +0 and is never -0)
-      T D[5], xn[5];
-#pragma unroll
-      for (int e = 0; e < 5; ++e) D[e] = ((T(0) + sh.sO[0][e][lane]) + sh.sO[1][e][lane]) + sh.sO[2][e][lane];
-      if (FULL) {
-        if (FWD) {
-#pragma unroll
-          for (int e = 0; e < 5; ++e) xn[e] = (T(sl.v5[e][lane]) + (D[e] - sl.O[FULL ? e : 0][lane])) * ainv;
-        } else {
-#pragma unroll
-          for (int e = 0; e < 5; ++e) xn[e] = ((T(sl.v5[e][lane]) + sl.O[FULL ? e : 0][lane]) - D[e]) * ainv;
-        }
-      } else if (FWD) {
-#pragma unroll
-        for (int e = 0; e < 5; ++e) xn[e] = (T(sl.v5[e][lane]) + D[e]) * ainv;
-      } else {
-#pragma unroll
-        for (int e = 0; e < 5; ++e) xn[e] = T(sl.v5[e][lane]) - D[e] * ainv;
-      }
-#pragma unroll
-      for (int e = 0; e < 5; ++e) sh.sX[e][lane] = xn[e];
-      LdsStore(&sh.xReady, st + 1);
-      const long p = (long)L.i + (long)L.j * b.ni + (long)(k < 0 ? 0 : k) * b.ni * b.nj;
-#pragma unroll
-      for (int e = 0; e < 5; ++e) StoreCoherent(k >= 0 ? &x[e * b.ncell + p] : &sink[e * kPenLanes + lane], xn[e]);
-      if ((st + 1) % kPubEvery == 0 || st + 1 == ns) {
-        // the owner wave's du stores have completed before the count
-        WaitStores();
-        if (lane == 0)
-          __hip_atomic_store(&s.prog[pid], st + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-      }
+    // ---- stager: steps j, j + kStagers, ...
+    const int j = wave - 3;
+    for (int st = j; st < ns; st += kStagers) {
+      PenStage<T, FWD, FULL>(b, P, pen, sh.slot[j], lane, st, &sh.xReady, G.err);
+      LdsStore(&sh.stageReady[j], st + 1);
     }
+    // empty this pencil's message slots of the other direction's pass
+    T *const old = (T *)G.msg[FWD ? 1 : 0] + ((long)ent.w + (long)pen.pid * 2 * b.pns) * kMsg;
+    for (long q = j * kPenLanes + lane; q < 2L * b.pns * kMsg; q += kStagers * kPenLanes) old[q] = EmptySlot<T>();
   }
 }
 

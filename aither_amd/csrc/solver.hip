@@ -112,6 +112,7 @@ struct ath_ctx {
   int *dflag = nullptr;             // bit 2: a sweep dependency wait exceeded its spin limit
   // all-block pencil sweep
   ath::PencilGroup pen{};
+  size_t msgBytes = 0;
   int fp32 = 0;
   int matres = 1;
   int sweepOrder = ATH_SWEEP_PENCIL;  // ATH_SWEEP_*
@@ -138,7 +139,7 @@ struct ath_ctx {
   // unit grids of the all-block launches (ath::BlockMap), kNumMaps of them,
   // nb entries each, and each one's total unit count
   int4 *dmaps = nullptr;
-  int mapTotal[4] = {0, 0, 0, 0};
+  int mapTotal[5] = {0, 0, 0, 0, 0};
   // the ghost-cell task lists of every block (ath::BlockTasks), kNumTaskMaps
   // tables of nb entries, and each one's item total
   ath::BlockTasks *dbt = nullptr;
@@ -189,8 +190,9 @@ int Grid(long n, int b = kBlk) { return (int)((n + b - 1) / b); }
 // the unit grids of the all-block launches: 8x8x4 tiles (residual and
 // viscous flux), ranges of 128 cells (block diagonal), of 256 cells (matrix
 // residual, update, initialisation; their partials are the reductions'
-// slots) and of 256 padded cells (auxiliary variables)
-enum { kMapTile = 0, kMapCell128 = 1, kMapCell256 = 2, kMapPad256 = 3, kNumMaps = 4 };
+// slots), of 256 padded cells (auxiliary variables) and of 256 lanes of the
+// pencil sweep's records
+enum { kMapTile = 0, kMapCell128 = 1, kMapCell256 = 2, kMapPad256 = 3, kMapPen256 = 4, kNumMaps = 5 };
 // the ghost-cell task tables: boundary patches, edge lines of the inviscid
 // and of the viscous pass, no-slip wall cells
 enum { kTaskBc = 0, kTaskEdgeInv = 1, kTaskEdgeVisc = 2, kTaskWall = 3, kNumTaskMaps = 4 };
@@ -507,6 +509,22 @@ void CaseConnections(const ath::HostCase &hc, CaseRes &cr) {
 
 int RebuildGroup(ath_ctx *c);
 
+// cases whose relax can run in the pencil order (EffectiveOrder)
+bool PencilCase(const ath::HostCase &hc) {
+  return hc.Implicit() && hc.solver == ath::Solver::LUSGS && !hc.block && !hc.roeJac;
+}
+// pencils run along the block's longest axis: the fewest column handoffs
+// (each costs several steps) and the fewest idle steps (2 kPW - 2 a pencil)
+void PencilGrid(const ath::HostBlock &h, int *pl, int *pa, int *pb, int *pns) {
+  int l = 2;
+  for (int d = 0; d < 2; ++d)
+    if (h.N(d) > h.N(l)) l = d;
+  *pl = l;
+  *pa = (h.N((l + 1) % 3) + ath::kPW - 1) / ath::kPW;
+  *pb = (h.N((l + 2) % 3) + ath::kPW - 1) / ath::kPW;
+  *pns = h.N(l) + 2 * ath::kPW - 2;
+}
+
 int AllocFp32(ath_ctx *c, ath::DevBlock &d) {
   if (d.x32) return ATH_OK;
   if (int r = c->Alloc(&d.Ainv32, d.ncell)) return r;
@@ -700,6 +718,21 @@ int UploadCase(ath_ctx *c, CaseRes &cr, bool fp32) {
     }
     if (hc.viscous)
       if (int r = UploadViscous(c, hc, h, br)) return r;
+    // scalar LU-SGS: the pencil sweep's arrays, pencils along the longest axis
+    d.skF = d.skS = d.skX = d.skO = nullptr;
+    d.pl = d.pa = d.pb = d.pns = 0;
+    if (PencilCase(hc)) {
+      PencilGrid(h, &d.pl, &d.pa, &d.pb, &d.pns);
+      const size_t lanes = (size_t)d.pa * d.pb * d.pns * kPenLanes;
+      const int nS = kPenS + (hc.viscous ? 1 : 0), nF = kPenF + (hc.viscous ? 3 : 0);
+      if (int r = c->Alloc(&d.skF, 2 * nF * lanes)) return r;
+      if (int r = c->Alloc(&d.skS, nS * lanes)) return r;
+      if (int r = c->Alloc(&d.skX, 5 * lanes)) return r;
+      if (hc.InitMatrix())
+        if (int r = c->Alloc(&d.skO, 5 * lanes)) return r;
+      hipLaunchKernelGGL(KPencilFaces, dim3(Grid((long)lanes)), dim3(kBlk), 0, nullptr, d, hc.viscous ? 1 : 0);
+      HIP_OK(hipGetLastError());
+    }
     // hyperplane order
     std::vector<int> cells;
     HyperplaneOrder(h.ni, h.nj, h.nk, &cells, &br.planeOff);
@@ -878,7 +911,8 @@ int RebuildGroup(ath_ctx *c) {
                       (d.nk + ath::kTK - 1) / ath::kTK, f);
       else if (q == kMapCell128) u = make_int4(Grid(d.ncell, 128), 1, 1, f);
       else if (q == kMapCell256) u = make_int4(Grid(d.ncell, ath::kRedThreads), 1, 1, f);
-      else u = make_int4(Grid(d.npad, 256), 1, 1, f);
+      else if (q == kMapPad256) u = make_int4(Grid(d.npad, 256), 1, 1, f);
+      else u = make_int4(d.skS ? Grid((long)d.pa * d.pb * d.pns * kPenLanes, 256) : 0, 1, 1, f);
       v[(size_t)q * nb + b] = u;
       f += u.x * u.y * u.z;
     }
@@ -929,24 +963,24 @@ int RebuildGroup(ath_ctx *c) {
   if (int r = c->Alloc(&c->dbt, bt.size())) return r;
   HIP_OK(hipMemcpy(c->dbt, bt.data(), bt.size() * sizeof(ath::BlockTasks), hipMemcpyHostToDevice));
   // pencil sweep queue: every block's kPW x kPW columns by column hyperplane
-  // a + b, then block, then b, a
-  {
+  // a + b, then block, then b, a; per block its first message step
+  if (c->mapTotal[kMapPen256] > 0) {
     std::vector<int4> ent;
     std::vector<int> base(nb);
-    int total = 0, maxPlane = 0;
+    int maxPlane = 0;
+    long steps = 0;
     for (int b = 0; b < nb; ++b) {
       const auto &d = c->blk[b].d;
-      const int pa = (d.ni + kPW - 1) / kPW, pb = (d.nj + kPW - 1) / kPW;
-      base[b] = total;
-      total += pa * pb;
-      maxPlane = std::max(maxPlane, pa + pb - 1);
+      base[b] = (int)steps;
+      steps += 2L * d.pa * d.pb * d.pns;
+      maxPlane = std::max(maxPlane, d.pa + d.pb - 1);
     }
+    if (steps > std::numeric_limits<int>::max()) return Fail(ATH_ERR_NOMEM, "too many cells for the pencil sweep");
     for (int pl = 0; pl < maxPlane; ++pl)
       for (int b = 0; b < nb; ++b) {
         const auto &d = c->blk[b].d;
-        const int pa = (d.ni + kPW - 1) / kPW, pb = (d.nj + kPW - 1) / kPW;
-        for (int bb = 0; bb < pb; ++bb)
-          for (int aa = 0; aa < pa; ++aa)
+        for (int bb = 0; bb < d.pb; ++bb)
+          for (int aa = 0; aa < d.pa; ++aa)
             if (aa + bb == pl) ent.push_back(make_int4(aa, bb, b, base[b]));
       }
     int4 *de = nullptr;
@@ -955,13 +989,16 @@ int RebuildGroup(ath_ctx *c) {
     PencilGroup &g = c->pen;
     g.entries = de;
     g.nent = (int)ent.size();
-    if (int r = c->Alloc(&g.prog, total)) return r;
     if (int r = c->Alloc(&g.ticket, 1)) return r;
-    double *sink = nullptr;
-    if (int r = c->Alloc(&sink, (size_t)total * 5 * kPenLanes)) return r;
-    g.sinkv = sink;
-    HIP_OK(hipMemset(g.prog, 0, total * sizeof(int)));
-    HIP_OK(hipMemset(g.ticket, 0, sizeof(int)));
+    HIP_OK(hipMemset(g.ticket, 0, sizeof *g.ticket));
+    c->msgBytes = (size_t)steps * kMsg * sizeof(double);
+    for (void *&m : g.msg) {
+      double *msg = nullptr;
+      if (int r = c->Alloc(&msg, c->msgBytes / sizeof(double))) return r;
+      m = msg;
+      HIP_OK(hipMemset(m, 0xff, c->msgBytes));
+    }
+    HIP_OK(hipStreamSynchronize(nullptr));  // the context's stream does not wait for the null stream
     g.err = c->dflag;
     g.blocks = c->dblocks;
   }
@@ -1200,31 +1237,41 @@ int LaunchRelaxT(ath_ctx *c, bool timed, size_t evBase) {
   // initialisation forms once per relax
   ath::Params P0 = c->P;
   P0.rhsOnce = (hc.solver == ath::Solver::LUSGS && c->P.block && EffectiveOrder(c) == ATH_SWEEP_ROWS) ? 1 : 0;
-  // (formed by the residual stage unless the sweep order changed since)
-  if (!(RhsInDiag(c) && c->rhsFormed))
+  // (formed by the residual stage unless the sweep order changed since); a
+  // one-sweep pencil relax writes every du before anything but the
+  // connection terms reads it
+  const bool pencilOnce = hc.solver == ath::Solver::LUSGS && !hc.InitMatrix() && EffectiveOrder(c) == ATH_SWEEP_PENCIL &&
+                          c->nconn == 0;
+  if (!(RhsInDiag(c) && c->rhsFormed) && !pencilOnce)
     hipLaunchKernelGGL(ath::KInitUpdate<T>, dim3(c->mapTotal[kMapCell256]), dim3(kBlk), 0, c->stream,
                        c->Map(kMapCell256), P0);
   for (int sw = 0; sw < hc.sweeps; ++sw) {
     const int full = (sw > 0 || hc.InitMatrix()) ? 1 : 0;
     const int order = EffectiveOrder(c);
     if (hc.solver == ath::Solver::LUSGS && order == ATH_SWEEP_PENCIL) {
-      if (sw == 0)
-        hipLaunchKernelGGL(ath::KLusgsRhs, dim3(c->mapTotal[kMapCell256]), dim3(kBlk), 0, c->stream,
-                           c->Map(kMapCell256), c->P);
+      const dim3 units(c->mapTotal[kMapPen256]);
+      const ath::BlockMap mp = c->Map(kMapPen256);
+      if (sw == 0) hipLaunchKernelGGL(ath::KPencilPrep<T>, units, dim3(kBlk), 0, c->stream, mp, c->P);
       for (int dir = 0; dir < 2; ++dir) {
         LaunchConnTerms<T>(c);
         mark(true);
         // every block's pencils in one launch
-        hipLaunchKernelGGL(ath::KPencilPrologue, dim3(1), dim3(256), 0, c->stream, c->pen);
         const dim3 grid(c->pen.nent), blk(ath::kPenWaves * ath::kPenLanes);
-        if (dir == 0 && full)
-          hipLaunchKernelGGL((ath::KLusgsPencil<T, true, true>), grid, blk, 0, c->stream, c->pen, c->P);
-        else if (dir == 0)
-          hipLaunchKernelGGL((ath::KLusgsPencil<T, true, false>), grid, blk, 0, c->stream, c->pen, c->P);
-        else if (full)
-          hipLaunchKernelGGL((ath::KLusgsPencil<T, false, true>), grid, blk, 0, c->stream, c->pen, c->P);
-        else
-          hipLaunchKernelGGL((ath::KLusgsPencil<T, false, false>), grid, blk, 0, c->stream, c->pen, c->P);
+        // a one-sweep forward pass hands du to the backward pass in sweep
+        // order; the connection terms and the other-side sums read the
+        // natural layout
+        const int store = dir == 0 && !full ? (c->nconn > 0 ? 3 : 2) : 1;
+        if (dir == 0 && full) {
+          hipLaunchKernelGGL((ath::KPencilOther<T, true>), units, dim3(kBlk), 0, c->stream, mp, c->P);
+          hipLaunchKernelGGL((ath::KLusgsPencil<T, true, true>), grid, blk, 0, c->stream, c->pen, c->P, store);
+        } else if (dir == 0) {
+          hipLaunchKernelGGL((ath::KLusgsPencil<T, true, false>), grid, blk, 0, c->stream, c->pen, c->P, store);
+        } else if (full) {
+          hipLaunchKernelGGL((ath::KPencilOther<T, false>), units, dim3(kBlk), 0, c->stream, mp, c->P);
+          hipLaunchKernelGGL((ath::KLusgsPencil<T, false, true>), grid, blk, 0, c->stream, c->pen, c->P, store);
+        } else {
+          hipLaunchKernelGGL((ath::KLusgsPencil<T, false, false>), grid, blk, 0, c->stream, c->pen, c->P, store);
+        }
         ++launches;
         mark(false);
       }
@@ -1422,6 +1469,11 @@ int TakeFlags(ath_ctx *c, CaseRes &cr, int *flag) {
   const int zero = 0;
   if (fc) HIP_OK(hipMemcpy(cr.dflag, &zero, sizeof zero, hipMemcpyHostToDevice));
   if (fg) HIP_OK(hipMemcpy(c->dflag, &zero, sizeof zero, hipMemcpyHostToDevice));
+  if (fg && c->pen.nent > 0) {
+    // a pass that gave up waiting may leave unread messages behind
+    for (void *m : c->pen.msg) HIP_OK(hipMemset(m, 0xff, c->msgBytes));
+    HIP_OK(hipStreamSynchronize(nullptr));
+  }
   *flag = fc | fg;
   return ATH_OK;
 }
@@ -2301,6 +2353,13 @@ double EstimateBytes(const ath::HostCase &hc, bool fp32) {
     const double nbf = 2.0 * ((double)h.nj * h.nk + (double)h.nk * h.ni + (double)h.ni * h.nj);
     t += np * 8 * 8 + nf * 32 + nc * 8 * 35 + nc * 4 + nbf * 80 + tiles * 32 + 8192;
     if (fp32) t += nc * 4 * 11 + nbf * 20;
+    if (PencilCase(hc)) {
+      int pl, pa, pb, pns;
+      PencilGrid(h, &pl, &pa, &pb, &pns);
+      // the case's sweep arrays and its share of the group's message slots
+      t += (double)pa * pb * pns * 8 *
+           (ath::kPenLanes * (2.0 * (ath::kPenF + 3) + ath::kPenS + 1 + 5 + (hc.InitMatrix() ? 5 : 0)) + 4.0 * ath::kMsg);
+    }
     if (hc.block) t += nc * 25 * 8 + tiles * 256 * 25 * 8;
     if (hc.viscous) t += np * 8 * 3 + nfp * 32 + nf * 8 + nbf + (double)h.g * h.g * 4 * (h.ni + h.nj + h.nk) * 2 * 64 +
                          nbf * 40.0 * h.g;

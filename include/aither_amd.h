@@ -89,8 +89,8 @@ int ath_block_dims(const ath_ctx *ctx, int block, int *ni, int *nj, int *nk);
 /* implicit-operator precision (default ATH_IMPLICIT_FP64).  No reference
  * counterpart: the reference is FP64 throughout. */
 int ath_set_implicit_precision(ath_ctx *ctx, int precision);
-/* LU-SGS execution order.  ATH_SWEEP_PENCIL (default): 8x8 columns walking k
- * on a skewed wavefront, one launch per sweep pass.  ATH_SWEEP_TILED: 8x8x4
+/* LU-SGS execution order.  ATH_SWEEP_PENCIL (default): 8x8 columns walking
+ * the block's longest axis on a skewed wavefront, one launch per sweep pass.  ATH_SWEEP_TILED: 8x8x4
  * tiles in tile-hyperplane order, dataflow-synchronised, one launch per pass.
  * ATH_SWEEP_HYPERPLANE: one launch per i+j+k hyperplane in the order of
  * HyperplaneReorder (src/utility.cpp:377-398).  ATH_SWEEP_ROWS (block
