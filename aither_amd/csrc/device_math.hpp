@@ -33,20 +33,75 @@ __device__ __forceinline__ GasT<T> Cast(const Gas &g) {
 __device__ __forceinline__ double Dmax(double a, double b) { return (a < b) ? b : a; }  // std::max
 __device__ __forceinline__ double Dmin(double a, double b) { return (b < a) ? b : a; }  // std::min
 
+// ---------------------------------------------------------------------------
+// Several quotients by one divisor: the reciprocal y is refined once by two
+// Newton steps (one in FP32), then each quotient takes one product and one
+// (two) residual corrections (Markstein, "Computation of elementary functions
+// on the IBM RISC System/6000 processor", 1990), and div_fixup settles signs
+// of zeros, infinities and NaN.  These are the operations of the compiler's
+// division without its scaling of operands near the ends of the exponent
+// range, so a quotient is that of operator/ bit for bit while divisor,
+// numerator residual (numerator 2^-53) and quotient are normal numbers; below
+// that it may be off by a few units of the smallest denormal.  A division by
+// operator/ is eleven operations, four of them in a row through one condition
+// register; four by one divisor are 17 here.
+template <typename T>
+struct Divisor {
+  T d, y;
+};
+__device__ __forceinline__ Divisor<double> MakeDivisor(double d) {
+  double y = __builtin_amdgcn_rcp(d);
+  y = fma(y, fma(-d, y, 1.0), y);
+  y = fma(y, fma(-d, y, 1.0), y);
+  return {d, y};
+}
+__device__ __forceinline__ Divisor<float> MakeDivisor(float d) {
+  const float y = __builtin_amdgcn_rcpf(d);
+  return {d, fmaf(fmaf(-d, y, 1.0f), y, y)};
+}
+__device__ __forceinline__ double Quot(double n, const Divisor<double> &v) {
+  const double q = n * v.y;
+  return __builtin_amdgcn_div_fixup(fma(fma(-v.d, q, n), v.y, q), v.d, n);
+}
+__device__ __forceinline__ float Quot(float n, const Divisor<float> &v) {
+  float q = n * v.y;
+  q = fmaf(fmaf(-v.d, q, n), v.y, q);
+  return __builtin_amdgcn_div_fixupf(fmaf(fmaf(-v.d, q, n), v.y, q), v.d, n);
+}
+// sqrt for x = 0 or x >= 2^-760: the Goldschmidt iteration of sqrt() without
+// its scaling of small arguments (inf and NaN pass through)
+__device__ __forceinline__ double SqrtInRange(double x) {
+  const double y = __builtin_amdgcn_rsq(x);
+  double g = x * y, h = 0.5 * y;
+  const double r = fma(-h, g, 0.5);
+  g = fma(g, r, g);
+  h = fma(h, r, h);
+  g = fma(fma(-g, g, x), h, g);
+  g = fma(fma(-g, g, x), h, g);
+  return (x == 0.0 || x == __builtin_inf()) ? x : g;
+}
+__device__ __forceinline__ double Sqrt(double x) { return SqrtInRange(x); }
+__device__ __forceinline__ float Sqrt(float x) { return sqrtf(x); }
+// one quotient
+template <typename T>
+__device__ __forceinline__ T Div(T n, T d) {
+  return Quot(n, MakeDivisor(d));
+}
+
 // idealGas::Temperature (src/eos.cpp:103-111), SoS (include/arrayView.hpp:384)
 template <typename T>
 __device__ __forceinline__ T Temperature(const GasT<T> &g, T rho, T p) {
 #pragma clang fp contract(off)
-  return p / (rho * g.R);
+  return Div(p, rho * g.R);
 }
 template <typename T>
 __device__ __forceinline__ T SoS(const GasT<T> &g, T rho, T p) {
-  return sqrt(g.gamma * p / rho);
+  return Sqrt(Div(g.gamma * p, rho));
 }
 template <typename T>
 __device__ __forceinline__ T VelMag(T u, T v, T w) {
 #pragma clang fp contract(off)
-  return sqrt((u * u + v * v) + w * w);
+  return Sqrt((u * u + v * v) + w * w);
 }
 // EnthalpyFunc / InternalEnergy (include/arrayView.hpp:420-444; hf = 0)
 template <typename T>
@@ -77,14 +132,14 @@ __device__ __forceinline__ void PrimToCons(const GasT<T> &g, const T W[5], T U[5
 template <typename T>
 __device__ __forceinline__ void ConsToPrim(const GasT<T> &g, const T U[5], T W[5]) {
 #pragma clang fp contract(off)
-  const T rho = U[0];
+  const Divisor<T> byRho = MakeDivisor(U[0]);
   W[0] = U[0];
-  W[1] = U[1] / rho;
-  W[2] = U[2] / rho;
-  W[3] = U[3] / rho;
-  const T en = U[4] / rho;
+  W[1] = Quot(U[1], byRho);
+  W[2] = Quot(U[2], byRho);
+  W[3] = Quot(U[3], byRho);
+  const T en = Quot(U[4], byRho);
   const T vel = VelMag(W[1], W[2], W[3]);
-  const T t = (en - T(0.5) * vel * vel) / g.cvs;
+  const T t = Div(en - T(0.5) * vel * vel, g.cvs);
   W[4] = (W[0] * g.R) * t;
 }
 // UpdatePrimWithCons (include/primitive.hpp:206-231); with a single species
@@ -115,17 +170,17 @@ __device__ __forceinline__ void PhysFlux(const GasT<T> &g, const T W[5], T nx, T
 // RoeAveragedState (include/primitive.hpp:245-280)
 __device__ inline void RoeFlux(const GasT<double> &g, const double L[5], const double R[5],
                                double nx, double ny, double nz, double F[5]) {
-  const double denRatio = sqrt(R[0] / L[0]);
+  const double denRatio = Sqrt(Div(R[0], L[0]));
   const double rr = L[0] * denRatio;
-  const double inv = 1.0 + denRatio;
-  const double ur = (L[1] + denRatio * R[1]) / inv;
-  const double vr = (L[2] + denRatio * R[2]) / inv;
-  const double wr = (L[3] + denRatio * R[3]) / inv;
-  const double pr = (L[4] + denRatio * R[4]) / inv;
+  const Divisor<double> inv = MakeDivisor(1.0 + denRatio);
+  const double ur = Quot(L[1] + denRatio * R[1], inv);
+  const double vr = Quot(L[2] + denRatio * R[2], inv);
+  const double wr = Quot(L[3] + denRatio * R[3], inv);
+  const double pr = Quot(L[4] + denRatio * R[4], inv);
   const double hR = Enthalpy(g, rr, ur, vr, wr, pr);
   const double aR = SoS(g, rr, pr);
   const double velNormR = (ur * nx + vr * ny) + wr * nz;
-  const double mfR = rr / rr;
+  const double mfR = Div(rr, rr);
   const double d0 = R[0] - L[0], d1 = R[1] - L[1], d2 = R[2] - L[2], d3 = R[3] - L[3],
                d4 = R[4] - L[4];
   const double normVelDiff = (d1 * nx + d2 * ny) + d3 * nz;
@@ -135,8 +190,9 @@ __device__ inline void RoeFlux(const GasT<double> &g, const double L[5], const d
 
   // left moving acoustic wave
   double ws = fabs(velNormR - aR);
-  if (ws < entropyFix) ws = 0.5 * (ws * ws / entropyFix + entropyFix);
-  double wst = (d4 - rr * aR * normVelDiff) / (2.0 * aR * aR);
+  if (ws < entropyFix) ws = 0.5 * (Div(ws * ws, entropyFix) + entropyFix);
+  const Divisor<double> by2a2 = MakeDivisor(2.0 * aR * aR), byA2 = MakeDivisor(aR2);
+  double wst = Quot(d4 - rr * aR * normVelDiff, by2a2);
   double wss = ws * wst;
   D0 = wss * mfR;
   D1 = wss * (ur - aR * nx);
@@ -146,10 +202,10 @@ __device__ inline void RoeFlux(const GasT<double> &g, const double L[5], const d
 
   // entropy wave
   ws = fabs(velNormR);
-  wst = -d4 / aR2;
+  wst = Quot(-d4, byA2);
   wss = ws * wst;
   D0 += wss * mfR + ws * d0;
-  wst = d0 - d4 / aR2;
+  wst = d0 - Quot(d4, byA2);
   wss = ws * wst;
   D1 += wss * ur;
   D2 += wss * vr;
@@ -165,8 +221,8 @@ __device__ inline void RoeFlux(const GasT<double> &g, const double L[5], const d
 
   // right moving acoustic wave
   ws = fabs(velNormR + aR);
-  if (ws < entropyFix) ws = 0.5 * (ws * ws / entropyFix + entropyFix);
-  wst = (d4 + rr * aR * normVelDiff) / (2.0 * aR * aR);
+  if (ws < entropyFix) ws = 0.5 * (Div(ws * ws, entropyFix) + entropyFix);
+  wst = Quot(d4 + rr * aR * normVelDiff, by2a2);
   wss = ws * wst;
   D0 += wss * mfR;
   D1 += wss * (ur + aR * nx);
@@ -288,9 +344,15 @@ __host__ __device__ inline double PowCR(double x, double y) {
 // PowCR(x, 1.5), so both round to the same double, at a few dozen operations
 // instead of the series of PowCR.
 __host__ __device__ __forceinline__ double Pow15CR(double x) {
+#ifdef __HIP_DEVICE_COMPILE__
+  const double s = Sqrt(x);
+  const double e = fma(-s, s, x);
+  const DD S = QuickTwoSum(s, Div(e, 2.0 * s));
+#else
   const double s = sqrt(x);
   const double e = fma(-s, s, x);
   const DD S = QuickTwoSum(s, e / (2.0 * s));
+#endif
   const DD p = DDMulD(S, x);
   return p.hi + p.lo;
 }
@@ -309,21 +371,23 @@ __device__ inline void AusmFlux(const GasT<double> &g, const double L[5], const 
                                 double nx, double ny, double nz, double F[5]) {
   const double velNormL = (L[1] * nx + L[2] * ny) + L[3] * nz;
   const double velNormR = (R[1] * nx + R[2] * ny) + R[3] * nz;
-  const double sosStar = sqrt(SoS(g, L[0], L[4]) * SoS(g, R[0], R[4]));
+  const double sosStar = Sqrt(SoS(g, L[0], L[4]) * SoS(g, R[0], R[4]));
   const double vel = 0.5 * (velNormL + velNormR);
   double sos = sosStar;
-  if (vel < 0.0) sos = sosStar * sosStar / Dmax(velNormR, sosStar);
-  else if (vel > 0.0) sos = sosStar * sosStar / Dmax(velNormL, sosStar);
-  const double ml = velNormL / sos, mr = velNormR / sos;
+  if (vel < 0.0) sos = Div(sosStar * sosStar, Dmax(velNormR, sosStar));
+  else if (vel > 0.0) sos = Div(sosStar * sosStar, Dmax(velNormL, sosStar));
+  const Divisor<double> bySos = MakeDivisor(sos);
+  const double ml = Quot(velNormL, bySos), mr = Quot(velNormR, bySos);
   const double mlp = (ml + 1.0) * (ml + 1.0), mrm = (mr - 1.0) * (mr - 1.0);
   const double mPlusL = fabs(ml) <= 1.0 ? 0.25 * mlp : 0.5 * (ml + fabs(ml));
   const double mMinusR = fabs(mr) <= 1.0 ? -0.25 * mrm : 0.5 * (mr - fabs(mr));
   const double pPlus = fabs(ml) <= 1.0 ? 0.25 * mlp * (2.0 - ml) : 0.5 * (1.0 + Sign(ml));
   const double pMinus = fabs(mr) <= 1.0 ? 0.25 * mrm * (2.0 + mr) : 0.5 * (1.0 - Sign(mr));
   const double ps = pPlus * L[4] + pMinus * R[4];
-  const double w = 1.0 - CubeCR(Dmin(L[4] / R[4], R[4] / L[4]));
-  const double fl = fabs(ml) < 1.0 ? L[4] / ps - 1.0 : 0.0;
-  const double fr = fabs(mr) < 1.0 ? R[4] / ps - 1.0 : 0.0;
+  const double w = 1.0 - CubeCR(Dmin(Div(L[4], R[4]), Div(R[4], L[4])));
+  const Divisor<double> byPs = MakeDivisor(ps);
+  const double fl = fabs(ml) < 1.0 ? Quot(L[4], byPs) - 1.0 : 0.0;
+  const double fr = fabs(mr) < 1.0 ? Quot(R[4], byPs) - 1.0 : 0.0;
   const double mavg = mPlusL + mMinusR;
   const double mPlusLBar = mavg >= 0.0 ? mPlusL + mMinusR * ((1.0 - w) * (1.0 + fr) - fl)
                                        : mPlusL * w * (1.0 + fl);
@@ -342,7 +406,7 @@ __device__ inline void AusmFlux(const GasT<double> &g, const double L[5], const 
 // LimiterVanAlbada / LimiterMinmod (src/limiter.cpp:24-53)
 __device__ __forceinline__ double VanAlbada(double r) {
   const double r2 = r * r;
-  return Dmax(0.0, (r + r2) / (1.0 + r2));
+  return Dmax(0.0, Div(r + r2, 1.0 + r2));
 }
 __device__ __forceinline__ double Minmod(double r) { return Dmax(0.0, Dmin(1.0, r)); }
 
@@ -350,14 +414,14 @@ __device__ __forceinline__ double Minmod(double r) { return Dmax(0.0, Dmin(1.0, 
 template <int LIM>
 __device__ __forceinline__ double Muscl(double u2, double u1, double d1, double kappa,
                                         double dPlus, double dMinus) {
-  const double r = (kEps + (d1 - u1) * dPlus) / (kEps + (u1 - u2) * dMinus);
+  const double r = Div(kEps + (d1 - u1) * dPlus, kEps + (u1 - u2) * dMinus);
   double lim = 1.0, inv = 1.0;
   if (LIM == 1) {
     lim = VanAlbada(r);
-    inv = VanAlbada(1.0 / r);
+    inv = VanAlbada(Div(1.0, r));
   } else if (LIM == 2) {
     lim = Minmod(r);
-    inv = Minmod(1.0 / r);
+    inv = Minmod(Div(1.0, r));
   }
   return u1 + (0.25 * ((u1 - u2) * dMinus)) * ((1.0 - kappa) * lim + (1.0 + kappa) * r * inv);
 }
@@ -404,7 +468,7 @@ __device__ __forceinline__ double LagrangeCoeffN(const double *w, int jj) {
       numer += prod;
       denom *= StencilWN<N>(w, II - RR + ll, II - RR + mm);
     }
-    c += numer / denom;
+    c += Div(numer, denom);
   }
   return c * w[II - RR + jj];
 }
@@ -431,8 +495,8 @@ __device__ __forceinline__ WenoGeom MakeWenoGeom(const double w[5]) {
   }
   // linear weights as the reference forms them (:273-276): lw1 is the
   // weight of the downwind stencil and is applied to the central one
-  G.lw0 = LagrangeCoeffAt<4, 2>(w, 0) / G.c0[0];
-  G.lw1 = LagrangeCoeffAt<4, 2>(w, 4) / G.c2[2];
+  G.lw0 = Div(LagrangeCoeffAt<4, 2>(w, 0), G.c0[0]);
+  G.lw1 = Div(LagrangeCoeffAt<4, 2>(w, 4), G.c2[2]);
   G.lw2 = 1.0 - G.lw0 - G.lw1;
   return G;
 }
@@ -440,14 +504,14 @@ __device__ __forceinline__ WenoGeom MakeWenoGeom(const double w[5]) {
 // Derivative2nd (include/utility.hpp:116-122)
 __device__ __forceinline__ double Deriv2nd(double x0, double x1, double x2, double y0, double y1,
                                            double y2) {
-  const double fwd = (y2 - y1) / (0.5 * (x2 + x1));
-  const double bck = (y1 - y0) / (0.5 * (x1 + x0));
-  return (fwd - bck) / (0.25 * (x2 + x0) + 0.5 * x1);
+  const double fwd = Div(y2 - y1, 0.5 * (x2 + x1));
+  const double bck = Div(y1 - y0, 0.5 * (x1 + x0));
+  return Div(fwd - bck, 0.25 * (x2 + x0) + 0.5 * x1);
 }
 
 // BetaIntegral (include/reconstruction.hpp:157-181); x^3 correctly rounded
 __device__ __forceinline__ double BetaIntAt(double d1, double d2, double dx, double x) {
-  return (d1 * d1 * x + d1 * d2 * x * x + d2 * d2 * CubeCR(x) / 3.0) * dx +
+  return (d1 * d1 * x + d1 * d2 * x * x + Div(d2 * d2 * CubeCR(x), 3.0)) * dx +
          d2 * d2 * x * CubeCR(dx);
 }
 
@@ -458,13 +522,13 @@ __device__ __forceinline__ double WenoBeta(double x0, double x1, double x2, doub
   const double d2 = Deriv2nd(x0, x1, x2, y0, y1, y2);
   double d1, h;
   if (WHICH == 0) {
-    d1 = (y2 - y1) / (0.5 * (x2 + x1)) + 0.5 * x2 * d2;
+    d1 = Div(y2 - y1, 0.5 * (x2 + x1)) + 0.5 * x2 * d2;
     h = x2;
   } else if (WHICH == 1) {
-    d1 = (y2 - y1) / (0.5 * (x2 + x1)) - 0.5 * x1 * d2;
+    d1 = Div(y2 - y1, 0.5 * (x2 + x1)) - 0.5 * x1 * d2;
     h = x1;
   } else {
-    d1 = (y1 - y0) / (0.5 * (x1 + x0)) - 0.5 * x0 * d2;
+    d1 = Div(y1 - y0, 0.5 * (x1 + x0)) - 0.5 * x0 * d2;
     h = x0;
   }
   return BetaIntAt(d1, d2, h, 0.5 * h) - BetaIntAt(d1, d2, h, -0.5 * h);
@@ -483,21 +547,20 @@ __device__ __forceinline__ double Weno(const WenoGeom &G, const double w[5], dou
   double n0, n1, n2;
   if (WENOZ) {
     const double tau5 = fabs(b0 - b2);
-    const double t0 = tau5 / (1.0e-40 + b0), t1 = tau5 / (1.0e-40 + b1),
-                 t2 = tau5 / (1.0e-40 + b2);
+    const double t0 = Div(tau5, 1.0e-40 + b0), t1 = Div(tau5, 1.0e-40 + b1), t2 = Div(tau5, 1.0e-40 + b2);
     n0 = G.lw0 * (1.0 + t0 * t0);
     n1 = G.lw1 * (1.0 + t1 * t1);
     n2 = G.lw2 * (1.0 + t2 * t2);
   } else {
     const double e0 = 1.0e-6 + b0, e1 = 1.0e-6 + b1, e2 = 1.0e-6 + b2;
-    n0 = G.lw0 / (e0 * e0);
-    n1 = G.lw1 / (e1 * e1);
-    n2 = G.lw2 / (e2 * e2);
+    n0 = Div(G.lw0, e0 * e0);
+    n1 = Div(G.lw1, e1 * e1);
+    n2 = Div(G.lw2, e2 * e2);
   }
-  const double sum = n0 + n1 + n2;
-  n0 /= sum;
-  n1 /= sum;
-  n2 /= sum;
+  const Divisor<double> sum = MakeDivisor(n0 + n1 + n2);
+  n0 = Quot(n0, sum);
+  n1 = Quot(n1, sum);
+  n2 = Quot(n2, sum);
   return n0 * s0 + n1 * s1 + n2 * s2;
 }
 
@@ -506,8 +569,8 @@ __device__ __forceinline__ double InvCellSpecRad(const GasT<double> &g, double r
                                                  double v, double w, double p, double4 aL,
                                                  double4 aR) {
   const double sx = 0.5 * (aL.x + aR.x), sy = 0.5 * (aL.y + aR.y), sz = 0.5 * (aL.z + aR.z);
-  const double m = sqrt((sx * sx + sy * sy) + sz * sz);
-  const double nx = sx / m, ny = sy / m, nz = sz / m;
+  const Divisor<double> m = MakeDivisor(Sqrt((sx * sx + sy * sy) + sz * sz));
+  const double nx = Quot(sx, m), ny = Quot(sy, m), nz = Quot(sz, m);
   const double fMag = 0.5 * (aL.w + aR.w);
   return (fabs((u * nx + v * ny) + w * nz) + SoS(g, rho, p)) * fMag;
 }
@@ -534,53 +597,6 @@ __device__ __forceinline__ void RoeOffDiag(const GasT<double> &g, const double W
   }
 }
 
-// ---------------------------------------------------------------------------
-// Several quotients by one divisor: the reciprocal y is refined once by two
-// Newton steps (one in FP32), then each quotient takes one product and one
-// (two) residual corrections (Markstein, "Computation of elementary functions
-// on the IBM RISC System/6000 processor", 1990), and div_fixup settles signs
-// of zeros, infinities and NaN.  These are the operations of the compiler's
-// division without its scaling of operands near the ends of the exponent
-// range, so a quotient is that of operator/ bit for bit while divisor,
-// numerator residual (numerator 2^-53) and quotient are normal numbers; below
-// that it may be off by a few units of the smallest denormal.  A division by
-// operator/ is eleven operations, four of them in a row through one condition
-// register; four by one divisor are 17 here.
-template <typename T>
-struct Divisor {
-  T d, y;
-};
-__device__ __forceinline__ Divisor<double> MakeDivisor(double d) {
-  double y = __builtin_amdgcn_rcp(d);
-  y = fma(y, fma(-d, y, 1.0), y);
-  y = fma(y, fma(-d, y, 1.0), y);
-  return {d, y};
-}
-__device__ __forceinline__ Divisor<float> MakeDivisor(float d) {
-  const float y = __builtin_amdgcn_rcpf(d);
-  return {d, fmaf(fmaf(-d, y, 1.0f), y, y)};
-}
-__device__ __forceinline__ double Quot(double n, const Divisor<double> &v) {
-  const double q = n * v.y;
-  return __builtin_amdgcn_div_fixup(fma(fma(-v.d, q, n), v.y, q), v.d, n);
-}
-__device__ __forceinline__ float Quot(float n, const Divisor<float> &v) {
-  float q = n * v.y;
-  q = fmaf(fmaf(-v.d, q, n), v.y, q);
-  return __builtin_amdgcn_div_fixupf(fmaf(fmaf(-v.d, q, n), v.y, q), v.d, n);
-}
-// sqrt for x = 0 or x >= 2^-760: the Goldschmidt iteration of sqrt() without
-// its scaling of small arguments (inf and NaN pass through)
-__device__ __forceinline__ double SqrtInRange(double x) {
-  const double y = __builtin_amdgcn_rsq(x);
-  double g = x * y, h = 0.5 * y;
-  const double r = fma(-h, g, 0.5);
-  g = fma(g, r, g);
-  h = fma(h, r, h);
-  g = fma(fma(-g, g, x), h, g);
-  g = fma(fma(-g, g, x), h, g);
-  return (x == 0.0 || __builtin_isinf(x)) ? x : g;
-}
 // ConsToPrim and the Enthalpy of its result in one, with the same operations
 // on the same values; `byCvs` is the divisor cvs
 __device__ __forceinline__ void ConsToPrimH(const GasT<double> &g, const Divisor<double> &byCvs, const double U[5],
@@ -648,7 +664,7 @@ __device__ __forceinline__ StateChange<T> ChangeOf(const GasT<T> &g, const T W[5
 // the base state's part: rho E + p
 template <typename T>
 __device__ __forceinline__ T EnergyPlusP(const GasT<T> &g, const T W[5]) {
-  const T rE = W[4] / (g.gamma - T(1)) + T(0.5) * W[0] * ((W[1] * W[1] + W[2] * W[2]) + W[3] * W[3]);
+  const T rE = Div(W[4], g.gamma - T(1)) + T(0.5) * W[0] * ((W[1] * W[1] + W[2] * W[2]) + W[3] * W[3]);
   return rE + W[4];
 }
 // dF through a face of unit normal n; vn = v.n of the base state, rEp its
@@ -815,7 +831,7 @@ __device__ __forceinline__ bool GJInverse5(T m[25], T I[25]) {
       }
 #pragma unroll
     for (int i = 0; i < r; ++i) {
-      const T factor = m[r * 5 + i] / m[i * 5 + i];
+      const T factor = Div(m[r * 5 + i], m[i * 5 + i]);
 #pragma unroll
       for (int c = 0; c < 5; ++c) {
         m[r * 5 + c] = m[r * 5 + c] - factor * m[i * 5 + c];
@@ -823,7 +839,7 @@ __device__ __forceinline__ bool GJInverse5(T m[25], T I[25]) {
       }
     }
     if (m[r * 5 + r] == T(0)) ok = false;
-    const T nf = T(1) / m[r * 5 + r];
+    const T nf = Div(T(1), m[r * 5 + r]);
 #pragma unroll
     for (int c = r; c < 5; ++c) m[r * 5 + c] *= nf;
 #pragma unroll

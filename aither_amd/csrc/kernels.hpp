@@ -126,19 +126,19 @@ struct Params {
 // idealGas::Temperature (src/eos.cpp:54-60)
 __device__ __forceinline__ double TempOf(const GasT<double> &g, double rho, double p) {
   const double rhoR = 0.0 + rho * g.R;
-  return p / rhoR;
+  return Div(p, rhoR);
 }
 // sutherland::SpeciesViscosity / SpeciesConductivity (src/transport.cpp:
 // 97-117), nondimensional; t^1.5 correctly rounded
 __device__ __forceinline__ double SutherlandMu(const ViscParams &v, double t) {
   const double temp = t * v.tRef;
-  const double mu = (v.c1 * Pow15CR(temp)) / (temp + v.s1);
-  return mu / v.muRef;
+  const double mu = Div(v.c1 * Pow15CR(temp), temp + v.s1);
+  return Div(mu, v.muRef);
 }
 __device__ __forceinline__ double SutherlandK(const ViscParams &v, double t) {
   const double temp = t * v.tRef;
-  const double k = (v.c2 * Pow15CR(temp)) / (temp + v.s2);
-  return k / v.kNonDim;
+  const double k = Div(v.c2 * Pow15CR(temp), temp + v.s2);
+  return Div(k, v.kNonDim);
 }
 // max(4/(3 rho), gamma/rho) and NondimScaling (mu / Pr + mut / Prt), mut = 0
 // (include/spectralRadius.hpp:93-151)
@@ -146,19 +146,19 @@ template <typename T>
 __device__ __forceinline__ T ViscFaceSR(const GasT<T> &g, const T W[5], T mag, T dist, T mu,
                                         const ViscParams &v) {
   const T rho = T(0) + W[0];
-  const T a = T(4) / (T(3) * rho), bq = g.gamma / rho;
+  const T a = Div(T(4), T(3) * rho), bq = Div(g.gamma, rho);
   const T maxTerm = a < bq ? bq : a;
-  const T viscTerm = T(v.vscale) * (mu / T(v.prandtl) + T(0) / T(0.9));
-  return mag / dist * maxTerm * viscTerm;
+  const T viscTerm = T(v.vscale) * (Div(mu, T(v.prandtl)) + T(0) / T(0.9));
+  return Div(mag, dist) * maxTerm * viscTerm;
 }
 __device__ __forceinline__ double ViscCellSR(const GasT<double> &g, const double W[5], double magL,
                                              double magR, double vol, double mu, const ViscParams &v) {
   const double fMag = 0.5 * (magL + magR);
   const double rho = 0.0 + W[0];
-  const double a = 4.0 / (3.0 * rho), bq = g.gamma / rho;
+  const double a = Div(4.0, 3.0 * rho), bq = Div(g.gamma, rho);
   const double maxTerm = a < bq ? bq : a;
-  const double viscTerm = v.vscale * (mu / v.prandtl + 0.0 / 0.9);
-  return maxTerm * viscTerm * fMag * fMag / vol;
+  const double viscTerm = v.vscale * (Div(mu, v.prandtl) + 0.0 / 0.9);
+  return Div(maxTerm * viscTerm * fMag * fMag, vol);
 }
 
 struct BcStateDev {
@@ -419,8 +419,9 @@ __device__ __forceinline__ void FaceStates(const DevBlock &b, double kappa, int 
   } else {
     const double *cw = b.cw + d * b.npad;
     const double wm2 = cw[c0 - 2 * s], wm1 = cw[c0 - s], w0 = cw[c0], wp1 = cw[c0 + s];
-    const double dPL = (wm1 + wm1) / (wm1 + w0), dML = (wm1 + wm1) / (wm1 + wm2);
-    const double dPR = (w0 + w0) / (w0 + wm1), dMR = (w0 + w0) / (w0 + wp1);
+    const Divisor<double> byC = MakeDivisor(wm1 + w0);  // the sum is that of w0 + wm1
+    const double dPL = Quot(wm1 + wm1, byC), dML = Div(wm1 + wm1, wm1 + wm2);
+    const double dPR = Quot(w0 + w0, byC), dMR = Div(w0 + w0, w0 + wp1);
 #pragma unroll
     for (int e = 0; e < 5; ++e) {
       const double *We = b.W + e * b.npad;
@@ -462,14 +463,14 @@ __device__ __forceinline__ void FaceSide(const DevBlock &b, double kappa, int d,
     const double *cw = b.cw + d * b.npad;
     const double wm2 = cw[c0 - 2 * s], wm1 = cw[c0 - s], w0 = cw[c0], wp1 = cw[c0 + s];
     if (!upper) {
-      const double dPL = (wm1 + wm1) / (wm1 + w0), dML = (wm1 + wm1) / (wm1 + wm2);
+      const double dPL = Div(wm1 + wm1, wm1 + w0), dML = Div(wm1 + wm1, wm1 + wm2);
 #pragma unroll
       for (int e = 0; e < 5; ++e) {
         const double *We = b.W + e * b.npad;
         Wout[e] = Muscl<LIM>(We[c0 - 2 * s], We[c0 - s], We[c0], kappa, dPL, dML);
       }
     } else {
-      const double dPR = (w0 + w0) / (w0 + wm1), dMR = (w0 + w0) / (w0 + wp1);
+      const double dPR = Div(w0 + w0, w0 + wm1), dMR = Div(w0 + w0, w0 + wp1);
 #pragma unroll
       for (int e = 0; e < 5; ++e) {
         const double *We = b.W + e * b.npad;
@@ -497,15 +498,15 @@ __device__ __forceinline__ void FaceFlux(const DevBlock &b, const GasT<double> &
 __device__ __forceinline__ void CellTail(const DevBlock &b, const Params &P, long p, double vol, double sr,
                                          double Ad) {
   b.sr[p] = sr;
-  const double dt = P.dtFixed > 0.0 ? P.dtFixed : (*b.cfl) * (vol / Dmax(sr, 0.0));
+  const double dt = P.dtFixed > 0.0 ? P.dtFixed : (*b.cfl) * Div(vol, Dmax(sr, 0.0));
   b.dt[p] = dt;
   if (P.implicit && !P.block) {
-    double dvt = (vol * (1.0 + P.zeta)) / (dt * P.theta);
-    if (P.dualCFL > 0.0) dvt += Dmax(sr, 0.0) / P.dualCFL;
+    double dvt = Div(vol * (1.0 + P.zeta), dt * P.theta);
+    if (P.dualCFL > 0.0) dvt += Div(Dmax(sr, 0.0), P.dualCFL);
     double A = Ad * P.relax;
     A += dvt;
     b.A[p] = A;
-    const double ainv = 1.0 / A;
+    const double ainv = Div(1.0, A);
     if (!P.fp32) {
       if (b.Ainv) b.Ainv[p] = ainv;
     } else if (b.Ainv32) {
@@ -811,7 +812,7 @@ __device__ __forceinline__ void FaceGrads(const DevBlock &b, const C &cv, int d,
       }
     }
   }
-  const double invVol = 1.0 / vol;
+  const double invVol = Div(1.0, vol);
 #pragma unroll
   for (int r = 0; r < 3; ++r) {
 #pragma unroll
@@ -944,9 +945,10 @@ __device__ __forceinline__ void TSLJacobian(const GasT<double> &g, const ViscPar
   double J[25];
 #pragma unroll
   for (int q = 0; q < 25; ++q) J[q] = 0.0;
-  J[0] = (0.0 + 0.0) * (1.0 - W[0] / rho) / mr;
-  J[20] = -(k + kt) * t / mr + J[0] * (g.cps * t);
-  const double sh = fac * 0.5 * dist / (mu + mut);
+  const Divisor<double> byMr = MakeDivisor(mr);
+  J[0] = Quot((0.0 + 0.0) * (1.0 - Div(W[0], rho)), byMr);
+  J[20] = Quot(-(k + kt) * t, byMr) + J[0] * (g.cps * t);
+  const double sh = Div(fac * 0.5 * dist, mu + mut);
   J[6] = third * nx * nx + 1.0;
   J[11] = third * nx * ny;
   J[16] = third * nx * nz;
@@ -959,13 +961,13 @@ __device__ __forceinline__ void TSLJacobian(const GasT<double> &g, const ViscPar
   J[13] = third * nz * ny;
   J[18] = third * nz * nz + 1.0;
   J[23] = sh * tau[2] + third * nz * vn + w;
-  J[24] = (k + kt) / mr;
-  const double f = a.w * (mu + mut) / dist;
+  J[24] = Quot(k + kt, byMr);
+  const double f = Div(a.w * (mu + mut), dist);
 #pragma unroll
   for (int q = 0; q < 25; ++q) J[q] *= f;
   // DelprimitiveDelConservative: its nonzero entries (row-major index)
   const double gm1 = g.gamma - 1.0;
-  const double invRho = 1.0 / rho;
+  const double invRho = Div(1.0, rho);
   const double p5 = -invRho * u, p10 = -invRho * v, p15 = -invRho * w;
   const double p20 = 0.5 * gm1 * ((u * u + v * v) + w * w);
   const double p6 = invRho, p12 = invRho, p18 = invRho;
@@ -1092,9 +1094,10 @@ __device__ __forceinline__ void RhsFrom(const Params &P, const double W[5], doub
   const GasT<double> g = Cast<double>(P.gas);
   double U[5];
   PrimToCons(g, W, U);
-  const double coeff = (vol * (1.0 + P.zeta)) / (dt * P.theta);
+  const Divisor<double> byDt = MakeDivisor(dt * P.theta);
+  const double coeff = Quot(vol * (1.0 + P.zeta), byDt);
   const double thetaInv = 1.0 / P.theta;
-  const double c2 = P.multilevel ? (vol * P.zeta) / (dt * P.theta) : 0.0;
+  const double c2 = P.multilevel ? Quot(vol * P.zeta, byDt) : 0.0;
 #pragma unroll
   for (int e = 0; e < 5; ++e) {
     const double nm1 = P.multilevel ? c2 * (cN[e] - cNm1[e]) : 0.0;
@@ -1208,8 +1211,8 @@ __global__ void __launch_bounds__(128) KBlockDiag(BlockMap M, Params P) {
     for (int q = 0; q < 9; ++q) b.vgrad[q * b.npad + c] = G[q];
   }
   const double sr = b.sr[p];
-  double dvt = (b.vol[p] * (1.0 + P.zeta)) / (b.dt[p] * P.theta);
-  if (P.dualCFL > 0.0) dvt += Dmax(sr, 0.0) / P.dualCFL;
+  double dvt = Div(b.vol[p] * (1.0 + P.zeta), b.dt[p] * P.theta);
+  if (P.dualCFL > 0.0) dvt += Div(Dmax(sr, 0.0), P.dualCFL);
 #pragma unroll
   for (int q = 0; q < 5; ++q) D[q * 6] *= P.relax;
 #pragma unroll
@@ -1653,7 +1656,7 @@ __global__ void __launch_bounds__(kRedThreads) KUpdate(BlockMap M, Params P, Par
     if (P.explicitEuler) {
       double U[5];
       PrimToCons(g, W, U);
-      const double f = b.dt[p] / b.vol[p];
+      const double f = Div(b.dt[p], b.vol[p]);
 #pragma unroll
       for (int e = 0; e < 5; ++e) U[e] -= f * R[e];
       ConsToPrim(g, U, Wn);
