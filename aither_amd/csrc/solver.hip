@@ -1612,25 +1612,27 @@ int ath_set_matrix_residual(ath_ctx *c, int on) {
   return ATH_OK;
 }
 
+// the physical cells' state of a block to or from a host array (AoS), through
+// the block's scratch xold, which every relax writes before it reads
+static int ExchangeState(ath_ctx *c, const ath::DevBlock &d, double *host, bool toHost) {
+  const size_t bytes = 5 * (size_t)d.ncell * sizeof(double);
+  if (toHost) {
+    hipLaunchKernelGGL(ath::KPackState, dim3(Grid(d.ncell)), dim3(kBlk), 0, c->stream, d, 0);
+    if (int r = CheckLaunch()) return r;
+    HIP_OK(hipMemcpyAsync(host, d.xold, bytes, hipMemcpyDeviceToHost, c->stream));
+  } else {
+    HIP_OK(hipMemcpyAsync(d.xold, host, bytes, hipMemcpyHostToDevice, c->stream));
+    hipLaunchKernelGGL(ath::KPackState, dim3(Grid(d.ncell)), dim3(kBlk), 0, c->stream, d, 1);
+    if (int r = CheckLaunch()) return r;
+  }
+  HIP_OK(hipStreamSynchronize(c->stream));
+  return ATH_OK;
+}
+
 static int CopyState(ath_ctx *c, int b, double *host, bool toHost) {
   if (!c || !host || b < 0 || b >= (int)c->blk.size()) return Fail(ATH_ERR_ARG, "bad argument");
   HIP_OK(hipSetDevice(c->device));
-  HIP_OK(hipStreamSynchronize(c->stream));
-  const auto &d = c->blk[b].d;
-  std::vector<double> W(5 * (size_t)d.npad);
-  HIP_OK(hipMemcpy(W.data(), d.W, W.size() * sizeof(double), hipMemcpyDeviceToHost));
-  for (int k = 0; k < d.nk; ++k)
-    for (int j = 0; j < d.nj; ++j)
-      for (int i = 0; i < d.ni; ++i) {
-        const long p = i + (long)j * d.ni + (long)k * d.ni * d.nj;
-        const long q = (i + d.g) + (long)(j + d.g) * d.NI + (long)(k + d.g) * d.NI * d.NJ;
-        for (int e = 0; e < 5; ++e) {
-          if (toHost) host[5 * p + e] = W[e * d.npad + q];
-          else W[e * d.npad + q] = host[5 * p + e];
-        }
-      }
-  if (!toHost) HIP_OK(hipMemcpy(d.W, W.data(), W.size() * sizeof(double), hipMemcpyHostToDevice));
-  return ATH_OK;
+  return ExchangeState(c, c->blk[b].d, host, toHost);
 }
 
 int ath_get_state(ath_ctx *c, int b, double *prim) { return CopyState(c, b, prim, true); }
@@ -2627,22 +2629,7 @@ static int SlotState(ath_server *s, int slot, int b, double *prim, bool toHost) 
   if (b < 0 || b >= (int)cr->blocks.size()) return Fail(ATH_ERR_ARG, "bad block index");
   ath_ctx *c = s->c.get();
   HIP_OK(hipSetDevice(c->device));
-  HIP_OK(hipStreamSynchronize(c->stream));
-  const auto &d = cr->blocks[b].d;
-  std::vector<double> W(5 * (size_t)d.npad);
-  HIP_OK(hipMemcpy(W.data(), d.W, W.size() * sizeof(double), hipMemcpyDeviceToHost));
-  for (int k = 0; k < d.nk; ++k)
-    for (int j = 0; j < d.nj; ++j)
-      for (int i = 0; i < d.ni; ++i) {
-        const long p = i + (long)j * d.ni + (long)k * d.ni * d.nj;
-        const long q = (i + d.g) + (long)(j + d.g) * d.NI + (long)(k + d.g) * d.NI * d.NJ;
-        for (int e = 0; e < 5; ++e) {
-          if (toHost) prim[5 * p + e] = W[e * d.npad + q];
-          else W[e * d.npad + q] = prim[5 * p + e];
-        }
-      }
-  if (!toHost) HIP_OK(hipMemcpy(d.W, W.data(), W.size() * sizeof(double), hipMemcpyHostToDevice));
-  return ATH_OK;
+  return ExchangeState(c, cr->blocks[b].d, prim, toHost);
 }
 
 int ath_slot_block_dims(ath_server *s, int slot, int block, int *ni, int *nj, int *nk) {
