@@ -28,6 +28,11 @@ __host__ __device__ inline ATH_GLOBAL T *Dev(T *p) {
   return (ATH_GLOBAL T *)p;
 }
 
+// Records of the pencil sweeps: pencils of kPW x kPW columns, kPenLanes lanes
+// a record (one hyperplane step of one pencil)
+constexpr int kPW = 8;
+constexpr int kPenLanes = kPW * kPW;
+
 struct DevBlock {
   int ni, nj, nk, g;
   int NI, NJ;
@@ -45,22 +50,22 @@ struct DevBlock {
   float ATH_GLOBAL *x32;            // 5 * ncell (FP32 operator)
   double ATH_GLOBAL *xold;          // 5 * ncell, DP-LUR Jacobi copy
   float ATH_GLOBAL *xold32;
-  double ATH_GLOBAL *rhs;           // 5 * ncell, right-hand side of the row-parallel block sweep
-  // scalar LU-SGS: the pencil sweep's inputs in the order the sweep takes
-  // them.  Pencils run along axis pl, pa x pb of them along the axes pl + 1
-  // and pl + 2 (mod 3), pns steps stored for each; record (pencil, step) holds
-  // its values 64 lanes at a time (KPencilFaces, KPencilPrep, KPencilOther)
+  // LU-SGS: the pencil sweep's inputs in the order the sweep takes them.
+  // Pencils run along axis pl, pa x pb of them along the axes pl + 1 and
+  // pl + 2 (mod 3), pns steps stored for each; record (pencil, step) holds its
+  // values 64 lanes at a time (KPencilFaces, KPencilPrep, KBlockDiag,
+  // KPencilOther).  pns = 0 and null pointers without it.
   int pl, pa, pb, pns;
   double ATH_GLOBAL *skF;  // face data, both sides
-  double ATH_GLOBAL *skS;  // state, right-hand side, D^-1 (and viscosity)
+  double ATH_GLOBAL *skS;  // scalar: state, right-hand side, D^-1 (and viscosity);
+                           // block: state, right-hand side (viscosity, conductivity, velocity gradient)
   double ATH_GLOBAL *skX;  // forward du (operator precision)
   double ATH_GLOBAL *skO;  // other-side sums of a full sweep (operator precision), null with one sweep
   // block matrix solvers: main diagonal after AddDiagonalTerms, 25 * ncell,
-  // entry (r, c) of cell p at (5 r + c) ncell + p; its inverse in the
-  // tile-blocked layout of TileBase (the sweep's 8 x 8 x 4 tiles: one tile's
-  // values of one entry are 256 consecutive doubles, so a wavefront reads
-  // whole cache lines no other tile shares).  The off-diagonal blocks are
-  // formed where they are used (NeighbourBlock).
+  // entry (r, c) of cell p at (5 r + c) ncell + p; its inverse in the layout
+  // of InverseBase (LU-SGS: the pencil sweep's records; DP-LUR: 8 x 8 x 4
+  // tiles, one tile's values of one entry 256 consecutive doubles).  The
+  // off-diagonal blocks are formed where they are used (NeighbourBlock).
   double ATH_GLOBAL *Ab, *Abi;
   float ATH_GLOBAL *Abi32;       // FP32 operator: Abi rounded to float, same layout
   int tni, tnj, tnk;  // tile grid of the layout
@@ -116,8 +121,9 @@ struct Params {
   int block;  // matrixSolver blusgs / bdplur: 5x5 main diagonal and off-diagonals
   int fp32;   // the scalar implicit operator runs in FP32: the residual stage writes Ainv32, else Ainv
   int roeJac; // inviscidFluxJacobian approximateRoe: the off-diagonals are Roe flux changes (FP64)
-  int rhsOnce; // the relax forms the right-hand side once, into rhs (the row-parallel block sweep reads it)
-  int rhsInDiag; // the viscous block diagonal forms that right-hand side and du = 0 (the relax does not)
+  int rhsOnce; // the relax forms the right-hand side once, in sweep order (the block pencil sweep reads it)
+  int rhsInDiag; // the block diagonal forms that right-hand side (the relax does not)
+  int copyState; // the relax refreshes the state in sweep order (it was set since the residual stage)
 };
 
 // ---------------------------------------------------------------------------
@@ -191,10 +197,54 @@ __device__ __forceinline__ long BtSlot(const DevBlock &b, int d, int upper, int 
   if (d == 1) return 2 * sI + upper * sJ + k + (long)b.nk * i;
   return 2 * sI + 2 * sJ + upper * sK + i + (long)b.ni * j;
 }
-// tile-blocked layout of the block solvers' per-cell 5x5 blocks: entry q of
-// cell (i, j, k) at TileBase(b, i, j, k) + 256 q
-__device__ __forceinline__ long TileBase(const DevBlock &b, int i, int j, int k) {
+// record and lane of cell (i, j, k) in the pencil sweep's arrays
+__device__ __forceinline__ long PencilRecord(const DevBlock &b, int i, int j, int k, int &lane) {
+  const int ca = b.pl == 0 ? j : (b.pl == 1 ? k : i), cb = b.pl == 0 ? k : (b.pl == 1 ? i : j),
+            cc = b.pl == 0 ? i : (b.pl == 1 ? j : k);
+  const int la = ca % kPW, lb = cb % kPW;
+  lane = la + kPW * lb;
+  return (long)(ca / kPW + b.pa * (cb / kPW)) * b.pns + la + lb + cc;
+}
+// Values in LDS go 16 bytes a lane: a 16-byte read takes 13 cycles of the
+// LDS pipe for a wave, two 8-byte reads 33.  Value q of a lane's record is
+// v[q % kVecN] of its vector q / kVecN.
+template <typename T>
+struct alignas(16) LdsVec {
+  T v[16 / sizeof(T)];
+};
+template <typename T>
+constexpr int kVecN = 16 / (int)sizeof(T);
+template <typename T>
+constexpr int Vecs(int n) { return (n + kVecN<T> - 1) / kVecN<T>; }
+
+// n consecutive values written as whole vectors, zeros behind them
+template <typename T, int N>
+__device__ __forceinline__ void PutVecs(T *p, const T *v) {
+#pragma unroll
+  for (int q = 0; q < Vecs<T>(N); ++q) {
+    LdsVec<T> w;
+#pragma unroll
+    for (int r = 0; r < kVecN<T>; ++r) w.v[r] = q * kVecN<T> + r < N ? v[q * kVecN<T> + r] : T(0);
+    ((LdsVec<T> *)p)[q] = w;
+  }
+}
+// layout of the block solvers' inverse diagonal: entry q of cell (i, j, k) at
+// InverseBase + q * stride.  In the pencil sweep's records a cell's 25 values
+// are consecutive, padded to whole 16-byte vectors (an odd number of them, so
+// that a record copied to LDS is read without bank conflicts).
+template <typename T>
+constexpr int kInv = Vecs<T>(25) * kVecN<T>;
+static_assert(Vecs<float>(25) % 2 == 1 && Vecs<double>(25) % 2 == 1, "bank spread of a record in LDS");
+template <typename T>
+__device__ __forceinline__ long InverseBase(const DevBlock &b, int i, int j, int k, int &stride) {
+  if (b.pns) {
+    int lane;
+    const long rec = PencilRecord(b, i, j, k, lane);
+    stride = 1;
+    return (rec * kPenLanes + lane) * kInv<T>;
+  }
   const long tile = (long)(i >> 3) + (long)b.tni * ((j >> 3) + (long)b.tnj * (k >> 2));
+  stride = 256;
   return tile * (25 * 256) + ((i & 7) + 8 * ((j & 7) + 8 * (k & 3)));
 }
 __device__ __forceinline__ void Map3(int dir, int d3, int d1, int d2, int &i, int &j, int &k) {
@@ -1120,13 +1170,53 @@ __device__ __forceinline__ void Rhs(const DevBlock &b, const Params &P, long p, 
   RhsFrom(P, W, b.vol[p], b.dt[p], R, cN, cNm1, out);
 }
 
+// values of a block solver's record: state, right-hand side, and with the
+// viscous terms viscosity, conductivity and velocity gradient
+__host__ __device__ constexpr int BlockRecord(bool viscous) { return viscous ? 21 : 10; }
+
+// The block diagonal's tiles (extents in i, j, k for pencils along each axis)
+// and a tile's cells by their place in the records: pencil, step, lane.  Each
+// record takes a cell's values 512 bytes apart, its lanes from as many rows, so
+// stores straight from the cells are single words: KBlockDiag on 1.03M cells
+// 800 us.  Through LDS in the records' order they are runs of up to eight lanes:
+// 534 us (8 x 8 x 4 tiles 554, 16 x 8 x 1 590, a wave's 8 x 8 cells 803),
+// against 395 us without any records, which the sweep's two passes (508 -> 353
+// us) and the initialisation gone from the relax pay for.
+constexpr int kDiagTile[3][3] = {{32, 8, 1}, {8, 8, 4}, {32, 1, 8}};
+struct TileOrder {
+  unsigned char cell[3][256];
+};
+constexpr TileOrder MakeTileOrder() {
+  TileOrder o{};
+  for (int l = 0; l < 3; ++l) {
+    const int ti = kDiagTile[l][0], tj = kDiagTile[l][1], tk = kDiagTile[l][2];
+    int n = 0;
+    for (int pen = 0; pen < (l == 0 ? 1 : ti / kPW); ++pen)  // pencils lie side by side along i
+      for (int key = 0; key < 64 * kPenLanes; ++key) {       // step * kPenLanes + lane
+        const int la = key % kPW, lb = key / kPW % kPW, cc = key / kPenLanes - la - lb;
+        const int i = l == 0 ? cc : kPW * pen + (l == 1 ? lb : la), j = l == 0 ? la : (l == 1 ? cc : lb),
+                  k = l == 0 ? lb : (l == 1 ? la : cc);
+        if (cc >= 0 && i < ti && j < tj && k < tk) o.cell[l][n++] = (unsigned char)(i + ti * (j + tj * k));
+      }
+  }
+  return o;
+}
+__constant__ const TileOrder kTileOrder = MakeTileOrder();
+// cell `t` of tile U
+__device__ __forceinline__ void DiagCell(const DevBlock &b, const Unit &U, int t, int &i, int &j, int &k) {
+  const int ti = b.pl == 1 ? 8 : 32, tj = b.pl == 2 ? 1 : 8, tk = b.pl == 0 ? 1 : (b.pl == 1 ? 4 : 8);
+  i = U.x * ti + t % ti;
+  j = U.y * tj + t / ti % tj;
+  k = U.z * tk + t / (ti * tj);
+}
+
 // Block main diagonal (src/procBlock.cpp:449-486, 588-625, 726-763):
 // every face adds the Rusanov Jacobian of its lower state to its lower cell
 // and subtracts that of its upper state from its upper cell, faces in i, j, k
 // order, so a cell sees -J(face i-) +J(face i+) -J(j-) +J(j+) -J(k-) +J(k+)
 // from a zero matrix.  Then AddDiagonalTerms (src/linearSolver.cpp:146-171)
 // and the Gauss-Jordan inverse (src/linearSolver.cpp:173-184).  One thread per
-// cell, after the residual kernels have written sr and dt.  A zero pivot sets
+// cell of a tile, after the residual kernels have written sr and dt.  A zero pivot sets
 // bit 4 of `flag`.
 //
 // MODE 0: the inviscid sum, then AddDiagonalTerms and the inverse.
@@ -1140,104 +1230,150 @@ __device__ __forceinline__ void Rhs(const DevBlock &b, const Params &P, long p, 
 // faces' thin-shear-layer Jacobians, the cell as upper cell adding
 // (src/procBlock.cpp:1467-1474) and as lower cell subtracting (:1416-1424),
 // stores the cell velocity gradient, a sixth of each face's in the same order
-// (:1396-1414, 1427-1436), and finishes.
+// (:1396-1414, 1427-1436), and finishes.  Bound by latency: two waves a SIMD (its
+// registers), VALU 45 % busy, 1.75 GB at 3.3 TB/s on the 1.03M-cell channel.
 template <int RECON, int LIM, int MODE>
-__global__ void __launch_bounds__(128) KBlockDiag(BlockMap M, Params P) {
+__global__ void __launch_bounds__(256, MODE == 3 && RECON < 2 ? 2 : 1) KBlockDiag(BlockMap M, Params P) {
 #pragma clang fp contract(off)
   const Unit U = MapUnit(M);
   const DevBlock &b = *U.b;
-  const long p = (long)U.local * blockDim.x + threadIdx.x;
-  if (p >= b.ncell) return;
-  const bool parked = MODE >= 1 && b.invPark && b.invPark[p];
+  const int tid = threadIdx.x;
+  const bool tiled = MODE != 1 && b.pns;
+  long p = (long)U.local * blockDim.x + tid;
+  int i, j, k;
+  if (tiled) {
+    DiagCell(b, U, tid, i, j, k);
+    p = i + (long)b.ni * (j + (long)b.nj * k);
+  } else {
+    i = (int)(p % b.ni);
+    j = (int)((p / b.ni) % b.nj);
+    k = (int)(p / ((long)b.ni * b.nj));
+  }
+  const bool cell = i < b.ni && j < b.nj && k < b.nk;
+  if (!tiled && !cell) return;
+  const long c = PadIdx(b, i, j, k);
+  const bool parked = MODE >= 1 && cell && b.invPark && b.invPark[p];
   if (MODE == 1 && !parked) return;
-  const int i = (int)(p % b.ni), j = (int)((p / b.ni) % b.nj), k = (int)(p / ((long)b.ni * b.nj));
-  const GasT<double> g = Cast<double>(P.gas);
-  double D[25];
+  if (cell) {
+    const GasT<double> g = Cast<double>(P.gas);
+    double D[25];
 #pragma unroll
-  for (int q = 0; q < 25; ++q) D[q] = MODE >= 2 && parked ? b.Ab[q * b.ncell + p] : 0.0;
-  if (!(MODE >= 2 && parked)) {
+    for (int q = 0; q < 25; ++q) D[q] = MODE >= 2 && parked ? b.Ab[q * b.ncell + p] : 0.0;
+    if (!(MODE >= 2 && parked)) {
 #pragma unroll
-    for (int d = 0; d < 3; ++d) {
-      // the cell is the upper cell of its lower face (upper state WR) and the
-      // lower cell of its upper face (lower state WL): one side of each
-      double Wf[5], J[25];
-      FaceSide<RECON, LIM>(b, P.kappa, d, i, j, k, true, Wf);
-      double4 a = b.fa[d][FaceIdx(b, d, i, j, k)];
-      RusanovJacobian<double>(g, Wf, a.x, a.y, a.z, a.w, false, J);
+      for (int d = 0; d < 3; ++d) {
+        // the cell is the upper cell of its lower face (upper state WR) and the
+        // lower cell of its upper face (lower state WL): one side of each
+        double Wf[5], J[25];
+        FaceSide<RECON, LIM>(b, P.kappa, d, i, j, k, true, Wf);
+        double4 a = b.fa[d][FaceIdx(b, d, i, j, k)];
+        RusanovJacobian<double>(g, Wf, a.x, a.y, a.z, a.w, false, J);
 #pragma unroll
-      for (int q = 0; q < 25; ++q) D[q] = D[q] - J[q];
-      const int ui = i + (d == 0), uj = j + (d == 1), uk = k + (d == 2);
-      FaceSide<RECON, LIM>(b, P.kappa, d, ui, uj, uk, false, Wf);
-      a = b.fa[d][FaceIdx(b, d, ui, uj, uk)];
-      RusanovJacobian<double>(g, Wf, a.x, a.y, a.z, a.w, true, J);
+        for (int q = 0; q < 25; ++q) D[q] = D[q] - J[q];
+        const int ui = i + (d == 0), uj = j + (d == 1), uk = k + (d == 2);
+        FaceSide<RECON, LIM>(b, P.kappa, d, ui, uj, uk, false, Wf);
+        a = b.fa[d][FaceIdx(b, d, ui, uj, uk)];
+        RusanovJacobian<double>(g, Wf, a.x, a.y, a.z, a.w, true, J);
 #pragma unroll
-      for (int q = 0; q < 25; ++q) D[q] = D[q] + J[q];
-    }
-  }
-  if (MODE == 1) {
-#pragma unroll
-    for (int q = 0; q < 25; ++q) b.Ab[q * b.ncell + p] = D[q];
-    return;
-  }
-  if (MODE >= 2) {
-    constexpr double sixth = 1.0 / 6.0;
-    double G[9];
-#pragma unroll
-    for (int q = 0; q < 9; ++q) G[q] = 0.0;
-#pragma unroll 1
-    for (int d = 0; d < 3; ++d) {
-#pragma unroll
-      for (int side = 0; side < 2; ++side) {
-        const int fi = i + (side && d == 0), fj = j + (side && d == 1), fk = k + (side && d == 2);
-        const long fq = FaceIdx(b, d, fi, fj, fk);
-        const long nf = (long)(b.ni + (d == 0)) * (b.nj + (d == 1)) * (b.nk + (d == 2));
-        // the face's gradient as the viscous pass formed it; its state,
-        // viscosity and conductivity formed again, as that pass forms them
-        const double *fv = b.fvis[d];
-        double vgr[9], Wf[5], J[25], muF;
-#pragma unroll
-        for (int q = 0; q < 9; ++q) vgr[q] = fv[q * nf + fq];
-        ViscFaceState<MODE == 3>(b, d, fi, fj, fk, Wf, muF);
-        const double kF = SutherlandK(P.visc, TempOf(g, Wf[0], Wf[4]));
-        TSLJacobian(g, P.visc, Wf, muF, kF, b.fa[d][fq], b.c2c[d][fq], side == 1, vgr, J);
-#pragma unroll
-        for (int q = 0; q < 25; ++q) D[q] = side ? D[q] - J[q] : D[q] + J[q];
-#pragma unroll
-        for (int q = 0; q < 9; ++q) G[q] += sixth * vgr[q];
+        for (int q = 0; q < 25; ++q) D[q] = D[q] + J[q];
       }
     }
-    const long c = PadIdx(b, i, j, k);
+    if (MODE == 1) {
 #pragma unroll
-    for (int q = 0; q < 9; ++q) b.vgrad[q * b.npad + c] = G[q];
-  }
-  const double sr = b.sr[p];
-  double dvt = Div(b.vol[p] * (1.0 + P.zeta), b.dt[p] * P.theta);
-  if (P.dualCFL > 0.0) dvt += Div(Dmax(sr, 0.0), P.dualCFL);
+      for (int q = 0; q < 25; ++q) b.Ab[q * b.ncell + p] = D[q];
+      return;
+    }
+    if (MODE >= 2) {
+      constexpr double sixth = 1.0 / 6.0;
+      double G[9];
 #pragma unroll
-  for (int q = 0; q < 5; ++q) D[q * 6] *= P.relax;
+      for (int q = 0; q < 9; ++q) G[q] = 0.0;
+#pragma unroll 1
+      for (int d = 0; d < 3; ++d) {
 #pragma unroll
-  for (int q = 0; q < 5; ++q) D[q * 6] += dvt;
+        for (int side = 0; side < 2; ++side) {
+          const int fi = i + (side && d == 0), fj = j + (side && d == 1), fk = k + (side && d == 2);
+          const long fq = FaceIdx(b, d, fi, fj, fk);
+          const long nf = (long)(b.ni + (d == 0)) * (b.nj + (d == 1)) * (b.nk + (d == 2));
+          // the face's gradient as the viscous pass formed it; its state,
+          // viscosity and conductivity formed again, as that pass forms them
+          const double *fv = b.fvis[d];
+          double vgr[9], Wf[5], J[25], muF;
 #pragma unroll
-  for (int q = 0; q < 25; ++q) b.Ab[q * b.ncell + p] = D[q];
-  double I[25];
-  if (!GJInverse5<double>(D, I)) atomicOr(b.flag, 4);
+          for (int q = 0; q < 9; ++q) vgr[q] = fv[q * nf + fq];
+          ViscFaceState<MODE == 3>(b, d, fi, fj, fk, Wf, muF);
+          const double kF = SutherlandK(P.visc, TempOf(g, Wf[0], Wf[4]));
+          TSLJacobian(g, P.visc, Wf, muF, kF, b.fa[d][fq], b.c2c[d][fq], side == 1, vgr, J);
 #pragma unroll
-  for (int q = 0; q < 25; ++q) b.Abi[TileBase(b, i, j, k) + 256 * q] = I[q];
-  if (P.fp32 && b.Abi32) {
+          for (int q = 0; q < 25; ++q) D[q] = side ? D[q] - J[q] : D[q] + J[q];
 #pragma unroll
-    for (int q = 0; q < 25; ++q) b.Abi32[TileBase(b, i, j, k) + 256 * q] = float(I[q]);
-  }
-  if (MODE >= 2 && P.rhsInDiag) {
-    // the initialisation of a one-sweep relax (KInitUpdate with rhsOnce,
-    // FP64 operator) from the values at hand: the right-hand side and du = 0
-    double rb[5];
-    Rhs(b, P, p, PadIdx(b, i, j, k), rb);
+          for (int q = 0; q < 9; ++q) G[q] += sixth * vgr[q];
+        }
+      }
 #pragma unroll
-    for (int e = 0; e < 5; ++e) {
-      b.rhs[e * b.ncell + p] = rb[e];
-      b.x[e * b.ncell + p] = 0.0;
+      for (int q = 0; q < 9; ++q) b.vgrad[q * b.npad + c] = G[q];
+    }
+    const double sr = b.sr[p];
+    double dvt = Div(b.vol[p] * (1.0 + P.zeta), b.dt[p] * P.theta);
+    if (P.dualCFL > 0.0) dvt += Div(Dmax(sr, 0.0), P.dualCFL);
+#pragma unroll
+    for (int q = 0; q < 5; ++q) D[q * 6] *= P.relax;
+#pragma unroll
+    for (int q = 0; q < 5; ++q) D[q * 6] += dvt;
+#pragma unroll
+    for (int q = 0; q < 25; ++q) b.Ab[q * b.ncell + p] = D[q];
+    double I[25];
+    if (!GJInverse5<double>(D, I)) atomicOr(b.flag, 4);
+    int stride;
+    const long ib = InverseBase<double>(b, i, j, k, stride), ib32 = InverseBase<float>(b, i, j, k, stride);
+    float If[25];
+#pragma unroll
+    for (int q = 0; q < 25; ++q) If[q] = float(I[q]);
+    const bool f32 = P.fp32 && b.Abi32;
+    if (b.pns) {
+      PutVecs<double, 25>(b.Abi + ib, I);
+      if (f32) PutVecs<float, 25>(b.Abi32 + ib32, If);
+    } else {
+#pragma unroll
+      for (int q = 0; q < 25; ++q) b.Abi[ib + (long)q * stride] = I[q];
+      if (f32) {
+#pragma unroll
+        for (int q = 0; q < 25; ++q) b.Abi32[ib32 + (long)q * stride] = If[q];
+      }
     }
   }
+  if (!b.pns) return;
+  // what the pencil sweep forms the off-diagonal blocks and the right-hand
+  // side from; this thread writes cell (oi, oj, ok)
+  constexpr int nr = BlockRecord(MODE >= 2);
+  __shared__ double sh[nr][256];
+  if (cell) {
+#pragma unroll
+    for (int e = 0; e < 5; ++e) sh[e][tid] = b.W[e * b.npad + c];
+    if (P.rhsInDiag) {
+      // the initialisation of a one-sweep relax, from the values at hand
+      double rb[5];
+      Rhs(b, P, p, c, rb);
+#pragma unroll
+      for (int e = 0; e < 5; ++e) sh[5 + e][tid] = rb[e];
+    }
+    if constexpr (MODE >= 2) {
+      sh[10][tid] = b.mu[c];
+      sh[11][tid] = b.kc[c];
+#pragma unroll
+      for (int q = 0; q < 9; ++q) sh[12 + q][tid] = b.vgrad[q * b.npad + c];
+    }
+  }
+  __syncthreads();
+  const int src = kTileOrder.cell[b.pl][tid];
+  int oi, oj, ok, lane;
+  DiagCell(b, U, src, oi, oj, ok);
+  if (oi >= b.ni || oj >= b.nj || ok >= b.nk) return;
+  double *o = b.skS + PencilRecord(b, oi, oj, ok, lane) * nr * kPenLanes;
+  o += lane;
+#pragma unroll
+  for (int e = 0; e < nr; ++e)
+    if (e < 5 || e >= 10 || P.rhsInDiag) o[e * kPenLanes] = sh[e][src];
 }
 
 // RusanovBlockOffDiagonal (src/fluxJacobian.cpp:164-194): the neighbour's
@@ -1312,11 +1448,13 @@ template <typename T>
 __device__ __forceinline__ void CellBlockMult(const DevBlock &b, const double *M, long p, const T v[5], T out[5]) {
   BlockMultG<T, double>(M, b.ncell, p, v, out);
 }
-// block product with a tile-blocked per-cell block (Abi)
+// block product with the cell's inverse diagonal (Abi)
 template <typename T, typename MT>
-__device__ __forceinline__ void TileBlockMult(const DevBlock &b, const MT *M, int i, int j, int k, const T v[5],
-                                              T out[5]) {
-  BlockMultG<T>(M, 256, TileBase(b, i, j, k), v, out);
+__device__ __forceinline__ void InverseMult(const DevBlock &b, const MT *M, int i, int j, int k, const T v[5],
+                                            T out[5]) {
+  int stride;
+  const long base = InverseBase<MT>(b, i, j, k, stride);
+  BlockMultG<T>(M, stride, base, v, out);
 }
 
 template <typename T>
@@ -1413,19 +1551,26 @@ __global__ void __launch_bounds__(256) KInitUpdate(BlockMap M, Params P) {
   const long p = (long)U.local * blockDim.x + threadIdx.x;
   if (p >= b.ncell) return;
   T *x = OpBuf<T>::X(b);
-  if (!P.initMatrix && !P.rhsOnce) {
+  if (!P.initMatrix && !P.rhsOnce && !P.copyState) {
 #pragma unroll
     for (int e = 0; e < 5; ++e) x[e * b.ncell + p] = T(0);
     return;
   }
   const int i = (int)(p % b.ni), j = (int)((p / b.ni) % b.nj), k = (int)(p / ((long)b.ni * b.nj));
   double rb[5];
-  Rhs(b, P, p, PadIdx(b, i, j, k), rb);
-  if (P.rhsOnce) {
-    // the right-hand side is fixed for the relax: formed once here, read by
-    // every sweep (b.rhs is FP64; the operator rounds it to its precision)
+  if (P.initMatrix || P.rhsOnce) Rhs(b, P, p, PadIdx(b, i, j, k), rb);
+  if (P.rhsOnce || P.copyState) {
+    // the block pencil sweep's right-hand side, fixed for the relax (FP64; the
+    // operator rounds it to its precision), and the state it runs from
+    int lane;
+    const long rec = PencilRecord(b, i, j, k, lane), c = PadIdx(b, i, j, k);
+    double *o = b.skS + rec * BlockRecord(P.visc.on) * kPenLanes + lane;
 #pragma unroll
-    for (int e = 0; e < 5; ++e) b.rhs[e * b.ncell + p] = rb[e];
+    for (int e = 0; e < 5; ++e) {
+      o[e * kPenLanes] = b.W[e * b.npad + c];
+      if (P.rhsOnce) o[(5 + e) * kPenLanes] = rb[e];
+    }
+    if (!P.rhsOnce) return;
   }
   if (!P.initMatrix) {
 #pragma unroll
@@ -1436,7 +1581,7 @@ __global__ void __launch_bounds__(256) KInitUpdate(BlockMap M, Params P) {
     T v[5], o[5];
 #pragma unroll
     for (int e = 0; e < 5; ++e) v[e] = T(rb[e]);
-    TileBlockMult<T>(b, OpBuf<T>::Abi(b), i, j, k, v, o);
+    InverseMult<T>(b, OpBuf<T>::Abi(b), i, j, k, v, o);
 #pragma unroll
     for (int e = 0; e < 5; ++e) x[e * b.ncell + p] = o[e];
     return;
@@ -1471,7 +1616,7 @@ __global__ void __launch_bounds__(64) KLusgsForward(DevBlock b, Params P,
     T v[5], o[5];
 #pragma unroll
     for (int e = 0; e < 5; ++e) v[e] = T(rb[e]) + L[e];
-    TileBlockMult<T>(b, OpBuf<T>::Abi(b), i, j, k, v, o);
+    InverseMult<T>(b, OpBuf<T>::Abi(b), i, j, k, v, o);
 #pragma unroll
     for (int e = 0; e < 5; ++e) x[e * b.ncell + p] = o[e];
     return;
@@ -1503,11 +1648,11 @@ __global__ void __launch_bounds__(64) KLusgsBackward(DevBlock b, Params P,
       Rhs(b, P, p, PadIdx(b, i, j, k), rb);
 #pragma unroll
       for (int e = 0; e < 5; ++e) v[e] = (T(rb[e]) + L[e]) - U[e];
-      TileBlockMult<T>(b, OpBuf<T>::Abi(b), i, j, k, v, o);
+      InverseMult<T>(b, OpBuf<T>::Abi(b), i, j, k, v, o);
 #pragma unroll
       for (int e = 0; e < 5; ++e) x[e * b.ncell + p] = o[e];
     } else {
-      TileBlockMult<T>(b, OpBuf<T>::Abi(b), i, j, k, U, o);
+      InverseMult<T>(b, OpBuf<T>::Abi(b), i, j, k, U, o);
 #pragma unroll
       for (int e = 0; e < 5; ++e) x[e * b.ncell + p] = x[e * b.ncell + p] - o[e];
     }
@@ -1546,7 +1691,7 @@ __global__ void __launch_bounds__(256) KDplur(DevBlock b, Params P) {
     T v[5], o[5];
 #pragma unroll
     for (int e = 0; e < 5; ++e) v[e] = (T(rb[e]) + T(0)) + (L[e] - U[e]);
-    TileBlockMult<T>(b, OpBuf<T>::Abi(b), i, j, k, v, o);
+    InverseMult<T>(b, OpBuf<T>::Abi(b), i, j, k, v, o);
 #pragma unroll
     for (int e = 0; e < 5; ++e) x[e * b.ncell + p] = o[e];
     return;
@@ -2259,591 +2404,6 @@ __global__ void __launch_bounds__(kLT) KLusgsTile(DevBlock b, Params P, SweepCtl
 }
 
 // ---------------------------------------------------------------------------
-// Block LU-SGS sweep over all blocks in one launch (blusgs).
-//
-// The blocks of a pass are independent (a connection's partner update enters
-// lagged, through the precomputed connection terms), so one persistent launch
-// sweeps them together: the tiles of every block are queued by their tile
-// hyperplane (then block, then k, j, i), each workgroup takes the next ticket,
-// waits for the (at most three) tiles of the same block it depends on, and
-// walks the tile's cell hyperplanes.  Per cell, the dependency side's three
-// off-diagonal blocks (formed once per relax) and D^-1 are read before the
-// wait and stay in registers; the arithmetic of each cell is that of
-// KLusgsForward / KLusgsBackward, so every order gives the same bits.
-
-struct MultiSweepCtl {
-  int *ticket;          // reset to 0 before each sweep
-  int *epoch;           // incremented before each sweep
-  int *flags;           // one per tile of every block, the epoch of its publication
-  int *err;             // bit 1: a dependency wait exceeded the spin limit
-  const int4 *tiles;    // (a, b, c, block) in pass order
-  const int4 *grid;     // per block: tile grid dims and the block's first flag
-  int ntiles;
-};
-
-__global__ void KMultiSweepPrologue(MultiSweepCtl s) {
-  *s.ticket = 0;
-  *s.epoch = *s.epoch + 1;
-}
-
-// tiles of 8 x 8 x 4 cells (four wavefronts).  Measured on the multiblock
-// channel: 4 x 4 x 4 tiles (more tickets and flags) take 1.3 times as long
-// per pass, 16 x 4 x 4 tiles (whole cache lines per tile row, but a longer
-// walk of 22 cell hyperplanes) 1.12 times as long.
-constexpr int kBTI = 8, kBTJ = 8, kBTK = 4;
-constexpr int kBT = kBTI * kBTJ * kBTK;
-constexpr int kBTPlanes = kBTI + kBTJ + kBTK - 2;
-constexpr int kBHaloI = kBTJ * kBTK, kBHaloJ = kBTI * kBTK, kBHaloK = kBTI * kBTJ;
-constexpr int kBHalo = kBHaloI + kBHaloJ + kBHaloK;
-
-template <typename T, bool FWD>
-__global__ void __launch_bounds__(kBT, sizeof(T) == 4 ? 2 : 1) KBlockSweepTiles(const DevBlock *__restrict__ blocks, Params P,
-                                                        MultiSweepCtl s, int full) {
-  __shared__ T sA[5][kBT + kBHalo];  // du of the tile's cells, then of the halo columns
-  __shared__ int sTicket, sNext;
-  __shared__ int sEpoch;
-
-  const int tid = threadIdx.x;
-  const int li = tid % kBTI, lj = (tid / kBTI) % kBTJ, lk = tid / (kBTI * kBTJ);
-  const GasT<T> g = Cast<T>(P.gas);
-  const int sgn = FWD ? -1 : 1;  // direction of the dependency neighbours
-
-  // thread 0 owns the ticket and the flag (see KLusgsTile)
-  if (tid == 0) {
-    sTicket = __hip_atomic_fetch_add(s.ticket, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    sEpoch = __hip_atomic_load(s.epoch, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-  }
-  __syncthreads();
-  const int epoch = sEpoch;
-  for (;;) {
-    const int t = sTicket;
-    if (t >= s.ntiles) break;
-    const int4 tl = s.tiles[FWD ? t : s.ntiles - 1 - t];
-    const DevBlock &b = blocks[tl.w];
-    const int4 gr = s.grid[tl.w];
-    T *x = OpBuf<T>::X(b);
-    const int i = tl.x * kBTI + li, j = tl.y * kBTJ + lj, k = tl.z * kBTK + lk;
-    const bool valid = i < b.ni && j < b.nj && k < b.nk;
-    const long p = (long)i + (long)j * b.ni + (long)k * b.ni * b.nj;
-
-    // --- static data before the dependency wait
-    const int ni = b.ni, nj = b.nj, nk = b.nk;
-    const long ncell = b.ncell, nbf = b.nbf;
-    const T *bt = OpBuf<T>::Bt(b);
-    // connection term (static during the pass) of the face of cell (ci, cj,
-    // ck) in direction d on the dependency side; zero without connections,
-    // and zero in the first forward pass, where every du starts at zero (J 0
-    // sums to +0), so the connection terms are not formed for it
-    const bool connZero = FWD && !full;
-    auto conn = [&](int d, int ci, int cj, int ck, int e) -> T {
-      return (bt && !connZero) ? bt[e * nbf + BtSlot(b, d, FWD ? 0 : 1, ci, cj, ck)] : T(0);
-    };
-    // LDS column of the dependency neighbour in each direction: a cell of
-    // the tile or a halo column
-    int nb[3];
-#pragma unroll
-    for (int d = 0; d < 3; ++d) {
-      const int l3 = d == 0 ? li : (d == 1 ? lj : lk);
-      const int L3 = d == 0 ? kBTI : (d == 1 ? kBTJ : kBTK);
-      const bool inTile = FWD ? (l3 > 0) : (l3 < L3 - 1);
-      nb[d] = inTile ? tid + sgn * (d == 0 ? 1 : (d == 1 ? kBTI : kBTI * kBTJ))
-                     : kBT + (d == 0 ? lj + kBTJ * lk
-                                     : (d == 1 ? kBHaloI + li + kBTI * lk : kBHaloI + kBHaloJ + li + kBTI * lj));
-    }
-    // the right-hand side is formed in FP64 and rounded once to the
-    // operator's precision; the dependency blocks are formed in FP64 and
-    // held in the operator's precision, as is D^-1
-    T rb[5] = {T(0), T(0), T(0), T(0), T(0)};
-    T mdep[3][25], mai[25];
-    T Ost[5];  // full sweeps: the other side's sum, from the previous sweep's du
-    if (valid) {
-      if (FWD || full) {
-        double r64[5];
-        Rhs(b, P, p, PadIdx(b, i, j, k), r64);
-#pragma unroll
-        for (int e = 0; e < 5; ++e) rb[e] = T(r64[e]);
-      }
-      const GasT<double> gd = Cast<double>(P.gas);
-#pragma unroll
-      for (int d = 0; d < 3; ++d) {
-        const int gi = i + (d == 0 ? sgn : 0), gj = j + (d == 1 ? sgn : 0), gk = k + (d == 2 ? sgn : 0);
-        const bool inside = gi >= 0 && gj >= 0 && gk >= 0 && gi < ni && gj < nj && gk < nk;
-        // a neighbour outside the block enters through its connection term,
-        // which its LDS column holds; the identity block passes it on
-        // unchanged (x + 0 y = x, and the sum never starts from -0)
-        if (inside) {
-          double J[25];
-          NeighbourBlock(b, gd, P.visc, d, !FWD, i, j, k, J);
-#pragma unroll
-          for (int q = 0; q < 25; ++q) mdep[d][q] = T(J[q]);
-        } else {
-#pragma unroll
-          for (int q = 0; q < 25; ++q) mdep[d][q] = q % 6 == 0 ? T(1) : T(0);
-        }
-      }
-      // the other side's du is not written before this tile publishes: its
-      // cells in other tiles wait for this one, those in it are stored after
-      // the walk
-      if (full) OffDiagSum<T>(b, g, P.visc, x, i, j, k, FWD, Ost, 1, 0, &P.gas);
-      const auto *Mi = OpBuf<T>::Abi(b) + TileBase(b, i, j, k);
-#pragma unroll
-      for (int q = 0; q < 25; ++q) mai[q] = T(Mi[256 * q]);
-      // backward: the forward result, which only this tile overwrites
-      if (!FWD) {
-#pragma unroll
-        for (int e = 0; e < 5; ++e) sA[e][tid] = x[e * ncell + p];
-      }
-    } else if (!FWD) {
-      // a partial tile's position just past the block's upper face along one
-      // axis is the dependency neighbour of the face cell below it
-      const int oi = i >= ni, oj = j >= nj, ok = k >= nk;
-      const int d = oi ? 0 : (oj ? 1 : 2);
-      const bool edge = oi + oj + ok == 1 && (oi ? i == ni : (oj ? j == nj : k == nk));
-#pragma unroll
-      for (int e = 0; e < 5; ++e)
-        sA[e][tid] = edge ? conn(d, i - (d == 0), j - (d == 1), k - (d == 2), e) : T(0);
-    }
-    // halo columns: positions outside the block hold connection terms now,
-    // those inside the du of the dependency tiles after the wait
-    int hi = 0, hj = 0, hk = 0, hd = 0;
-    bool hin = false;
-    if (tid < kBHalo) {
-      const int di = FWD ? -1 : kBTI, dj = FWD ? -1 : kBTJ, dk = FWD ? -1 : kBTK;
-      if (tid < kBHaloI) { hd = 0; hi = di; hj = tid % kBTJ; hk = tid / kBTJ; }
-      else if (tid < kBHaloI + kBHaloJ) { const int q = tid - kBHaloI; hd = 1; hi = q % kBTI; hj = dj; hk = q / kBTI; }
-      else { const int q = tid - kBHaloI - kBHaloJ; hd = 2; hi = q % kBTI; hj = q / kBTI; hk = dk; }
-      hi += tl.x * kBTI; hj += tl.y * kBTJ; hk += tl.z * kBTK;
-      hin = hi >= 0 && hj >= 0 && hk >= 0 && hi < ni && hj < nj && hk < nk;
-      if (!hin) {
-        // the tile cell next to it along hd
-        const int ci = hi - (hd == 0 ? sgn : 0), cj = hj - (hd == 1 ? sgn : 0), ck = hk - (hd == 2 ? sgn : 0);
-        const bool face = ci >= 0 && cj >= 0 && ck >= 0 && ci < ni && cj < nj && ck < nk;
-#pragma unroll
-        for (int e = 0; e < 5; ++e) sA[e][kBT + tid] = face ? conn(hd, ci, cj, ck, e) : T(0);
-      }
-    }
-
-    // --- wait for the tiles of the same block this one depends on
-    if (tid == 0) {
-      const int deps[3][3] = {{tl.x + sgn, tl.y, tl.z}, {tl.x, tl.y + sgn, tl.z}, {tl.x, tl.y, tl.z + sgn}};
-      for (int q = 0; q < 3; ++q) {
-        const int a = deps[q][0], bb = deps[q][1], cc = deps[q][2];
-        if (a < 0 || bb < 0 || cc < 0 || a >= gr.x || bb >= gr.y || cc >= gr.z) continue;
-        const int id = gr.w + a + gr.x * (bb + gr.y * cc);
-        long spins = 0;
-        while (__hip_atomic_load(&s.flags[id], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) < epoch) {
-          if ((++spins & 255) == 0 &&
-              (__hip_atomic_load(s.err, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) & 2))
-            break;
-          if (spins > kSpinLimit) {
-            __hip_atomic_fetch_or(s.err, 2, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            break;
-          }
-          __builtin_amdgcn_s_sleep(1);
-        }
-      }
-      // one acquire for the workgroup: the barrier below orders it before
-      // every wave's halo loads (each wave's own fence would invalidate the
-      // XCD's L2 once more)
-      __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
-      // the next ticket now, so that its atomic overlaps this tile's walk (a
-      // held ticket only ever waits on smaller ones, so no cycle can form)
-      sNext = __hip_atomic_fetch_add(s.ticket, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    }
-    __syncthreads();
-
-    // halo du, published by the dependency tiles
-    if (hin) {
-      const long q = (long)hi + (long)hj * ni + (long)hk * ni * nj;
-#pragma unroll
-      for (int e = 0; e < 5; ++e) sA[e][kBT + tid] = x[e * ncell + q];
-    }
-    __syncthreads();
-
-    // --- intra-tile hyperplanes
-    const int plane = li + lj + lk;
-    for (int st = 0; st < kBTPlanes; ++st) {
-      const int pl = FWD ? st : kBTPlanes - 1 - st;
-      if (valid && plane == pl) {
-        T D[5];  // dependency-side sum: L (forward) or U (backward), i, j, k order
-#pragma unroll
-        for (int e = 0; e < 5; ++e) D[e] = T(0);
-#pragma unroll
-        for (int d = 0; d < 3; ++d) {
-          T dn[5], o[5];
-#pragma unroll
-          for (int e = 0; e < 5; ++e) dn[e] = sA[e][nb[d]];
-          BlockMult<T>(mdep[d], dn, o);
-#pragma unroll
-          for (int e = 0; e < 5; ++e) D[e] += o[e];
-        }
-        T xn[5], v[5];
-        const T *ai = mai;
-        if (full) {
-          if (FWD) {
-#pragma unroll
-            for (int e = 0; e < 5; ++e) v[e] = T(rb[e]) + (D[e] - Ost[e]);
-          } else {
-#pragma unroll
-            for (int e = 0; e < 5; ++e) v[e] = (T(rb[e]) + Ost[e]) - D[e];
-          }
-          BlockMult<T>(ai, v, xn);
-        } else if (FWD) {
-#pragma unroll
-          for (int e = 0; e < 5; ++e) v[e] = T(rb[e]) + D[e];
-          BlockMult<T>(ai, v, xn);
-        } else {
-          T o[5];
-          BlockMult<T>(ai, D, o);
-#pragma unroll
-          for (int e = 0; e < 5; ++e) xn[e] = sA[e][tid] - o[e];
-        }
-        // in LDS only during the walk: per-step global stores of scattered
-        // cells would write partial cache lines
-#pragma unroll
-        for (int e = 0; e < 5; ++e) sA[e][tid] = xn[e];
-      }
-      __syncthreads();
-    }
-    if (valid) {
-#pragma unroll
-      for (int e = 0; e < 5; ++e) StoreCoherent(&x[e * ncell + p], sA[e][tid]);
-    }
-
-    // --- publish: every wave's du stores have completed before the barrier,
-    // and thread 0 stores the flag after it, then takes the next ticket
-    WaitStores();
-    __syncthreads();
-    if (tid == 0) {
-      __hip_atomic_store(&s.flags[gr.w + tl.x + gr.x * (tl.y + gr.y * tl.z)], epoch, __ATOMIC_RELAXED,
-                         __HIP_MEMORY_SCOPE_AGENT);
-      sTicket = sNext;
-    }
-    __syncthreads();
-  }
-}
-
-// A full block LU-SGS sweep's other-side sums (OffDiagSum over the upper
-// neighbours in a forward pass, the lower ones in a backward pass, from the
-// previous sweep's du and this pass's connection terms), formed for every
-// cell before the pass into xold: none of the du they read is written by the
-// pass before the cell's own tile publishes, so the values are those the
-// sweep would form in place.
-template <typename T, bool FWD>
-__global__ void __launch_bounds__(256) KOtherSide(BlockMap M, Params P) {
-  const Unit U = MapUnit(M);
-  const DevBlock &b = *U.b;
-  const long p = (long)U.local * blockDim.x + threadIdx.x;
-  if (p >= b.ncell) return;
-  const int i = (int)(p % b.ni), j = (int)((p / b.ni) % b.nj), k = (int)(p / ((long)b.ni * b.nj));
-  const GasT<T> g = Cast<T>(P.gas);
-  T o[5];
-  OffDiagSum<T>(b, g, P.visc, OpBuf<T>::X(b), i, j, k, FWD, o, 1, 0, &P.gas);
-  T *xo = OpBuf<T>::Xold(b);
-#pragma unroll
-  for (int e = 0; e < 5; ++e) xo[e * b.ncell + p] = o[e];
-}
-
-// ---------------------------------------------------------------------------
-// Row-parallel block LU-SGS sweep over all blocks (blusgs).
-//
-// The tiles, queue and flags of KBlockSweepTiles (8 x 8 x 4 cells), with two
-// lanes per cell: lane h of a cell's pair holds rows 3h .. 3h+2 (rows 3 and
-// 4 for h = 1) of its three dependency-side blocks, of D^-1, of the
-// right-hand side and of the forward result, in registers.
-//
-// * Forming: lane h forms the block of direction 2h (i or k) and both lanes
-//   form the j block; a lane keeps its rows and hands the pair's other rows
-//   to its partner with a lane shuffle.  The right-hand side is formed once
-//   per relax (by the viscous block diagonal for a one-sweep FP64 relax,
-//   else by KInitUpdate), a full sweep's other-side sums by KOtherSide
-//   before the pass.
-// * The walk: per cell hyperplane a lane forms its rows of the dependency
-//   sum and of v, the pair exchanges v, and each lane forms its rows of
-//   D^-1 v.  Pairs are given to cells in hyperplane order, so a hyperplane
-//   occupies one or two of the eight wavefronts.
-//
-// Each row is summed in the order BlockMult sums it and the dependency sum
-// adds the directions in i, j, k order from +0, so the result is that of
-// KLusgsForward / KLusgsBackward bit for bit.
-constexpr int kPThreads = 2 * kBT;
-static_assert(kPThreads == 512 && kBHalo <= kBT, "row sweep layout");
-
-template <typename T, bool FWD>
-__global__ void __launch_bounds__(kPThreads) KBlockSweepRows(const DevBlock *__restrict__ blocks, Params P,
-                                                             MultiSweepCtl s, int full) {
-  __shared__ T sA[5][kBT + kBHalo];  // du of the tile's cells, then of the halo columns
-  __shared__ unsigned char sCell[kBT];  // pair -> cell, in hyperplane order
-  __shared__ int sTicket, sNext, sEpoch;
-
-  const int tid = threadIdx.x;
-  const int sgn = FWD ? -1 : 1;  // direction of the dependency neighbours
-  const int g = tid >> 1, h = tid & 1;
-  const int r0 = 3 * h;           // this lane's first row
-  const int nrow = h ? 2 : 3;     // its rows r0 .. r0 + nrow - 1
-  const bool connZero = FWD && !full;
-
-  if (tid < kBT) {
-    // rank of cell tid among the tile's cells by (hyperplane, index)
-    const int li = tid % kBTI, lj = (tid / kBTI) % kBTJ, lk = tid / (kBTI * kBTJ);
-    const int pl = li + lj + lk;
-    int rank = 0;
-    for (int q = 0; q < kBT; ++q) {
-      const int qp = q % kBTI + (q / kBTI) % kBTJ + q / (kBTI * kBTJ);
-      rank += (qp < pl || (qp == pl && q < tid)) ? 1 : 0;
-    }
-    sCell[rank] = (unsigned char)tid;
-  }
-  if (tid == 0) {
-    sTicket = __hip_atomic_fetch_add(s.ticket, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    sEpoch = __hip_atomic_load(s.epoch, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-  }
-  __syncthreads();
-  const int epoch = sEpoch;
-  const GasT<double> gd = Cast<double>(P.gas);
-  const int wc = sCell[g];
-  const int li = wc % kBTI, lj = (wc / kBTI) % kBTJ, lk = wc / (kBTI * kBTJ);
-  const int plane = li + lj + lk;
-  // LDS column of the dependency neighbour in each direction: a cell of the
-  // tile or a halo column
-  int nb[3];
-#pragma unroll
-  for (int d = 0; d < 3; ++d) {
-    const int l3 = d == 0 ? li : (d == 1 ? lj : lk);
-    const int L3 = d == 0 ? kBTI : (d == 1 ? kBTJ : kBTK);
-    const bool inTile = FWD ? (l3 > 0) : (l3 < L3 - 1);
-    nb[d] = inTile ? wc + sgn * (d == 0 ? 1 : (d == 1 ? kBTI : kBTI * kBTJ))
-                   : kBT + (d == 0 ? lj + kBTJ * lk
-                                   : (d == 1 ? kBHaloI + li + kBTI * lk : kBHaloI + kBHaloJ + li + kBTI * lj));
-  }
-
-  for (;;) {
-    const int t = sTicket;
-    if (t >= s.ntiles) break;
-    const int4 tl = s.tiles[FWD ? t : s.ntiles - 1 - t];
-    const DevBlock &b = blocks[tl.w];
-    const int4 gr = s.grid[tl.w];
-    T *x = OpBuf<T>::X(b);
-    const int ni = b.ni, nj = b.nj, nk = b.nk;
-    const long ncell = b.ncell, nbf = b.nbf;
-    const T *bt = OpBuf<T>::Bt(b);
-    auto conn = [&](int d, int ci, int cj, int ck, int e) -> T {
-      return (bt && !connZero) ? bt[e * nbf + BtSlot(b, d, FWD ? 0 : 1, ci, cj, ck)] : T(0);
-    };
-
-    // --- static data before the dependency wait
-    const int i = tl.x * kBTI + li, j = tl.y * kBTJ + lj, k = tl.z * kBTK + lk;
-    const bool valid = i < ni && j < nj && k < nk;
-    const long p = (long)i + (long)j * ni + (long)k * ni * nj;
-    T m[3][3][5];  // [direction][slot][column]: rows r0 + slot of the dependency blocks
-    T ai[3][5], rb[3], ost[3], xf[3];
-#pragma unroll
-    for (int sl = 0; sl < 3; ++sl) {
-      rb[sl] = ost[sl] = xf[sl] = T(0);
-#pragma unroll
-      for (int q = 0; q < 5; ++q) {
-        ai[sl][q] = T(0);
-#pragma unroll
-        for (int d = 0; d < 3; ++d) m[d][sl][q] = T(0);
-      }
-    }
-    if (valid) {
-      // one dependency-side block of direction d, formed in FP64 and held in
-      // the operator's precision; a neighbour outside the block enters
-      // through its connection term in the LDS column, the identity block
-      // passing it on unchanged (x + 0 y = x, and the sum never starts from -0)
-      auto form = [&](int d, T Jt[25]) {
-        const int gi = i + (d == 0 ? sgn : 0), gj = j + (d == 1 ? sgn : 0), gk = k + (d == 2 ? sgn : 0);
-        const bool inside = gi >= 0 && gj >= 0 && gk >= 0 && gi < ni && gj < nj && gk < nk;
-        if (inside) {
-          double J[25];
-          NeighbourBlock(b, gd, P.visc, d, !FWD, i, j, k, J);
-#pragma unroll
-          for (int q = 0; q < 25; ++q) Jt[q] = T(J[q]);
-        } else {
-#pragma unroll
-          for (int q = 0; q < 25; ++q) Jt[q] = q % 6 == 0 ? T(1) : T(0);
-        }
-      };
-      // (every register index below is a compile-time constant; the lane's
-      // half selects between values)
-      {
-        // lane h forms direction 2h; each keeps its rows and sends the
-        // partner's rows (rows 3-4 from lane 0, rows 0-2 from lane 1)
-        T J[25];
-        form(2 * h, J);
-        T send[15], own[3][5];
-#pragma unroll
-        for (int q = 0; q < 15; ++q) send[q] = h ? J[q] : (q < 10 ? J[15 + q] : T(0));
-#pragma unroll
-        for (int sl = 0; sl < 3; ++sl)
-#pragma unroll
-          for (int q = 0; q < 5; ++q) own[sl][q] = h ? (sl < 2 ? J[15 + 5 * sl + q] : T(0)) : J[5 * sl + q];
-        T recv[15];
-#pragma unroll
-        for (int q = 0; q < 15; ++q) recv[q] = __shfl_xor(send[q], 1, 64);
-        // lane 0 receives direction k, rows 0-2; lane 1 direction i, rows 3-4
-#pragma unroll
-        for (int sl = 0; sl < 3; ++sl)
-#pragma unroll
-          for (int q = 0; q < 5; ++q) {
-            const T got = (sl == 2) ? (h ? T(0) : recv[5 * sl + q]) : recv[5 * sl + q];
-            m[0][sl][q] = h ? got : own[sl][q];
-            m[2][sl][q] = h ? own[sl][q] : got;
-          }
-      }
-      {
-        // both lanes form direction j and keep their rows
-        T J[25];
-        form(1, J);
-#pragma unroll
-        for (int sl = 0; sl < 3; ++sl)
-#pragma unroll
-          for (int q = 0; q < 5; ++q) m[1][sl][q] = h ? (sl < 2 ? J[15 + 5 * sl + q] : T(0)) : J[5 * sl + q];
-      }
-      const auto *Mi = OpBuf<T>::Abi(b) + TileBase(b, i, j, k);
-#pragma unroll
-      for (int sl = 0; sl < 3; ++sl) {
-        const int row = r0 + sl;
-        if (row < 5) {
-#pragma unroll
-          for (int q = 0; q < 5; ++q) ai[sl][q] = T(Mi[256 * (5 * row + q)]);
-          if (FWD || full) rb[sl] = T(b.rhs[row * ncell + p]);
-          if (full) ost[sl] = OpBuf<T>::Xold(b)[row * ncell + p];
-          if (!FWD && !full) xf[sl] = x[row * ncell + p];
-        }
-      }
-    }
-    // backward: a partial tile's position just past the block's upper face
-    // along one axis is the dependency neighbour of the face cell below it
-    if (!FWD && tid < kBT) {
-      const int pi = tl.x * kBTI + tid % kBTI, pj = tl.y * kBTJ + (tid / kBTI) % kBTJ,
-                pk = tl.z * kBTK + tid / (kBTI * kBTJ);
-      if (!(pi < ni && pj < nj && pk < nk)) {
-        const int oi = pi >= ni, oj = pj >= nj, ok = pk >= nk;
-        const int d = oi ? 0 : (oj ? 1 : 2);
-        const bool edge = oi + oj + ok == 1 && (oi ? pi == ni : (oj ? pj == nj : pk == nk));
-#pragma unroll
-        for (int e = 0; e < 5; ++e)
-          sA[e][tid] = edge ? conn(d, pi - (d == 0), pj - (d == 1), pk - (d == 2), e) : T(0);
-      }
-    }
-    // halo columns: positions outside the block hold connection terms now,
-    // those inside the du of the dependency tiles after the wait
-    int hi = 0, hj = 0, hk = 0, hd = 0;
-    bool hin = false;
-    if (tid < kBHalo) {
-      const int di = FWD ? -1 : kBTI, dj = FWD ? -1 : kBTJ, dk = FWD ? -1 : kBTK;
-      if (tid < kBHaloI) { hd = 0; hi = di; hj = tid % kBTJ; hk = tid / kBTJ; }
-      else if (tid < kBHaloI + kBHaloJ) { const int q = tid - kBHaloI; hd = 1; hi = q % kBTI; hj = dj; hk = q / kBTI; }
-      else { const int q = tid - kBHaloI - kBHaloJ; hd = 2; hi = q % kBTI; hj = q / kBTI; hk = dk; }
-      hi += tl.x * kBTI; hj += tl.y * kBTJ; hk += tl.z * kBTK;
-      hin = hi >= 0 && hj >= 0 && hk >= 0 && hi < ni && hj < nj && hk < nk;
-      if (!hin) {
-        const int ci = hi - (hd == 0 ? sgn : 0), cj = hj - (hd == 1 ? sgn : 0), ck = hk - (hd == 2 ? sgn : 0);
-        const bool face = ci >= 0 && cj >= 0 && ck >= 0 && ci < ni && cj < nj && ck < nk;
-#pragma unroll
-        for (int e = 0; e < 5; ++e) sA[e][kBT + tid] = face ? conn(hd, ci, cj, ck, e) : T(0);
-      }
-    }
-
-    // --- wait for the tiles of the same block this one depends on
-    if (tid == 0) {
-      const int deps[3][3] = {{tl.x + sgn, tl.y, tl.z}, {tl.x, tl.y + sgn, tl.z}, {tl.x, tl.y, tl.z + sgn}};
-      for (int q = 0; q < 3; ++q) {
-        const int a = deps[q][0], bb = deps[q][1], cc = deps[q][2];
-        if (a < 0 || bb < 0 || cc < 0 || a >= gr.x || bb >= gr.y || cc >= gr.z) continue;
-        const int id = gr.w + a + gr.x * (bb + gr.y * cc);
-        long spins = 0;
-        while (__hip_atomic_load(&s.flags[id], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) < epoch) {
-          if ((++spins & 255) == 0 &&
-              (__hip_atomic_load(s.err, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) & 2))
-            break;
-          if (spins > kSpinLimit) {
-            __hip_atomic_fetch_or(s.err, 2, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            break;
-          }
-          __builtin_amdgcn_s_sleep(1);
-        }
-      }
-      // one acquire for the workgroup; the barrier below orders it before
-      // every wave's halo loads
-      __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
-      // the next ticket now, so that its atomic overlaps this tile's walk
-      sNext = __hip_atomic_fetch_add(s.ticket, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    }
-    __syncthreads();
-    if (hin) {
-      const long q = (long)hi + (long)hj * ni + (long)hk * ni * nj;
-#pragma unroll
-      for (int e = 0; e < 5; ++e) sA[e][kBT + tid] = x[e * ncell + q];
-    }
-    __syncthreads();
-
-    // --- intra-tile hyperplanes
-    for (int st = 0; st < kBTPlanes; ++st) {
-      const int pl = FWD ? st : kBTPlanes - 1 - st;
-      if (valid && plane == pl) {
-        T dn[3][5];
-#pragma unroll
-        for (int d = 0; d < 3; ++d)
-#pragma unroll
-          for (int q = 0; q < 5; ++q) dn[d][q] = sA[q][nb[d]];
-        // this lane's rows of the dependency-side sum, L (forward) or U
-        // (backward), and of v (of D, backward)
-        T v[3];
-#pragma unroll
-        for (int sl = 0; sl < 3; ++sl) {
-          T D = T(0);
-#pragma unroll
-          for (int d = 0; d < 3; ++d) {
-            T o = T(0);
-#pragma unroll
-            for (int q = 0; q < 5; ++q) o += m[d][sl][q] * dn[d][q];
-            D += o;
-          }
-          if (full) v[sl] = FWD ? rb[sl] + (D - ost[sl]) : (rb[sl] + ost[sl]) - D;
-          else v[sl] = FWD ? rb[sl] + D : D;
-        }
-        // the pair's five rows of v
-        T w[3];
-#pragma unroll
-        for (int sl = 0; sl < 3; ++sl) w[sl] = __shfl_xor(v[sl], 1, 64);
-        const T vv[5] = {h ? w[0] : v[0], h ? w[1] : v[1], h ? w[2] : v[2], h ? v[0] : w[0], h ? v[1] : w[1]};
-#pragma unroll
-        for (int sl = 0; sl < 3; ++sl) {
-          const int row = r0 + sl;
-          if (sl < nrow) {
-            T o = T(0);
-#pragma unroll
-            for (int q = 0; q < 5; ++q) o += ai[sl][q] * vv[q];
-            sA[row < 5 ? row : 4][wc] = (!full && !FWD) ? xf[sl] - o : o;
-          }
-        }
-      }
-      __syncthreads();
-    }
-    for (int q = tid; q < 5 * kBT; q += kPThreads) {
-      const int e = q / kBT, c = q % kBT;
-      const int ci = tl.x * kBTI + c % kBTI, cj = tl.y * kBTJ + (c / kBTI) % kBTJ, ck = tl.z * kBTK + c / (kBTI * kBTJ);
-      if (ci < ni && cj < nj && ck < nk)
-        StoreCoherent(&x[e * ncell + (long)ci + (long)cj * ni + (long)ck * ni * nj], sA[e][c]);
-    }
-
-    // --- publish: every wave's du stores have completed before the barrier,
-    // and thread 0 stores the flag after it, then takes the next ticket
-    WaitStores();
-    __syncthreads();
-    if (tid == 0) {
-      __hip_atomic_store(&s.flags[gr.w + tl.x + gr.x * (tl.y + gr.y * tl.z)], epoch, __ATOMIC_RELAXED,
-                         __HIP_MEMORY_SCOPE_AGENT);
-      sTicket = sNext;
-    }
-    __syncthreads();
-  }
-}
-
-// ---------------------------------------------------------------------------
 // Pencil-wavefront LU-SGS sweep (scalar operator).
 //
 // The block is cut into kPW x kPW columns ("pencils") that run the whole
@@ -2897,8 +2457,6 @@ __global__ void __launch_bounds__(kPThreads) KBlockSweepRows(const DevBlock *__r
 // which hold the wave's issue for 13-29 cycles each), a handoff 1.6 us more
 // than its step.  Three compute waves, one per outgoing product, took 0.82 us
 // a step (the exchange between them costs what the arithmetic saves).
-constexpr int kPW = 8;
-constexpr int kPenLanes = kPW * kPW;
 constexpr int kStagers = 4;
 constexpr int kPenSlots = kStagers;
 constexpr int kPenWaves = 3 + kStagers;
@@ -2937,8 +2495,7 @@ __device__ __forceinline__ T CoherentLoad(const T *p) {
 // the empty message slot: all bits one, a NaN that no product is stored as
 __device__ __forceinline__ bool IsEmpty(double v) { return __double_as_longlong(v) == -1LL; }
 __device__ __forceinline__ bool IsEmpty(float v) { return __float_as_int(v) == -1; }
-// Arithmetic passes on the payload of a NaN it is given and makes no all-ones
-// one of its own, so it is enough that no input of a product holds one.
+// (a product could hold that pattern only as a NaN handed down from an input)
 template <typename T>
 __device__ __forceinline__ T NotEmpty(T v) {
   return IsEmpty(v) ? T(__builtin_nan("")) : v;
@@ -2969,13 +2526,13 @@ __device__ __forceinline__ PenCell PencilCell(const DevBlock &b, int pid, int s,
 // lower faces (what the backward pass's products cross), side 1 the upper
 // ones (forward), axes in the order A, B, C.  Records of idle lanes, which the
 // sweep reads and whose results it drops, start from zeros.
-__global__ void __launch_bounds__(256) KPencilFaces(const DevBlock b, int visc) {
+__global__ void __launch_bounds__(256) KPencilFaces(const DevBlock b, int visc, int nS) {
   const long t = (long)blockIdx.x * blockDim.x + threadIdx.x;
   const int lane = (int)(t % kPenLanes);
   const long rec = t / kPenLanes, nrec = (long)b.pa * b.pb * b.pns;
   if (rec >= nrec) return;
   const PenCell c = PencilCell(b, (int)(rec / b.pns), (int)(rec % b.pns), lane);
-  const int nF = kPenF + (visc ? 3 : 0), nS = kPenS + (visc ? 1 : 0);
+  const int nF = kPenF + (visc ? 3 : 0);
   if (!c.active) {
     for (int q = 0; q < nF; ++q)
       b.skF[(rec * nF + q) * kPenLanes + lane] = b.skF[((nrec + rec) * nF + q) * kPenLanes + lane] = 0.0;
@@ -3044,23 +2601,11 @@ __global__ void __launch_bounds__(256) KPencilOther(BlockMap M, Params P) {
   const PenCell q = PencilCell(b, (int)(rec / b.pns), (int)(rec % b.pns), lane);
   if (!q.active) return;
   T O[5];
-  OffDiagSum<T>(b, Cast<T>(P.gas), P.visc, OpBuf<T>::X(b), q.i, q.j, q.k, FWD, O);
+  OffDiagSum<T>(b, Cast<T>(P.gas), P.visc, OpBuf<T>::X(b), q.i, q.j, q.k, FWD, O, P.block, 0, &P.gas);
   T *o = (T *)b.skO + rec * 5 * kPenLanes + lane;
 #pragma unroll
   for (int e = 0; e < 5; ++e) o[e * kPenLanes] = O[e];
 }
-
-// Values in LDS go 16 bytes a lane: a 16-byte read takes 13 cycles of the
-// LDS pipe for a wave, two 8-byte reads 33.  Value q of a lane's record is
-// v[q % kVecN] of its vector q / kVecN.
-template <typename T>
-struct alignas(16) LdsVec {
-  T v[16 / sizeof(T)];
-};
-template <typename T>
-constexpr int kVecN = 16 / (int)sizeof(T);
-template <typename T>
-constexpr int Vecs(int n) { return (n + kVecN<T> - 1) / kVecN<T>; }
 
 // everything of one step that does not depend on this sweep's du.  Early:
 // right-hand side or the cell's forward du (5), D^-1, state
@@ -3078,11 +2623,11 @@ struct PenSlot {
   LdsVec<T> late[3][Vecs<T>(kLate<T>)][kPenLanes];
 };
 // n values of a lane from / to its vectors
-template <typename T, int N>
+template <typename T, int N, int STRIDE = kPenLanes>
 __device__ __forceinline__ void LdsGet(const LdsVec<T> *p, T *v) {
 #pragma unroll
   for (int q = 0; q < Vecs<T>(N); ++q) {
-    const LdsVec<T> w = p[q * kPenLanes];
+    const LdsVec<T> w = p[q * STRIDE];
 #pragma unroll
     for (int r = 0; r < kVecN<T>; ++r)
       if (q * kVecN<T> + r < N) v[q * kVecN<T> + r] = w.v[r];
@@ -3099,40 +2644,39 @@ __device__ __forceinline__ void LdsPut(LdsVec<T> *p, const T *v) {
   }
 }
 
-template <typename T, bool FULL>
-struct PenShared {
-  PenSlot<T, FULL> slot[kPenSlots];
+// what links the steps and the waves of a pencil
+template <typename T>
+struct PenLink {
   // the products across axes A and B: of the last kProdRing steps, a lane
   // each, and those that enter through the pencil's faces: entry q of step s
   // in column kPW (s mod kHaloRing) + q
   LdsVec<T> prod[kProdRing][2][Vecs<T>(5)][kPenLanes];
   LdsVec<T> halo[2][Vecs<T>(5)][kPenLanes];
-  int stageReady[kPenSlots];  // slot j holds step stageReady[j] - 1
-  int haloReady;              // steps whose halo products are in the ring
-  int xReady;                 // steps the compute wave has finished
-  int sentReady;              // steps whose outgoing products have been sent
+  int haloReady;  // steps whose halo products are in the ring
+  int xReady;     // steps the compute wave has finished
+  int sentReady;  // steps whose outgoing products have been sent
   int ticket;
+};
+template <typename T, bool FULL>
+struct PenShared {
+  PenSlot<T, FULL> slot[kPenSlots];
+  PenLink<T> link;
+  int stageReady[kPenSlots];  // slot j holds step stageReady[j] - 1
 };
 
 __device__ __forceinline__ int LdsLoad(const int *p) {
   return __hip_atomic_load(p, __ATOMIC_ACQUIRE, __HIP_MEMORY_SCOPE_WORKGROUP);
-}
-// publish a step counter for the whole wave: the wave barrier is a
-// convergent point the compiler cannot duplicate into a lane-divergent
-// branch, the release fence waits for every lane's earlier LDS writes, and
-// then one lane stores the count
-__device__ __forceinline__ void LdsStore(int *p, int v) {
-  __builtin_amdgcn_wave_barrier();
-  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
-  if (__lane_id() == 0) __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
 }
 // a counter read without waiting for it, to be tested later (an acquire fence
 // comes between the test and the reads of what it covers)
 __device__ __forceinline__ int LdsPeek(const int *p) {
   return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
 }
-// store a counter that covers only this wave's LDS reads whose values have
-// been used: nothing of other waves is released by it, so no wait is needed
+// publish a step counter for the whole wave.  A wave's LDS operations complete
+// in order, so every LDS read and write it issued before is done when another
+// wave sees the count; no wait is needed.  The wave barrier is a convergent
+// point the compiler cannot duplicate into a lane-divergent branch, the fence
+// keeps it from moving LDS accesses across, and one lane stores the count.
 __device__ __forceinline__ void LdsPost(int *p, int v) {
   __builtin_amdgcn_wave_barrier();
   __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
@@ -3157,10 +2701,149 @@ __device__ __forceinline__ void LdsWait(const int *p, int need, int *err) {
 struct Pencil {
   int a, b;             // position in the pencil grid
   int pid;              // number within the block
+  int C, na, nb;        // axis the pencil runs along, the block's cells across it
   int wa, wb, nc, ns;   // widths, length, steps
   long rec;             // first record of the pencil
   long nrec;            // records of the block
+  long msg;             // first message step of the block
+  bool toA, toB;        // a pencil lies downstream across A, across B
+  bool from[2];         // a pencil lies upstream across A, across B
 };
+// the next pencil of the launch for this workgroup: every thread gets it
+// after the barrier that follows
+__device__ __forceinline__ int PencilTicket(const PencilGroup &G) {
+  return (int)(__hip_atomic_fetch_add(G.ticket, 1ULL, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) %
+               (unsigned long long)G.nent);
+}
+template <bool FWD>
+__device__ __forceinline__ Pencil MakePencil(const DevBlock &b, int4 ent) {
+  constexpr int sgn = FWD ? -1 : 1;
+  Pencil p;
+  p.a = ent.x;
+  p.b = ent.y;
+  p.pid = p.a + b.pa * p.b;
+  p.C = b.pl;
+  p.na = AxisN(b, (b.pl + 1) % 3);
+  p.nb = AxisN(b, (b.pl + 2) % 3);
+  p.wa = PenWidth(p.na, p.a);
+  p.wb = PenWidth(p.nb, p.b);
+  p.nc = AxisN(b, b.pl);
+  p.ns = p.wa + p.wb + p.nc - 2;
+  p.rec = (long)p.pid * b.pns;
+  p.nrec = (long)b.pa * b.pb * b.pns;
+  p.msg = ent.w;
+  p.toA = p.a - sgn >= 0 && p.a - sgn < b.pa;
+  p.toB = p.b - sgn >= 0 && p.b - sgn < b.pb;
+  p.from[0] = p.a + sgn >= 0 && p.a + sgn < b.pa;
+  p.from[1] = p.b + sgn >= 0 && p.b + sgn < b.pb;
+  return p;
+}
+// messages of pencil (pa, pb) of the block through its face f (0 A, 1 B)
+template <typename T, bool FWD>
+__device__ __forceinline__ T *Messages(const PencilGroup &G, const DevBlock &b, const Pencil &p, int pa, int pb,
+                                       int f) {
+  return (T *)G.msg[FWD ? 0 : 1] + (p.msg + ((long)(pa + b.pa * pb) * 2 + f) * b.pns) * kMsg;
+}
+
+// The send wave: lane = (value e, entry q); entry q of face A is the row
+// lb = q, of face B the row la = q.
+template <typename T, bool FWD>
+__device__ __forceinline__ void PenSend(const PencilGroup &G, const DevBlock &b, const Pencil &p, PenLink<T> &ln,
+                                        int lane) {
+  if (!p.toA && !p.toB) return;
+  constexpr int sgn = FWD ? -1 : 1;
+  const int e = lane / kPW, q = lane % kPW;
+  // the columns whose products leave the pencil, and their first steps
+  const int cA = (FWD ? p.wa - 1 : 0) + kPW * q, cB = q + kPW * (FWD ? p.wb - 1 : 0);
+  const int offA = FWD ? p.wa - 1 + q : p.wa - 1 + p.wb - 1 - q, offB = FWD ? q + p.wb - 1 : p.wa - 1 - q + p.wb - 1;
+  const bool useA = p.toA && e < 5 && q < p.wb, useB = p.toB && e < 5 && q < p.wa;
+  // the receiver's step lags by this pencil's width less one
+  T *mA = p.toA ? Messages<T, FWD>(G, b, p, p.a - sgn, p.b, 0) + e * kPW + q - (long)(p.wa - 1) * kMsg : nullptr;
+  T *mB = p.toB ? Messages<T, FWD>(G, b, p, p.a, p.b - sgn, 1) + e * kPW + q - (long)(p.wb - 1) * kMsg : nullptr;
+  const int ev = e < 5 ? e / kVecN<T> : 0, er = e % kVecN<T>;
+  for (int st = 0; st < p.ns; ++st) {
+    LdsWait<1>(&ln.xReady, st + 1, G.err);
+    const T vA = ln.prod[st & (kProdRing - 1)][0][ev][cA].v[er], vB = ln.prod[st & (kProdRing - 1)][1][ev][cB].v[er];
+    // (no wait for the stores of the steps before)
+    asm volatile("" ::"v"(vA), "v"(vB));
+    LdsPost(&ln.sentReady, st + 1);
+    const int kA = st - offA, kB = st - offB;
+    if (useA && kA >= 0 && kA < p.nc) StoreCoherent(mA + (long)st * kMsg, NotEmpty(vA));
+    if (useB && kB >= 0 && kB < p.nc) StoreCoherent(mB + (long)st * kMsg, NotEmpty(vB));
+  }
+}
+
+// The halo wave: the products that enter through the pencil's faces, polled
+// from the messages of the pencils upstream; on a block face the connection
+// terms `bt` (zero off connections, null for none).  One step at a time: a
+// poll of two or four steps lasts as long as its slowest load.
+template <typename T, bool FWD>
+__device__ __forceinline__ void PenHalo(const PencilGroup &G, const DevBlock &b, const Pencil &p, PenLink<T> &ln,
+                                        int lane, const T *bt) {
+  const int e = lane / kPW, q = lane % kPW;
+  const int w[2] = {p.wb, p.wa};
+  const T *in[2];
+  int off[2];
+  bool use[2];
+#pragma unroll
+  for (int f = 0; f < 2; ++f) {
+    in[f] = Messages<T, FWD>(G, b, p, p.a, p.b, f) + min(lane, kMsg - 1);
+    off[f] = FWD ? q : w[f] - 1 - q;
+    use[f] = e < 5 && q < w[f];
+  }
+  bool dead = false;
+  for (int st = 0; st < p.ns; ++st) {
+    LdsWait<1>(&ln.xReady, st + 1 - kHaloRing, G.err);
+    T v[2];
+    for (int spins = 0;;) {
+      bool empty = false;
+#pragma unroll
+      for (int f = 0; f < 2; ++f) {
+        v[f] = p.from[f] ? CoherentLoad(in[f]) : T(0);
+        empty |= use[f] && (unsigned)(st - off[f]) < (unsigned)p.nc && IsEmpty(v[f]) && p.from[f];
+      }
+      if (dead || !__any(empty)) break;
+      if (((++spins & 255) == 0 && (__builtin_amdgcn_readfirstlane(CoherentLoad(G.err)) & 2)) || spins > kSpinLimit) {
+        // a wait of this launch has timed out: stop waiting at all
+        __hip_atomic_fetch_or(G.err, 2, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        dead = true;
+      }
+    }
+#pragma unroll
+    for (int f = 0; f < 2; ++f) {
+      const int kk = st - off[f];
+      if (bt && !p.from[f] && use[f] && kk >= 0 && kk < p.nc) {
+        int i, j, k;
+        const int edgeA = FWD ? 0 : p.na - 1, edgeB = FWD ? 0 : p.nb - 1;
+        Map3(p.C, FWD ? kk : p.nc - 1 - kk, f == 0 ? edgeA : p.a * kPW + q, f == 0 ? p.b * kPW + q : edgeB, i, j, k);
+        v[f] = bt[e * b.nbf + BtSlot(b, (p.C + 1 + f) % 3, FWD ? 0 : 1, i, j, k)];
+      }
+      if (e < 5) ln.halo[f][e / kVecN<T>][kPW * (st % kHaloRing) + q].v[e % kVecN<T>] = v[f];
+      in[f] += kMsg;
+    }
+    LdsPost(&ln.haloReady, st + 1);
+  }
+}
+
+// empty this pencil's message slots of the other direction's pass (thread t
+// of n)
+template <typename T, bool FWD>
+__device__ __forceinline__ void PenEmpty(const PencilGroup &G, const DevBlock &b, const Pencil &p, int t, int n) {
+  T *const old = Messages<T, !FWD>(G, b, p, p.a, p.b, 0);
+  for (long q = t; q < 2L * b.pns * kMsg; q += n) old[q] = EmptySlot<T>();
+}
+
+// the connection term across C of a lane's first cell (zero off connections)
+template <typename T, bool FWD>
+__device__ __forceinline__ void PenFirst(const DevBlock &b, const Pencil &p, int lane, const T *bt, T out[5]) {
+  const int la = lane % kPW, lb = lane / kPW;
+  const bool conn = bt && la < p.wa && lb < p.wb;
+  int i, j, k;
+  Map3(p.C, FWD ? 0 : p.nc - 1, p.a * kPW + la, p.b * kPW + lb, i, j, k);
+  const long q = conn ? BtSlot(b, p.C, FWD ? 0 : 1, i, j, k) : 0;
+#pragma unroll
+  for (int e = 0; e < 5; ++e) out[e] = conn ? bt[e * b.nbf + q] : T(0);
+}
 
 // one step's slot from the sweep-ordered inputs
 template <typename T, bool FWD, bool FULL>
@@ -3197,12 +2880,6 @@ __device__ __forceinline__ void PenStage(const DevBlock &b, const Params &P, con
 #pragma unroll
     for (int q = 0; q < 3; ++q) dist[q] = T(F[(kPenF + q) * kPenLanes]);
   }
-  // (NotEmpty: no product may look like an empty message slot)
-#pragma unroll
-  for (int e = 0; e < 5; ++e) W[e] = NotEmpty(W[e]);
-#pragma unroll
-  for (int e = 0; e < kEarly<T, FULL>; ++e)
-    if (e < 6 || e >= 11) early[e] = NotEmpty(early[e]);
   T late[3][kLate<T>];
   if constexpr (sizeof(T) == 8) {
     PrimToCons(g, W, &early[6]);
@@ -3244,9 +2921,11 @@ __device__ __forceinline__ void PenStage(const DevBlock &b, const Params &P, con
 // formed.
 template <typename T, bool FWD, bool FULL, int C>
 __device__ __forceinline__ void PenCompute(const DevBlock &b, const Params &P, const Pencil &pen,
-                                           PenShared<T, FULL> &sh, int lane, int store, bool sends, int *err) {
+                                           PenShared<T, FULL> &sh, int lane, int store, int *err) {
   constexpr int sgn = FWD ? -1 : 1;  // direction of the dependency neighbours
   constexpr int V5 = Vecs<T>(5);
+  PenLink<T> &ln = sh.link;
+  const bool sends = pen.toA || pen.toB;
   const GasT<T> g = Cast<T>(P.gas);
   const auto byCvs = MakeDivisor(g.cvs);
   const int ns = pen.ns, nc = pen.nc;
@@ -3257,22 +2936,12 @@ __device__ __forceinline__ void PenCompute(const DevBlock &b, const Params &P, c
   // where the lane's incoming products lie: the neighbour lane's of the step
   // before, or the halo ring's
   const int nlA = min(max(lane + sgn, 0), kPenLanes - 1), nlB = min(max(lane + sgn * kPW, 0), kPenLanes - 1);
-  const LdsVec<T> *const inA = firstA ? &sh.halo[0][0][lb] : &sh.prod[0][0][0][nlA];
-  const LdsVec<T> *const inB = firstB ? &sh.halo[1][0][la] : &sh.prod[0][1][0][nlB];
+  const LdsVec<T> *const inA = firstA ? &ln.halo[0][0][lb] : &ln.prod[0][0][0][nlA];
+  const LdsVec<T> *const inB = firstB ? &ln.halo[1][0][la] : &ln.prod[0][1][0][nlB];
   constexpr int kProdStep = 2 * V5 * kPenLanes;  // vectors of one step of the product ring
   const int gA = pen.a * kPW + la, gB = pen.b * kPW + lb;
-  // the first cell of a lane takes the connection term across C (zero off
-  // connections)
   T oC[5];
-  {
-    const T *bt = OpBuf<T>::Bt(b);
-    int i, j, k;
-    Map3(C, FWD ? 0 : nc - 1, gA, gB, i, j, k);
-    const bool conn = bt && col;
-    const long q = conn ? BtSlot(b, C, FWD ? 0 : 1, i, j, k) : 0;
-#pragma unroll
-    for (int e = 0; e < 5; ++e) oC[e] = conn ? NotEmpty(bt[e * b.nbf + q]) : T(0);
-  }
+  PenFirst<T, FWD>(b, pen, lane, OpBuf<T>::Bt(b), oC);
   // du in the natural layout: a lane's cells follow each other along C
   T *const x = OpBuf<T>::X(b);
   int i0, j0, k0;
@@ -3283,7 +2952,7 @@ __device__ __forceinline__ void PenCompute(const DevBlock &b, const Params &P, c
   T xA[5], xB[5], early[kEarly<T, FULL>], late[3][kLate<T>];
   int next = 1;  // slot of the next step
   LdsWait<0>(&sh.stageReady[0], 1, err);
-  LdsWait<0>(&sh.haloReady, 1, err);
+  LdsWait<0>(&ln.haloReady, 1, err);
   int stage = LdsPeek(&sh.stageReady[next]), halo, sent;
   LdsGet<T, kEarly<T, FULL>>(&sh.slot[0].early[0][lane], early);
   LdsGet<T, 5>(inA, xA);
@@ -3316,7 +2985,7 @@ __device__ __forceinline__ void PenCompute(const DevBlock &b, const Params &P, c
     LdsGet<T, kEarly<T, FULL>>(&sl.early[0][lane], early);
     next = next + 1 == kPenSlots ? 0 : next + 1;
     stage = LdsPeek(&sh.stageReady[next]);
-    sent = LdsPeek(&sh.sentReady);
+    sent = LdsPeek(&ln.sentReady);
     // the updated state
     T Wu[5], H = T(0);
     StateChange<T> ch;
@@ -3339,21 +3008,21 @@ __device__ __forceinline__ void PenCompute(const DevBlock &b, const Params &P, c
     };
     // the product ring's place is free once its products have been sent
     if (sends && __builtin_amdgcn_readfirstlane(sent) < st + 1 - kProdRing)
-      LdsWait<0>(&sh.sentReady, st + 1 - kProdRing, err);
-    LdsVec<T> *const out = &sh.prod[st & (kProdRing - 1)][0][0][lane];
+      LdsWait<0>(&ln.sentReady, st + 1 - kProdRing, err);
+    LdsVec<T> *const out = &ln.prod[st & (kProdRing - 1)][0][0][lane];
     T o[5];
     product(1, o);
     LdsPut<T, 5>(out + V5 * kPenLanes, o);
     __builtin_amdgcn_sched_barrier(0);
-    halo = LdsPeek(&sh.haloReady);
+    halo = LdsPeek(&ln.haloReady);
     LdsGet<T, kLate<T>>(&sl.late[1][0][lane], late[1]);
     product(0, o);
     LdsPut<T, 5>(out, o);
     // this step's slot (read in the step before) and ring columns are free,
     // and its products are in LDS (a wave's LDS operations complete in order)
-    LdsPost(&sh.xReady, st + 1);
+    LdsPost(&ln.xReady, st + 1);
     __builtin_amdgcn_sched_barrier(0);
-    if (more && __builtin_amdgcn_readfirstlane(halo) < st + 2) LdsWait<0>(&sh.haloReady, st + 2, err);
+    if (more && __builtin_amdgcn_readfirstlane(halo) < st + 2) LdsWait<0>(&ln.haloReady, st + 2, err);
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
     const int ro = kPW * ((st + 1) % kHaloRing), po = kProdStep * (st & (kProdRing - 1));
     LdsGet<T, 5>(inB + (firstB ? ro : po), xB);
@@ -3385,126 +3054,316 @@ __global__ void __launch_bounds__(kPenWaves * kPenLanes) KLusgsPencil(PencilGrou
   const int tid = threadIdx.x, lane = tid % kPenLanes;
   const int wave = __builtin_amdgcn_readfirstlane(tid / kPenLanes);
   if (tid == 0) {
-    sh.ticket = (int)(__hip_atomic_fetch_add(G.ticket, 1ULL, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) %
-                      (unsigned long long)G.nent);
-    sh.haloReady = 0;
-    sh.xReady = 0;
-    sh.sentReady = 0;
+    sh.link.ticket = PencilTicket(G);
+    sh.link.haloReady = sh.link.xReady = sh.link.sentReady = 0;
   }
   if (tid < kPenSlots) sh.stageReady[tid] = 0;
   __syncthreads();
-  const int t = __builtin_amdgcn_readfirstlane(sh.ticket);
+  const int t = __builtin_amdgcn_readfirstlane(sh.link.ticket);
   const int4 ent = G.entries[FWD ? t : G.nent - 1 - t];
   const DevBlock b = G.blocks[ent.z];
-  const int C = b.pl, A = (C + 1) % 3, B = (C + 2) % 3;
-  const int na = AxisN(b, A), nb = AxisN(b, B);
-  Pencil pen;
-  pen.a = ent.x;
-  pen.b = ent.y;
-  pen.pid = pen.a + b.pa * pen.b;
-  pen.wa = PenWidth(na, pen.a);
-  pen.wb = PenWidth(nb, pen.b);
-  pen.nc = AxisN(b, C);
-  pen.ns = pen.wa + pen.wb + pen.nc - 2;
-  pen.rec = (long)pen.pid * b.pns;
-  pen.nrec = (long)b.pa * b.pb * b.pns;
-  const int sgn = FWD ? -1 : 1;  // direction of the dependency neighbours
-  const int ns = pen.ns, nc = pen.nc;
-  const T *bt = OpBuf<T>::Bt(b);
-  // messages of pencil (pa, pb) of this block through its face f (0 A, 1 B)
-  T *const msg0 = (T *)G.msg[FWD ? 0 : 1] + (long)ent.w * kMsg;
-  auto messages = [&](int pa, int pb, int f) { return msg0 + ((long)(pa + b.pa * pb) * 2 + f) * b.pns * kMsg; };
-
-  const int da = pen.a - sgn, db = pen.b - sgn;  // the pencils downstream
-  const bool toA = da >= 0 && da < b.pa, toB = db >= 0 && db < b.pb;
+  const Pencil pen = MakePencil<FWD>(b, ent);
   if (wave == 0) {
-    // ---- compute wave
     __builtin_amdgcn_s_setprio(3);
-    const bool sends = toA || toB;
-    if (C == 0) PenCompute<T, FWD, FULL, 0>(b, P, pen, sh, lane, store, sends, G.err);
-    else if (C == 1) PenCompute<T, FWD, FULL, 1>(b, P, pen, sh, lane, store, sends, G.err);
-    else PenCompute<T, FWD, FULL, 2>(b, P, pen, sh, lane, store, sends, G.err);
-  } else if (wave == 2) {
-    // ---- send wave: lane = (value e, entry q), as in the halo wave
-    if (!toA && !toB) return;
-    const int e = lane / kPW, q = lane % kPW;
-    // the columns whose products leave the pencil
-    const int cA = (FWD ? pen.wa - 1 : 0) + kPW * q, cB = q + kPW * (FWD ? pen.wb - 1 : 0);
-    const int offA = FWD ? pen.wa - 1 + q : pen.wa - 1 + pen.wb - 1 - q,
-              offB = FWD ? q + pen.wb - 1 : pen.wa - 1 - q + pen.wb - 1;
-    const bool useA = toA && e < 5 && q < pen.wb, useB = toB && e < 5 && q < pen.wa;
-    T *const mA = toA ? messages(da, pen.b, 0) + e * kPW + q - (long)(pen.wa - 1) * kMsg : nullptr;
-    T *const mB = toB ? messages(pen.a, db, 1) + e * kPW + q - (long)(pen.wb - 1) * kMsg : nullptr;
-    const int ev = e < 5 ? e / kVecN<T> : 0, er = e % kVecN<T>;
-    for (int st = 0; st < ns; ++st) {
-      LdsWait<1>(&sh.xReady, st + 1, G.err);
-      const T vA = sh.prod[st & (kProdRing - 1)][0][ev][cA].v[er], vB = sh.prod[st & (kProdRing - 1)][1][ev][cB].v[er];
-      // (no wait for the stores of the steps before)
-      asm volatile("" ::"v"(vA), "v"(vB));
-      LdsPost(&sh.sentReady, st + 1);
-      const int kA = st - offA, kB = st - offB;
-      if (useA && kA >= 0 && kA < nc) StoreCoherent(mA + (long)st * kMsg, vA);
-      if (useB && kB >= 0 && kB < nc) StoreCoherent(mB + (long)st * kMsg, vB);
-    }
+    if (pen.C == 0) PenCompute<T, FWD, FULL, 0>(b, P, pen, sh, lane, store, G.err);
+    else if (pen.C == 1) PenCompute<T, FWD, FULL, 1>(b, P, pen, sh, lane, store, G.err);
+    else PenCompute<T, FWD, FULL, 2>(b, P, pen, sh, lane, store, G.err);
   } else if (wave == 1) {
-    // ---- halo wave: lane = (value e, entry q); entry q of face A is the
-    // row lb = q, of face B the row la = q
-    const int e = lane / kPW, q = lane % kPW;
-    const int ua = pen.a + sgn, ub = pen.b + sgn;  // the pencils upstream
-    const bool from[2] = {ua >= 0 && ua < b.pa, ub >= 0 && ub < b.pb};
-    const int w[2] = {pen.wb, pen.wa};
-    const T *in[2];
-    int off[2];
-    bool use[2];
-#pragma unroll
-    for (int f = 0; f < 2; ++f) {
-      in[f] = messages(pen.a, pen.b, f) + min(lane, kMsg - 1);
-      off[f] = FWD ? q : w[f] - 1 - q;
-      use[f] = e < 5 && q < w[f];
-    }
-    bool dead = false;
-    for (int st = 0; st < ns; ++st) {
-      LdsWait<1>(&sh.xReady, st + 1 - kHaloRing, G.err);
-      T v[2];
-      for (int spins = 0;;) {
-        bool empty = false;
-#pragma unroll
-        for (int f = 0; f < 2; ++f) {
-          v[f] = from[f] ? CoherentLoad(in[f]) : T(0);
-          empty |= use[f] && (unsigned)(st - off[f]) < (unsigned)nc && IsEmpty(v[f]);
-        }
-        if (dead || !__any(empty)) break;
-        if (((++spins & 255) == 0 && (__builtin_amdgcn_readfirstlane(CoherentLoad(G.err)) & 2)) || spins > kSpinLimit) {
-          // a wait of this launch has timed out: stop waiting at all
-          __hip_atomic_fetch_or(G.err, 2, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-          dead = true;
-        }
-      }
-#pragma unroll
-      for (int f = 0; f < 2; ++f) {
-        const int kk = st - off[f];
-        if (bt && !from[f] && use[f] && kk >= 0 && kk < nc) {
-          // on a block face: the connection term (zero off connections)
-          int i, j, k;
-          const int edgeA = FWD ? 0 : na - 1, edgeB = FWD ? 0 : nb - 1;
-          Map3(C, FWD ? kk : nc - 1 - kk, f == 0 ? edgeA : pen.a * kPW + q, f == 0 ? pen.b * kPW + q : edgeB, i, j, k);
-          v[f] = NotEmpty(bt[e * b.nbf + BtSlot(b, f == 0 ? A : B, FWD ? 0 : 1, i, j, k)]);
-        }
-        if (e < 5) sh.halo[f][e / kVecN<T>][kPW * (st % kHaloRing) + q].v[e % kVecN<T>] = v[f];
-        in[f] += kMsg;
-      }
-      LdsPost(&sh.haloReady, st + 1);
-    }
+    PenHalo<T, FWD>(G, b, pen, sh.link, lane, OpBuf<T>::Bt(b));
+  } else if (wave == 2) {
+    PenSend<T, FWD>(G, b, pen, sh.link, lane);
   } else {
-    // ---- stager: steps j, j + kStagers, ...
+    // stager j: steps j, j + kStagers, ...
     const int j = wave - 3;
-    for (int st = j; st < ns; st += kStagers) {
-      PenStage<T, FWD, FULL>(b, P, pen, sh.slot[j], lane, st, &sh.xReady, G.err);
-      LdsStore(&sh.stageReady[j], st + 1);
+    for (int st = j; st < pen.ns; st += kStagers) {
+      PenStage<T, FWD, FULL>(b, P, pen, sh.slot[j], lane, st, &sh.link.xReady, G.err);
+      LdsPost(&sh.stageReady[j], st + 1);
     }
-    // empty this pencil's message slots of the other direction's pass
-    T *const old = (T *)G.msg[FWD ? 1 : 0] + ((long)ent.w + (long)pen.pid * 2 * b.pns) * kMsg;
-    for (long q = j * kPenLanes + lane; q < 2L * b.pns * kMsg; q += kStagers * kPenLanes) old[q] = EmptySlot<T>();
+    PenEmpty<T, FWD>(G, b, pen, j * kPenLanes + lane, kStagers * kPenLanes);
+  }
+}
+
+// ---------------------------------------------------------------------------
+// Block LU-SGS pencil sweep (blusgs): the scheme of KLusgsPencil with 5x5
+// blocks.  A cell's outgoing product across axis q is J_q du, J_q the block its
+// neighbour has for it (NeighbourBlock: this cell's Rusanov Jacobian at the
+// shared face with its thin-shear-layer Jacobian), and du = D^-1 (b + sum of
+// the incoming products).  Four stager waves a step (one for each of the three
+// blocks, one for D^-1, right-hand side or forward du, and the other-side sum
+// of a full sweep) form the next step in LDS; the compute wave applies the four
+// matrices, row by row in BlockMult's order, so the result is that of
+// KLusgsForward / KLusgsBackward bit for bit.
+//
+// Bound by the step, one wave's 195 FP64 operations and 54 16-byte LDS reads:
+// 1.08 us a step in FP64, 0.84 in FP32.  A pass over the eight blocks of the
+// 1.03M-cell channel takes 353 us (FP32 320), of eight blocks of 59 x 39 x 19
+// and smaller 188 (171), of 24 x 16 x 8 and smaller 71 (59); the tile sweep
+// with per-tile flags that was here before took 508 (494), 207 (317) and 83
+// (138), so it is gone.  FP32 waves of 168 registers hold two sets of stagers
+// without scratch (one set: 343, 195, 73 us); FP64 waves of 168 spill (820 us),
+// so one set with 256.
+constexpr int kBlkSlots = 2;
+template <typename T>
+constexpr int kBlkSets = sizeof(T) == 4 ? 2 : 1;  // groups of four stager waves, each taking every kBlkSets-th step
+template <typename T>
+constexpr int kBlkWaves = 3 + 4 * kBlkSets<T>;
+static_assert(kBlkSlots % kBlkSets<float> == 0 && kBlkSlots % kBlkSets<double> == 0, "a stager's slots");
+template <bool FULL>
+constexpr int kBlkR = FULL ? 10 : 5;  // right-hand side (forward du), other-side sum
+template <typename T, bool FULL>
+struct BlkSlot {
+  LdsVec<T> J[3][Vecs<T>(25)][kPenLanes];
+  LdsVec<T> D[kPenLanes * Vecs<T>(25)];  // the record of D^-1 as it is in memory, one cell behind the other
+  LdsVec<T> r[Vecs<T>(kBlkR<FULL>)][kPenLanes];
+};
+constexpr int kBlkParts = 4;  // blocks of A, B, C; the rest
+template <typename T, bool FULL>
+struct BlkShared {
+  BlkSlot<T, FULL> slot[kBlkSlots];
+  PenLink<T> link;
+  int ready[kBlkSlots];  // parts put into the slot so far: step st is there at kBlkParts (st / kBlkSlots + 1)
+};
+
+// one more part in a slot (the LDS writes before it are done, see LdsPost)
+__device__ __forceinline__ void LdsAdd(int *p) {
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  if (__lane_id() == 0) __hip_atomic_fetch_add(p, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+}
+
+// stager of the blocks of axis A + q: the cell's values and the face's
+struct BlkRaw {
+  double W[5], mu, kc, vg[9], a[4], dist;
+};
+template <bool FWD>
+__device__ __forceinline__ void BlkLoad(const DevBlock &b, const Params &P, const Pencil &pen, int q, int lane, int st,
+                                        BlkRaw &r) {
+  const long rec = pen.rec + (FWD ? st : pen.ns - 1 - st);
+  const int nF = kPenF + (P.visc.on ? 3 : 0);
+  const double *S = b.skS + rec * BlockRecord(P.visc.on) * kPenLanes + lane;
+  const double *F = b.skF + ((FWD ? pen.nrec : 0) + rec) * nF * kPenLanes + lane;
+#pragma unroll
+  for (int e = 0; e < 5; ++e) r.W[e] = S[e * kPenLanes];
+#pragma unroll
+  for (int e = 0; e < 4; ++e) r.a[e] = F[(4 * q + e) * kPenLanes];
+  if (P.visc.on) {
+    r.mu = S[10 * kPenLanes];
+    r.kc = S[11 * kPenLanes];
+#pragma unroll
+    for (int e = 0; e < 9; ++e) r.vg[e] = S[(12 + e) * kPenLanes];
+    r.dist = F[(kPenF + q) * kPenLanes];
+  }
+}
+// the block, formed in FP64 as NeighbourBlock forms it, in the operator's
+// precision
+template <typename T, bool FWD>
+__device__ __forceinline__ void BlkForm(const Params &P, const BlkRaw &r, T out[25]) {
+#pragma clang fp contract(off)
+  const GasT<double> g = Cast<double>(P.gas);
+  double J[25];
+  RusanovJacobian<double>(g, r.W, r.a[0], r.a[1], r.a[2], r.a[3], FWD, J);
+  if (P.visc.on) {
+    double V[25];
+    TSLJacobian(g, P.visc, r.W, r.mu, r.kc, make_double4(r.a[0], r.a[1], r.a[2], r.a[3]), r.dist, FWD, r.vg, V);
+#pragma unroll
+    for (int q = 0; q < 25; ++q) J[q] = FWD ? J[q] - V[q] : J[q] + V[q];
+  }
+#pragma unroll
+  for (int q = 0; q < 25; ++q) out[q] = T(J[q]);
+}
+
+template <typename T, bool FWD, bool FULL>
+__device__ __forceinline__ void BlkStage(const DevBlock &b, const Params &P, const Pencil &pen,
+                                         BlkShared<T, FULL> &sh, int lane, int set, int part, int *err) {
+  const int *xReady = &sh.link.xReady;
+  if (part < 3) {
+    BlkRaw r;
+    if (set < pen.ns) BlkLoad<FWD>(b, P, pen, part, lane, set, r);
+    for (int st = set; st < pen.ns; st += kBlkSets<T>) {
+      T J[25];
+      BlkForm<T, FWD>(P, r, J);
+      // the next step's loads are in flight while the slot is waited for
+      BlkLoad<FWD>(b, P, pen, part, lane, min(st + kBlkSets<T>, pen.ns - 1), r);
+      const int slot = st % kBlkSlots;
+      LdsWait<1>(xReady, st - kBlkSlots + 1, err);
+      LdsPut<T, 25>(&sh.slot[slot].J[part][0][lane], J);
+      LdsAdd(&sh.ready[slot]);
+    }
+    return;
+  }
+  constexpr int V = Vecs<T>(25);
+  T d[V * kVecN<T>], r[kBlkR<FULL>];
+  auto load = [&](int st) {
+    const long rec = pen.rec + (FWD ? st : pen.ns - 1 - st);
+    const LdsVec<T> *ai = (const LdsVec<T> *)OpBuf<T>::Abi(b) + rec * V * kPenLanes + lane;
+#pragma unroll
+    for (int q = 0; q < V; ++q) {
+      const LdsVec<T> w = ai[q * kPenLanes];
+#pragma unroll
+      for (int e = 0; e < kVecN<T>; ++e) d[q * kVecN<T> + e] = w.v[e];
+    }
+    if (FWD || FULL) {
+      const double *S = b.skS + (rec * BlockRecord(P.visc.on) + 5) * kPenLanes + lane;
+#pragma unroll
+      for (int e = 0; e < 5; ++e) r[e] = T(S[e * kPenLanes]);
+    } else {
+      const T *X = (const T *)b.skX + rec * 5 * kPenLanes + lane;
+#pragma unroll
+      for (int e = 0; e < 5; ++e) r[e] = X[e * kPenLanes];
+    }
+    if constexpr (FULL) {
+      const T *o = (const T *)b.skO + rec * 5 * kPenLanes + lane;
+#pragma unroll
+      for (int e = 0; e < 5; ++e) r[5 + e] = o[e * kPenLanes];
+    }
+  };
+  if (set < pen.ns) load(set);
+  for (int st = set; st < pen.ns; st += kBlkSets<T>) {
+    const int slot = st % kBlkSlots;
+    LdsWait<1>(xReady, st - kBlkSlots + 1, err);
+    LdsPut<T, V * kVecN<T>>(&sh.slot[slot].D[lane], d);
+    LdsPut<T, kBlkR<FULL>>(&sh.slot[slot].r[0][lane], r);
+    LdsAdd(&sh.ready[slot]);
+    load(min(st + kBlkSets<T>, pen.ns - 1));
+  }
+}
+
+template <typename T, bool FWD, bool FULL, int C>
+__device__ __forceinline__ void BlkCompute(const DevBlock &b, const Pencil &pen, BlkShared<T, FULL> &sh, int lane,
+                                           int store, const T *bt, int *err) {
+  constexpr int sgn = FWD ? -1 : 1;  // direction of the dependency neighbours
+  constexpr int V5 = Vecs<T>(5);
+  PenLink<T> &ln = sh.link;
+  const bool sends = pen.toA || pen.toB;
+  const int ns = pen.ns, nc = pen.nc;
+  const int la = lane % kPW, lb = lane / kPW;
+  const bool col = la < pen.wa && lb < pen.wb;
+  const int off = FWD ? la + lb : (pen.wa - 1 - la) + (pen.wb - 1 - lb);
+  const bool firstA = FWD ? la == 0 : la == pen.wa - 1, firstB = FWD ? lb == 0 : lb == pen.wb - 1;
+  const int nlA = min(max(lane + sgn, 0), kPenLanes - 1), nlB = min(max(lane + sgn * kPW, 0), kPenLanes - 1);
+  const LdsVec<T> *const inA = firstA ? &ln.halo[0][0][lb] : &ln.prod[0][0][0][nlA];
+  const LdsVec<T> *const inB = firstB ? &ln.halo[1][0][la] : &ln.prod[0][1][0][nlB];
+  constexpr int kProdStep = 2 * V5 * kPenLanes;  // vectors of one step of the product ring
+  T oC[5];
+  PenFirst<T, FWD>(b, pen, lane, bt, oC);
+  T *const x = OpBuf<T>::X(b);
+  int i0, j0, k0;
+  Map3(C, FWD ? -off : nc - 1 + off, pen.a * kPW + la, pen.b * kPW + lb, i0, j0, k0);
+  const int sC = -sgn * (C == 0 ? 1 : (C == 1 ? b.ni : b.ni * b.nj));
+  int p = i0 + j0 * b.ni + k0 * b.ni * b.nj;  // cell of step st (of the active steps)
+  T *Xs = (T *)b.skX + pen.rec * 5 * kPenLanes + lane;
+  T xA[5], xB[5], d[25], r[kBlkR<FULL>], JA[25], JB[25];
+  LdsWait<0>(&sh.ready[0], kBlkParts, err);
+  LdsGet<T, 25, 1>(&sh.slot[0].D[lane * Vecs<T>(25)], d);
+  LdsGet<T, kBlkR<FULL>>(&sh.slot[0].r[0][lane], r);
+  LdsWait<0>(&ln.haloReady, 1, err);
+  LdsGet<T, 5>(inA, xA);
+  LdsGet<T, 5>(inB, xB);
+  for (int st = 0; st < ns; ++st) {
+    const bool more = st + 1 < ns;
+    const int cur = st % kBlkSlots, next = (st + 1) % kBlkSlots;
+    const BlkSlot<T, FULL> &sl = sh.slot[cur], &nx = sh.slot[next];
+    // the dependency-side sum, i, j, k order from +0 (see PenCompute)
+    T xn[5], v[5], o[5];
+#pragma unroll
+    for (int e = 0; e < 5; ++e) {
+      const T o0 = C == 2 ? xA[e] : (C == 0 ? oC[e] : xB[e]), o1 = C == 2 ? xB[e] : (C == 0 ? xA[e] : oC[e]),
+              o2 = C == 2 ? oC[e] : (C == 0 ? xB[e] : xA[e]);
+      const T D = ((T(0) + o0) + o1) + o2;
+      if constexpr (FULL) v[e] = FWD ? r[e] + (D - r[5 + e]) : (r[e] + r[5 + e]) - D;
+      else v[e] = FWD ? r[e] + D : D;
+    }
+    BlockMult<T>(d, v, xn);
+    if constexpr (!FULL && !FWD) {
+#pragma unroll
+      for (int e = 0; e < 5; ++e) xn[e] = r[e] - xn[e];
+    }
+    __builtin_amdgcn_sched_barrier(0);
+    LdsGet<T, 25>(&sl.J[1][0][lane], JB);
+    LdsGet<T, 25>(&sl.J[0][0][lane], JA);
+    const int ready = LdsPeek(&sh.ready[next]), need = kBlkParts * ((st + 1) / kBlkSlots + 1);
+    const int sent = LdsPeek(&ln.sentReady);
+    BlockMult<T>(JB, xn, o);
+    // the product ring's place is free once its products have been sent
+    if (sends && __builtin_amdgcn_readfirstlane(sent) < st + 1 - kProdRing)
+      LdsWait<0>(&ln.sentReady, st + 1 - kProdRing, err);
+    LdsVec<T> *const out = &ln.prod[st & (kProdRing - 1)][0][0][lane];
+    LdsPut<T, 5>(out + V5 * kPenLanes, o);
+    __builtin_amdgcn_sched_barrier(0);
+    LdsGet<T, 25>(&sl.J[2][0][lane], JB);
+    const int halo = LdsPeek(&ln.haloReady);
+    BlockMult<T>(JA, xn, o);
+    LdsPut<T, 5>(out, o);
+    // the slot has been read, its products are in LDS
+    LdsPost(&ln.xReady, st + 1);
+    __builtin_amdgcn_sched_barrier(0);
+    if (more && __builtin_amdgcn_readfirstlane(ready) < need) LdsWait<0>(&sh.ready[next], need, err);
+    const int kk = st - off;
+    const bool act = col && kk >= 0 && kk < nc;
+    if constexpr (sizeof(T) == 8) {
+      if (act) BlockMult<T>(JB, xn, oC);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    LdsGet<T, kBlkR<FULL>>(&nx.r[0][lane], r);
+    LdsGet<T, 25, 1>(&nx.D[lane * Vecs<T>(25)], d);
+    if (more && __builtin_amdgcn_readfirstlane(halo) < st + 2) LdsWait<0>(&ln.haloReady, st + 2, err);
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    const int ro = kPW * ((st + 1) % kHaloRing), po = kProdStep * (st & (kProdRing - 1));
+    LdsGet<T, 5>(inB + (firstB ? ro : po), xB);
+    LdsGet<T, 5>(inA + (firstA ? ro : po), xA);
+    __builtin_amdgcn_sched_barrier(0);
+    if (act) {
+      if constexpr (sizeof(T) == 4) BlockMult<T>(JB, xn, oC);
+      if (store & 1) {
+#pragma unroll
+        for (int e = 0; e < 5; ++e) x[e * b.ncell + p] = xn[e];
+      }
+    }
+    if (FWD && !FULL && (store & 2)) {
+#pragma unroll
+      for (int e = 0; e < 5; ++e) Xs[e * kPenLanes] = xn[e];
+    }
+    p += sC;
+    Xs += 5 * kPenLanes;
+  }
+}
+
+// `store` as in KLusgsPencil.  The first forward pass starts from du = 0, so
+// its connection terms are zero (J 0 sums to +0) and are not formed.
+template <typename T, bool FWD, bool FULL>
+__global__ void __launch_bounds__(kBlkWaves<T> * kPenLanes) KBlockPencil(PencilGroup G, Params P, int store) {
+  __shared__ BlkShared<T, FULL> sh;
+  const int tid = threadIdx.x, lane = tid % kPenLanes;
+  const int wave = __builtin_amdgcn_readfirstlane(tid / kPenLanes);
+  if (tid == 0) {
+    sh.link.ticket = PencilTicket(G);
+    sh.link.haloReady = sh.link.xReady = sh.link.sentReady = 0;
+  }
+  if (tid < kBlkSlots) sh.ready[tid] = 0;
+  __syncthreads();
+  const int t = __builtin_amdgcn_readfirstlane(sh.link.ticket);
+  const int4 ent = G.entries[FWD ? t : G.nent - 1 - t];
+  const DevBlock b = G.blocks[ent.z];
+  const Pencil pen = MakePencil<FWD>(b, ent);
+  const T *bt = FWD && !FULL ? nullptr : OpBuf<T>::Bt(b);
+  if (wave == 0) {
+    __builtin_amdgcn_s_setprio(3);
+    if (pen.C == 0) BlkCompute<T, FWD, FULL, 0>(b, pen, sh, lane, store, bt, G.err);
+    else if (pen.C == 1) BlkCompute<T, FWD, FULL, 1>(b, pen, sh, lane, store, bt, G.err);
+    else BlkCompute<T, FWD, FULL, 2>(b, pen, sh, lane, store, bt, G.err);
+  } else if (wave == 1) {
+    PenHalo<T, FWD>(G, b, pen, sh.link, lane, bt);
+  } else if (wave == 2) {
+    PenSend<T, FWD>(G, b, pen, sh.link, lane);
+  } else {
+    // waves 4 and 8 share the compute wave's SIMD (waves are dealt to the four
+    // SIMDs in turn): they take the light part
+    constexpr int kSets = kBlkSets<T>;
+    const int heavy = wave == 3 ? 0 : wave - 4 - (wave - 5) / 4;  // 3, 5, 6, 7, 9, 10
+    const bool light = wave % 4 == 0;
+    BlkStage<T, FWD, FULL>(b, P, pen, sh, lane, light ? wave / 4 - 1 : heavy % kSets, light ? 3 : heavy / kSets, G.err);
+    PenEmpty<T, FWD>(G, b, pen, (wave - 3) * kPenLanes + lane, 4 * kBlkSets<T> * kPenLanes);
   }
 }
 

@@ -93,7 +93,9 @@ struct ath_ctx {
   int device = 0;
   hipStream_t stream = nullptr;
   int anyPark = 0;  // some block parks its wall cells' inviscid block sums (DevBlock::invPark)
-  int rhsFormed = 0;  // the last residual stage formed the relax's right-hand side (RhsInDiag)
+  int rhsFormed = 0;  // the last residual stage formed the relax's right-hand side (RhsInDiag); 2: to keep
+                      // even when the state changes before the relax
+  int stateSet = 0;   // a state or a stored solution level changed since
   ath::HostCase hc;  // the case (a single-case context) or the numerics every case shares (a server)
   ath::Params P{};
   // the resident cases; blk concatenates the blocks of the cases that
@@ -129,13 +131,6 @@ struct ath_ctx {
   int nhalo = 0;
   ath::ConnTask *dconn = nullptr;
   int nconn = 0;
-  // block solvers: one tiled sweep over all blocks, 8 x 8 x 4 tiles with a
-  // lane per cell (msweep, ATH_SWEEP_TILED) or two lanes per cell, each
-  // holding some of the cell's rows (rsweep, ATH_SWEEP_ROWS)
-  ath::MultiSweepCtl msweep{};
-  int msweepGrid = 0;
-  ath::MultiSweepCtl rsweep{};
-  int rsweepGrid = 0;
   // unit grids of the all-block launches (ath::BlockMap), kNumMaps of them,
   // nb entries each, and each one's total unit count
   int4 *dmaps = nullptr;
@@ -187,12 +182,11 @@ constexpr int kBlk = 256;
 
 int Grid(long n, int b = kBlk) { return (int)((n + b - 1) / b); }
 
-// the unit grids of the all-block launches: 8x8x4 tiles (residual and
-// viscous flux), ranges of 128 cells (block diagonal), of 256 cells (matrix
-// residual, update, initialisation; their partials are the reductions'
-// slots), of 256 padded cells (auxiliary variables) and of 256 lanes of the
+// the unit grids of the all-block launches: 8x8x4 tiles (residual, viscous
+// flux), the block diagonal's tiles, ranges of 256 cells (matrix residual,
+// update, initialisation; the partials of the reductions are their slots), of 256 padded cells (auxiliary variables) and of 256 lanes of the
 // pencil sweep's records
-enum { kMapTile = 0, kMapCell128 = 1, kMapCell256 = 2, kMapPad256 = 3, kMapPen256 = 4, kNumMaps = 5 };
+enum { kMapTile = 0, kMapDiag = 1, kMapCell256 = 2, kMapPad256 = 3, kMapPen256 = 4, kNumMaps = 5 };
 // the ghost-cell task tables: boundary patches, edge lines of the inviscid
 // and of the viscous pass, no-slip wall cells
 enum { kTaskBc = 0, kTaskEdgeInv = 1, kTaskEdgeVisc = 2, kTaskWall = 3, kNumTaskMaps = 4 };
@@ -511,7 +505,11 @@ int RebuildGroup(ath_ctx *c);
 
 // cases whose relax can run in the pencil order (EffectiveOrder)
 bool PencilCase(const ath::HostCase &hc) {
-  return hc.Implicit() && hc.solver == ath::Solver::LUSGS && !hc.block && !hc.roeJac;
+  return hc.Implicit() && hc.solver == ath::Solver::LUSGS && !hc.roeJac;
+}
+// values of one record of DevBlock::skS
+int RecordValues(const ath::HostCase &hc) {
+  return hc.block ? ath::BlockRecord(hc.viscous) : ath::kPenS + (hc.viscous ? 1 : 0);
 }
 // pencils run along the block's longest axis: the fewest column handoffs
 // (each costs several steps) and the fewest idle steps (2 kPW - 2 a pencil)
@@ -525,6 +523,12 @@ void PencilGrid(const ath::HostBlock &h, int *pl, int *pa, int *pb, int *pns) {
   *pns = h.N(l) + 2 * ath::kPW - 2;
 }
 
+// values of the block solvers' inverse diagonal (InverseBase in the kernels)
+template <typename T>
+long InverseSize(const ath::DevBlock &d) {
+  return d.pns ? (long)ath::kInv<T> * ath::kPenLanes * d.pa * d.pb * d.pns : 25L * 256 * d.tni * d.tnj * d.tnk;
+}
+
 int AllocFp32(ath_ctx *c, ath::DevBlock &d) {
   if (d.x32) return ATH_OK;
   if (int r = c->Alloc(&d.Ainv32, d.ncell)) return r;
@@ -536,10 +540,9 @@ int AllocFp32(ath_ctx *c, ath::DevBlock &d) {
     HIP_OK(hipMemset(d.bt32, 0, 5 * d.nbf * sizeof(float)));
   }
   if (d.Abi) {
-    // block solvers: D^-1 rounded to float in the tile-blocked layout
-    const long tb = 25L * 256 * d.tni * d.tnj * d.tnk;
-    if (int r = c->Alloc(&d.Abi32, tb)) return r;
-    HIP_OK(hipMemset(d.Abi32, 0, tb * sizeof(float)));
+    // block solvers: D^-1 rounded to float
+    if (int r = c->Alloc(&d.Abi32, InverseSize<float>(d))) return r;
+    HIP_OK(hipMemset(d.Abi32, 0, InverseSize<float>(d) * sizeof(float)));
   }
   return ATH_OK;
 }
@@ -668,10 +671,12 @@ int UploadCase(ath_ctx *c, CaseRes &cr, bool fp32) {
     if (int r = c->Alloc(&d.consNm1, 5 * nc)) return r;
     if (int r = c->Alloc(&d.x, 5 * nc)) return r;
     if (int r = c->Alloc(&d.xold, 5 * nc)) return r;
-    if (int r = c->Alloc(&d.rhs, 5 * nc)) return r;
     HIP_OK(hipMemset(d.x, 0, 5 * nc * sizeof(double)));
     HIP_OK(hipMemset(d.A, 0, nc * sizeof(double)));
     d.Ab = d.Abi = nullptr;
+    d.skF = d.skS = d.skX = d.skO = nullptr;
+    d.pl = d.pa = d.pb = d.pns = 0;
+    if (PencilCase(hc)) PencilGrid(h, &d.pl, &d.pa, &d.pb, &d.pns);
     d.vgrad = nullptr;
     d.invPark = nullptr;
     d.kc = nullptr;
@@ -680,10 +685,8 @@ int UploadCase(ath_ctx *c, CaseRes &cr, bool fp32) {
     d.tnj = (h.nj + 7) / 8;
     d.tnk = (h.nk + 3) / 4;
     if (hc.block) {
-      // tile-blocked per-cell blocks: 25 entries of 256 cells per 8x8x4 tile
-      const long tb = 25L * 256 * d.tni * d.tnj * d.tnk;
       if (int r = c->Alloc(&d.Ab, 25 * nc)) return r;
-      if (int r = c->Alloc(&d.Abi, tb)) return r;
+      if (int r = c->Alloc(&d.Abi, InverseSize<double>(d))) return r;
       for (int dd = 0; dd < 3; ++dd) {
         const long nf = (long)(h.ni + (dd == 0)) * (h.nj + (dd == 1)) * (h.nk + (dd == 2));
         if (hc.viscous)
@@ -718,19 +721,16 @@ int UploadCase(ath_ctx *c, CaseRes &cr, bool fp32) {
     }
     if (hc.viscous)
       if (int r = UploadViscous(c, hc, h, br)) return r;
-    // scalar LU-SGS: the pencil sweep's arrays, pencils along the longest axis
-    d.skF = d.skS = d.skX = d.skO = nullptr;
-    d.pl = d.pa = d.pb = d.pns = 0;
-    if (PencilCase(hc)) {
-      PencilGrid(h, &d.pl, &d.pa, &d.pb, &d.pns);
+    // the pencil sweep's arrays
+    if (d.pns) {
       const size_t lanes = (size_t)d.pa * d.pb * d.pns * kPenLanes;
-      const int nS = kPenS + (hc.viscous ? 1 : 0), nF = kPenF + (hc.viscous ? 3 : 0);
+      const int nS = RecordValues(hc), nF = kPenF + (hc.viscous ? 3 : 0);
       if (int r = c->Alloc(&d.skF, 2 * nF * lanes)) return r;
       if (int r = c->Alloc(&d.skS, nS * lanes)) return r;
       if (int r = c->Alloc(&d.skX, 5 * lanes)) return r;
       if (hc.InitMatrix())
         if (int r = c->Alloc(&d.skO, 5 * lanes)) return r;
-      hipLaunchKernelGGL(KPencilFaces, dim3(Grid((long)lanes)), dim3(kBlk), 0, nullptr, d, hc.viscous ? 1 : 0);
+      hipLaunchKernelGGL(KPencilFaces, dim3(Grid((long)lanes)), dim3(kBlk), 0, nullptr, d, hc.viscous ? 1 : 0, nS);
       HIP_OK(hipGetLastError());
     }
     // hyperplane order
@@ -859,8 +859,6 @@ int RebuildGroup(ath_ctx *c) {
   c->nhalo = c->nconn = 0;
   c->nparts = 0;
   c->pen = PencilGroup{};
-  c->msweep = MultiSweepCtl{};
-  c->rsweep = MultiSweepCtl{};
   for (int q = 0; q < kNumMaps; ++q) c->mapTotal[q] = 0;
   for (int q = 0; q < kNumTaskMaps; ++q) c->taskTotal[q] = 0;
   if (nb == 0) return ATH_OK;
@@ -909,8 +907,10 @@ int RebuildGroup(ath_ctx *c) {
       if (q == kMapTile)
         u = make_int4((d.ni + ath::kTI - 1) / ath::kTI, (d.nj + ath::kTJ - 1) / ath::kTJ,
                       (d.nk + ath::kTK - 1) / ath::kTK, f);
-      else if (q == kMapCell128) u = make_int4(Grid(d.ncell, 128), 1, 1, f);
-      else if (q == kMapCell256) u = make_int4(Grid(d.ncell, ath::kRedThreads), 1, 1, f);
+      else if (q == kMapDiag && d.pns)
+        u = make_int4(Grid(d.ni, ath::kDiagTile[d.pl][0]), Grid(d.nj, ath::kDiagTile[d.pl][1]),
+                      Grid(d.nk, ath::kDiagTile[d.pl][2]), f);
+      else if (q == kMapDiag || q == kMapCell256) u = make_int4(Grid(d.ncell, ath::kRedThreads), 1, 1, f);
       else if (q == kMapPad256) u = make_int4(Grid(d.npad, 256), 1, 1, f);
       else u = make_int4(d.skS ? Grid((long)d.pa * d.pb * d.pns * kPenLanes, 256) : 0, 1, 1, f);
       v[(size_t)q * nb + b] = u;
@@ -1002,50 +1002,6 @@ int RebuildGroup(ath_ctx *c) {
     g.err = c->dflag;
     g.blocks = c->dblocks;
   }
-  // block solvers: one tiled sweep over all blocks, tiles by tile hyperplane,
-  // then block, then k, j, i; per block its tile grid and first flag
-  if (c->hc.block) {
-    hipDeviceProp_t prop;
-    HIP_OK(hipGetDeviceProperties(&prop, c->device));
-    // the tiles of every block by tile hyperplane, then block, then k, j, i;
-    // per block its tile grid and first flag
-    auto queue = [&](int TI, int TJ, int TK, MultiSweepCtl &m) -> int {
-      std::vector<int4> grid, tiles;
-      int base = 0, maxPlane = 0;
-      for (auto &br : c->blk) {
-        const int ta = (br.d.ni + TI - 1) / TI, tb = (br.d.nj + TJ - 1) / TJ, tc = (br.d.nk + TK - 1) / TK;
-        grid.push_back(make_int4(ta, tb, tc, base));
-        base += ta * tb * tc;
-        maxPlane = std::max(maxPlane, ta + tb + tc - 2);
-      }
-      for (int pl = 0; pl < maxPlane; ++pl)
-        for (size_t q = 0; q < grid.size(); ++q)
-          for (int cc = 0; cc < grid[q].z; ++cc)
-            for (int bb = 0; bb < grid[q].y; ++bb)
-              for (int aa = 0; aa < grid[q].x; ++aa)
-                if (aa + bb + cc == pl) tiles.push_back(make_int4(aa, bb, cc, (int)q));
-      m.ntiles = (int)tiles.size();
-      int4 *dt = nullptr, *dg = nullptr;
-      if (int r = c->Alloc(&dt, tiles.size())) return r;
-      if (int r = c->Alloc(&dg, grid.size())) return r;
-      HIP_OK(hipMemcpy(dt, tiles.data(), tiles.size() * sizeof(int4), hipMemcpyHostToDevice));
-      HIP_OK(hipMemcpy(dg, grid.data(), grid.size() * sizeof(int4), hipMemcpyHostToDevice));
-      m.tiles = dt;
-      m.grid = dg;
-      if (int r = c->Alloc(&m.flags, base)) return r;
-      if (int r = c->Alloc(&m.ticket, 2)) return r;
-      HIP_OK(hipMemset(m.flags, 0, base * sizeof(int)));
-      HIP_OK(hipMemset(m.ticket, 0, 2 * sizeof(int)));
-      m.epoch = m.ticket + 1;
-      m.err = c->dflag;
-      return ATH_OK;
-    };
-    if (int r = queue(kBTI, kBTJ, kBTK, c->msweep)) return r;
-    if (int r = queue(kBTI, kBTJ, kBTK, c->rsweep)) return r;
-    c->msweepGrid = std::max(1, std::min(c->msweep.ntiles, 2 * prop.multiProcessorCount));
-    // one 512-thread workgroup fits a CU (registers)
-    c->rsweepGrid = std::max(1, std::min(c->rsweep.ntiles, prop.multiProcessorCount));
-  }
   return ATH_OK;
 }
 
@@ -1128,30 +1084,31 @@ void LaunchConnTerms(ath_ctx *c) {
 
 int EffectiveOrder(const ath_ctx *c);
 
-// the relax's initialisation (right-hand side once per relax, du = 0) is
-// formed by the viscous block diagonal: one-sweep block LU-SGS with the FP64
-// operator in the row-parallel order, viscous terms on.  A one-sweep relax
-// never reads its initial du, so a relax repeated without a new residual
-// gives the same result.
-bool RhsInDiag(const ath_ctx *c) {
-  return c->P.block && c->P.visc.on && !c->fp32 && c->hc.solver == ath::Solver::LUSGS &&
-         !c->hc.InitMatrix() && EffectiveOrder(c) == ATH_SWEEP_ROWS;
+// block LU-SGS in the pencil sweep (every order but the hyperplane one)
+bool BlockPencil(const ath_ctx *c) {
+  return c->P.block && c->hc.solver == ath::Solver::LUSGS && EffectiveOrder(c) != ATH_SWEEP_HYPERPLANE;
 }
+// the right-hand side of a one-sweep relax in that sweep is formed by the
+// block diagonal; such a relax reads no du it has not written
+bool RhsInDiag(const ath_ctx *c) { return BlockPencil(c) && !c->hc.InitMatrix(); }
 
 template <int RECON, int LIM, int FLUX>
 void LaunchResidualT(ath_ctx *c) {
   const ath::Params &P = c->P;
-  const ath::BlockMap mt = c->Map(kMapTile), mc = c->Map(kMapCell128), mp = c->Map(kMapPad256);
-  const dim3 tiles(c->mapTotal[kMapTile]), cells(c->mapTotal[kMapCell128]);
+  const ath::BlockMap mt = c->Map(kMapTile), mc = c->Map(kMapCell256), md = c->Map(kMapDiag), mp = c->Map(kMapPad256);
+  const dim3 tiles(c->mapTotal[kMapTile]), cells(c->mapTotal[kMapCell256]),
+             diag(c->mapTotal[kMapDiag]);
   hipLaunchKernelGGL((ath::KResidual<RECON, LIM, FLUX>), tiles, dim3(256), 0, c->stream, mt, P);
   if (P.block) {
     // inviscid block sum from the inviscid ghost states: finished here, or,
     // for the cells next to a viscous wall, parked in Ab until the viscous
     // pass has formed dt (the other cells form it then)
-    if (!P.visc.on)
-      hipLaunchKernelGGL((ath::KBlockDiag<RECON, LIM, 0>), cells, dim3(128), 0, c->stream, mc, P);
-    else if (c->anyPark)
-      hipLaunchKernelGGL((ath::KBlockDiag<RECON, LIM, 1>), cells, dim3(128), 0, c->stream, mc, P);
+    if (!P.visc.on) {
+      ath::Params PD = P;
+      c->rhsFormed = PD.rhsInDiag = RhsInDiag(c) ? 1 : 0;
+      hipLaunchKernelGGL((ath::KBlockDiag<RECON, LIM, 0>), diag, dim3(256), 0, c->stream, md, PD);
+    } else if (c->anyPark)
+      hipLaunchKernelGGL((ath::KBlockDiag<RECON, LIM, 1>), cells, dim3(256), 0, c->stream, mc, P);
   }
   if (!P.visc.on) return;
   // viscous ghost cells, temperature and viscosity, viscous fluxes
@@ -1173,11 +1130,11 @@ void LaunchResidualT(ath_ctx *c) {
   if (P.block) {
     ath::Params PD = P;
     PD.rhsInDiag = RhsInDiag(c) ? 1 : 0;
-    c->rhsFormed = PD.rhsInDiag;
+    c->rhsFormed = PD.rhsInDiag ? (c->fp32 ? 1 : 2) : 0;
     if (P.visc.recon4)
-      hipLaunchKernelGGL((ath::KBlockDiag<RECON, LIM, 3>), cells, dim3(128), 0, c->stream, mc, PD);
+      hipLaunchKernelGGL((ath::KBlockDiag<RECON, LIM, 3>), diag, dim3(256), 0, c->stream, md, PD);
     else
-      hipLaunchKernelGGL((ath::KBlockDiag<RECON, LIM, 2>), cells, dim3(128), 0, c->stream, mc, PD);
+      hipLaunchKernelGGL((ath::KBlockDiag<RECON, LIM, 2>), diag, dim3(256), 0, c->stream, md, PD);
   }
 }
 
@@ -1192,6 +1149,7 @@ void LaunchAfterResiduals(ath_ctx *c) {
 // the residual stage of every block: one launch per kernel over all blocks
 void LaunchResidual(ath_ctx *c) {
   c->rhsFormed = 0;
+  c->stateSet = 0;
   const auto &hc = c->hc;
   const int recon = (int)hc.recon;
   const int lim = (int)hc.limiter;
@@ -1208,12 +1166,11 @@ void LaunchResidual(ath_ctx *c) {
 #undef ATH_RES
 }
 
-// the order the sweeps run in: the block solvers have the row-parallel,
-// tiled and hyperplane orders (the pencil order maps to the row-parallel
-// one with the FP64 operator and to the tiled one with the FP32 operator,
-// the faster of the two for each on the 1 M-cell channel), scalar LU-SGS
-// the pencil, tiled and hyperplane orders (the row-parallel order maps to
-// the tiled one); the Roe flux-change off-diagonals (approximateRoe) run in
+// the order in effect: the block solvers have the pencil order, under the names
+// ATH_SWEEP_ROWS and ATH_SWEEP_TILED, and the hyperplane order (the pencil
+// order is reported as the first with the FP64 operator and as the second with
+// the FP32 operator, as callers know them), scalar LU-SGS the pencil, tiled and
+// hyperplane orders (ATH_SWEEP_ROWS maps to the tiled one); the Roe flux-change off-diagonals (approximateRoe) run in
 // the hyperplane order only
 int EffectiveOrder(const ath_ctx *c) {
   if (c->P.roeJac) return ATH_SWEEP_HYPERPLANE;
@@ -1233,79 +1190,56 @@ int LaunchRelaxT(ath_ctx *c, bool timed, size_t evBase) {
     if (timed) hipEventRecord(c->evs[evBase + 2 * pass + (begin ? 0 : 1)], c->stream);
     if (!begin) ++pass;
   };
-  // the row-parallel block sweep reads the right-hand side that the
-  // initialisation forms once per relax
+  // The block pencil sweep reads the right-hand side formed once, by the
+  // residual stage or here (the sweep order, the state or a stored solution
+  // level may have changed in between; the viscous FP64 stage's is kept then),
+  // and the state, refreshed here if it changed in between.  A one-sweep pencil
+  // relax writes every du before anything but the scalar connection terms
+  // reads it.
+  const bool blkPencil = BlockPencil(c),
+             formed = RhsInDiag(c) && c->rhsFormed && (!c->stateSet || (c->rhsFormed == 2 && !c->fp32));
   ath::Params P0 = c->P;
-  P0.rhsOnce = (hc.solver == ath::Solver::LUSGS && c->P.block && EffectiveOrder(c) == ATH_SWEEP_ROWS) ? 1 : 0;
-  // (formed by the residual stage unless the sweep order changed since); a
-  // one-sweep pencil relax writes every du before anything but the
-  // connection terms reads it
-  const bool pencilOnce = hc.solver == ath::Solver::LUSGS && !hc.InitMatrix() && EffectiveOrder(c) == ATH_SWEEP_PENCIL &&
-                          c->nconn == 0;
-  if (!(RhsInDiag(c) && c->rhsFormed) && !pencilOnce)
+  P0.rhsOnce = blkPencil && !formed ? 1 : 0;
+  P0.copyState = blkPencil && c->stateSet ? 1 : 0;
+  const bool pencilOnce = hc.solver == ath::Solver::LUSGS && !hc.InitMatrix() &&
+                          (blkPencil ? formed && !c->stateSet
+                                     : EffectiveOrder(c) == ATH_SWEEP_PENCIL && c->nconn == 0);
+  if (!pencilOnce)
     hipLaunchKernelGGL(ath::KInitUpdate<T>, dim3(c->mapTotal[kMapCell256]), dim3(kBlk), 0, c->stream,
                        c->Map(kMapCell256), P0);
   for (int sw = 0; sw < hc.sweeps; ++sw) {
     const int full = (sw > 0 || hc.InitMatrix()) ? 1 : 0;
     const int order = EffectiveOrder(c);
-    if (hc.solver == ath::Solver::LUSGS && order == ATH_SWEEP_PENCIL) {
+    if (blkPencil || (hc.solver == ath::Solver::LUSGS && order == ATH_SWEEP_PENCIL)) {
       const dim3 units(c->mapTotal[kMapPen256]);
       const ath::BlockMap mp = c->Map(kMapPen256);
-      if (sw == 0) hipLaunchKernelGGL(ath::KPencilPrep<T>, units, dim3(kBlk), 0, c->stream, mp, c->P);
+      if (sw == 0 && !blkPencil)
+        hipLaunchKernelGGL(ath::KPencilPrep<T>, units, dim3(kBlk), 0, c->stream, mp, c->P);
       for (int dir = 0; dir < 2; ++dir) {
-        LaunchConnTerms<T>(c);
+        // the first forward pass of a block solver starts from du = 0: its
+        // connection terms are zero and the sweep does not read them
+        if (!blkPencil || dir > 0 || full) LaunchConnTerms<T>(c);
         mark(true);
-        // every block's pencils in one launch
-        const dim3 grid(c->pen.nent), blk(ath::kPenWaves * ath::kPenLanes);
-        // a one-sweep forward pass hands du to the backward pass in sweep
-        // order; the connection terms and the other-side sums read the
-        // natural layout
-        const int store = dir == 0 && !full ? (c->nconn > 0 ? 3 : 2) : 1;
-        if (dir == 0 && full) {
-          hipLaunchKernelGGL((ath::KPencilOther<T, true>), units, dim3(kBlk), 0, c->stream, mp, c->P);
-          hipLaunchKernelGGL((ath::KLusgsPencil<T, true, true>), grid, blk, 0, c->stream, c->pen, c->P, store);
-        } else if (dir == 0) {
-          hipLaunchKernelGGL((ath::KLusgsPencil<T, true, false>), grid, blk, 0, c->stream, c->pen, c->P, store);
-        } else if (full) {
-          hipLaunchKernelGGL((ath::KPencilOther<T, false>), units, dim3(kBlk), 0, c->stream, mp, c->P);
-          hipLaunchKernelGGL((ath::KLusgsPencil<T, false, true>), grid, blk, 0, c->stream, c->pen, c->P, store);
-        } else {
-          hipLaunchKernelGGL((ath::KLusgsPencil<T, false, false>), grid, blk, 0, c->stream, c->pen, c->P, store);
+        if (full) {
+          if (dir == 0)
+            hipLaunchKernelGGL((ath::KPencilOther<T, true>), units, dim3(kBlk), 0, c->stream, mp, c->P);
+          else
+            hipLaunchKernelGGL((ath::KPencilOther<T, false>), units, dim3(kBlk), 0, c->stream, mp, c->P);
         }
-        ++launches;
-        mark(false);
-      }
-    } else if (hc.solver == ath::Solver::LUSGS && c->P.block &&
-               (order == ATH_SWEEP_TILED || order == ATH_SWEEP_ROWS)) {
-      for (int dir = 0; dir < 2; ++dir) {
-        // the first forward pass starts from du = 0: its connection terms
-        // are zero and the sweep does not read them
-        if (dir > 0 || full) LaunchConnTerms<T>(c);
-        mark(true);
-        if (order == ATH_SWEEP_ROWS) {
-          if (full) {
-            if (dir == 0)
-              hipLaunchKernelGGL((ath::KOtherSide<T, true>), dim3(c->mapTotal[kMapCell256]), dim3(kBlk), 0,
-                                 c->stream, c->Map(kMapCell256), c->P);
-            else
-              hipLaunchKernelGGL((ath::KOtherSide<T, false>), dim3(c->mapTotal[kMapCell256]), dim3(kBlk), 0,
-                                 c->stream, c->Map(kMapCell256), c->P);
-          }
-          hipLaunchKernelGGL(ath::KMultiSweepPrologue, dim3(1), dim3(1), 0, c->stream, c->rsweep);
-          if (dir == 0)
-            hipLaunchKernelGGL((ath::KBlockSweepRows<T, true>), dim3(c->rsweepGrid), dim3(ath::kPThreads), 0,
-                               c->stream, c->dblocks, c->P, c->rsweep, full);
-          else
-            hipLaunchKernelGGL((ath::KBlockSweepRows<T, false>), dim3(c->rsweepGrid), dim3(ath::kPThreads), 0,
-                               c->stream, c->dblocks, c->P, c->rsweep, full);
+        // every block's pencils in one launch.  A one-sweep forward pass hands
+        // du to the backward pass in sweep order; the connection terms and the
+        // other-side sums read the natural layout.
+        const int store = dir == 0 && !full ? (c->nconn > 0 ? 3 : 2) : 1;
+        const dim3 grid(c->pen.nent), blk((blkPencil ? ath::kBlkWaves<T> : ath::kPenWaves) * ath::kPenLanes);
+        auto launch = [&](auto kernel) {
+          hipLaunchKernelGGL(kernel, grid, blk, 0, c->stream, c->pen, c->P, store);
+        };
+        if (blkPencil) {
+          if (dir == 0) full ? launch(ath::KBlockPencil<T, true, true>) : launch(ath::KBlockPencil<T, true, false>);
+          else full ? launch(ath::KBlockPencil<T, false, true>) : launch(ath::KBlockPencil<T, false, false>);
         } else {
-          hipLaunchKernelGGL(ath::KMultiSweepPrologue, dim3(1), dim3(1), 0, c->stream, c->msweep);
-          if (dir == 0)
-            hipLaunchKernelGGL((ath::KBlockSweepTiles<T, true>), dim3(c->msweepGrid), dim3(ath::kBT), 0,
-                               c->stream, c->dblocks, c->P, c->msweep, full);
-          else
-            hipLaunchKernelGGL((ath::KBlockSweepTiles<T, false>), dim3(c->msweepGrid), dim3(ath::kBT), 0,
-                               c->stream, c->dblocks, c->P, c->msweep, full);
+          if (dir == 0) full ? launch(ath::KLusgsPencil<T, true, true>) : launch(ath::KLusgsPencil<T, true, false>);
+          else full ? launch(ath::KLusgsPencil<T, false, true>) : launch(ath::KLusgsPencil<T, false, false>);
         }
         ++launches;
         mark(false);
@@ -1370,6 +1304,7 @@ int LaunchRelaxT(ath_ctx *c, bool timed, size_t evBase) {
 
 template <typename T>
 void LaunchUpdateT(ath_ctx *c) {
+  c->stateSet = 1;
   hipLaunchKernelGGL(ath::KUpdate<T>, dim3(c->mapTotal[kMapCell256]), dim3(ath::kRedThreads), 0, c->stream,
                      c->Map(kMapCell256), c->P, c->dpart);
   hipLaunchKernelGGL(ath::KReduceNorms, dim3(c->active.size()), dim3(ath::kRedThreads), 0, c->stream, c->dpart,
@@ -1396,6 +1331,7 @@ int SweepPasses(const ath_ctx *c) {
 }
 
 void LaunchCopyNm1(ath_ctx *c) {
+  c->stateSet = 1;
   for (auto &br : c->blk)
     hipLaunchKernelGGL(ath::KCopyNm1, dim3(Grid(5 * br.d.ncell)), dim3(kBlk), 0, c->stream, br.d);
 }
@@ -1632,6 +1568,7 @@ static int ExchangeState(ath_ctx *c, const ath::DevBlock &d, double *host, bool 
 static int CopyState(ath_ctx *c, int b, double *host, bool toHost) {
   if (!c || !host || b < 0 || b >= (int)c->blk.size()) return Fail(ATH_ERR_ARG, "bad argument");
   HIP_OK(hipSetDevice(c->device));
+  if (!toHost) c->stateSet = 1;
   return ExchangeState(c, c->blk[b].d, host, toHost);
 }
 
@@ -1650,6 +1587,7 @@ int ath_begin_step(ath_ctx *c, int nn) {
   // (input::NeedToStoreTimeN, include/input.hpp:174-176)
   if (c->P.implicit) {
     const int copyNm1 = (c->P.multilevel && nn == 0) ? 1 : 0;
+    c->stateSet = 1;
     hipLaunchKernelGGL(ath::KBeginStep, dim3(c->mapTotal[kMapCell256]), dim3(kBlk), 0, c->stream,
                        c->Map(kMapCell256), c->P, copyNm1);
   }
@@ -1848,10 +1786,8 @@ int ath_run(ath_ctx *c, int nn0, int nsteps, ath_norms *last) {
 }
 
 // Autotuning of the sweep execution order: every order the case admits
-// (pencil, tiled and hyperplane for scalar LU-SGS; the row-parallel sweep,
-// the tiled sweep with one or two workgroups per CU and the hyperplane order
-// for the block solvers) runs `iterations`
-// nonlinear iterations from the current state, timed by events around each
+// (pencil, tiled and hyperplane for scalar LU-SGS; pencil and hyperplane for
+// the block solvers) runs `iterations` nonlinear iterations from the current state, timed by events around each
 // sweep pass; the fastest is kept.  All orders give the same results bit for
 // bit (topological orders of the same dependencies), so the choice changes
 // speed only.  The state, the old time levels and the norm normalisation are
@@ -1885,23 +1821,19 @@ int ath_autotune(ath_ctx *c, int iterations, int *chosen, double *pass_ms) {
     std::memcpy(cr.l2first, l2keep, sizeof l2keep);
     return ATH_OK;
   };
-  struct Cand { int order, gridMul; };
+  struct Cand { int order; };
   std::vector<Cand> cands;
   if (!c->P.implicit) return Fail(ATH_ERR_ARG, "autotuning needs an implicit time integration");
   if (c->P.roeJac || c->hc.solver != ath::Solver::LUSGS) {
-    cands.push_back({EffectiveOrder(c), 0});
+    cands.push_back({EffectiveOrder(c)});
   } else if (c->P.block) {
-    cands.push_back({ATH_SWEEP_ROWS, 0});
-    cands.push_back({ATH_SWEEP_TILED, 1});
-    cands.push_back({ATH_SWEEP_TILED, 2});
-    cands.push_back({ATH_SWEEP_HYPERPLANE, 0});
+    cands.push_back({EffectiveOrder(c) == ATH_SWEEP_TILED ? ATH_SWEEP_TILED : ATH_SWEEP_ROWS});
+    cands.push_back({ATH_SWEEP_HYPERPLANE});
   } else {
-    cands.push_back({ATH_SWEEP_PENCIL, 0});
-    cands.push_back({ATH_SWEEP_TILED, 0});
-    cands.push_back({ATH_SWEEP_HYPERPLANE, 0});
+    cands.push_back({ATH_SWEEP_PENCIL});
+    cands.push_back({ATH_SWEEP_TILED});
+    cands.push_back({ATH_SWEEP_HYPERPLANE});
   }
-  hipDeviceProp_t prop;
-  HIP_OK(hipGetDeviceProperties(&prop, c->device));
   const int keepTiming = c->timing;
   const int nl = c->hc.nonlinear;
   const int steps = std::max(1, (iterations + nl - 1) / nl);
@@ -1909,8 +1841,6 @@ int ath_autotune(ath_ctx *c, int iterations, int *chosen, double *pass_ms) {
   Cand pick = cands[0];
   for (const Cand &k : cands) {
     c->sweepOrder = k.order;
-    if (k.gridMul > 0)
-      c->msweepGrid = std::max(1, std::min(c->msweep.ntiles, k.gridMul * prop.multiProcessorCount));
     c->timing = 1;
     const int r = ath_run(c, 0, steps, nullptr);
     c->timing = keepTiming;
@@ -1923,8 +1853,6 @@ int ath_autotune(ath_ctx *c, int iterations, int *chosen, double *pass_ms) {
     }
   }
   c->sweepOrder = pick.order;
-  if (pick.gridMul > 0)
-    c->msweepGrid = std::max(1, std::min(c->msweep.ntiles, pick.gridMul * prop.multiProcessorCount));
   c->DropGraph();
   if (chosen) *chosen = pick.order;
   if (pass_ms) *pass_ms = best;
@@ -2002,19 +1930,25 @@ int ath_get_block_diagonal(ath_ctx *c, int b, int inverse, double *a) {
       for (int q = 0; q < 25; ++q) a[25 * p + q] = t[q * n + p];
     return ATH_OK;
   }
-  // the inverse is kept in the sweep's tile-blocked layout
-  std::vector<double> t(25L * 256 * d.tni * d.tnj * d.tnk);
+  // the inverse is kept in the sweep's layout (InverseBase in the kernels)
+  std::vector<double> t(InverseSize<double>(d));
   HIP_OK(hipMemcpy(t.data(), d.Abi, t.size() * sizeof(double), hipMemcpyDeviceToHost));
   for (int k = 0; k < d.nk; ++k)
     for (int j = 0; j < d.nj; ++j)
       for (int i = 0; i < d.ni; ++i) {
+        const int x[3] = {i, j, k};
+        const int ca = x[(d.pl + 1) % 3], cb = x[(d.pl + 2) % 3], cc = x[d.pl];
+        constexpr int w = ath::kPW, lanes = ath::kPenLanes;
+        const long rec = (long)(ca / w + d.pa * (cb / w)) * d.pns + ca % w + cb % w + cc;
         const long tile = (long)(i >> 3) + (long)d.tni * ((j >> 3) + (long)d.tnj * (k >> 2));
-        const long base = tile * (25 * 256) + ((i & 7) + 8 * ((j & 7) + 8 * (k & 3)));
+        const long base = d.pns ? (rec * lanes + ca % w + w * (cb % w)) * ath::kInv<double>
+                                : tile * (25 * 256) + ((i & 7) + 8 * ((j & 7) + 8 * (k & 3)));
         const long p = i + (long)j * d.ni + (long)k * d.ni * d.nj;
-        for (int q = 0; q < 25; ++q) a[25 * p + q] = t[base + 256 * q];
+        for (int q = 0; q < 25; ++q) a[25 * p + q] = t[base + (d.pns ? 1L : 256L) * q];
       }
   return ATH_OK;
 }
+
 int ath_get_update(ath_ctx *c, int b, double *du) { return GetPhys(c, b, du, 4); }
 
 // the cell-centre fields of every block of a single-case context, physical
@@ -2113,6 +2047,7 @@ int ath_read_restart(ath_ctx *c, const char *path, int *iteration) {
           for (int q = 0; q < 5; ++q) soa[q * nc + p] = io[b].consNm1[5 * p + q];
         HIP_OK(hipMemcpy(d.consNm1, soa.data(), soa.size() * sizeof(double), hipMemcpyHostToDevice));
       } else {
+        c->stateSet = 1;
         hipLaunchKernelGGL(ath::KBeginStep, dim3(c->mapTotal[kMapCell256]), dim3(kBlk), 0, c->stream,
                            c->Map(kMapCell256), c->P, 1);
         HIP_OK(hipStreamSynchronize(c->stream));
@@ -2353,16 +2288,19 @@ double EstimateBytes(const ath::HostCase &hc, bool fp32) {
     }
     const double tiles = (double)((h.ni + 7) / 8) * ((h.nj + 7) / 8) * ((h.nk + 3) / 4);
     const double nbf = 2.0 * ((double)h.nj * h.nk + (double)h.nk * h.ni + (double)h.ni * h.nj);
-    t += np * 8 * 8 + nf * 32 + nc * 8 * 35 + nc * 4 + nbf * 80 + tiles * 32 + 8192;
+    t += np * 8 * 8 + nf * 32 + nc * 8 * 30 + nc * 4 + nbf * 80 + tiles * 32 + 8192;
     if (fp32) t += nc * 4 * 11 + nbf * 20;
     if (PencilCase(hc)) {
       int pl, pa, pb, pns;
       PencilGrid(h, &pl, &pa, &pb, &pns);
       // the case's sweep arrays and its share of the group's message slots
+      const double visc = hc.viscous ? 6 : 0;
       t += (double)pa * pb * pns * 8 *
-           (ath::kPenLanes * (2.0 * (ath::kPenF + 3) + ath::kPenS + 1 + 5 + (hc.InitMatrix() ? 5 : 0)) + 4.0 * ath::kMsg);
+           (ath::kPenLanes * (2.0 * ath::kPenF + visc + RecordValues(hc) + 5 + (hc.InitMatrix() ? 5 : 0) +
+                              (hc.block ? ath::kInv<double> + (fp32 ? ath::kInv<float> / 2 : 0) : 0)) +
+            4.0 * ath::kMsg);
     }
-    if (hc.block) t += nc * 25 * 8 + tiles * 256 * 25 * 8;
+    if (hc.block) t += nc * 25 * 8 + (PencilCase(hc) ? 0 : tiles * 256 * 25 * 8 * (fp32 ? 1.5 : 1.0));
     if (hc.viscous) t += np * 8 * 3 + nfp * 32 + nf * 8 + nbf + (double)h.g * h.g * 4 * (h.ni + h.nj + h.nk) * 2 * 64 +
                          nbf * 40.0 * h.g;
     if (hc.block && hc.viscous) t += nf * 9 * 8 + np * 10 * 8;
@@ -2421,6 +2359,7 @@ double Drop(const CaseRes &cr, const ath_norms &n) {
 void LaunchServeIteration(ath_ctx *c) {
   const int na = (int)c->active.size();
   hipLaunchKernelGGL(ath::KCaseCfl, dim3(Grid(na, 64)), dim3(64), 0, c->stream, c->dcflc, na);
+  c->stateSet = 1;
   if (c->P.implicit)
     hipLaunchKernelGGL(ath::KBeginStep, dim3(c->mapTotal[kMapCell256]), dim3(kBlk), 0, c->stream,
                        c->Map(kMapCell256), c->P, 0);

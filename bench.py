@@ -62,32 +62,30 @@ VORTEX_SWEEP_TRAFFIC = 0.5 * (263.6e6 + 257.8e6)
 #   backward pass (first sweep, no initialisation: x - D^-1 U): W 40 +
 #   geometry 96 + D^-1 200 + mu 8 + k 8 + velocity gradient 72 + centre
 #   distances 24 + x read 40 + x write 40 = 528
-#   the row-parallel sweep reads the right-hand side formed once per relax
-#   (rhs 40 in place of R, U^n, U^n-1, V and dt): 528 forward and backward
+#   the pencil sweep reads sweep-ordered records: D^-1 200 + face areas and
+#   distances 120 + state, viscosity, conductivity and velocity gradient 128,
+#   forward rhs 40 and du 40 written twice, backward du 40 read and written
 CHANNEL_FLUX_BYTES = 712
-# with the row-parallel sweep (FP64 operator, one sweep) the viscous block
-# diagonal also forms the relax's right-hand side and du = 0: U^n 40 +
-# U^n-1 40 read, rhs 40 + x 40 written (W, R, V and dt are counted above)
-CHANNEL_FLUX_RHS_BYTES = 160
+# for the pencil sweep the viscous block diagonal also forms the relax's
+# right-hand side and writes the records: U^n 40 + U^n-1 40 read, rhs 40 +
+# state, viscosity, conductivity and velocity gradient 128 written (W, R, V
+# and dt are counted above)
+CHANNEL_FLUX_RHS_BYTES = 248
 CHANNEL_SWEEP_BYTES = {"fwd": 624, "bwd": 528}
-CHANNEL_ROWS_SWEEP_BYTES = {"fwd": 528, "bwd": 528}
+CHANNEL_PENCIL_SWEEP_BYTES = {"fwd": 568, "bwd": 528}
 # HBM bytes per launch on the full-size channel (refine 1), from rocprofv3
 # FETCH_SIZE / WRITE_SIZE scaled by the device-copy calibration (2.0, 1.0);
 # see profiles/channel-multiblock-1M_hbm_counters.md
-CHANNEL_SWEEP_TRAFFIC = 0.5 * (1338.3e6 + 1119.8e6)   # one pass, forward and backward averaged
-CHANNEL_ROWS_SWEEP_TRAFFIC = 0.5 * (1177.5e6 + 1123.9e6)  # the row-parallel sweep
-CHANNEL_FLUX_TRAFFIC = 2827.7e6                       # residual stage over all blocks
+CHANNEL_PENCIL_SWEEP_TRAFFIC = 0.5 * (782e6 + 728e6)  # one pass, forward and backward averaged
+CHANNEL_FLUX_TRAFFIC = 3046e6                         # residual stage over all blocks
 # what the occupancy and VALU counters show binds each (rocprofv3 SQ_WAVES,
 # SQ_INSTS_VALU, VALUBusy, OccupancyPercent on the same case; see
 # profiles/channel-multiblock-1M_sq_counters.md)
-ROWS_SWEEP_LIMITER = ("dependency latency: one workgroup of 8 waves per CU (22 % occupancy), VALU 20 % busy, HBM about "
-                      "28 %; a tile's forming is a chain of memory round trips, and the tile hyperplanes of the largest "
-                      "block set the ramps")
-SWEEP_LIMITER = ("dependency latency: one workgroup per CU (10.6 % occupancy), VALU 17 % busy, HBM about 20 %; "
-                 "the pass is the chain of tile hyperplanes of the largest block")
+PENCIL_SWEEP_LIMITER = ("dependency latency: 184 pencils of one workgroup each, 110 steps of 1.08 us (one wave's four "
+                        "5x5 products) and the handoffs between pencils; HBM about 30 %")
 FLUX_LIMITER = ("mixed: KResidual FP64-VALU issue (VALUBusy 80 %), the viscous block diagonal with the inviscid "
-                "block sum and the relax's right-hand side VALU (52 %) and HBM (45 %), the viscous flux the latency "
-                "of its gathers (occupancy 22 %, VALU 27 %, HBM 40 %)")
+                "block sum, the relax's right-hand side and the sweep's records latency (VALU 45 %, HBM 41 %), "
+                "the viscous flux the latency of its gathers (occupancy 22 %, VALU 27 %, HBM 40 %)")
 
 
 def parse():
@@ -299,17 +297,17 @@ def bench_channel(args, Solver, cases):
     pass_avg_s = tm.sweep_ms / max(tm.sweep_passes, 1) * 1e-3
     flux_share = tm.flux_ms / max(tm.run_ms, 1e-30)
     sweep_share = tm.sweep_ms / max(tm.run_ms, 1e-30)
-    rows = s.sweep_ordering() == Solver.ROWS
-    per_cell = CHANNEL_ROWS_SWEEP_BYTES if rows else CHANNEL_SWEEP_BYTES
+    pencil = s.sweep_ordering() != Solver.HYPERPLANE
+    per_cell = CHANNEL_PENCIL_SWEEP_BYTES if pencil else CHANNEL_SWEEP_BYTES
     pass_bytes = 0.5 * (per_cell["fwd"] + per_cell["bwd"]) * ncell
     full = args.refine == 1.0
-    kname = "KBlockSweepRows<double, FWD>, two lanes per cell" if rows else "KBlockSweepTiles<double, FWD>"
-    sweep = roofline(f"block LU-SGS sweep pass over all eight blocks ({kname}, one launch), average of forward "
+    kname = "KBlockPencil<double, FWD>, one launch" if pencil else "one launch per hyperplane"
+    sweep = roofline(f"block LU-SGS sweep pass over all eight blocks ({kname}), average of forward "
                      "and backward", pass_bytes, pass_avg_s, sweep_share,
-                     traffic=(CHANNEL_ROWS_SWEEP_TRAFFIC if rows else CHANNEL_SWEEP_TRAFFIC) if full else None,
+                     traffic=CHANNEL_PENCIL_SWEEP_TRAFFIC if full and pencil else None,
                      launches_per_pass=tm.sweep_launches / max(tm.sweep_passes, 1),
-                     limiter=ROWS_SWEEP_LIMITER if rows else SWEEP_LIMITER)
-    rhs_in_stage = rows  # the FP64 operator (this run) with the row-parallel sweep
+                     limiter=PENCIL_SWEEP_LIMITER if pencil else "launch latency: one launch per hyperplane")
+    rhs_in_stage = pencil
     flux = roofline("residual stage over all eight blocks (inviscid + viscous fluxes, spectral radii, dt, block "
                     "diagonal and inverse" + (", the relax's right-hand side" if rhs_in_stage else "") +
                     "; one launch per kernel)",

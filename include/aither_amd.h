@@ -93,25 +93,25 @@ int ath_set_implicit_precision(ath_ctx *ctx, int precision);
  * the block's longest axis on a skewed wavefront, one launch per sweep pass.  ATH_SWEEP_TILED: 8x8x4
  * tiles in tile-hyperplane order, dataflow-synchronised, one launch per pass.
  * ATH_SWEEP_HYPERPLANE: one launch per i+j+k hyperplane in the order of
- * HyperplaneReorder (src/utility.cpp:377-398).  ATH_SWEEP_ROWS (block
- * solvers): 8x4x4 tiles in tile-hyperplane order with each cell's five rows
- * on their own lanes, one launch per pass.  All are topological orders of the
- * same Gauss-Seidel dependencies and give identical results. */
+ * HyperplaneReorder (src/utility.cpp:377-398).  ATH_SWEEP_ROWS is kept for
+ * callers that set it.  The block solvers run the pencil order for every
+ * setting but ATH_SWEEP_HYPERPLANE.  All are topological orders of the same
+ * Gauss-Seidel dependencies and give identical results. */
 #define ATH_SWEEP_TILED 0
 #define ATH_SWEEP_HYPERPLANE 1
 #define ATH_SWEEP_PENCIL 2
 #define ATH_SWEEP_ROWS 3
 int ath_set_sweep_ordering(ath_ctx *ctx, int ordering);
-/* the order the sweeps actually run in: block solvers (blusgs, bdplur) map
- * ATH_SWEEP_PENCIL to ATH_SWEEP_ROWS with the FP64 operator and to
- * ATH_SWEEP_TILED with the FP32 operator, scalar LU-SGS maps ATH_SWEEP_ROWS
- * to ATH_SWEEP_TILED, and the approximateRoe flux Jacobian always runs
+/* the order in effect: block solvers (blusgs, bdplur) report ATH_SWEEP_PENCIL
+ * as ATH_SWEEP_ROWS with the FP64 operator and as ATH_SWEEP_TILED with the
+ * FP32 operator (both names run their pencil sweep), scalar LU-SGS maps
+ * ATH_SWEEP_ROWS to ATH_SWEEP_TILED, and the approximateRoe flux Jacobian always runs
  * ATH_SWEEP_HYPERPLANE, whatever was set */
 int ath_get_sweep_ordering(const ath_ctx *ctx, int *ordering);
 /* Autotune the sweep execution order for this case: time `iterations`
  * nonlinear iterations in each order the case admits (pencil, tiled and
- * hyperplane for scalar LU-SGS; the all-block tiled sweep with one or two
- * workgroups per CU, and the hyperplane order, for the block solvers) and
+ * hyperplane for scalar LU-SGS; pencil and hyperplane for the block solvers)
+ * and
  * keep the fastest per sweep pass.  Results do not depend on the order; the
  * state and the norm normalisation are restored.  No reference counterpart. */
 int ath_autotune(ath_ctx *ctx, int iterations, int *chosen, double *pass_ms);
@@ -151,7 +151,7 @@ int ath_calc_residual(ath_ctx *ctx);
 /* linearSolver::InitializeMatrixUpdate + Relax (src/linearSolver.cpp:111-144,
  * 430-470, 509-535); returns the matrix residual (CycleAtLevel value).  Uses
  * the last ath_calc_residual's residual, time step and diagonal (for a
- * one-sweep FP64 block LU-SGS relax in the row-parallel order also the
+ * one-sweep FP64 viscous block LU-SGS relax in the pencil order also the
  * right-hand side that call formed). */
 int ath_relax(ath_ctx *ctx, double *cycle_value);
 /* gridLevel::UpdateBlocks + ResetDiagonal (src/gridLevel.cpp:418-431) */
