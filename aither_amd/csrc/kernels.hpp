@@ -2911,6 +2911,18 @@ __device__ __forceinline__ void PenStage(const DevBlock &b, const Params &P, con
   for (int q = 0; q < 3; ++q) LdsPut<T, kLate<T>>(&sl.late[q][0][lane], late[q]);
 }
 
+// Where a pass writes its sweep-ordered output, first step.  The
+// dependency-side sums of a full pass are the other-side sums of the next: its
+// cells' neighbours on that side still have this pass's du then, so without
+// connections (whose ghost du changes in between) only the first full pass of a
+// relax needs KPencilOther.  The stager reads a record before the compute wave
+// writes it.  40 iterations of two sweeps, 48^3 viscous cells: 34.6 ms with
+// KPencilOther before each pass, 30.7 so.
+template <typename T, bool FWD, bool FULL>
+__device__ __forceinline__ T *PenStore(const DevBlock &b, const Pencil &pen) {
+  return (FULL ? (T *)b.skO : (T *)b.skX) + (pen.rec + (FWD ? 0 : pen.ns - 1)) * 5 * kPenLanes;
+}
+
 // The compute wave.  A wave issues one instruction in 4.6 cycles whatever it
 // depends on, so a step costs its instruction count plus what it waits for,
 // and it is ordered so that it waits for nothing: each value of the next step
@@ -2948,8 +2960,10 @@ __device__ __forceinline__ void PenCompute(const DevBlock &b, const Params &P, c
   Map3(C, FWD ? -off : nc - 1 + off, gA, gB, i0, j0, k0);
   const int sC = -sgn * (C == 0 ? 1 : (C == 1 ? b.ni : b.ni * b.nj));
   int p = i0 + j0 * b.ni + k0 * b.ni * b.nj;  // cell of step st (of the active steps)
-  T *Xs = (T *)b.skX + pen.rec * 5 * kPenLanes + lane;
-  T xA[5], xB[5], early[kEarly<T, FULL>], late[3][kLate<T>];
+  // one-sweep forward pass: du for the backward pass; full pass: the
+  // dependency-side sums for the next pass (PenStore)
+  T *Xs = PenStore<T, FWD, FULL>(b, pen) + lane;
+  T xA[5], xB[5], S[5], early[kEarly<T, FULL>], late[3][kLate<T>];
   int next = 1;  // slot of the next step
   LdsWait<0>(&sh.stageReady[0], 1, err);
   LdsWait<0>(&ln.haloReady, 1, err);
@@ -2973,6 +2987,7 @@ __device__ __forceinline__ void PenCompute(const DevBlock &b, const Params &P, c
       const T o0 = C == 2 ? xA[e] : (C == 0 ? oC[e] : xB[e]), o1 = C == 2 ? xB[e] : (C == 0 ? xA[e] : oC[e]),
               o2 = C == 2 ? oC[e] : (C == 0 ? xB[e] : xA[e]);
       const T D = ((T(0) + o0) + o1) + o2, v = early[e], ainv = early[5];
+      S[e] = D;
       if constexpr (FULL) xn[e] = FWD ? (v + (D - early[11 + e])) * ainv : ((v + early[11 + e]) - D) * ainv;
       else xn[e] = FWD ? (v + D) * ainv : v - D * ainv;
       W0[e] = early[6 + e];
@@ -3037,17 +3052,18 @@ __device__ __forceinline__ void PenCompute(const DevBlock &b, const Params &P, c
         for (int e = 0; e < 5; ++e) x[e * b.ncell + p] = xn[e];
       }
     }
-    if (FWD && !FULL && (store & 2)) {
+    if ((FWD || FULL) && (store & 2)) {
 #pragma unroll
-      for (int e = 0; e < 5; ++e) Xs[e * kPenLanes] = xn[e];
+      for (int e = 0; e < 5; ++e) Xs[e * kPenLanes] = FULL ? S[e] : xn[e];
     }
     p += sC;
-    Xs += 5 * kPenLanes;
+    Xs += (FWD ? 5 : -5) * kPenLanes;
   }
 }
 
-// `store`: bit 0 du in the natural layout, bit 1 in sweep order (a forward
-// pass whose backward pass reads it)
+// `store`: bit 0 du in the natural layout, bit 1 in sweep order (a one-sweep
+// forward pass, whose backward pass reads it) or, of a full pass, the sums for
+// the next (PenStore)
 template <typename T, bool FWD, bool FULL>
 __global__ void __launch_bounds__(kPenWaves * kPenLanes) KLusgsPencil(PencilGroup G, Params P, int store) {
   __shared__ PenShared<T, FULL> sh;
@@ -3251,8 +3267,8 @@ __device__ __forceinline__ void BlkCompute(const DevBlock &b, const Pencil &pen,
   Map3(C, FWD ? -off : nc - 1 + off, pen.a * kPW + la, pen.b * kPW + lb, i0, j0, k0);
   const int sC = -sgn * (C == 0 ? 1 : (C == 1 ? b.ni : b.ni * b.nj));
   int p = i0 + j0 * b.ni + k0 * b.ni * b.nj;  // cell of step st (of the active steps)
-  T *Xs = (T *)b.skX + pen.rec * 5 * kPenLanes + lane;
-  T xA[5], xB[5], d[25], r[kBlkR<FULL>], JA[25], JB[25];
+  T *Xs = PenStore<T, FWD, FULL>(b, pen) + lane;
+  T xA[5], xB[5], S[5], d[25], r[kBlkR<FULL>], JA[25], JB[25];
   LdsWait<0>(&sh.ready[0], kBlkParts, err);
   LdsGet<T, 25, 1>(&sh.slot[0].D[lane * Vecs<T>(25)], d);
   LdsGet<T, kBlkR<FULL>>(&sh.slot[0].r[0][lane], r);
@@ -3270,6 +3286,7 @@ __device__ __forceinline__ void BlkCompute(const DevBlock &b, const Pencil &pen,
       const T o0 = C == 2 ? xA[e] : (C == 0 ? oC[e] : xB[e]), o1 = C == 2 ? xB[e] : (C == 0 ? xA[e] : oC[e]),
               o2 = C == 2 ? oC[e] : (C == 0 ? xB[e] : xA[e]);
       const T D = ((T(0) + o0) + o1) + o2;
+      S[e] = D;
       if constexpr (FULL) v[e] = FWD ? r[e] + (D - r[5 + e]) : (r[e] + r[5 + e]) - D;
       else v[e] = FWD ? r[e] + D : D;
     }
@@ -3320,12 +3337,12 @@ __device__ __forceinline__ void BlkCompute(const DevBlock &b, const Pencil &pen,
         for (int e = 0; e < 5; ++e) x[e * b.ncell + p] = xn[e];
       }
     }
-    if (FWD && !FULL && (store & 2)) {
+    if ((FWD || FULL) && (store & 2)) {
 #pragma unroll
-      for (int e = 0; e < 5; ++e) Xs[e * kPenLanes] = xn[e];
+      for (int e = 0; e < 5; ++e) Xs[e * kPenLanes] = FULL ? S[e] : xn[e];
     }
     p += sC;
-    Xs += 5 * kPenLanes;
+    Xs += (FWD ? 5 : -5) * kPenLanes;
   }
 }
 

@@ -1220,7 +1220,10 @@ int LaunchRelaxT(ath_ctx *c, bool timed, size_t evBase) {
         // connection terms are zero and the sweep does not read them
         if (!blkPencil || dir > 0 || full) LaunchConnTerms<T>(c);
         mark(true);
-        if (full) {
+        // without connections a full pass hands its dependency-side sums to
+        // the next, and only the relax's last du is read
+        const bool carry = full && c->nconn == 0, last = sw + 1 == hc.sweeps && dir == 1;
+        if (full && !(carry && (sw > 0 || dir > 0))) {
           if (dir == 0)
             hipLaunchKernelGGL((ath::KPencilOther<T, true>), units, dim3(kBlk), 0, c->stream, mp, c->P);
           else
@@ -1229,7 +1232,7 @@ int LaunchRelaxT(ath_ctx *c, bool timed, size_t evBase) {
         // every block's pencils in one launch.  A one-sweep forward pass hands
         // du to the backward pass in sweep order; the connection terms and the
         // other-side sums read the natural layout.
-        const int store = dir == 0 && !full ? (c->nconn > 0 ? 3 : 2) : 1;
+        const int store = carry && !last ? 2 : (dir == 0 && !full ? (c->nconn > 0 ? 3 : 2) : 1);
         const dim3 grid(c->pen.nent), blk((blkPencil ? ath::kBlkWaves<T> : ath::kPenWaves) * ath::kPenLanes);
         auto launch = [&](auto kernel) {
           hipLaunchKernelGGL(kernel, grid, blk, 0, c->stream, c->pen, c->P, store);
