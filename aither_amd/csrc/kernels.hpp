@@ -32,6 +32,7 @@ __host__ __device__ inline ATH_GLOBAL T *Dev(T *p) {
 // a record (one hyperplane step of one pencil)
 constexpr int kPW = 8;
 constexpr int kPenLanes = kPW * kPW;
+constexpr int kPenS = 11;      // per-relax values of a cell: W, right-hand side, D^-1 (and viscosity)
 
 struct DevBlock {
   int ni, nj, nk, g;
@@ -122,6 +123,7 @@ struct Params {
   int fp32;   // the scalar implicit operator runs in FP32: the residual stage writes Ainv32, else Ainv
   int roeJac; // inviscidFluxJacobian approximateRoe: the off-diagonals are Roe flux changes (FP64)
   int rhsOnce; // the relax forms the right-hand side once, in sweep order (the block pencil sweep reads it)
+  int prep;      // the inviscid residual kernel writes the scalar pencil sweep's records (KPencilPrep's)
   int rhsInDiag; // the block diagonal forms that right-hand side (the relax does not)
   int copyState; // the relax refreshes the state in sweep order (it was set since the residual stage)
 };
@@ -546,10 +548,11 @@ __device__ __forceinline__ void FaceFlux(const DevBlock &b, const GasT<double> &
 // (src/linearSolver.cpp:146-188) for one cell; `sr` is the cell spectral
 // radius, `Ad` the accumulated main diagonal
 __device__ __forceinline__ void CellTail(const DevBlock &b, const Params &P, long p, double vol, double sr,
-                                         double Ad) {
+                                         double Ad, double *dtOut = nullptr, double *ainvOut = nullptr) {
   b.sr[p] = sr;
   const double dt = P.dtFixed > 0.0 ? P.dtFixed : (*b.cfl) * Div(vol, Dmax(sr, 0.0));
   b.dt[p] = dt;
+  if (dtOut) *dtOut = dt;
   if (P.implicit && !P.block) {
     double dvt = Div(vol * (1.0 + P.zeta), dt * P.theta);
     if (P.dualCFL > 0.0) dvt += Div(Dmax(sr, 0.0), P.dualCFL);
@@ -557,6 +560,7 @@ __device__ __forceinline__ void CellTail(const DevBlock &b, const Params &P, lon
     A += dvt;
     b.A[p] = A;
     const double ainv = Div(1.0, A);
+    if (ainvOut) *ainvOut = P.fp32 ? double((float)ainv) : ainv;
     if (!P.fp32) {
       if (b.Ainv) b.Ainv[p] = ainv;
     } else if (b.Ainv32) {
@@ -603,6 +607,66 @@ __device__ __forceinline__ Unit MapUnit(const BlockMap &m) {
           (int)(l / ((unsigned)u.x * (unsigned)u.y)), l, n};
 }
 
+// b = -R/theta + forcing + SolDeltaNm1 - SolDeltaMmN
+// (src/linearSolver.cpp:360-378, src/procBlock.cpp:1010-1034); forcing is
+// zero on the single grid level
+// the same from values already loaded (cNm1 is read only when multilevel)
+__device__ __forceinline__ void RhsFrom(const Params &P, const double W[5], double vol, double dt,
+                                        const double R[5], const double cN[5], const double cNm1[5],
+                                        double out[5]) {
+#pragma clang fp contract(off)
+  const GasT<double> g = Cast<double>(P.gas);
+  double U[5];
+  PrimToCons(g, W, U);
+  const Divisor<double> byDt = MakeDivisor(dt * P.theta);
+  const double coeff = Quot(vol * (1.0 + P.zeta), byDt);
+  const double thetaInv = 1.0 / P.theta;
+  const double c2 = P.multilevel ? Quot(vol * P.zeta, byDt) : 0.0;
+#pragma unroll
+  for (int e = 0; e < 5; ++e) {
+    const double nm1 = P.multilevel ? c2 * (cN[e] - cNm1[e]) : 0.0;
+    const double mmn = coeff * (U[e] - cN[e]);
+    double v = -thetaInv * R[e];
+    out[e] = (v + nm1) - mmn;
+  }
+}
+
+__device__ __forceinline__ void Rhs(const DevBlock &b, const Params &P, long p, long c,
+                                    double out[5]) {
+  double W[5], R[5], cN[5], cNm1[5] = {0, 0, 0, 0, 0};
+#pragma unroll
+  for (int e = 0; e < 5; ++e) {
+    W[e] = b.W[e * b.npad + c];
+    R[e] = b.R[e * b.ncell + p];
+    cN[e] = b.consN[e * b.ncell + p];
+    if (P.multilevel) cNm1[e] = b.consNm1[e * b.ncell + p];
+  }
+  RhsFrom(P, W, b.vol[p], b.dt[p], R, cN, cNm1, out);
+}
+
+// A tile's 256 cells by their place in the pencil sweep's records: pencil, step,
+// lane, for pencils along each axis; extents of the tiles in i, j, k.
+struct TileOrder {
+  unsigned char cell[3][256];
+};
+constexpr TileOrder MakeTileOrder(const int (&tile)[3][3]) {
+  TileOrder o{};
+  for (int l = 0; l < 3; ++l) {
+    const int ti = tile[l][0], tj = tile[l][1], tk = tile[l][2];
+    int n = 0;
+    for (int pen = 0; pen < (l == 0 ? 1 : ti / kPW); ++pen)  // pencils lie side by side along i
+      for (int key = 0; key < 64 * kPenLanes; ++key) {       // step * kPenLanes + lane
+        const int la = key % kPW, lb = key / kPW % kPW, cc = key / kPenLanes - la - lb;
+        const int i = l == 0 ? cc : kPW * pen + (l == 1 ? lb : la), j = l == 0 ? la : (l == 1 ? cc : lb),
+                  k = l == 0 ? lb : (l == 1 ? la : cc);
+        if (cc >= 0 && i < ti && j < tj && k < tk) o.cell[l][n++] = (unsigned char)(i + ti * (j + tj * k));
+      }
+  }
+  return o;
+}
+constexpr int kCellTile[3][3] = {{kTI, kTJ, kTK}, {kTI, kTJ, kTK}, {kTI, kTJ, kTK}};
+__constant__ const TileOrder kCellOrder = MakeTileOrder(kCellTile);
+
 template <int RECON, int LIM, int FLUX>
 __global__ void __launch_bounds__(256) KResidual(BlockMap M, Params P) {
   __shared__ double sF[5][kNF];
@@ -633,37 +697,78 @@ __global__ void __launch_bounds__(256) KResidual(BlockMap M, Params P) {
   __syncthreads();
   const int li = threadIdx.x % kTI, lj = (threadIdx.x / kTI) % kTJ, lk = threadIdx.x / (kTI * kTJ);
   const int i = i0 + li, j = j0 + lj, k = k0 + lk;
-  if (i >= b.ni || j >= b.nj || k >= b.nk) return;
-  const int fi = lk * (kTI + 1) * kTJ + lj * (kTI + 1) + li;
-  const int fj = kNFI + lk * kTI * (kTJ + 1) + lj * kTI + li;
-  const int fk = kNFI + kNFJ + lk * kTI * kTJ + lj * kTI + li;
-  const long p = (long)i + (long)j * b.ni + (long)k * b.ni * b.nj;
+  const bool cell = i < b.ni && j < b.nj && k < b.nk, prep = P.prep && b.pns;
+  if (!cell && !prep) return;
+  double W[5], R[5], rb[5], ainv;
+  if (cell) {
+    const int fi = lk * (kTI + 1) * kTJ + lj * (kTI + 1) + li;
+    const int fj = kNFI + lk * kTI * (kTJ + 1) + lj * kTI + li;
+    const int fk = kNFI + kNFJ + lk * kTI * kTJ + lj * kTI + li;
+    const long p = (long)i + (long)j * b.ni + (long)k * b.ni * b.nj;
 #pragma unroll
-  for (int e = 0; e < 5; ++e) {
-    double r = -sF[e][fi];
-    r += sF[e][fi + 1];
-    r -= sF[e][fj];
-    r += sF[e][fj + kTI];
-    r -= sF[e][fk];
-    r += sF[e][fk + kTI * kTJ];
-    b.R[e * b.ncell + p] = r;
+    for (int e = 0; e < 5; ++e) {
+      double r = -sF[e][fi];
+      r += sF[e][fi + 1];
+      r -= sF[e][fj];
+      r += sF[e][fj + kTI];
+      r -= sF[e][fk];
+      r += sF[e][fk + kTI * kTJ];
+      b.R[e * b.ncell + p] = R[e] = r;
+    }
+    const long c = PadIdx(b, i, j, k);
+#pragma unroll
+    for (int e = 0; e < 5; ++e) W[e] = b.W[e * b.npad + c];
+    const double rho = W[0], u = W[1], v = W[2], w = W[3], pr = W[4];
+    const double li_ = InvCellSpecRad(g, rho, u, v, w, pr, b.fa[0][FaceIdx(b, 0, i, j, k)],
+                                      b.fa[0][FaceIdx(b, 0, i + 1, j, k)]);
+    const double lj_ = InvCellSpecRad(g, rho, u, v, w, pr, b.fa[1][FaceIdx(b, 1, i, j, k)],
+                                      b.fa[1][FaceIdx(b, 1, i, j + 1, k)]);
+    const double lk_ = InvCellSpecRad(g, rho, u, v, w, pr, b.fa[2][FaceIdx(b, 2, i, j, k)],
+                                      b.fa[2][FaceIdx(b, 2, i, j, k + 1)]);
+    const double sr = (li_ + lj_) + lk_;
+    if (P.visc.on) {
+      // the viscous pass adds its spectral radii and forms dt and the diagonal
+      b.sr[p] = sr;
+      return;
+    }
+    double dt;
+    const double vol = b.vol[p];
+    CellTail(b, P, p, vol, sr, sr, &dt, &ainv);
+    if (prep) {
+      double cN[5], cNm1[5] = {0, 0, 0, 0, 0};
+#pragma unroll
+      for (int e = 0; e < 5; ++e) {
+        cN[e] = b.consN[e * b.ncell + p];
+        if (P.multilevel) cNm1[e] = b.consNm1[e * b.ncell + p];
+      }
+      RhsFrom(P, W, vol, dt, R, cN, cNm1, rb);
+    }
   }
-  const long c = PadIdx(b, i, j, k);
-  const double rho = b.W[c], u = b.W[b.npad + c], v = b.W[2 * b.npad + c],
-               w = b.W[3 * b.npad + c], pr = b.W[4 * b.npad + c];
-  const double li_ = InvCellSpecRad(g, rho, u, v, w, pr, b.fa[0][FaceIdx(b, 0, i, j, k)],
-                                    b.fa[0][FaceIdx(b, 0, i + 1, j, k)]);
-  const double lj_ = InvCellSpecRad(g, rho, u, v, w, pr, b.fa[1][FaceIdx(b, 1, i, j, k)],
-                                    b.fa[1][FaceIdx(b, 1, i, j + 1, k)]);
-  const double lk_ = InvCellSpecRad(g, rho, u, v, w, pr, b.fa[2][FaceIdx(b, 2, i, j, k)],
-                                    b.fa[2][FaceIdx(b, 2, i, j, k + 1)]);
-  const double sr = (li_ + lj_) + lk_;
-  if (P.visc.on) {
-    // the viscous pass adds its spectral radii and forms dt and the diagonal
-    b.sr[p] = sr;
-    return;
+  if (!prep) return;
+  // the pencil sweep's records of the tile (KPencilPrep's values), through LDS
+  // in their order.  Everything but U^n is at hand here: an iteration of 64^3
+  // cells 522 us with KPencilPrep (23 us, gathers) in the relax, 506 so; of
+  // the eight served cases 393 and 370.
+  __syncthreads();
+  double(*sh)[256] = (double(*)[256])sF;
+  const int tid = threadIdx.x;
+  if (cell) {
+#pragma unroll
+    for (int e = 0; e < 5; ++e) {
+      sh[e][tid] = W[e];
+      sh[5 + e][tid] = rb[e];
+    }
+    sh[10][tid] = ainv;
   }
-  CellTail(b, P, p, b.vol[p], sr, sr);
+  __syncthreads();
+  const int src = kCellOrder.cell[b.pl][tid];
+  const int oi = i0 + src % kTI, oj = j0 + src / kTI % kTJ, ok = k0 + src / (kTI * kTJ);
+  if (oi >= b.ni || oj >= b.nj || ok >= b.nk) return;
+  int lane;
+  const long rec = PencilRecord(b, oi, oj, ok, lane);
+  double *o = b.skS + rec * kPenS * kPenLanes + lane;
+#pragma unroll
+  for (int e = 0; e < kPenS; ++e) o[e * kPenLanes] = sh[e][src];
 }
 
 // ---------------------------------------------------------------------------
@@ -1133,75 +1238,18 @@ __global__ void __launch_bounds__(256) KViscFlux(BlockMap M, Params P) {
 // ---------------------------------------------------------------------------
 // implicit operator
 
-// b = -R/theta + forcing + SolDeltaNm1 - SolDeltaMmN
-// (src/linearSolver.cpp:360-378, src/procBlock.cpp:1010-1034); forcing is
-// zero on the single grid level
-// the same from values already loaded (cNm1 is read only when multilevel)
-__device__ __forceinline__ void RhsFrom(const Params &P, const double W[5], double vol, double dt,
-                                        const double R[5], const double cN[5], const double cNm1[5],
-                                        double out[5]) {
-#pragma clang fp contract(off)
-  const GasT<double> g = Cast<double>(P.gas);
-  double U[5];
-  PrimToCons(g, W, U);
-  const Divisor<double> byDt = MakeDivisor(dt * P.theta);
-  const double coeff = Quot(vol * (1.0 + P.zeta), byDt);
-  const double thetaInv = 1.0 / P.theta;
-  const double c2 = P.multilevel ? Quot(vol * P.zeta, byDt) : 0.0;
-#pragma unroll
-  for (int e = 0; e < 5; ++e) {
-    const double nm1 = P.multilevel ? c2 * (cN[e] - cNm1[e]) : 0.0;
-    const double mmn = coeff * (U[e] - cN[e]);
-    double v = -thetaInv * R[e];
-    out[e] = (v + nm1) - mmn;
-  }
-}
-
-__device__ __forceinline__ void Rhs(const DevBlock &b, const Params &P, long p, long c,
-                                    double out[5]) {
-  double W[5], R[5], cN[5], cNm1[5] = {0, 0, 0, 0, 0};
-#pragma unroll
-  for (int e = 0; e < 5; ++e) {
-    W[e] = b.W[e * b.npad + c];
-    R[e] = b.R[e * b.ncell + p];
-    cN[e] = b.consN[e * b.ncell + p];
-    if (P.multilevel) cNm1[e] = b.consNm1[e * b.ncell + p];
-  }
-  RhsFrom(P, W, b.vol[p], b.dt[p], R, cN, cNm1, out);
-}
-
 // values of a block solver's record: state, right-hand side, and with the
 // viscous terms viscosity, conductivity and velocity gradient
 __host__ __device__ constexpr int BlockRecord(bool viscous) { return viscous ? 21 : 10; }
 
-// The block diagonal's tiles (extents in i, j, k for pencils along each axis)
-// and a tile's cells by their place in the records: pencil, step, lane.  Each
-// record takes a cell's values 512 bytes apart, its lanes from as many rows, so
+// The block diagonal's tiles.  Each record takes a cell's values 512 bytes apart, its lanes from as many rows, so
 // stores straight from the cells are single words: KBlockDiag on 1.03M cells
 // 800 us.  Through LDS in the records' order they are runs of up to eight lanes:
 // 534 us (8 x 8 x 4 tiles 554, 16 x 8 x 1 590, a wave's 8 x 8 cells 803),
 // against 395 us without any records, which the sweep's two passes (508 -> 353
 // us) and the initialisation gone from the relax pay for.
 constexpr int kDiagTile[3][3] = {{32, 8, 1}, {8, 8, 4}, {32, 1, 8}};
-struct TileOrder {
-  unsigned char cell[3][256];
-};
-constexpr TileOrder MakeTileOrder() {
-  TileOrder o{};
-  for (int l = 0; l < 3; ++l) {
-    const int ti = kDiagTile[l][0], tj = kDiagTile[l][1], tk = kDiagTile[l][2];
-    int n = 0;
-    for (int pen = 0; pen < (l == 0 ? 1 : ti / kPW); ++pen)  // pencils lie side by side along i
-      for (int key = 0; key < 64 * kPenLanes; ++key) {       // step * kPenLanes + lane
-        const int la = key % kPW, lb = key / kPW % kPW, cc = key / kPenLanes - la - lb;
-        const int i = l == 0 ? cc : kPW * pen + (l == 1 ? lb : la), j = l == 0 ? la : (l == 1 ? cc : lb),
-                  k = l == 0 ? lb : (l == 1 ? la : cc);
-        if (cc >= 0 && i < ti && j < tj && k < tk) o.cell[l][n++] = (unsigned char)(i + ti * (j + tj * k));
-      }
-  }
-  return o;
-}
-__constant__ const TileOrder kTileOrder = MakeTileOrder();
+__constant__ const TileOrder kTileOrder = MakeTileOrder(kDiagTile);
 // cell `t` of tile U
 __device__ __forceinline__ void DiagCell(const DevBlock &b, const Unit &U, int t, int &i, int &j, int &k) {
   const int ti = b.pl == 1 ? 8 : 32, tj = b.pl == 2 ? 1 : 8, tk = b.pl == 0 ? 1 : (b.pl == 1 ? 4 : 8);
@@ -2463,7 +2511,6 @@ constexpr int kPenWaves = 3 + kStagers;
 constexpr int kProdRing = 4;   // steps of products kept in LDS for the send wave (a power of two)
 constexpr int kHaloRing = 8;   // steps of halo products in LDS
 constexpr int kMsg = 5 * kPW;  // values of one message
-constexpr int kPenS = 11;      // per-relax values of a cell: W, right-hand side, D^-1 (and viscosity)
 constexpr int kPenF = 12;      // values of a cell's three faces on one side: unit normal, area (and centre distance)
 constexpr int kLdsSpinLimit = 1 << 24;
 static_assert(kHaloRing * kPW == kPenLanes, "halo ring layout");

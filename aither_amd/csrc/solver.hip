@@ -94,7 +94,8 @@ struct ath_ctx {
   hipStream_t stream = nullptr;
   int anyPark = 0;  // some block parks its wall cells' inviscid block sums (DevBlock::invPark)
   int rhsFormed = 0;  // the last residual stage formed the relax's right-hand side (RhsInDiag); 2: to keep
-                      // even when the state changes before the relax
+                      // even when the state changes before the relax; the scalar sweep's records (ScalarPrep)
+                      // with the 3: FP64, 4: FP32 operator's D^-1
   int stateSet = 0;   // a state or a stored solution level changed since
   ath::HostCase hc;  // the case (a single-case context) or the numerics every case shares (a server)
   ath::Params P{};
@@ -1092,13 +1093,24 @@ bool BlockPencil(const ath_ctx *c) {
 // block diagonal; such a relax reads no du it has not written
 bool RhsInDiag(const ath_ctx *c) { return BlockPencil(c) && !c->hc.InitMatrix(); }
 
+// the scalar pencil sweep's records are written by the inviscid residual kernel
+// (the viscous terms add to the diagonal after it)
+bool ScalarPrep(const ath_ctx *c) {
+  return PencilCase(c->hc) && !c->P.block && !c->P.visc.on && EffectiveOrder(c) == ATH_SWEEP_PENCIL;
+}
+
 template <int RECON, int LIM, int FLUX>
 void LaunchResidualT(ath_ctx *c) {
   const ath::Params &P = c->P;
   const ath::BlockMap mt = c->Map(kMapTile), mc = c->Map(kMapCell256), md = c->Map(kMapDiag), mp = c->Map(kMapPad256);
   const dim3 tiles(c->mapTotal[kMapTile]), cells(c->mapTotal[kMapCell256]),
              diag(c->mapTotal[kMapDiag]);
-  hipLaunchKernelGGL((ath::KResidual<RECON, LIM, FLUX>), tiles, dim3(256), 0, c->stream, mt, P);
+  ath::Params PR = P;
+  if (ScalarPrep(c)) {
+    PR.prep = 1;
+    c->rhsFormed = c->fp32 ? 4 : 3;
+  }
+  hipLaunchKernelGGL((ath::KResidual<RECON, LIM, FLUX>), tiles, dim3(256), 0, c->stream, mt, PR);
   if (P.block) {
     // inviscid block sum from the inviscid ghost states: finished here, or,
     // for the cells next to a viscous wall, parked in Ab until the viscous
@@ -1213,7 +1225,7 @@ int LaunchRelaxT(ath_ctx *c, bool timed, size_t evBase) {
     if (blkPencil || (hc.solver == ath::Solver::LUSGS && order == ATH_SWEEP_PENCIL)) {
       const dim3 units(c->mapTotal[kMapPen256]);
       const ath::BlockMap mp = c->Map(kMapPen256);
-      if (sw == 0 && !blkPencil)
+      if (sw == 0 && !blkPencil && !(ScalarPrep(c) && c->rhsFormed == (c->fp32 ? 4 : 3) && !c->stateSet))
         hipLaunchKernelGGL(ath::KPencilPrep<T>, units, dim3(kBlk), 0, c->stream, mp, c->P);
       for (int dir = 0; dir < 2; ++dir) {
         // the first forward pass of a block solver starts from du = 0: its

@@ -44,3 +44,32 @@ def test_viscous_pencil_equals_hyperplane(tmp_path, sweeps, precisions):
     print("viscous pencil", sweeps, precisions, flush=True)
     a, b = run(path, Solver.PENCIL, precisions), run(path, Solver.HYPERPLANE, precisions)
     assert all(np.array_equal(x, y) for x, y in zip(a, b))
+
+
+@pytest.mark.parametrize("between", ["state", "level", "order"])
+@pytest.mark.parametrize("precision", [0, 1])
+def test_changes_between_residual_and_relax(tmp_path, precision, between):
+    """The residual stage writes the sweep's inputs; a relax after the state,
+    the stored solution or the order changed forms them again."""
+    path = cases.vortex_case(str(tmp_path), n=13, iterations=2, ni=21, nj=9, nk=13)
+    print("pencil, change before the relax", precision, between, flush=True)
+    out = []
+    for order in (Solver.PENCIL, Solver.HYPERPLANE):
+        s = Solver(path)
+        s.set_implicit_precision(precision)
+        s.set_sweep_ordering(Solver.TILED if between == "order" else order)
+        s.begin_step(0)
+        s.assign_ghost_cells()
+        s.calc_residual()
+        if between == "state":
+            s.set_state(1.01 * s.get_state())
+        elif between == "level":
+            s.relax()
+            s.update(0)
+            s.begin_step(1)
+        s.set_sweep_ordering(order)
+        s.relax()
+        out.append(s.update_vector())
+        s.close()
+    assert np.abs(out[0]).max() > 0
+    assert np.array_equal(out[0], out[1])
