@@ -1823,13 +1823,57 @@ __global__ void __launch_bounds__(kRedThreads) KMatrixResidual(BlockMap M, Param
   if (threadIdx.x == 0) part[n].mres = s[0];
 }
 
+// Norms of a workgroup in the tree of halving strides (thread t takes t + w,
+// w = 128, ..., 1): the first two levels through LDS, the others within the first
+// wave, whose lane 0 has the result.  With eight levels and barriers KUpdate took
+// 26.0 us on 96^3 cells, 6.1 on 40^3; so 23.7 and 5.5.
+__device__ __forceinline__ void TreeNorms(double l2[5], double &m, double &bv, long long &bi) {
+  __shared__ double s[8][kRedThreads];
+  const int t = threadIdx.x;
+  auto put = [&] {
+#pragma unroll
+    for (int e = 0; e < 5; ++e) s[e][t] = l2[e];
+    s[5][t] = m;
+    s[6][t] = bv;
+    s[7][t] = __longlong_as_double(bi);
+  };
+  auto take = [&](const double o[8]) {
+#pragma unroll
+    for (int e = 0; e < 5; ++e) l2[e] += o[e];
+    m += o[5];
+    if (LinfBetter(o[6], __double_as_longlong(o[7]), bv, bi)) {
+      bv = o[6];
+      bi = __double_as_longlong(o[7]);
+    }
+  };
+  static_assert(kRedThreads == 256, "two levels through LDS");
+  double o[8];
+  if (t >= 128) put();
+  __syncthreads();
+  if (t < 128) {
+#pragma unroll
+    for (int e = 0; e < 8; ++e) o[e] = s[e][t + 128];
+    take(o);
+    if (t >= 64) put();
+  }
+  __syncthreads();
+  if (t >= 64) return;
+#pragma unroll
+  for (int e = 0; e < 8; ++e) o[e] = s[e][t + 64];
+  take(o);
+#pragma unroll
+  for (int w = 32; w > 0; w >>= 1) {
+    const double own[8] = {l2[0], l2[1], l2[2], l2[3], l2[4], m, bv, __longlong_as_double(bi)};
+#pragma unroll
+    for (int e = 0; e < 8; ++e) o[e] = __shfl_down(own[e], w);
+    take(o);
+  }
+}
+
 // procBlock::UpdateBlock (src/procBlock.cpp:826-871) with
 // ImplicitTimeAdvance (:902-916) or ExplicitEulerTimeAdvance (:880-896)
 template <typename T>
 __global__ void __launch_bounds__(kRedThreads) KUpdate(BlockMap M, Params P, Partial *part) {
-  __shared__ double sl2[5][kRedThreads];
-  __shared__ double sv[kRedThreads];
-  __shared__ long long si[kRedThreads];
   const Unit U = MapUnit(M);
   const DevBlock &b = *U.b;
   const long p = (long)U.local * blockDim.x + threadIdx.x;
@@ -1872,28 +1916,14 @@ __global__ void __launch_bounds__(kRedThreads) KUpdate(BlockMap M, Params P, Par
       }
     }
   }
-#pragma unroll
-  for (int e = 0; e < 5; ++e) sl2[e][threadIdx.x] = l2[e];
-  sv[threadIdx.x] = bv;
-  si[threadIdx.x] = bi;
-  __syncthreads();
-  for (int w = kRedThreads / 2; w > 0; w >>= 1) {
-    if (threadIdx.x < w) {
-#pragma unroll
-      for (int e = 0; e < 5; ++e) sl2[e][threadIdx.x] += sl2[e][threadIdx.x + w];
-      if (LinfBetter(sv[threadIdx.x + w], si[threadIdx.x + w], sv[threadIdx.x], si[threadIdx.x])) {
-        sv[threadIdx.x] = sv[threadIdx.x + w];
-        si[threadIdx.x] = si[threadIdx.x + w];
-      }
-    }
-    __syncthreads();
-  }
+  double m = 0.0;
+  TreeNorms(l2, m, bv, bi);
   if (threadIdx.x == 0) {
     Partial &o = part[U.global];
 #pragma unroll
-    for (int e = 0; e < 5; ++e) o.l2[e] = sl2[e][0];
-    o.linf = sv[0];
-    o.linfIdx = si[0];
+    for (int e = 0; e < 5; ++e) o.l2[e] = l2[e];
+    o.linf = bv;
+    o.linfIdx = bi;
   }
 }
 
@@ -1917,10 +1947,6 @@ __global__ void __launch_bounds__(kRedThreads) KReduceNorms(const Partial *__res
   const int n = nc.n;
   double *hist = nc.hist;
   int *counter = nc.counter;
-  __shared__ double sl2[5][kRedThreads];
-  __shared__ double sm[kRedThreads];
-  __shared__ double sv[kRedThreads];
-  __shared__ long long si[kRedThreads];
   double l2[5] = {0, 0, 0, 0, 0}, m = 0.0, bv = 0.0;
   long long bi = -1;
   for (int q = threadIdx.x; q < n; q += kRedThreads) {
@@ -1932,32 +1958,15 @@ __global__ void __launch_bounds__(kRedThreads) KReduceNorms(const Partial *__res
       bi = part[q].linfIdx;
     }
   }
-#pragma unroll
-  for (int e = 0; e < 5; ++e) sl2[e][threadIdx.x] = l2[e];
-  sm[threadIdx.x] = m;
-  sv[threadIdx.x] = bv;
-  si[threadIdx.x] = bi;
-  __syncthreads();
-  for (int w = kRedThreads / 2; w > 0; w >>= 1) {
-    if (threadIdx.x < w) {
-#pragma unroll
-      for (int e = 0; e < 5; ++e) sl2[e][threadIdx.x] += sl2[e][threadIdx.x + w];
-      sm[threadIdx.x] += sm[threadIdx.x + w];
-      if (LinfBetter(sv[threadIdx.x + w], si[threadIdx.x + w], sv[threadIdx.x], si[threadIdx.x])) {
-        sv[threadIdx.x] = sv[threadIdx.x + w];
-        si[threadIdx.x] = si[threadIdx.x + w];
-      }
-    }
-    __syncthreads();
-  }
+  TreeNorms(l2, m, bv, bi);
   if (threadIdx.x == 0) {
     const int slot = *counter;
     double *o = hist + (long)slot * 8;
 #pragma unroll
-    for (int e = 0; e < 5; ++e) o[e] = sl2[e][0];
-    o[5] = sv[0];
-    o[6] = __longlong_as_double(si[0]);
-    o[7] = sm[0];
+    for (int e = 0; e < 5; ++e) o[e] = l2[e];
+    o[5] = bv;
+    o[6] = __longlong_as_double(bi);
+    o[7] = m;
     *counter = slot + 1;
   }
 }
@@ -1978,19 +1987,27 @@ __global__ void KZeroCounters(const NormCase *__restrict__ cs, int n) {
   if (q < n) *cs[q].counter = 0;
 }
 
-__global__ void KCaseCfl(const CflCase *__restrict__ cs, int n) {
-  const int q = blockIdx.x * blockDim.x + threadIdx.x;
-  if (q >= n) return;
-  const CflCase c = cs[q];
+__device__ __forceinline__ void CaseCfl(const CflCase &c) {
   const int nn = *c.nn;
   const double v = c.start + nn * c.step;
   *c.cfl = (c.max < v) ? c.max : v;
   *c.nn = nn + 1;
 }
+__global__ void KCaseCfl(const CflCase *__restrict__ cs, int n) {
+  const int q = blockIdx.x * blockDim.x + threadIdx.x;
+  if (q < n) CaseCfl(cs[q]);
+}
 
-// StoreOldSolution (src/procBlock.cpp:1037-1053)
-__global__ void __launch_bounds__(256) KBeginStep(BlockMap M, Params P, int copyNm1) {
+// StoreOldSolution (src/procBlock.cpp:1037-1053).  The first workgroup also
+// sets the step's CFL number, one case's (`cfl`) or a group's (`cs`): a launch of
+// its own is 4.4 us of an iteration of 285 us (40^3 cells).
+__global__ void __launch_bounds__(256) KBeginStep(BlockMap M, Params P, int copyNm1, double *cfl, double cflValue,
+                                                  const CflCase *__restrict__ cs, int ncs) {
 #pragma clang fp contract(off)
+  if (blockIdx.x == 0) {
+    if (cfl && threadIdx.x == 0) *cfl = cflValue;
+    for (int q = threadIdx.x; q < ncs; q += blockDim.x) CaseCfl(cs[q]);
+  }
   const Unit Un = MapUnit(M);
   const DevBlock &b = *Un.b;
   const long p = (long)Un.local * blockDim.x + threadIdx.x;

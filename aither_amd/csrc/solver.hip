@@ -1597,14 +1597,15 @@ int ath_begin_step(ath_ctx *c, int nn) {
   HIP_OK(hipSetDevice(c->device));
   CaseRes &cr = *c->cases[0];
   cr.cfl = c->hc.Cfl(nn);
-  hipLaunchKernelGGL(ath::KSetScalar, dim3(1), dim3(1), 0, c->stream, cr.dcfl, cr.cfl);
   // StoreOldSolution only when the scheme needs U^n
   // (input::NeedToStoreTimeN, include/input.hpp:174-176)
   if (c->P.implicit) {
     const int copyNm1 = (c->P.multilevel && nn == 0) ? 1 : 0;
     c->stateSet = 1;
     hipLaunchKernelGGL(ath::KBeginStep, dim3(c->mapTotal[kMapCell256]), dim3(kBlk), 0, c->stream,
-                       c->Map(kMapCell256), c->P, copyNm1);
+                       c->Map(kMapCell256), c->P, copyNm1, cr.dcfl, cr.cfl, nullptr, 0);
+  } else {
+    hipLaunchKernelGGL(ath::KSetScalar, dim3(1), dim3(1), 0, c->stream, cr.dcfl, cr.cfl);
   }
   return CheckLaunch();
 }
@@ -2064,7 +2065,7 @@ int ath_read_restart(ath_ctx *c, const char *path, int *iteration) {
       } else {
         c->stateSet = 1;
         hipLaunchKernelGGL(ath::KBeginStep, dim3(c->mapTotal[kMapCell256]), dim3(kBlk), 0, c->stream,
-                           c->Map(kMapCell256), c->P, 1);
+                           c->Map(kMapCell256), c->P, 1, nullptr, 0.0, nullptr, 0);
         HIP_OK(hipStreamSynchronize(c->stream));
       }
     }
@@ -2373,11 +2374,12 @@ double Drop(const CaseRes &cr, const ath_norms &n) {
 // relax, update and the per-case norm reductions
 void LaunchServeIteration(ath_ctx *c) {
   const int na = (int)c->active.size();
-  hipLaunchKernelGGL(ath::KCaseCfl, dim3(Grid(na, 64)), dim3(64), 0, c->stream, c->dcflc, na);
   c->stateSet = 1;
   if (c->P.implicit)
     hipLaunchKernelGGL(ath::KBeginStep, dim3(c->mapTotal[kMapCell256]), dim3(kBlk), 0, c->stream,
-                       c->Map(kMapCell256), c->P, 0);
+                       c->Map(kMapCell256), c->P, 0, nullptr, 0.0, c->dcflc, na);
+  else
+    hipLaunchKernelGGL(ath::KCaseCfl, dim3(Grid(na, 64)), dim3(64), 0, c->stream, c->dcflc, na);
   LaunchBoundary(c);
   LaunchResidual(c);
   LaunchAfterResiduals(c);
