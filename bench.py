@@ -39,18 +39,19 @@ HBM_PEAK_GBS = 8000.0
 
 # Algorithmic bytes per physical cell (FP64; each array element once, halos
 # and re-reads excluded).
-# vortex (inviscid, scalar LU-SGS, implicit Euler):
-#   residual kernel: W 40 + geometry 128 + R 40 + lambda 8 + diagonal 8 = 224
-#   forward pass: W 40 + R 40 + U^n 40 + geometry 96 + V 8 + dt 8 + D^-1 8 +
-#   x 40 = 280; backward pass: W 40 + geometry 96 + D^-1 8 + x read 40 + x
-#   write 40 = 224
-VORTEX_FLUX_BYTES = 224
-VORTEX_SWEEP_BYTES = {"fwd": 280, "bwd": 224}
+# vortex (inviscid, scalar LU-SGS, implicit Euler, pencil order):
+#   residual kernel: W 40 + geometry 128 + R 40 + lambda 8 + diagonal 8 = 224,
+#   and for the sweep's records U^n 40 read, W 40 + right-hand side 40 + D^-1 8
+#   written = 352
+#   forward pass: W 40 + right-hand side 40 + geometry 96 + D^-1 8 + x 40 = 224;
+#   backward pass: W 40 + geometry 96 + D^-1 8 + x read 40 + x write 40 = 224
+VORTEX_FLUX_BYTES = 352
+VORTEX_SWEEP_BYTES = {"fwd": 224, "bwd": 224}
 # HBM bytes per launch on the 64^3 vortex (FP64), from rocprofv3 FETCH_SIZE /
 # WRITE_SIZE scaled by the same counters on a 256 MiB device copy (factor 2.0
 # for FETCH_SIZE, 1.0 for WRITE_SIZE); see profiles/euler-vortex-64_hbm_counters.md
-VORTEX_FLUX_TRAFFIC = 85.4e6
-VORTEX_SWEEP_TRAFFIC = 0.5 * (263.6e6 + 257.8e6)
+VORTEX_FLUX_TRAFFIC = 150.4e6
+VORTEX_SWEEP_TRAFFIC = 0.5 * (81.7e6 + 79.1e6)
 # channel (laminar, block LU-SGS, BDF2):
 #   residual stage (inviscid and viscous face fluxes, spectral radii, dt,
 #   block diagonal and inverse): W 40 + geometry 128 + R 40 + lambda 8 + dt 8
