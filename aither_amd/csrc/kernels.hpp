@@ -54,7 +54,7 @@ struct DevBlock {
   // LU-SGS: the pencil sweep's inputs in the order the sweep takes them.
   // Pencils run along axis pl, pa x pb of them along the axes pl + 1 and
   // pl + 2 (mod 3), pns steps stored for each; record (pencil, step) holds its
-  // values 64 lanes at a time (KPencilFaces, KPencilPrep, KBlockDiag,
+  // values 64 lanes at a time (KPencilFaces, KResidual, KPencilPrep, KBlockDiag,
   // KPencilOther).  pns = 0 and null pointers without it.
   int pl, pa, pb, pns;
   double ATH_GLOBAL *skF;  // face data, both sides
