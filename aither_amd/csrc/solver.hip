@@ -1459,6 +1459,23 @@ void LogLine(ath_ctx *c, const ath_norms &n, int nn, int mm, double iterSeconds)
   }
 }
 
+// `launch` captured into the context's graph.  It runs nothing, so what the
+// host knows of the last relax's inputs (rhsFormed, stateSet) stays.
+template <typename F>
+int CaptureGraph(ath_ctx *c, F launch) {
+  const int rhsFormed = c->rhsFormed, stateSet = c->stateSet;
+  HIP_OK(hipStreamBeginCapture(c->stream, hipStreamCaptureModeThreadLocal));
+  launch();
+  c->rhsFormed = rhsFormed;
+  c->stateSet = stateSet;
+  hipGraph_t g = nullptr;
+  hipError_t e = hipStreamEndCapture(c->stream, &g);
+  if (e != hipSuccess) return Fail(ATH_ERR_HIP, std::string("graph capture: ") + hipGetErrorString(e));
+  c->graph = g;
+  HIP_OK(hipGraphInstantiate(&c->graphExec, c->graph, nullptr, nullptr, 0));
+  return ATH_OK;
+}
+
 int BuildGraph(ath_ctx *c) {
   if (c->graphExec && c->graphFp32 == c->fp32 && c->graphMatres == c->matres && c->graphOrder == c->sweepOrder)
     return ATH_OK;
@@ -1466,16 +1483,13 @@ int BuildGraph(ath_ctx *c) {
   if (c->graph) { hipGraphDestroy(c->graph); c->graph = nullptr; }
   // the whole nonlinear iteration: ghost cells, residual stage, relax,
   // update and norms
-  HIP_OK(hipStreamBeginCapture(c->stream, hipStreamCaptureModeThreadLocal));
-  LaunchBoundary(c);
-  LaunchResidual(c);
-  LaunchAfterResiduals(c);
-  LaunchTail(c, false, 0);
-  hipGraph_t g = nullptr;
-  hipError_t e = hipStreamEndCapture(c->stream, &g);
-  if (e != hipSuccess) return Fail(ATH_ERR_HIP, std::string("graph capture: ") + hipGetErrorString(e));
-  c->graph = g;
-  HIP_OK(hipGraphInstantiate(&c->graphExec, c->graph, nullptr, nullptr, 0));
+  const int r = CaptureGraph(c, [c] {
+    LaunchBoundary(c);
+    LaunchResidual(c);
+    LaunchAfterResiduals(c);
+    LaunchTail(c, false, 0);
+  });
+  if (r) return r;
   c->graphFp32 = c->fp32;
   c->graphMatres = c->matres;
   c->graphOrder = c->sweepOrder;
@@ -1758,6 +1772,9 @@ int ath_run(ath_ctx *c, int nn0, int nsteps, ath_norms *last) {
         LaunchAfterResiduals(c);
         sweepLaunches += LaunchTail(c, true, eb + 2 * nflux);
       } else {
+        // its residual stage's inputs are those of the state before its update
+        c->rhsFormed = 0;
+        c->stateSet = 1;
         HIP_OK(hipGraphLaunch(c->graphExec, c->stream));
       }
       if (c->P.multilevel && mm == nl - 1) LaunchCopyNm1(c);
@@ -2388,14 +2405,7 @@ void LaunchServeIteration(ath_ctx *c) {
 
 int BuildServeGraph(ath_ctx *c) {
   if (c->graphExec) return ATH_OK;
-  HIP_OK(hipStreamBeginCapture(c->stream, hipStreamCaptureModeThreadLocal));
-  LaunchServeIteration(c);
-  hipGraph_t g = nullptr;
-  hipError_t e = hipStreamEndCapture(c->stream, &g);
-  if (e != hipSuccess) return Fail(ATH_ERR_HIP, std::string("graph capture: ") + hipGetErrorString(e));
-  c->graph = g;
-  HIP_OK(hipGraphInstantiate(&c->graphExec, c->graph, nullptr, nullptr, 0));
-  return ATH_OK;
+  return CaptureGraph(c, [c] { LaunchServeIteration(c); });
 }
 
 }  // namespace

@@ -1,0 +1,103 @@
+"""What a relax reads when something happens between the residual stage and it,
+through the C ABI: the sweep order changes, an iteration's graph is captured or
+replayed.  Every sweep order must
+give the bits of the one-launch-per-hyperplane order in the same calls, which
+forms everything in the relax."""
+import numpy as np
+import pytest
+
+from aither_amd import Solver, cases
+
+pytestmark = pytest.mark.gpu
+
+
+def write(tmp_path, kind):
+    if kind == "channel":
+        return cases.channel_case(str(tmp_path), refine=0.125, steps=1, subits=2)[0]
+    if kind == "bump":  # one block, viscous
+        path = cases.bump_case(str(tmp_path), seed=4, n=13, iterations=4, viscous=True)[0]
+        text = open(path).read()
+        open(path, "w").write(text.replace("matrixSolver: lusgs", "matrixSolver: blusgs"))
+        return path
+    return cases.vortex_case(str(tmp_path), n=13, iterations=2, ni=21, nj=9, nk=13,
+                             solver="blusgs" if kind == "block" else "lusgs")
+
+
+def relaxed(path, precision, calls):
+    """cycle value and update vectors after `calls` and a relax"""
+    s = Solver(path)
+    s.set_implicit_precision(precision)
+    s.begin_step(0)
+    s.assign_ghost_cells()
+    calls(s)
+    out = [np.array(s.relax())] + [s.update_vector(b) for b in range(s.info.num_blocks)]
+    s.close()
+    assert np.abs(out[1]).max() > 0
+    return out
+
+
+def same(a, b):
+    assert all(np.array_equal(x, y) for x, y in zip(a, b))
+
+
+@pytest.mark.parametrize("kind", ["scalar", "block", "bump", "channel"])
+@pytest.mark.parametrize("precision", [0, 1])
+@pytest.mark.parametrize("first,second", [("HYPERPLANE", "PENCIL"), ("PENCIL", "HYPERPLANE"), ("PENCIL", "PENCIL")])
+def test_order_changed(tmp_path, kind, precision, first, second):
+    """A residual under one order and a relax under another: the one-order bits."""
+    path = write(tmp_path, kind)
+    print("order changed before the relax", kind, precision, first, second, flush=True)
+
+    def calls(a, b):
+        def f(s):
+            s.set_sweep_ordering(getattr(Solver, a))
+            s.calc_residual()
+            s.set_sweep_ordering(getattr(Solver, b))
+        return f
+    same(relaxed(path, precision, calls(first, second)), relaxed(path, precision, calls("HYPERPLANE", "HYPERPLANE")))
+
+
+@pytest.mark.parametrize("kind", ["scalar", "block", "bump", "channel"])
+@pytest.mark.parametrize("precision", [0, 1])
+def test_graph_captured_between(tmp_path, kind, precision):
+    """``run`` of no steps captures the iteration and runs nothing: a relax
+    after it reads what the residual stage before it left."""
+    path = write(tmp_path, kind)
+    print("capture before the relax", kind, precision, flush=True)
+
+    def calls(a, b):
+        def f(s):
+            s.set_sweep_ordering(a)
+            s.calc_residual()
+            s.set_sweep_ordering(b)
+            s.run(0, 0)
+        return f
+    H, P = Solver.HYPERPLANE, Solver.PENCIL
+    ref = relaxed(path, precision, calls(H, H))
+    same(relaxed(path, precision, calls(H, P)), ref)
+    same(relaxed(path, precision, calls(P, H)), ref)
+    same(relaxed(path, precision, calls(P, P)), ref)
+
+
+@pytest.mark.parametrize("kind", ["scalar", "block", "bump", "channel"])
+@pytest.mark.parametrize("precision", [0, 1])
+def test_graph_replayed_between(tmp_path, kind, precision):
+    """A residual stage, then steps replayed from a graph captured under
+    another order, then a relax."""
+    path = write(tmp_path, kind)
+    print("replay before the relax", kind, precision, flush=True)
+
+    def calls(a, b):
+        def f(s):
+            s.set_sweep_ordering(b)
+            s.run(0, 0)
+            s.set_sweep_ordering(a)
+            s.calc_residual()
+            s.set_sweep_ordering(b)
+            s.run(0, 1)
+            s.set_sweep_ordering(a)
+        return f
+    H, P = Solver.HYPERPLANE, Solver.PENCIL
+    ref = relaxed(path, precision, calls(H, H))
+    same(relaxed(path, precision, calls(P, H)), ref)
+    same(relaxed(path, precision, calls(H, P)), ref)
