@@ -122,10 +122,9 @@ struct Params {
   int block;  // matrixSolver blusgs / bdplur: 5x5 main diagonal and off-diagonals
   int fp32;   // the scalar implicit operator runs in FP32: the residual stage writes Ainv32, else Ainv
   int roeJac; // inviscidFluxJacobian approximateRoe: the off-diagonals are Roe flux changes (FP64)
-  int rhsOnce; // the relax forms the right-hand side once, in sweep order (the block pencil sweep reads it)
+  int rhsOnce; // the relax writes the right-hand side and the state in sweep order (the block pencil sweep reads them)
   int prep;      // the inviscid residual kernel writes the scalar pencil sweep's records (KPencilPrep's)
   int rhsInDiag; // the block diagonal forms that right-hand side (the relax does not)
-  int copyState; // the relax refreshes the state in sweep order (it was set since the residual stage)
 };
 
 // ---------------------------------------------------------------------------
@@ -1599,15 +1598,15 @@ __global__ void __launch_bounds__(256) KInitUpdate(BlockMap M, Params P) {
   const long p = (long)U.local * blockDim.x + threadIdx.x;
   if (p >= b.ncell) return;
   T *x = OpBuf<T>::X(b);
-  if (!P.initMatrix && !P.rhsOnce && !P.copyState) {
+  if (!P.initMatrix && !P.rhsOnce) {
 #pragma unroll
     for (int e = 0; e < 5; ++e) x[e * b.ncell + p] = T(0);
     return;
   }
   const int i = (int)(p % b.ni), j = (int)((p / b.ni) % b.nj), k = (int)(p / ((long)b.ni * b.nj));
   double rb[5];
-  if (P.initMatrix || P.rhsOnce) Rhs(b, P, p, PadIdx(b, i, j, k), rb);
-  if (P.rhsOnce || P.copyState) {
+  Rhs(b, P, p, PadIdx(b, i, j, k), rb);
+  if (P.rhsOnce) {
     // the block pencil sweep's right-hand side, fixed for the relax (FP64; the
     // operator rounds it to its precision), and the state it runs from
     int lane;
@@ -1616,9 +1615,8 @@ __global__ void __launch_bounds__(256) KInitUpdate(BlockMap M, Params P) {
 #pragma unroll
     for (int e = 0; e < 5; ++e) {
       o[e * kPenLanes] = b.W[e * b.npad + c];
-      if (P.rhsOnce) o[(5 + e) * kPenLanes] = rb[e];
+      o[(5 + e) * kPenLanes] = rb[e];
     }
-    if (!P.rhsOnce) return;
   }
   if (!P.initMatrix) {
 #pragma unroll

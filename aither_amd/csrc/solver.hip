@@ -93,9 +93,8 @@ struct ath_ctx {
   int device = 0;
   hipStream_t stream = nullptr;
   int anyPark = 0;  // some block parks its wall cells' inviscid block sums (DevBlock::invPark)
-  int rhsFormed = 0;  // the last residual stage formed the relax's right-hand side (RhsInDiag); 2: to keep
-                      // even when the state changes before the relax; the scalar sweep's records (ScalarPrep)
-                      // with the 3: FP64, 4: FP32 operator's D^-1
+  int rhsFormed = 0;  // the last residual stage formed the relax's right-hand side (RhsInDiag: 1) or the scalar
+                      // sweep's records (ScalarPrep) with the FP64 (1) or FP32 (2) operator's D^-1
   int stateSet = 0;   // a state or a stored solution level changed since
   ath::HostCase hc;  // the case (a single-case context) or the numerics every case shares (a server)
   ath::Params P{};
@@ -1108,7 +1107,7 @@ void LaunchResidualT(ath_ctx *c) {
   ath::Params PR = P;
   if (ScalarPrep(c)) {
     PR.prep = 1;
-    c->rhsFormed = c->fp32 ? 4 : 3;
+    c->rhsFormed = c->fp32 ? 2 : 1;
   }
   hipLaunchKernelGGL((ath::KResidual<RECON, LIM, FLUX>), tiles, dim3(256), 0, c->stream, mt, PR);
   if (P.block) {
@@ -1141,8 +1140,7 @@ void LaunchResidualT(ath_ctx *c) {
   // the block diagonal needs dt, which the viscous pass completes
   if (P.block) {
     ath::Params PD = P;
-    PD.rhsInDiag = RhsInDiag(c) ? 1 : 0;
-    c->rhsFormed = PD.rhsInDiag ? (c->fp32 ? 1 : 2) : 0;
+    c->rhsFormed = PD.rhsInDiag = RhsInDiag(c) ? 1 : 0;
     if (P.visc.recon4)
       hipLaunchKernelGGL((ath::KBlockDiag<RECON, LIM, 3>), diag, dim3(256), 0, c->stream, md, PD);
     else
@@ -1202,20 +1200,16 @@ int LaunchRelaxT(ath_ctx *c, bool timed, size_t evBase) {
     if (timed) hipEventRecord(c->evs[evBase + 2 * pass + (begin ? 0 : 1)], c->stream);
     if (!begin) ++pass;
   };
-  // The block pencil sweep reads the right-hand side formed once, by the
-  // residual stage or here (the sweep order, the state or a stored solution
-  // level may have changed in between; the viscous FP64 stage's is kept then),
-  // and the state, refreshed here if it changed in between.  A one-sweep pencil
+  // The block pencil sweep reads the right-hand side and the state in sweep
+  // order, written once: by the residual stage, or here if the sweep order, the
+  // state or a stored solution level changed in between.  A one-sweep pencil
   // relax writes every du before anything but the scalar connection terms
   // reads it.
-  const bool blkPencil = BlockPencil(c),
-             formed = RhsInDiag(c) && c->rhsFormed && (!c->stateSet || (c->rhsFormed == 2 && !c->fp32));
+  const bool blkPencil = BlockPencil(c), formed = RhsInDiag(c) && c->rhsFormed && !c->stateSet;
   ath::Params P0 = c->P;
   P0.rhsOnce = blkPencil && !formed ? 1 : 0;
-  P0.copyState = blkPencil && c->stateSet ? 1 : 0;
   const bool pencilOnce = hc.solver == ath::Solver::LUSGS && !hc.InitMatrix() &&
-                          (blkPencil ? formed && !c->stateSet
-                                     : EffectiveOrder(c) == ATH_SWEEP_PENCIL && c->nconn == 0);
+                          (blkPencil ? formed : EffectiveOrder(c) == ATH_SWEEP_PENCIL && c->nconn == 0);
   if (!pencilOnce)
     hipLaunchKernelGGL(ath::KInitUpdate<T>, dim3(c->mapTotal[kMapCell256]), dim3(kBlk), 0, c->stream,
                        c->Map(kMapCell256), P0);
@@ -1225,7 +1219,7 @@ int LaunchRelaxT(ath_ctx *c, bool timed, size_t evBase) {
     if (blkPencil || (hc.solver == ath::Solver::LUSGS && order == ATH_SWEEP_PENCIL)) {
       const dim3 units(c->mapTotal[kMapPen256]);
       const ath::BlockMap mp = c->Map(kMapPen256);
-      if (sw == 0 && !blkPencil && !(ScalarPrep(c) && c->rhsFormed == (c->fp32 ? 4 : 3) && !c->stateSet))
+      if (sw == 0 && !blkPencil && !(ScalarPrep(c) && c->rhsFormed == (c->fp32 ? 2 : 1) && !c->stateSet))
         hipLaunchKernelGGL(ath::KPencilPrep<T>, units, dim3(kBlk), 0, c->stream, mp, c->P);
       for (int dir = 0; dir < 2; ++dir) {
         // the first forward pass of a block solver starts from du = 0: its

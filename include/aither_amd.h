@@ -150,9 +150,8 @@ int ath_assign_ghost_cells(ath_ctx *ctx);
 int ath_calc_residual(ath_ctx *ctx);
 /* linearSolver::InitializeMatrixUpdate + Relax (src/linearSolver.cpp:111-144,
  * 430-470, 509-535); returns the matrix residual (CycleAtLevel value).  Uses
- * the last ath_calc_residual's residual, time step and diagonal (for a
- * one-sweep FP64 viscous block LU-SGS relax in the pencil order also the
- * right-hand side that call formed). */
+ * the last ath_calc_residual's residual, time step and diagonal, with the
+ * state and the stored solution as they are now. */
 int ath_relax(ath_ctx *ctx, double *cycle_value);
 /* gridLevel::UpdateBlocks + ResetDiagonal (src/gridLevel.cpp:418-431) */
 int ath_update(ath_ctx *ctx, int mm, ath_norms *norms);

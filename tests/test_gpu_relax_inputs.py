@@ -1,6 +1,6 @@
 """What a relax reads when something happens between the residual stage and it,
-through the C ABI: the sweep order changes, an iteration's graph is captured or
-replayed.  Every sweep order must
+through the C ABI: the state or a stored solution level changes, the sweep order
+changes, an iteration's graph is captured or replayed.  Every sweep order must
 give the bits of the one-launch-per-hyperplane order in the same calls, which
 forms everything in the relax."""
 import numpy as np
@@ -38,6 +38,32 @@ def relaxed(path, precision, calls):
 
 def same(a, b):
     assert all(np.array_equal(x, y) for x, y in zip(a, b))
+
+
+def scale_state(s):
+    for b in range(s.info.num_blocks):
+        s.set_state(1.01 * s.get_state(b), b)
+
+
+@pytest.mark.parametrize("order", ["PENCIL", "TILED", "ROWS"])
+@pytest.mark.parametrize("kind", ["scalar", "block", "bump", "channel"])
+@pytest.mark.parametrize("precision", [0, 1])
+@pytest.mark.parametrize("between", ["state", "level", "state then level"])
+def test_state_or_level_changed(tmp_path, order, kind, precision, between):
+    """The relax uses the state and the stored solution as they are then."""
+    path = write(tmp_path, kind)
+    print("changed before the relax", order, kind, precision, between, flush=True)
+
+    def calls(o):
+        def f(s):
+            s.set_sweep_ordering(o)
+            s.calc_residual()
+            if between != "level":
+                scale_state(s)
+            if between != "state":
+                s.begin_step(1)
+        return f
+    same(relaxed(path, precision, calls(getattr(Solver, order))), relaxed(path, precision, calls(Solver.HYPERPLANE)))
 
 
 @pytest.mark.parametrize("kind", ["scalar", "block", "bump", "channel"])
