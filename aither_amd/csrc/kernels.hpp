@@ -57,6 +57,7 @@ struct DevBlock {
   // values 64 lanes at a time (KPencilFaces, KResidual, KPencilPrep, KBlockDiag,
   // KPencilOther).  pns = 0 and null pointers without it.
   int pl, pa, pb, pns;
+  int dtile;  // the block diagonal's tile, an index of kDiagTile
   double ATH_GLOBAL *skF;  // face data, both sides
   double ATH_GLOBAL *skS;  // scalar: state, right-hand side, D^-1 (and viscosity);
                            // block: state, right-hand side (viscosity, conductivity, velocity gradient)
@@ -643,28 +644,39 @@ __device__ __forceinline__ void Rhs(const DevBlock &b, const Params &P, long p, 
   RhsFrom(P, W, b.vol[p], b.dt[p], R, cN, cNm1, out);
 }
 
-// A tile's 256 cells by their place in the pencil sweep's records: pencil, step,
-// lane, for pencils along each axis; extents of the tiles in i, j, k.
-struct TileOrder {
-  unsigned char cell[3][256];
+// A tile of 256 cells and the axis its block's pencils run along
+struct CellTile {
+  int pl, n[3];
 };
-constexpr TileOrder MakeTileOrder(const int (&tile)[3][3]) {
-  TileOrder o{};
-  for (int l = 0; l < 3; ++l) {
-    const int ti = tile[l][0], tj = tile[l][1], tk = tile[l][2];
+// the tiles' cells (i fastest) by their place in the pencil sweep's records:
+// pencil, step, lane
+template <int N>
+struct TileOrder {
+  unsigned char cell[N][256];
+};
+template <int N>
+constexpr TileOrder<N> MakeTileOrder(const CellTile (&tile)[N]) {
+  TileOrder<N> o{};
+  for (int q = 0; q < N; ++q) {
+    const int c = tile[q].pl, a = (c + 1) % 3, b = (c + 2) % 3;
+    const int tc = tile[q].n[c], ta = tile[q].n[a], tb = tile[q].n[b];
     int n = 0;
-    for (int pen = 0; pen < (l == 0 ? 1 : ti / kPW); ++pen)  // pencils lie side by side along i
-      for (int key = 0; key < 64 * kPenLanes; ++key) {       // step * kPenLanes + lane
-        const int la = key % kPW, lb = key / kPW % kPW, cc = key / kPenLanes - la - lb;
-        const int i = l == 0 ? cc : kPW * pen + (l == 1 ? lb : la), j = l == 0 ? la : (l == 1 ? cc : lb),
-                  k = l == 0 ? lb : (l == 1 ? la : cc);
-        if (cc >= 0 && i < ti && j < tj && k < tk) o.cell[l][n++] = (unsigned char)(i + ti * (j + tj * k));
-      }
+    for (int b0 = 0; b0 < tb; b0 += kPW)
+      for (int a0 = 0; a0 < ta; a0 += kPW)
+        for (int key = 0; key < (tc + 2 * kPW) * kPenLanes; ++key) {  // step * kPenLanes + lane
+          const int la = key % kPW, lb = key / kPW % kPW, cc = key / kPenLanes - la - lb;
+          if (cc < 0 || cc >= tc || a0 + la >= ta || b0 + lb >= tb) continue;
+          int x[3] = {0, 0, 0};
+          x[c] = cc;
+          x[a] = a0 + la;
+          x[b] = b0 + lb;
+          o.cell[q][n++] = (unsigned char)(x[0] + tile[q].n[0] * (x[1] + tile[q].n[1] * x[2]));
+        }
   }
   return o;
 }
-constexpr int kCellTile[3][3] = {{kTI, kTJ, kTK}, {kTI, kTJ, kTK}, {kTI, kTJ, kTK}};
-__constant__ const TileOrder kCellOrder = MakeTileOrder(kCellTile);
+constexpr CellTile kCellTile[3] = {{0, {kTI, kTJ, kTK}}, {1, {kTI, kTJ, kTK}}, {2, {kTI, kTJ, kTK}}};
+__constant__ const TileOrder<3> kCellOrder = MakeTileOrder(kCellTile);
 
 template <int RECON, int LIM, int FLUX>
 __global__ void __launch_bounds__(256) KResidual(BlockMap M, Params P) {
@@ -1246,15 +1258,35 @@ __host__ __device__ constexpr int BlockRecord(bool viscous) { return viscous ? 2
 // 800 us.  Through LDS in the records' order they are runs of up to eight lanes:
 // 534 us (8 x 8 x 4 tiles 554, 16 x 8 x 1 590, a wave's 8 x 8 cells 803),
 // against 395 us without any records, which the sweep's two passes (508 -> 353
-// us) and the initialisation gone from the relax pay for.
-constexpr int kDiagTile[3][3] = {{32, 8, 1}, {8, 8, 4}, {32, 1, 8}};
-__constant__ const TileOrder kTileOrder = MakeTileOrder(kDiagTile);
+// us) and the initialisation gone from the relax pay for.  The first tile of an
+// axis is the one for blocks thick along every axis; a tile chosen by that axis
+// alone left 8 of 256 threads with a cell where ni = 1 and k is longest (the
+// rule is DiagTile's, beside the launches).
+constexpr int kDiagTiles = 11;
+constexpr CellTile kDiagTile[kDiagTiles] = {
+    {0, {32, 8, 1}}, {1, {8, 8, 4}},  {2, {32, 1, 8}}, {0, {32, 1, 8}},  {0, {256, 1, 1}}, {1, {8, 32, 1}},
+    {1, {1, 32, 8}}, {1, {1, 256, 1}}, {2, {8, 4, 8}}, {2, {1, 8, 32}}, {2, {1, 1, 256}}};
+__constant__ const TileOrder<kDiagTiles> kTileOrder = MakeTileOrder(kDiagTile);
+constexpr int Log2(int n) { return n > 1 ? 1 + Log2(n / 2) : 0; }
+struct TileShift {
+  unsigned char i[kDiagTiles], j[kDiagTiles], k[kDiagTiles];
+};
+constexpr TileShift MakeTileShift() {
+  TileShift s{};
+  for (int q = 0; q < kDiagTiles; ++q) {
+    s.i[q] = (unsigned char)Log2(kDiagTile[q].n[0]);
+    s.j[q] = (unsigned char)Log2(kDiagTile[q].n[1]);
+    s.k[q] = (unsigned char)Log2(kDiagTile[q].n[2]);
+  }
+  return s;
+}
+__constant__ const TileShift kTileShift = MakeTileShift();
 // cell `t` of tile U
 __device__ __forceinline__ void DiagCell(const DevBlock &b, const Unit &U, int t, int &i, int &j, int &k) {
-  const int ti = b.pl == 1 ? 8 : 32, tj = b.pl == 2 ? 1 : 8, tk = b.pl == 0 ? 1 : (b.pl == 1 ? 4 : 8);
-  i = U.x * ti + t % ti;
-  j = U.y * tj + t / ti % tj;
-  k = U.z * tk + t / (ti * tj);
+  const int si = kTileShift.i[b.dtile], sj = kTileShift.j[b.dtile], sk = kTileShift.k[b.dtile];
+  i = (U.x << si) + (t & ((1 << si) - 1));
+  j = (U.y << sj) + ((t >> si) & ((1 << sj) - 1));
+  k = (U.z << sk) + (t >> (si + sj));
 }
 
 // Block main diagonal (src/procBlock.cpp:449-486, 588-625, 726-763):
@@ -1412,7 +1444,7 @@ __global__ void __launch_bounds__(256, MODE == 3 && RECON < 2 ? 2 : 1) KBlockDia
     }
   }
   __syncthreads();
-  const int src = kTileOrder.cell[b.pl][tid];
+  const int src = kTileOrder.cell[b.dtile][tid];
   int oi, oj, ok, lane;
   DiagCell(b, U, src, oi, oj, ok);
   if (oi >= b.ni || oj >= b.nj || ok >= b.nk) return;

@@ -523,6 +523,30 @@ void PencilGrid(const ath::HostBlock &h, int *pl, int *pa, int *pb, int *pns) {
   *pns = h.N(l) + 2 * ath::kPW - 2;
 }
 
+// The block diagonal's tile for a block whose pencils run along axis pl: the
+// launch is bound by latency, a tile takes the same time however many of its
+// threads have a cell, so the fewest tiles win.  The first tile of the axis
+// stays unless another saves a fifth of them (40 x 100 x 3: 65 tiles of 8 x 8 x 4
+// 28 us, 60 of 8 x 32 x 1 33 us); tiles with runs of one cell along i load
+// single words and cost twice as much again (4 x 100 x 300: 520 of 1 x 8 x 32 118
+// us, 950 of 8 x 4 x 8 91 us) where the block has more.  1 x 256 x 256 viscous
+// cells 572 -> 75 us, 8 x 64 x 200 125 -> 55, 256 x 300 x 1 101 -> 77.
+int DiagTile(const ath::HostBlock &h, int pl) {
+  int best = pl;
+  double least = 1e300;
+  for (int q = 0; q < ath::kDiagTiles; ++q) {
+    const ath::CellTile &t = ath::kDiagTile[q];
+    if (t.pl != pl) continue;
+    const double cost = (double)Grid(h.ni, t.n[0]) * Grid(h.nj, t.n[1]) * Grid(h.nk, t.n[2]) *
+                        (q == pl ? 1.0 : (t.n[0] == 1 && h.ni > 1 ? 2.5 : 1.25));
+    if (cost < least) {
+      least = cost;
+      best = q;
+    }
+  }
+  return best;
+}
+
 // values of the block solvers' inverse diagonal (InverseBase in the kernels)
 template <typename T>
 long InverseSize(const ath::DevBlock &d) {
@@ -675,8 +699,11 @@ int UploadCase(ath_ctx *c, CaseRes &cr, bool fp32) {
     HIP_OK(hipMemset(d.A, 0, nc * sizeof(double)));
     d.Ab = d.Abi = nullptr;
     d.skF = d.skS = d.skX = d.skO = nullptr;
-    d.pl = d.pa = d.pb = d.pns = 0;
-    if (PencilCase(hc)) PencilGrid(h, &d.pl, &d.pa, &d.pb, &d.pns);
+    d.pl = d.pa = d.pb = d.pns = d.dtile = 0;
+    if (PencilCase(hc)) {
+      PencilGrid(h, &d.pl, &d.pa, &d.pb, &d.pns);
+      d.dtile = DiagTile(h, d.pl);
+    }
     d.vgrad = nullptr;
     d.invPark = nullptr;
     d.kc = nullptr;
@@ -908,8 +935,8 @@ int RebuildGroup(ath_ctx *c) {
         u = make_int4((d.ni + ath::kTI - 1) / ath::kTI, (d.nj + ath::kTJ - 1) / ath::kTJ,
                       (d.nk + ath::kTK - 1) / ath::kTK, f);
       else if (q == kMapDiag && d.pns)
-        u = make_int4(Grid(d.ni, ath::kDiagTile[d.pl][0]), Grid(d.nj, ath::kDiagTile[d.pl][1]),
-                      Grid(d.nk, ath::kDiagTile[d.pl][2]), f);
+        u = make_int4(Grid(d.ni, ath::kDiagTile[d.dtile].n[0]), Grid(d.nj, ath::kDiagTile[d.dtile].n[1]),
+                      Grid(d.nk, ath::kDiagTile[d.dtile].n[2]), f);
       else if (q == kMapDiag || q == kMapCell256) u = make_int4(Grid(d.ncell, ath::kRedThreads), 1, 1, f);
       else if (q == kMapPad256) u = make_int4(Grid(d.npad, 256), 1, 1, f);
       else u = make_int4(d.skS ? Grid((long)d.pa * d.pb * d.pns * kPenLanes, 256) : 0, 1, 1, f);

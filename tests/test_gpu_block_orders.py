@@ -89,3 +89,17 @@ def test_viscous_axes(tmp_path, dims, solver, sweeps, precision):
     path = write_plate(str(tmp_path), dims, wall, sweeps, solver)
     print("orders, viscous", dims, solver, sweeps, precision, flush=True)
     same(path, precision)
+
+
+# one block for each tile the block diagonal may be cut into, with remainders
+@pytest.mark.parametrize("dims", [(40, 16, 3), (9, 33, 9), (40, 3, 64), (33, 1, 9), (300, 1, 1), (9, 33, 1), (1, 40, 9),
+                                  (1, 300, 1), (9, 9, 25), (1, 9, 33), (1, 1, 300)])
+@pytest.mark.parametrize("eq", ["euler", "navierStokes"])
+def test_diagonal_tiles(tmp_path, dims, eq):
+    if eq == "euler":
+        ni, nj, nk = dims
+        path = cases.vortex_case(str(tmp_path), n=max(dims), iterations=4, ni=ni, nj=nj, nk=nk, solver="blusgs")
+    else:
+        path = write_plate(str(tmp_path), dims, next(d for d in (1, 2, 0) if dims[d] > 1), 1)
+    print("block diagonal's tiles", dims, eq, flush=True)
+    same(path, 0)
