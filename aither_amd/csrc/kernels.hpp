@@ -6,6 +6,8 @@
 //  * face vectors: one double4 (unit normal, magnitude) per physical face.
 #pragma once
 
+#include <type_traits>
+
 #include "device_math.hpp"
 
 namespace ath {
@@ -29,7 +31,8 @@ __host__ __device__ inline ATH_GLOBAL T *Dev(T *p) {
 }
 
 // Records of the pencil sweeps: pencils of kPW x kPW columns, kPenLanes lanes
-// a record (one hyperplane step of one pencil)
+// a record (one hyperplane step of one pencil, or several where the block is
+// thinner than a pencil: DevBlock::pln)
 constexpr int kPW = 8;
 constexpr int kPenLanes = kPW * kPW;
 constexpr int kPenS = 11;      // per-relax values of a cell: W, right-hand side, D^-1 (and viscosity)
@@ -53,10 +56,14 @@ struct DevBlock {
   float ATH_GLOBAL *xold32;
   // LU-SGS: the pencil sweep's inputs in the order the sweep takes them.
   // Pencils run along axis pl, pa x pb of them along the axes pl + 1 and
-  // pl + 2 (mod 3), pns steps stored for each; record (pencil, step) holds its
-  // values 64 lanes at a time (KPencilFaces, KResidual, KPencilPrep, KBlockDiag,
-  // KPencilOther).  pns = 0 and null pointers without it.
+  // pl + 2 (mod 3), pns steps stored for each in prec records, which hold each
+  // value 64 lanes at a time (KPencilFaces, KResidual, KPencilPrep, KBlockDiag,
+  // KPencilOther).  A step has 2^pln lanes, 2^pla of them along the first cut
+  // axis (the pencil's width or the block's, rounded up to a power of two), a
+  // record 64 >> pln steps: a 256 x 256 x 1 block takes 8 lanes a step, where 64
+  // would make eight times the memory.  pns = 0 and null pointers without it.
   int pl, pa, pb, pns;
+  int pla, pln, prec;
   int dtile;  // the block diagonal's tile, an index of kDiagTile
   double ATH_GLOBAL *skF;  // face data, both sides
   double ATH_GLOBAL *skS;  // scalar: state, right-hand side, D^-1 (and viscosity);
@@ -199,13 +206,20 @@ __device__ __forceinline__ long BtSlot(const DevBlock &b, int d, int upper, int 
   if (d == 1) return 2 * sI + upper * sJ + k + (long)b.nk * i;
   return 2 * sI + 2 * sJ + upper * sK + i + (long)b.ni * j;
 }
+// record (of a pencil's) and first lane of step s
+__host__ __device__ __forceinline__ int StepRecord(const DevBlock &b, int s, int &lane) {
+  const int sh = 6 - b.pln;
+  lane = (s & ((1 << sh) - 1)) << b.pln;
+  return s >> sh;
+}
 // record and lane of cell (i, j, k) in the pencil sweep's arrays
-__device__ __forceinline__ long PencilRecord(const DevBlock &b, int i, int j, int k, int &lane) {
+__host__ __device__ __forceinline__ long PencilRecord(const DevBlock &b, int i, int j, int k, int &lane) {
   const int ca = b.pl == 0 ? j : (b.pl == 1 ? k : i), cb = b.pl == 0 ? k : (b.pl == 1 ? i : j),
             cc = b.pl == 0 ? i : (b.pl == 1 ? j : k);
   const int la = ca % kPW, lb = cb % kPW;
-  lane = la + kPW * lb;
-  return (long)(ca / kPW + b.pa * (cb / kPW)) * b.pns + la + lb + cc;
+  const int r = StepRecord(b, la + lb + cc, lane);
+  lane += la + (lb << b.pla);
+  return (long)(ca / kPW + b.pa * (cb / kPW)) * b.prec + r;
 }
 // Values in LDS go 16 bytes a lane: a 16-byte read takes 13 cycles of the
 // LDS pipe for a wave, two 8-byte reads 33.  Value q of a lane's record is
@@ -238,7 +252,7 @@ template <typename T>
 constexpr int kInv = Vecs<T>(25) * kVecN<T>;
 static_assert(Vecs<float>(25) % 2 == 1 && Vecs<double>(25) % 2 == 1, "bank spread of a record in LDS");
 template <typename T>
-__device__ __forceinline__ long InverseBase(const DevBlock &b, int i, int j, int k, int &stride) {
+__host__ __device__ __forceinline__ long InverseBase(const DevBlock &b, int i, int j, int k, int &stride) {
   if (b.pns) {
     int lane;
     const long rec = PencilRecord(b, i, j, k, lane);
@@ -2601,20 +2615,22 @@ __device__ __forceinline__ double EmptySlot<double>() { return __longlong_as_dou
 template <>
 __device__ __forceinline__ float EmptySlot<float>() { return __int_as_float(-1); }
 
-// record (pid, s, lane) of the sweep-ordered arrays and its cell
+// the cell of a lane of a record of the sweep-ordered arrays
 struct PenCell {
   bool active;
   int i, j, k;
 };
-__device__ __forceinline__ PenCell PencilCell(const DevBlock &b, int pid, int s, int lane) {
+__device__ __forceinline__ PenCell PencilCell(const DevBlock &b, long rec, int lane) {
+  const int pid = (int)(rec / b.prec), s = ((int)(rec % b.prec) << (6 - b.pln)) + (lane >> b.pln);
   const int a = pid % b.pa, bb = pid / b.pa;
   const int na = AxisN(b, (b.pl + 1) % 3), nb = AxisN(b, (b.pl + 2) % 3), nc = AxisN(b, b.pl);
-  const int la = lane % kPW, lb = lane / kPW, c = s - la - lb;
+  const int l = lane & ((1 << b.pln) - 1), la = l & ((1 << b.pla) - 1), lb = l >> b.pla, c = s - la - lb;
   PenCell r;
   r.active = la < PenWidth(na, a) && lb < PenWidth(nb, bb) && c >= 0 && c < nc;
   Map3(b.pl, c, a * kPW + la, bb * kPW + lb, r.i, r.j, r.k);
   return r;
 }
+__device__ __forceinline__ long Records(const DevBlock &b) { return (long)b.pa * b.pb * b.prec; }
 
 // The face data of every pencil record, laid out once per case: side 0 the
 // lower faces (what the backward pass's products cross), side 1 the upper
@@ -2623,9 +2639,9 @@ __device__ __forceinline__ PenCell PencilCell(const DevBlock &b, int pid, int s,
 __global__ void __launch_bounds__(256) KPencilFaces(const DevBlock b, int visc, int nS) {
   const long t = (long)blockIdx.x * blockDim.x + threadIdx.x;
   const int lane = (int)(t % kPenLanes);
-  const long rec = t / kPenLanes, nrec = (long)b.pa * b.pb * b.pns;
+  const long rec = t / kPenLanes, nrec = Records(b);
   if (rec >= nrec) return;
-  const PenCell c = PencilCell(b, (int)(rec / b.pns), (int)(rec % b.pns), lane);
+  const PenCell c = PencilCell(b, rec, lane);
   const int nF = kPenF + (visc ? 3 : 0);
   if (!c.active) {
     for (int q = 0; q < nF; ++q)
@@ -2663,8 +2679,8 @@ __global__ void __launch_bounds__(256) KPencilPrep(BlockMap M, Params P) {
   const long t = (long)U.local * blockDim.x + threadIdx.x;
   const int lane = (int)(t % kPenLanes);
   const long rec = t / kPenLanes;
-  if (rec >= (long)b.pa * b.pb * b.pns) return;
-  const PenCell q = PencilCell(b, (int)(rec / b.pns), (int)(rec % b.pns), lane);
+  if (rec >= Records(b)) return;
+  const PenCell q = PencilCell(b, rec, lane);
   if (!q.active) return;
   const long p = (long)q.i + (long)q.j * b.ni + (long)q.k * b.ni * b.nj, c = PadIdx(b, q.i, q.j, q.k);
   const int nS = kPenS + (P.visc.on ? 1 : 0);
@@ -2691,8 +2707,8 @@ __global__ void __launch_bounds__(256) KPencilOther(BlockMap M, Params P) {
   const long t = (long)U.local * blockDim.x + threadIdx.x;
   const int lane = (int)(t % kPenLanes);
   const long rec = t / kPenLanes;
-  if (rec >= (long)b.pa * b.pb * b.pns) return;
-  const PenCell q = PencilCell(b, (int)(rec / b.pns), (int)(rec % b.pns), lane);
+  if (rec >= Records(b)) return;
+  const PenCell q = PencilCell(b, rec, lane);
   if (!q.active) return;
   T O[5];
   OffDiagSum<T>(b, Cast<T>(P.gas), P.visc, OpBuf<T>::X(b), q.i, q.j, q.k, FWD, O, P.block, 0, &P.gas);
@@ -2823,14 +2839,40 @@ __device__ __forceinline__ Pencil MakePencil(const DevBlock &b, int4 ent) {
   p.wb = PenWidth(p.nb, p.b);
   p.nc = AxisN(b, b.pl);
   p.ns = p.wa + p.wb + p.nc - 2;
-  p.rec = (long)p.pid * b.pns;
-  p.nrec = (long)b.pa * b.pb * b.pns;
+  p.rec = (long)p.pid * b.prec;
+  p.nrec = Records(b);
   p.msg = ent.w;
   p.toA = p.a - sgn >= 0 && p.a - sgn < b.pa;
   p.toB = p.b - sgn >= 0 && p.b - sgn < b.pb;
   p.from[0] = p.a + sgn >= 0 && p.a + sgn < b.pa;
   p.from[1] = p.b + sgn >= 0 && p.b + sgn < b.pb;
   return p;
+}
+// a column's lane among those of a step in the records; columns that the
+// records do not have read the first one's values, and their results are dropped
+__device__ __forceinline__ int RecordLane(const DevBlock &b, int lane) {
+  const int la = lane % kPW, lb = lane / kPW;
+  return (la >> b.pla) == 0 && (lb >> (b.pln - b.pla)) == 0 ? la + (lb << b.pla) : 0;
+}
+// record of pencil p's step s, and the column's lane in it
+__device__ __forceinline__ long StepAt(const DevBlock &b, const Pencil &p, int s, int recLane, int &lane) {
+  int l0;
+  const long rec = p.rec + StepRecord(b, s, l0);
+  lane = l0 + recLane;
+  return rec;
+}
+// f(axis, whether a record is one step) with both known to the compiler.  Where
+// records hold several steps the columns without lanes of their own must not
+// store; the test costs a whole step's pass 3 % (48^3, two sweeps: 140 -> 144 us).
+template <typename F>
+__device__ __forceinline__ void PencilAxis(const DevBlock &b, const Pencil &p, F f) {
+  auto with = [&](auto c) {
+    if (b.pln == 6) f(c, std::true_type{});
+    else f(c, std::false_type{});
+  };
+  if (p.C == 0) with(std::integral_constant<int, 0>{});
+  else if (p.C == 1) with(std::integral_constant<int, 1>{});
+  else with(std::integral_constant<int, 2>{});
 }
 // messages of pencil (pa, pb) of the block through its face f (0 A, 1 B)
 template <typename T, bool FWD>
@@ -2942,12 +2984,14 @@ __device__ __forceinline__ void PenFirst(const DevBlock &b, const Pencil &p, int
 // one step's slot from the sweep-ordered inputs
 template <typename T, bool FWD, bool FULL>
 __device__ __forceinline__ void PenStage(const DevBlock &b, const Params &P, const Pencil &pen,
-                                         PenSlot<T, FULL> &sl, int lane, int st, const int *xReady, int *err) {
+                                         PenSlot<T, FULL> &sl, int lane, int recLane, int st, const int *xReady,
+                                         int *err) {
   const GasT<T> g = Cast<T>(P.gas);
-  const long rec = pen.rec + (FWD ? st : pen.ns - 1 - st);
+  int rl;
+  const long rec = StepAt(b, pen, FWD ? st : pen.ns - 1 - st, recLane, rl);
   const int nS = kPenS + (P.visc.on ? 1 : 0), nF = kPenF + (P.visc.on ? 3 : 0);
-  const double *S = b.skS + rec * nS * kPenLanes + lane;
-  const double *F = b.skF + ((FWD ? pen.nrec : 0) + rec) * nF * kPenLanes + lane;
+  const double *S = b.skS + rec * nS * kPenLanes + rl;
+  const double *F = b.skF + ((FWD ? pen.nrec : 0) + rec) * nF * kPenLanes + rl;
   // every load before the wait for the slot
   T W[5], fa[12], early[kEarly<T, FULL>];
 #pragma unroll
@@ -2958,13 +3002,13 @@ __device__ __forceinline__ void PenStage(const DevBlock &b, const Params &P, con
 #pragma unroll
     for (int e = 0; e < 5; ++e) early[e] = T(S[(5 + e) * kPenLanes]);
   } else {
-    const T *X = (const T *)b.skX + rec * 5 * kPenLanes + lane;
+    const T *X = (const T *)b.skX + rec * 5 * kPenLanes + rl;
 #pragma unroll
     for (int e = 0; e < 5; ++e) early[e] = X[e * kPenLanes];
   }
   early[5] = T(S[10 * kPenLanes]);
   if constexpr (FULL) {
-    const T *o = (const T *)b.skO + rec * 5 * kPenLanes + lane;
+    const T *o = (const T *)b.skO + rec * 5 * kPenLanes + rl;
 #pragma unroll
     for (int e = 0; e < 5; ++e) early[11 + e] = o[e * kPenLanes];
   }
@@ -3005,16 +3049,18 @@ __device__ __forceinline__ void PenStage(const DevBlock &b, const Params &P, con
   for (int q = 0; q < 3; ++q) LdsPut<T, kLate<T>>(&sl.late[q][0][lane], late[q]);
 }
 
-// Where a pass writes its sweep-ordered output, first step.  The
+// Where a pass writes its sweep-ordered output of step st.  The
 // dependency-side sums of a full pass are the other-side sums of the next: its
 // cells' neighbours on that side still have this pass's du then, so without
 // connections (whose ghost du changes in between) only the first full pass of a
-// relax needs KPencilOther.  The stager reads a record before the compute wave
-// writes it.  40 iterations of two sweeps, 48^3 viscous cells: 34.6 ms with
+// relax needs KPencilOther.  The stager reads a step's values before the compute
+// wave writes them.  40 iterations of two sweeps, 48^3 viscous cells: 34.6 ms with
 // KPencilOther before each pass, 30.7 so.
 template <typename T, bool FWD, bool FULL>
-__device__ __forceinline__ T *PenStore(const DevBlock &b, const Pencil &pen) {
-  return (FULL ? (T *)b.skO : (T *)b.skX) + (pen.rec + (FWD ? 0 : pen.ns - 1)) * 5 * kPenLanes;
+__device__ __forceinline__ T *PenStore(const DevBlock &b, const Pencil &pen, int st, int recLane) {
+  int rl;
+  const long rec = StepAt(b, pen, FWD ? st : pen.ns - 1 - st, recLane, rl);
+  return (FULL ? (T *)b.skO : (T *)b.skX) + rec * 5 * kPenLanes + rl;
 }
 
 // The compute wave.  A wave issues one instruction in 4.6 cycles whatever it
@@ -3025,7 +3071,7 @@ __device__ __forceinline__ T *PenStore(const DevBlock &b, const Pencil &pen) {
 // across B and A go into LDS (where the next step's lanes and the send wave
 // take them) before the one across C, which stays in the lane's registers, is
 // formed.
-template <typename T, bool FWD, bool FULL, int C>
+template <typename T, bool FWD, bool FULL, int C, bool WHOLE>
 __device__ __forceinline__ void PenCompute(const DevBlock &b, const Params &P, const Pencil &pen,
                                            PenShared<T, FULL> &sh, int lane, int store, int *err) {
   constexpr int sgn = FWD ? -1 : 1;  // direction of the dependency neighbours
@@ -3056,7 +3102,8 @@ __device__ __forceinline__ void PenCompute(const DevBlock &b, const Params &P, c
   int p = i0 + j0 * b.ni + k0 * b.ni * b.nj;  // cell of step st (of the active steps)
   // one-sweep forward pass: du for the backward pass; full pass: the
   // dependency-side sums for the next pass (PenStore)
-  T *Xs = PenStore<T, FWD, FULL>(b, pen) + lane;
+  const int recLane = RecordLane(b, lane);
+  T *Xs = PenStore<T, FWD, FULL>(b, pen, 0, recLane);
   T xA[5], xB[5], S[5], early[kEarly<T, FULL>], late[3][kLate<T>];
   int next = 1;  // slot of the next step
   LdsWait<0>(&sh.stageReady[0], 1, err);
@@ -3139,19 +3186,21 @@ __device__ __forceinline__ void PenCompute(const DevBlock &b, const Params &P, c
     LdsGet<T, kLate<T>>(&sl.late[0][0][lane], late[0]);
     cur = &sl;
     const int kk = st - off;
-    if (col && kk >= 0 && kk < nc) {
+    const bool act = col && kk >= 0 && kk < nc;
+    if (act) {
       product(2, oC);
       if (store & 1) {
 #pragma unroll
         for (int e = 0; e < 5; ++e) x[e * b.ncell + p] = xn[e];
       }
     }
-    if ((FWD || FULL) && (store & 2)) {
+    if ((FWD || FULL) && (store & 2) && (WHOLE || act)) {
 #pragma unroll
       for (int e = 0; e < 5; ++e) Xs[e * kPenLanes] = FULL ? S[e] : xn[e];
     }
     p += sC;
-    Xs += (FWD ? 5 : -5) * kPenLanes;
+    if constexpr (WHOLE) Xs += (FWD ? 5 : -5) * kPenLanes;
+    else Xs = PenStore<T, FWD, FULL>(b, pen, min(st + 1, ns - 1), recLane);
   }
 }
 
@@ -3175,18 +3224,18 @@ __global__ void __launch_bounds__(kPenWaves * kPenLanes) KLusgsPencil(PencilGrou
   const Pencil pen = MakePencil<FWD>(b, ent);
   if (wave == 0) {
     __builtin_amdgcn_s_setprio(3);
-    if (pen.C == 0) PenCompute<T, FWD, FULL, 0>(b, P, pen, sh, lane, store, G.err);
-    else if (pen.C == 1) PenCompute<T, FWD, FULL, 1>(b, P, pen, sh, lane, store, G.err);
-    else PenCompute<T, FWD, FULL, 2>(b, P, pen, sh, lane, store, G.err);
+    PencilAxis(b, pen, [&](auto c, auto whole) {
+      PenCompute<T, FWD, FULL, c.value, whole.value>(b, P, pen, sh, lane, store, G.err);
+    });
   } else if (wave == 1) {
     PenHalo<T, FWD>(G, b, pen, sh.link, lane, OpBuf<T>::Bt(b));
   } else if (wave == 2) {
     PenSend<T, FWD>(G, b, pen, sh.link, lane);
   } else {
     // stager j: steps j, j + kStagers, ...
-    const int j = wave - 3;
+    const int j = wave - 3, recLane = RecordLane(b, lane);
     for (int st = j; st < pen.ns; st += kStagers) {
-      PenStage<T, FWD, FULL>(b, P, pen, sh.slot[j], lane, st, &sh.link.xReady, G.err);
+      PenStage<T, FWD, FULL>(b, P, pen, sh.slot[j], lane, recLane, st, &sh.link.xReady, G.err);
       LdsPost(&sh.stageReady[j], st + 1);
     }
     PenEmpty<T, FWD>(G, b, pen, j * kPenLanes + lane, kStagers * kPenLanes);
@@ -3223,7 +3272,7 @@ constexpr int kBlkR = FULL ? 10 : 5;  // right-hand side (forward du), other-sid
 template <typename T, bool FULL>
 struct BlkSlot {
   LdsVec<T> J[3][Vecs<T>(25)][kPenLanes];
-  LdsVec<T> D[kPenLanes * Vecs<T>(25)];  // the record of D^-1 as it is in memory, one cell behind the other
+  LdsVec<T> D[kPenLanes * Vecs<T>(25)];  // the step's D^-1 as they are in memory, one cell behind the other
   LdsVec<T> r[Vecs<T>(kBlkR<FULL>)][kPenLanes];
 };
 constexpr int kBlkParts = 4;  // blocks of A, B, C; the rest
@@ -3246,12 +3295,13 @@ struct BlkRaw {
   double W[5], mu, kc, vg[9], a[4], dist;
 };
 template <bool FWD>
-__device__ __forceinline__ void BlkLoad(const DevBlock &b, const Params &P, const Pencil &pen, int q, int lane, int st,
-                                        BlkRaw &r) {
-  const long rec = pen.rec + (FWD ? st : pen.ns - 1 - st);
+__device__ __forceinline__ void BlkLoad(const DevBlock &b, const Params &P, const Pencil &pen, int q, int recLane,
+                                        int st, BlkRaw &r) {
+  int rl;
+  const long rec = StepAt(b, pen, FWD ? st : pen.ns - 1 - st, recLane, rl);
   const int nF = kPenF + (P.visc.on ? 3 : 0);
-  const double *S = b.skS + rec * BlockRecord(P.visc.on) * kPenLanes + lane;
-  const double *F = b.skF + ((FWD ? pen.nrec : 0) + rec) * nF * kPenLanes + lane;
+  const double *S = b.skS + rec * BlockRecord(P.visc.on) * kPenLanes + rl;
+  const double *F = b.skF + ((FWD ? pen.nrec : 0) + rec) * nF * kPenLanes + rl;
 #pragma unroll
   for (int e = 0; e < 5; ++e) r.W[e] = S[e * kPenLanes];
 #pragma unroll
@@ -3286,14 +3336,15 @@ template <typename T, bool FWD, bool FULL>
 __device__ __forceinline__ void BlkStage(const DevBlock &b, const Params &P, const Pencil &pen,
                                          BlkShared<T, FULL> &sh, int lane, int set, int part, int *err) {
   const int *xReady = &sh.link.xReady;
+  const int recLane = RecordLane(b, lane);
   if (part < 3) {
     BlkRaw r;
-    if (set < pen.ns) BlkLoad<FWD>(b, P, pen, part, lane, set, r);
+    if (set < pen.ns) BlkLoad<FWD>(b, P, pen, part, recLane, set, r);
     for (int st = set; st < pen.ns; st += kBlkSets<T>) {
       T J[25];
       BlkForm<T, FWD>(P, r, J);
       // the next step's loads are in flight while the slot is waited for
-      BlkLoad<FWD>(b, P, pen, part, lane, min(st + kBlkSets<T>, pen.ns - 1), r);
+      BlkLoad<FWD>(b, P, pen, part, recLane, min(st + kBlkSets<T>, pen.ns - 1), r);
       const int slot = st % kBlkSlots;
       LdsWait<1>(xReady, st - kBlkSlots + 1, err);
       LdsPut<T, 25>(&sh.slot[slot].J[part][0][lane], J);
@@ -3304,8 +3355,11 @@ __device__ __forceinline__ void BlkStage(const DevBlock &b, const Params &P, con
   constexpr int V = Vecs<T>(25);
   T d[V * kVecN<T>], r[kBlkR<FULL>];
   auto load = [&](int st) {
-    const long rec = pen.rec + (FWD ? st : pen.ns - 1 - st);
-    const LdsVec<T> *ai = (const LdsVec<T> *)OpBuf<T>::Abi(b) + rec * V * kPenLanes + lane;
+    int rl;
+    const long rec = StepAt(b, pen, FWD ? st : pen.ns - 1 - st, recLane, rl);
+    // the step's cells, and what follows them in memory where they are fewer
+    // than 64 (the array has that much more behind its last record)
+    const LdsVec<T> *ai = (const LdsVec<T> *)OpBuf<T>::Abi(b) + (rec * kPenLanes + (rl - recLane)) * V + lane;
 #pragma unroll
     for (int q = 0; q < V; ++q) {
       const LdsVec<T> w = ai[q * kPenLanes];
@@ -3313,16 +3367,16 @@ __device__ __forceinline__ void BlkStage(const DevBlock &b, const Params &P, con
       for (int e = 0; e < kVecN<T>; ++e) d[q * kVecN<T> + e] = w.v[e];
     }
     if (FWD || FULL) {
-      const double *S = b.skS + (rec * BlockRecord(P.visc.on) + 5) * kPenLanes + lane;
+      const double *S = b.skS + (rec * BlockRecord(P.visc.on) + 5) * kPenLanes + rl;
 #pragma unroll
       for (int e = 0; e < 5; ++e) r[e] = T(S[e * kPenLanes]);
     } else {
-      const T *X = (const T *)b.skX + rec * 5 * kPenLanes + lane;
+      const T *X = (const T *)b.skX + rec * 5 * kPenLanes + rl;
 #pragma unroll
       for (int e = 0; e < 5; ++e) r[e] = X[e * kPenLanes];
     }
     if constexpr (FULL) {
-      const T *o = (const T *)b.skO + rec * 5 * kPenLanes + lane;
+      const T *o = (const T *)b.skO + rec * 5 * kPenLanes + rl;
 #pragma unroll
       for (int e = 0; e < 5; ++e) r[5 + e] = o[e * kPenLanes];
     }
@@ -3338,7 +3392,7 @@ __device__ __forceinline__ void BlkStage(const DevBlock &b, const Params &P, con
   }
 }
 
-template <typename T, bool FWD, bool FULL, int C>
+template <typename T, bool FWD, bool FULL, int C, bool WHOLE>
 __device__ __forceinline__ void BlkCompute(const DevBlock &b, const Pencil &pen, BlkShared<T, FULL> &sh, int lane,
                                            int store, const T *bt, int *err) {
   constexpr int sgn = FWD ? -1 : 1;  // direction of the dependency neighbours
@@ -3361,10 +3415,11 @@ __device__ __forceinline__ void BlkCompute(const DevBlock &b, const Pencil &pen,
   Map3(C, FWD ? -off : nc - 1 + off, pen.a * kPW + la, pen.b * kPW + lb, i0, j0, k0);
   const int sC = -sgn * (C == 0 ? 1 : (C == 1 ? b.ni : b.ni * b.nj));
   int p = i0 + j0 * b.ni + k0 * b.ni * b.nj;  // cell of step st (of the active steps)
-  T *Xs = PenStore<T, FWD, FULL>(b, pen) + lane;
+  const int recLane = RecordLane(b, lane);
+  T *Xs = PenStore<T, FWD, FULL>(b, pen, 0, recLane);  // (see PenCompute)
   T xA[5], xB[5], S[5], d[25], r[kBlkR<FULL>], JA[25], JB[25];
   LdsWait<0>(&sh.ready[0], kBlkParts, err);
-  LdsGet<T, 25, 1>(&sh.slot[0].D[lane * Vecs<T>(25)], d);
+  LdsGet<T, 25, 1>(&sh.slot[0].D[recLane * Vecs<T>(25)], d);
   LdsGet<T, kBlkR<FULL>>(&sh.slot[0].r[0][lane], r);
   LdsWait<0>(&ln.haloReady, 1, err);
   LdsGet<T, 5>(inA, xA);
@@ -3417,7 +3472,7 @@ __device__ __forceinline__ void BlkCompute(const DevBlock &b, const Pencil &pen,
     }
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
     LdsGet<T, kBlkR<FULL>>(&nx.r[0][lane], r);
-    LdsGet<T, 25, 1>(&nx.D[lane * Vecs<T>(25)], d);
+    LdsGet<T, 25, 1>(&nx.D[recLane * Vecs<T>(25)], d);
     if (more && __builtin_amdgcn_readfirstlane(halo) < st + 2) LdsWait<0>(&ln.haloReady, st + 2, err);
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
     const int ro = kPW * ((st + 1) % kHaloRing), po = kProdStep * (st & (kProdRing - 1));
@@ -3431,12 +3486,13 @@ __device__ __forceinline__ void BlkCompute(const DevBlock &b, const Pencil &pen,
         for (int e = 0; e < 5; ++e) x[e * b.ncell + p] = xn[e];
       }
     }
-    if ((FWD || FULL) && (store & 2)) {
+    if ((FWD || FULL) && (store & 2) && (WHOLE || act)) {
 #pragma unroll
       for (int e = 0; e < 5; ++e) Xs[e * kPenLanes] = FULL ? S[e] : xn[e];
     }
     p += sC;
-    Xs += (FWD ? 5 : -5) * kPenLanes;
+    if constexpr (WHOLE) Xs += (FWD ? 5 : -5) * kPenLanes;
+    else Xs = PenStore<T, FWD, FULL>(b, pen, min(st + 1, ns - 1), recLane);
   }
 }
 
@@ -3460,9 +3516,9 @@ __global__ void __launch_bounds__(kBlkWaves<T> * kPenLanes) KBlockPencil(PencilG
   const T *bt = FWD && !FULL ? nullptr : OpBuf<T>::Bt(b);
   if (wave == 0) {
     __builtin_amdgcn_s_setprio(3);
-    if (pen.C == 0) BlkCompute<T, FWD, FULL, 0>(b, pen, sh, lane, store, bt, G.err);
-    else if (pen.C == 1) BlkCompute<T, FWD, FULL, 1>(b, pen, sh, lane, store, bt, G.err);
-    else BlkCompute<T, FWD, FULL, 2>(b, pen, sh, lane, store, bt, G.err);
+    PencilAxis(b, pen, [&](auto c, auto whole) {
+      BlkCompute<T, FWD, FULL, c.value, whole.value>(b, pen, sh, lane, store, bt, G.err);
+    });
   } else if (wave == 1) {
     PenHalo<T, FWD>(G, b, pen, sh.link, lane, bt);
   } else if (wave == 2) {

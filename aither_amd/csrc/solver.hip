@@ -512,15 +512,26 @@ int RecordValues(const ath::HostCase &hc) {
   return hc.block ? ath::BlockRecord(hc.viscous) : ath::kPenS + (hc.viscous ? 1 : 0);
 }
 // pencils run along the block's longest axis: the fewest column handoffs
-// (each costs several steps) and the fewest idle steps (2 kPW - 2 a pencil)
-void PencilGrid(const ath::HostBlock &h, int *pl, int *pa, int *pb, int *pns) {
+// (each costs several steps) and the fewest idle steps (the pencil's widths
+// less two)
+void PencilGrid(const ath::HostBlock &h, ath::DevBlock *d) {
   int l = 2;
-  for (int d = 0; d < 2; ++d)
-    if (h.N(d) > h.N(l)) l = d;
-  *pl = l;
-  *pa = (h.N((l + 1) % 3) + ath::kPW - 1) / ath::kPW;
-  *pb = (h.N((l + 2) % 3) + ath::kPW - 1) / ath::kPW;
-  *pns = h.N(l) + 2 * ath::kPW - 2;
+  for (int q = 0; q < 2; ++q)
+    if (h.N(q) > h.N(l)) l = q;
+  const int na = h.N((l + 1) % 3), nb = h.N((l + 2) % 3);
+  auto log2Up = [](int n) {
+    int q = 0;
+    while (1 << q < n) ++q;
+    return q;
+  };
+  const int wa = std::min(na, ath::kPW), wb = std::min(nb, ath::kPW);
+  d->pl = l;
+  d->pa = Grid(na, ath::kPW);
+  d->pb = Grid(nb, ath::kPW);
+  d->pns = h.N(l) + wa + wb - 2;
+  d->pla = log2Up(wa);
+  d->pln = d->pla + log2Up(wb);
+  d->prec = Grid(d->pns, ath::kPenLanes >> d->pln);
 }
 
 // The block diagonal's tile for a block whose pencils run along axis pl: the
@@ -550,7 +561,9 @@ int DiagTile(const ath::HostBlock &h, int pl) {
 // values of the block solvers' inverse diagonal (InverseBase in the kernels)
 template <typename T>
 long InverseSize(const ath::DevBlock &d) {
-  return d.pns ? (long)ath::kInv<T> * ath::kPenLanes * d.pa * d.pb * d.pns : 25L * 256 * d.tni * d.tnj * d.tnk;
+  // (one more record: the sweep reads 64 cells from a step's first on)
+  return d.pns ? (long)ath::kInv<T> * ath::kPenLanes * ((long)d.pa * d.pb * d.prec + 1)
+               : 25L * 256 * d.tni * d.tnj * d.tnk;
 }
 
 int AllocFp32(ath_ctx *c, ath::DevBlock &d) {
@@ -699,9 +712,9 @@ int UploadCase(ath_ctx *c, CaseRes &cr, bool fp32) {
     HIP_OK(hipMemset(d.A, 0, nc * sizeof(double)));
     d.Ab = d.Abi = nullptr;
     d.skF = d.skS = d.skX = d.skO = nullptr;
-    d.pl = d.pa = d.pb = d.pns = d.dtile = 0;
+    d.pl = d.pa = d.pb = d.pns = d.pla = d.pln = d.prec = d.dtile = 0;
     if (PencilCase(hc)) {
-      PencilGrid(h, &d.pl, &d.pa, &d.pb, &d.pns);
+      PencilGrid(h, &d);
       d.dtile = DiagTile(h, d.pl);
     }
     d.vgrad = nullptr;
@@ -750,7 +763,7 @@ int UploadCase(ath_ctx *c, CaseRes &cr, bool fp32) {
       if (int r = UploadViscous(c, hc, h, br)) return r;
     // the pencil sweep's arrays
     if (d.pns) {
-      const size_t lanes = (size_t)d.pa * d.pb * d.pns * kPenLanes;
+      const size_t lanes = (size_t)d.pa * d.pb * d.prec * kPenLanes;
       const int nS = RecordValues(hc), nF = kPenF + (hc.viscous ? 3 : 0);
       if (int r = c->Alloc(&d.skF, 2 * nF * lanes)) return r;
       if (int r = c->Alloc(&d.skS, nS * lanes)) return r;
@@ -939,7 +952,7 @@ int RebuildGroup(ath_ctx *c) {
                       Grid(d.nk, ath::kDiagTile[d.dtile].n[2]), f);
       else if (q == kMapDiag || q == kMapCell256) u = make_int4(Grid(d.ncell, ath::kRedThreads), 1, 1, f);
       else if (q == kMapPad256) u = make_int4(Grid(d.npad, 256), 1, 1, f);
-      else u = make_int4(d.skS ? Grid((long)d.pa * d.pb * d.pns * kPenLanes, 256) : 0, 1, 1, f);
+      else u = make_int4(d.skS ? Grid((long)d.pa * d.pb * d.prec * kPenLanes, 256) : 0, 1, 1, f);
       v[(size_t)q * nb + b] = u;
       f += u.x * u.y * u.z;
     }
@@ -1990,15 +2003,9 @@ int ath_get_block_diagonal(ath_ctx *c, int b, int inverse, double *a) {
   for (int k = 0; k < d.nk; ++k)
     for (int j = 0; j < d.nj; ++j)
       for (int i = 0; i < d.ni; ++i) {
-        const int x[3] = {i, j, k};
-        const int ca = x[(d.pl + 1) % 3], cb = x[(d.pl + 2) % 3], cc = x[d.pl];
-        constexpr int w = ath::kPW, lanes = ath::kPenLanes;
-        const long rec = (long)(ca / w + d.pa * (cb / w)) * d.pns + ca % w + cb % w + cc;
-        const long tile = (long)(i >> 3) + (long)d.tni * ((j >> 3) + (long)d.tnj * (k >> 2));
-        const long base = d.pns ? (rec * lanes + ca % w + w * (cb % w)) * ath::kInv<double>
-                                : tile * (25 * 256) + ((i & 7) + 8 * ((j & 7) + 8 * (k & 3)));
-        const long p = i + (long)j * d.ni + (long)k * d.ni * d.nj;
-        for (int q = 0; q < 25; ++q) a[25 * p + q] = t[base + (d.pns ? 1L : 256L) * q];
+        int stride;
+        const long base = ath::InverseBase<double>(d, i, j, k, stride), p = i + (long)j * d.ni + (long)k * d.ni * d.nj;
+        for (int q = 0; q < 25; ++q) a[25 * p + q] = t[base + (long)stride * q];
       }
   return ATH_OK;
 }
@@ -2345,14 +2352,14 @@ double EstimateBytes(const ath::HostCase &hc, bool fp32) {
     t += np * 8 * 8 + nf * 32 + nc * 8 * 30 + nc * 4 + nbf * 80 + tiles * 32 + 8192;
     if (fp32) t += nc * 4 * 11 + nbf * 20;
     if (PencilCase(hc)) {
-      int pl, pa, pb, pns;
-      PencilGrid(h, &pl, &pa, &pb, &pns);
+      ath::DevBlock d{};
+      PencilGrid(h, &d);
       // the case's sweep arrays and its share of the group's message slots
       const double visc = hc.viscous ? 6 : 0;
-      t += (double)pa * pb * pns * 8 *
-           (ath::kPenLanes * (2.0 * ath::kPenF + visc + RecordValues(hc) + 5 + (hc.InitMatrix() ? 5 : 0) +
-                              (hc.block ? ath::kInv<double> + (fp32 ? ath::kInv<float> / 2 : 0) : 0)) +
-            4.0 * ath::kMsg);
+      const double inv = hc.block ? ath::kInv<double> + (fp32 ? ath::kInv<float> / 2 : 0) : 0;
+      t += 8.0 * d.pa * d.pb *
+           (ath::kPenLanes * d.prec * (2.0 * ath::kPenF + visc + RecordValues(hc) + 5 + (hc.InitMatrix() ? 5 : 0) + inv) +
+            4.0 * ath::kMsg * d.pns) + 8.0 * ath::kPenLanes * inv;
     }
     if (hc.block) t += nc * 25 * 8 + (PencilCase(hc) ? 0 : tiles * 256 * 25 * 8 * (fp32 ? 1.5 : 1.0));
     if (hc.viscous) t += np * 8 * 3 + nfp * 32 + nf * 8 + nbf + (double)h.g * h.g * 4 * (h.ni + h.nj + h.nk) * 2 * 64 +
