@@ -768,9 +768,10 @@ __device__ __forceinline__ void RusanovJacobian(const GasT<T> &g, const T W[5], 
   const T f = T(0.5) * mag;
 #pragma unroll
   for (int q = 0; q < 25; ++q) {
-    const T dis = (q % 6 == 0) ? sr : T(0);
-    const T jq = J[q] * f;
-    J[q] = positive ? jq + dis : jq - dis;
+    // (off the diagonal the dissipation is zero: only the sign of a zero entry
+    // could tell, and every product's sum starts from +0)
+    J[q] *= f;
+    if (q % 6 == 0) J[q] = positive ? J[q] + sr : J[q] - sr;
   }
 }
 

@@ -1105,7 +1105,7 @@ __device__ __forceinline__ void TSLJacobian(const GasT<double> &g, const ViscPar
   const double nx = a.x, ny = a.y, nz = a.z;
   const double u = W[1], v = W[2], w = W[3];
   const double vn = (u * nx + v * ny) + w * nz;
-  const double rho = 0.0 + W[0];
+  const double rho = W[0];  // (one species: the reference's sum from +0 is the same for rho > 0)
   const double k = kLam * vp.vscale;
   const double kt = mut * g.cps / 0.9;
   // TauNormal (src/utility.cpp:426-436)
@@ -1126,8 +1126,9 @@ __device__ __forceinline__ void TSLJacobian(const GasT<double> &g, const ViscPar
 #pragma unroll
   for (int q = 0; q < 25; ++q) J[q] = 0.0;
   const Divisor<double> byMr = MakeDivisor(mr);
-  J[0] = Quot((0.0 + 0.0) * (1.0 - Div(W[0], rho)), byMr);
-  J[20] = Quot(-(k + kt) * t, byMr) + J[0] * (g.cps * t);
+  // (J[0], the species' diffusion term 0 (1 - rho_s / rho) / mr, is zero with one
+  // species, and so is what it adds to J[20])
+  J[20] = Quot(-(k + kt) * t, byMr);
   const double sh = Div(fac * 0.5 * dist, mu + mut);
   J[6] = third * nx * nx + 1.0;
   J[11] = third * nx * ny;
@@ -3294,19 +3295,18 @@ __device__ __forceinline__ void LdsAdd(int *p) {
 struct BlkRaw {
   double W[5], mu, kc, vg[9], a[4], dist;
 };
-template <bool FWD>
-__device__ __forceinline__ void BlkLoad(const DevBlock &b, const Params &P, const Pencil &pen, int q, int recLane,
-                                        int st, BlkRaw &r) {
+template <bool FWD, bool VISC>
+__device__ __forceinline__ void BlkLoad(const DevBlock &b, const Pencil &pen, int q, int recLane, int st, BlkRaw &r) {
   int rl;
   const long rec = StepAt(b, pen, FWD ? st : pen.ns - 1 - st, recLane, rl);
-  const int nF = kPenF + (P.visc.on ? 3 : 0);
-  const double *S = b.skS + rec * BlockRecord(P.visc.on) * kPenLanes + rl;
+  constexpr int nF = kPenF + (VISC ? 3 : 0);
+  const double *S = b.skS + rec * BlockRecord(VISC) * kPenLanes + rl;
   const double *F = b.skF + ((FWD ? pen.nrec : 0) + rec) * nF * kPenLanes + rl;
 #pragma unroll
   for (int e = 0; e < 5; ++e) r.W[e] = S[e * kPenLanes];
 #pragma unroll
   for (int e = 0; e < 4; ++e) r.a[e] = F[(4 * q + e) * kPenLanes];
-  if (P.visc.on) {
+  if constexpr (VISC) {
     r.mu = S[10 * kPenLanes];
     r.kc = S[11 * kPenLanes];
 #pragma unroll
@@ -3316,13 +3316,13 @@ __device__ __forceinline__ void BlkLoad(const DevBlock &b, const Params &P, cons
 }
 // the block, formed in FP64 as NeighbourBlock forms it, in the operator's
 // precision
-template <typename T, bool FWD>
+template <typename T, bool FWD, bool VISC>
 __device__ __forceinline__ void BlkForm(const Params &P, const BlkRaw &r, T out[25]) {
 #pragma clang fp contract(off)
   const GasT<double> g = Cast<double>(P.gas);
   double J[25];
   RusanovJacobian<double>(g, r.W, r.a[0], r.a[1], r.a[2], r.a[3], FWD, J);
-  if (P.visc.on) {
+  if constexpr (VISC) {
     double V[25];
     TSLJacobian(g, P.visc, r.W, r.mu, r.kc, make_double4(r.a[0], r.a[1], r.a[2], r.a[3]), r.dist, FWD, r.vg, V);
 #pragma unroll
@@ -3338,18 +3338,32 @@ __device__ __forceinline__ void BlkStage(const DevBlock &b, const Params &P, con
   const int *xReady = &sh.link.xReady;
   const int recLane = RecordLane(b, lane);
   if (part < 3) {
-    BlkRaw r;
-    if (set < pen.ns) BlkLoad<FWD>(b, P, pen, part, recLane, set, r);
-    for (int st = set; st < pen.ns; st += kBlkSets<T>) {
-      T J[25];
-      BlkForm<T, FWD>(P, r, J);
-      // the next step's loads are in flight while the slot is waited for
-      BlkLoad<FWD>(b, P, pen, part, recLane, min(st + kBlkSets<T>, pen.ns - 1), r);
-      const int slot = st % kBlkSlots;
-      LdsWait<1>(xReady, st - kBlkSlots + 1, err);
-      LdsPut<T, 25>(&sh.slot[slot].J[part][0][lane], J);
-      LdsAdd(&sh.ready[slot]);
-    }
+    // With and without the viscous terms in loops of their own.  The stagers of
+    // a viscous block bound the pass (a step of one pencil alone: 3240 cycles, 760
+    // of them the compute wave waiting for its blocks; without the viscous terms
+    // 2820 and 2): a branch in the loop cost them 5 % of a pass.
+    auto blocks = [&](auto visc) {
+      constexpr bool kVisc = visc.value;
+      BlkRaw r;
+      auto load = [&](int st) { BlkLoad<FWD, kVisc>(b, pen, part, recLane, min(st, pen.ns - 1), r); };
+      load(set);
+      for (int st = set; st < pen.ns; st += kBlkSets<T>) {
+        T J[25];
+        BlkForm<T, FWD, kVisc>(P, r, J);
+        // formed here, not behind the wait for the slot (where the compiler
+        // would put it: FP32 pass 167 -> 255 us on 48^3 cells)
+#pragma unroll
+        for (int q = 0; q < 25; ++q) asm volatile("" : "+v"(J[q]));
+        // the next step's loads are in flight while the slot is waited for
+        load(st + kBlkSets<T>);
+        const int slot = st % kBlkSlots;
+        LdsWait<1>(xReady, st - kBlkSlots + 1, err);
+        LdsPut<T, 25>(&sh.slot[slot].J[part][0][lane], J);
+        LdsAdd(&sh.ready[slot]);
+      }
+    };
+    if (P.visc.on) blocks(std::true_type{});
+    else blocks(std::false_type{});
     return;
   }
   constexpr int V = Vecs<T>(25);
