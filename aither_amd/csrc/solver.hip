@@ -64,6 +64,7 @@ struct CaseRes {
   std::vector<BlockRes> blocks;
   std::vector<void *> allocs;         // device memory owned by this case
   size_t bytes = 0;
+  bool sweepArrays = true;            // with the pencil sweep's arrays, when its relax can use them
   int partFirst = 0, nparts = 0;      // reduction partials in the current group
   ath::BcStateDev *dstates = nullptr;
   double *dcfl = nullptr;
@@ -112,8 +113,9 @@ struct ath_ctx {
   ath::NormCase *dnorm = nullptr;   // per active case: its partials and norm ring
   ath::CflCase *dcflc = nullptr;    // per active served case: its CFL ramp
   int *dflag = nullptr;             // bit 2: a sweep dependency wait exceeded its spin limit
-  // all-block pencil sweep
+  // all-block pencil sweep; not when a case was too large for its arrays
   ath::PencilGroup pen{};
+  bool pencil = false;
   size_t msgBytes = 0;
   int fp32 = 0;
   int matres = 1;
@@ -167,8 +169,10 @@ struct ath_ctx {
   int Alloc(T **p, size_t n) {
     void *q = nullptr;
     const size_t bytes = std::max<size_t>(n, 1) * sizeof(T);
-    if (hipMalloc(&q, bytes) != hipSuccess)
+    if (hipMalloc(&q, bytes) != hipSuccess) {
+      (void)hipGetLastError();  // not the next launch's error
       return Fail(ATH_ERR_NOMEM, "device allocation of " + std::to_string(n * sizeof(T)) + " bytes failed");
+    }
     (allocTo ? allocTo : &allocs)->push_back(q);
     if (bytesTo) *bytesTo += bytes;
     *p = (T *)q;
@@ -503,7 +507,8 @@ void CaseConnections(const ath::HostCase &hc, CaseRes &cr) {
 
 int RebuildGroup(ath_ctx *c);
 
-// cases whose relax can run in the pencil order (EffectiveOrder)
+// cases whose relax can run in the pencil order (EffectiveOrder), memory
+// permitting (CaseRes::sweepArrays)
 bool PencilCase(const ath::HostCase &hc) {
   return hc.Implicit() && hc.solver == ath::Solver::LUSGS && !hc.roeJac;
 }
@@ -713,7 +718,7 @@ int UploadCase(ath_ctx *c, CaseRes &cr, bool fp32) {
     d.Ab = d.Abi = nullptr;
     d.skF = d.skS = d.skX = d.skO = nullptr;
     d.pl = d.pa = d.pb = d.pns = d.pla = d.pln = d.prec = d.dtile = 0;
-    if (PencilCase(hc)) {
+    if (PencilCase(hc) && cr.sweepArrays) {
       PencilGrid(h, &d);
       d.dtile = DiagTile(h, d.pl);
     }
@@ -899,6 +904,7 @@ int RebuildGroup(ath_ctx *c) {
   c->nhalo = c->nconn = 0;
   c->nparts = 0;
   c->pen = PencilGroup{};
+  c->pencil = false;
   for (int q = 0; q < kNumMaps; ++q) c->mapTotal[q] = 0;
   for (int q = 0; q < kNumTaskMaps; ++q) c->taskTotal[q] = 0;
   if (nb == 0) return ATH_OK;
@@ -1004,7 +1010,9 @@ int RebuildGroup(ath_ctx *c) {
   HIP_OK(hipMemcpy(c->dbt, bt.data(), bt.size() * sizeof(ath::BlockTasks), hipMemcpyHostToDevice));
   // pencil sweep queue: every block's kPW x kPW columns by column hyperplane
   // a + b, then block, then b, a; per block its first message step
-  if (c->mapTotal[kMapPen256] > 0) {
+  c->pencil = true;
+  for (const auto &br : c->blk) c->pencil = c->pencil && br.d.pns > 0;
+  if (c->pencil) {
     std::vector<int4> ent;
     std::vector<int> base(nb);
     int maxPlane = 0;
@@ -1015,7 +1023,10 @@ int RebuildGroup(ath_ctx *c) {
       steps += 2L * d.pa * d.pb * d.pns;
       maxPlane = std::max(maxPlane, d.pa + d.pb - 1);
     }
-    if (steps > std::numeric_limits<int>::max()) return Fail(ATH_ERR_NOMEM, "too many cells for the pencil sweep");
+    if (steps > std::numeric_limits<int>::max()) {
+      c->pencil = false;
+      return ATH_OK;
+    }
     for (int pl = 0; pl < maxPlane; ++pl)
       for (int b = 0; b < nb; ++b) {
         const auto &d = c->blk[b].d;
@@ -1086,13 +1097,25 @@ int Upload(ath_ctx *c) {
   FillParams(c->hc, &c->P);
   if (int r = c->Alloc(&c->dflag, 1)) return r;
   HIP_OK(hipMemset(c->dflag, 0, sizeof(int)));
-  auto cr = std::make_unique<CaseRes>();
-  cr->hc = &c->hc;
-  c->cases.push_back(std::move(cr));
-  CaseRes &k = *c->cases.back();
-  if (int r = UploadCase(c, k, false)) return r;
-  c->active.assign(1, &k);
-  return RebuildGroup(c);
+  auto upload = [&](bool sweepArrays) -> int {
+    auto cr = std::make_unique<CaseRes>();
+    cr->hc = &c->hc;
+    cr->sweepArrays = sweepArrays;
+    c->cases.push_back(std::move(cr));
+    CaseRes &k = *c->cases.back();
+    if (int r = UploadCase(c, k, false)) return r;
+    c->active.assign(1, &k);
+    return RebuildGroup(c);
+  };
+  const int r = upload(true);
+  if (r != ATH_ERR_NOMEM || !PencilCase(c->hc)) return r;
+  // too large with the pencil sweep's arrays (about half of a scalar case's
+  // bytes): without them, in another order (EffectiveOrder)
+  c->active.clear();
+  c->cases.clear();
+  for (void *p : c->groupAllocs) hipFree(p);
+  c->groupAllocs.clear();
+  return upload(false);
 }
 
 // --- launch helpers (all on c->stream) -------------------------------------
@@ -1220,10 +1243,16 @@ void LaunchResidual(ath_ctx *c) {
 // ATH_SWEEP_ROWS and ATH_SWEEP_TILED, and the hyperplane order (the pencil
 // order is reported as the first with the FP64 operator and as the second with
 // the FP32 operator, as callers know them), scalar LU-SGS the pencil, tiled and
-// hyperplane orders (ATH_SWEEP_ROWS maps to the tiled one); the Roe flux-change off-diagonals (approximateRoe) run in
-// the hyperplane order only
+// hyperplane orders (ATH_SWEEP_ROWS maps to the tiled one); the Roe flux-change
+// off-diagonals (approximateRoe) run in the hyperplane order only.  Without the
+// pencil sweep's arrays the block solvers run the hyperplane order, scalar
+// LU-SGS the tiled one instead.
 int EffectiveOrder(const ath_ctx *c) {
   if (c->P.roeJac) return ATH_SWEEP_HYPERPLANE;
+  if (PencilCase(c->hc) && !c->pencil) {
+    if (c->P.block) return ATH_SWEEP_HYPERPLANE;
+    if (c->sweepOrder == ATH_SWEEP_PENCIL) return ATH_SWEEP_TILED;
+  }
   if (c->P.block && c->sweepOrder == ATH_SWEEP_PENCIL) return c->fp32 ? ATH_SWEEP_TILED : ATH_SWEEP_ROWS;
   if (!c->P.block && c->sweepOrder == ATH_SWEEP_ROWS) return ATH_SWEEP_TILED;
   return c->sweepOrder;
@@ -2337,8 +2366,10 @@ namespace {
 
 // device bytes a case will hold (an upper bound of what UploadCase
 // allocates: state, geometry, residual and operator arrays, the block
-// operator and viscous arrays when selected, sweep tables, norm history)
-double EstimateBytes(const ath::HostCase &hc, bool fp32) {
+// operator and viscous arrays when selected, sweep tables, norm history),
+// with or without the pencil sweep's arrays
+double EstimateBytes(const ath::HostCase &hc, bool fp32, bool sweepArrays) {
+  const bool pencil = PencilCase(hc) && sweepArrays;
   double t = 4096.0 * 64 + 4096;  // norm history, scalars, states
   for (const auto &h : hc.blocks) {
     const double np = (double)h.NumPadded(), nc = (double)h.NumCells();
@@ -2351,7 +2382,7 @@ double EstimateBytes(const ath::HostCase &hc, bool fp32) {
     const double nbf = 2.0 * ((double)h.nj * h.nk + (double)h.nk * h.ni + (double)h.ni * h.nj);
     t += np * 8 * 8 + nf * 32 + nc * 8 * 30 + nc * 4 + nbf * 80 + tiles * 32 + 8192;
     if (fp32) t += nc * 4 * 11 + nbf * 20;
-    if (PencilCase(hc)) {
+    if (pencil) {
       ath::DevBlock d{};
       PencilGrid(h, &d);
       // the case's sweep arrays and its share of the group's message slots
@@ -2361,7 +2392,7 @@ double EstimateBytes(const ath::HostCase &hc, bool fp32) {
            (ath::kPenLanes * d.prec * (2.0 * ath::kPenF + visc + RecordValues(hc) + 5 + (hc.InitMatrix() ? 5 : 0) + inv) +
             4.0 * ath::kMsg * d.pns) + 8.0 * ath::kPenLanes * inv;
     }
-    if (hc.block) t += nc * 25 * 8 + (PencilCase(hc) ? 0 : tiles * 256 * 25 * 8 * (fp32 ? 1.5 : 1.0));
+    if (hc.block) t += nc * 25 * 8 + (pencil ? 0 : tiles * 256 * 25 * 8 * (fp32 ? 1.5 : 1.0));
     if (hc.viscous) t += np * 8 * 3 + nfp * 32 + nf * 8 + nbf + (double)h.g * h.g * 4 * (h.ni + h.nj + h.nk) * 2 * 64 +
                          nbf * 40.0 * h.g;
     if (hc.block && hc.viscous) t += nf * 9 * 8 + np * 10 * 8;
@@ -2479,7 +2510,7 @@ int ath_estimate_case_bytes(const char *inp_path, int precision, double *bytes) 
   ath::HostCase hc;
   std::string err = ath::LoadCase(inp_path, &hc);
   if (!err.empty()) return Fail(err.find("cannot open") == 0 ? ATH_ERR_IO : ATH_ERR_CONFIG, err);
-  *bytes = EstimateBytes(hc, precision == ATH_IMPLICIT_FP32);
+  *bytes = EstimateBytes(hc, precision == ATH_IMPLICIT_FP32, true);
   return ATH_OK;
 }
 
@@ -2512,10 +2543,17 @@ int ath_admit(ath_server *s, const char *inp_path, double residual_drop, int max
   for (auto &cp : c->cases) running += cp->state == ATH_SLOT_RUNNING;
   if (running >= s->maxSlots) return Fail(ATH_ERR_NOMEM, "no free slot");
   const bool fp32 = s->precision == ATH_IMPLICIT_FP32;
-  const double need = EstimateBytes(hc, fp32);
+  double need = EstimateBytes(hc, fp32, true);
   size_t fr = 0, tot = 0;
   HIP_OK(hipMemGetInfo(&fr, &tot));
   const double reserve = 2.0 * (1 << 30);
+  // a case that does not fit an empty server with the pencil sweep's arrays goes
+  // in without them if it fits so (and every case beside it runs the same order)
+  auto fits = [&](double n) { return n + reserve <= (double)fr && (s->budget <= 0 || s->used + n <= s->budget); };
+  if (c->cases.empty() && !fits(need) && fits(EstimateBytes(hc, fp32, false))) {
+    cr->sweepArrays = false;
+    need = EstimateBytes(hc, fp32, false);
+  }
   if (need + reserve > (double)fr) return Fail(ATH_ERR_NOMEM, "not enough free device memory for the case");
   if (s->budget > 0 && s->used + need > s->budget)
     return Fail(ATH_ERR_NOMEM, "the case does not fit in the remaining memory budget");

@@ -78,7 +78,9 @@ typedef struct {
  * (src/plot3d.cpp:363-445), the procBlock constructor and InitializeStates
  * (src/procBlock.cpp:59-174, 280-355), AssignGhostCellsGeom
  * (src/procBlock.cpp:2160-2268) and CalcCellWidths (src/procBlock.cpp:6397)
- * as called from src/main.cpp:101-164. */
+ * as called from src/main.cpp:101-164.  A case that fits the device only
+ * without the pencil sweep's arrays (about half of a scalar LU-SGS case's
+ * bytes) is opened without them: see ath_get_sweep_ordering. */
 int ath_open(const char *inp_path, int device, ath_ctx **out);
 void ath_close(ath_ctx *ctx);
 const char *ath_last_error(void);
@@ -106,7 +108,9 @@ int ath_set_sweep_ordering(ath_ctx *ctx, int ordering);
  * as ATH_SWEEP_ROWS with the FP64 operator and as ATH_SWEEP_TILED with the
  * FP32 operator (both names run their pencil sweep), scalar LU-SGS maps
  * ATH_SWEEP_ROWS to ATH_SWEEP_TILED, and the approximateRoe flux Jacobian always runs
- * ATH_SWEEP_HYPERPLANE, whatever was set */
+ * ATH_SWEEP_HYPERPLANE, whatever was set.  Without memory for the pencil
+ * sweep's arrays block solvers run ATH_SWEEP_HYPERPLANE and scalar LU-SGS
+ * ATH_SWEEP_TILED in its place */
 int ath_get_sweep_ordering(const ath_ctx *ctx, int *ordering);
 /* Autotune the sweep execution order for this case: time `iterations`
  * nonlinear iterations in each order the case admits (pencil, tiled and
@@ -302,13 +306,16 @@ void ath_server_close(ath_server *srv);
  * estimates), and the device's free memory */
 int ath_server_memory(const ath_server *srv, double *used, double *free_hbm);
 /* the device bytes admission reserves for a case: an upper bound of what it
- * allocates (no device needed) */
+ * allocates (no device needed; with the pencil sweep's arrays) */
 int ath_estimate_case_bytes(const char *inp_path, int precision, double *bytes);
 /* Read the case (as ath_open does) and upload it if its estimated device
  * memory fits the free memory and the budget and a slot is free; else
  * ATH_ERR_NOMEM (nothing changed: try again after a retire).  The case runs
  * until its residual drop is <= `residual_drop` (checked after every batch
- * step) or `max_iterations` are done.  *slot identifies it from then on. */
+ * step) or `max_iterations` are done.  *slot identifies it from then on.
+ * A case that does not fit an empty server with the pencil sweep's arrays is
+ * taken without them if it fits so; while it runs every case runs the tiled
+ * (block solvers: hyperplane) order, with the same results. */
 int ath_admit(ath_server *srv, const char *inp_path, double residual_drop, int max_iterations, int *slot);
 /* `iterations` nonlinear iterations of every running case, launched
  * together and replayed from a captured HIP graph; then each case's norms
