@@ -40,11 +40,19 @@ __device__ __forceinline__ double Dmin(double a, double b) { return (b < a) ? b 
 // on the IBM RISC System/6000 processor", 1990), and div_fixup settles signs
 // of zeros, infinities and NaN.  These are the operations of the compiler's
 // division without its scaling of operands near the ends of the exponent
-// range, so a quotient is that of operator/ bit for bit while divisor,
-// numerator residual (numerator 2^-53) and quotient are normal numbers; below
-// that it may be off by a few units of the smallest denormal.  A division by
-// operator/ is eleven operations, four of them in a row through one condition
-// register; four by one divisor are 17 here.
+// range, so a quotient is that of operator/ bit for bit while the divisor, its
+// reciprocal, the numerator's residual (numerator 2^-53) and the quotient are
+// normal numbers: numerators above 2^-969, divisors between 2^-1022 and 2^1022
+// (FP32: 2^-102, 2^-126 and 2^126).  Outside it
+//  * a smaller numerator's quotient may be off by a few units of the smallest
+//    denormal;
+//  * a quotient that overflows is NaN, not infinity, and so is one by a divisor
+//    below 2^-1024 (FP32: 2^-128), unless numerator or divisor is zero,
+//    infinite or NaN itself;
+//  * a divisor above 2^1022 (2^126) loses digits.
+// Nondimensional states, volumes and areas are hundreds of orders of magnitude
+// away.  A division by operator/ is eleven operations, four of them in a row
+// through one condition register; four by one divisor are 21 here.
 template <typename T>
 struct Divisor {
   T d, y;
@@ -68,8 +76,10 @@ __device__ __forceinline__ float Quot(float n, const Divisor<float> &v) {
   q = fmaf(fmaf(-v.d, q, n), v.y, q);
   return __builtin_amdgcn_div_fixupf(fmaf(fmaf(-v.d, q, n), v.y, q), v.d, n);
 }
-// sqrt for x = 0 or x >= 2^-760: the Goldschmidt iteration of sqrt() without
-// its scaling of small arguments (inf and NaN pass through)
+// sqrt for x = 0 or x >= 2^-760: the Goldschmidt iteration with two residual
+// corrections (Markstein, "Software division and square root using
+// Goldschmidt's algorithms", 2004) without a scaling of small arguments, whose
+// roots may be off in the last digit; infinity and NaN pass through
 __device__ __forceinline__ double SqrtInRange(double x) {
   const double y = __builtin_amdgcn_rsq(x);
   double g = x * y, h = 0.5 * y;
