@@ -3116,6 +3116,10 @@ __device__ __forceinline__ void PenCompute(const DevBlock &b, const Params &P, c
 #pragma unroll
   for (int q = 0; q < 2; ++q) LdsGet<T, kLate<T>>(&sh.slot[0].late[q][0][lane], late[q]);
   const PenSlot<T, FULL> *cur = &sh.slot[0];
+  // The loop from a cache line's start on: without it a pass takes up to 2 %
+  // longer along one axis or another as the code before it changes (57 x 49 x 38
+  // FP64 along i 141 against 139 us, 40^3 FP32 105 against 103).
+  asm volatile(".p2align 6");
   for (int st = 0; st < ns; ++st) {
     const bool more = st + 1 < ns;
     __builtin_amdgcn_sched_barrier(0);
