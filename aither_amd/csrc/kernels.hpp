@@ -1325,7 +1325,7 @@ __device__ __forceinline__ void DiagCell(const DevBlock &b, const Unit &U, int t
 // (src/procBlock.cpp:1467-1474) and as lower cell subtracting (:1416-1424),
 // stores the cell velocity gradient, a sixth of each face's in the same order
 // (:1396-1414, 1427-1436), and finishes.  Bound by latency: two waves a SIMD (its
-// registers), VALU 45 % busy, 1.75 GB at 3.3 TB/s on the 1.03M-cell channel.
+// registers), VALU 38 % busy, 1.75 GB at 3.4 TB/s on the 1.03M-cell channel.
 template <int RECON, int LIM, int MODE>
 __global__ void __launch_bounds__(256, MODE == 3 && RECON < 2 ? 2 : 1) KBlockDiag(BlockMap M, Params P) {
 #pragma clang fp contract(off)
@@ -2118,16 +2118,16 @@ namespace ath {
 // ---------------------------------------------------------------------------
 // Publishing a sweep's du to other workgroups.
 //
-// A workgroup publishes a tile's (or a pencil's) du by storing it and then a
-// flag or progress count that other workgroups poll; they read the du after
-// an agent-scope acquire.  An agent-scope release on this target writes back
-// the XCD's L2 and then waits for the wave's stores: the write-back is there
-// for stores that are not coherent at agent scope, and it cost about 100 us
-// of each 760 us block-sweep pass.  The sweeps therefore store du with
-// agent-scope atomic stores (written through to the agent's point of
-// coherence), wait for each wave's own stores to complete, and only then
-// store the flag; no write-back is needed for stores that are already
-// coherent.
+// A workgroup publishes a tile's du by storing it and then a flag that other
+// workgroups poll; they read the du after an agent-scope acquire.  An
+// agent-scope release on this target writes back the XCD's L2 and then waits
+// for the wave's stores: the write-back is there for stores that are not
+// coherent at agent scope, and it cost about 100 us of each 760 us pass of a
+// tile sweep.  The sweeps therefore store with agent-scope atomic stores
+// (written through to the agent's point of coherence), the tiled one waits for
+// each wave's own stores to complete and only then stores the flag; no
+// write-back is needed for stores that are already coherent.  (The pencil
+// sweeps' messages carry their own validity.)
 template <typename T>
 __device__ __forceinline__ void StoreCoherent(T *p, T v) {
   __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
@@ -2562,7 +2562,7 @@ __global__ void __launch_bounds__(kLT) KLusgsTile(DevBlock b, Params P, SweepCtl
 //
 // Measured per pass on a 64^3 block, against a sweep that handed du from an
 // owner wave to three neighbour waves and published progress counts: FP64 785
-// -> 184 us, FP32 790 -> 166 us.  A step takes 0.80 us (0.47 us of it
+// -> 185 us, FP32 790 -> 164 us.  A step takes 0.80 us (0.47 us of it
 // the compute wave's arithmetic, the rest its LDS and store instructions,
 // which hold the wave's issue for 13-29 cycles each), a handoff 1.6 us more
 // than its step.  Three compute waves, one per outgoing product, took 0.82 us
@@ -3258,14 +3258,16 @@ __global__ void __launch_bounds__(kPenWaves * kPenLanes) KLusgsPencil(PencilGrou
 // matrices, row by row in BlockMult's order, so the result is that of
 // KLusgsForward / KLusgsBackward bit for bit.
 //
-// Bound by the step, one wave's 195 FP64 operations and 54 16-byte LDS reads:
-// 1.08 us a step in FP64, 0.84 in FP32.  A pass over the eight blocks of the
-// 1.03M-cell channel takes 353 us (FP32 320), of eight blocks of 59 x 39 x 19
-// and smaller 188 (171), of 24 x 16 x 8 and smaller 71 (59); the tile sweep
-// with per-tile flags that was here before took 508 (494), 207 (317) and 83
-// (138), so it is gone.  FP32 waves of 168 registers hold two sets of stagers
-// without scratch (one set: 343, 195, 73 us); FP64 waves of 168 spill (820 us),
-// so one set with 256.
+// Bound by the step: one wave's 195 FP64 operations and 54 16-byte LDS reads,
+// 1.09 us alone in FP64 (48^3 without viscous terms), and what it waits for.  On
+// the eight blocks of the 1.03M-cell channel a step takes 1.87 us, 0.42 of them
+// for its blocks (the stagers issue and wait for their loads, 184 pencils at
+// once, for as long as they form) and 0.42 for the pencil upstream.  A pass there
+// takes 354 us (FP32 319), of eight blocks of 59 x 39 x 19 and smaller 189 (170),
+// of 24 x 16 x 8 and smaller 68 (58); the tile sweep with per-tile flags that was
+// here before took 508 (494), 207 (317) and 83 (138), so it is gone.  FP32 waves
+// of 168 registers hold two sets of stagers without scratch (one set: 343, 195,
+// 73 us); FP64 waves of 168 spill (820 us), so one set with 256.
 constexpr int kBlkSlots = 2;
 template <typename T>
 constexpr int kBlkSets = sizeof(T) == 4 ? 2 : 1;  // groups of four stager waves, each taking every kBlkSets-th step

@@ -77,16 +77,17 @@ CHANNEL_PENCIL_SWEEP_BYTES = {"fwd": 568, "bwd": 528}
 # HBM bytes per launch on the full-size channel (refine 1), from rocprofv3
 # FETCH_SIZE / WRITE_SIZE scaled by the device-copy calibration (2.0, 1.0);
 # see profiles/channel-multiblock-1M_hbm_counters.md
-CHANNEL_PENCIL_SWEEP_TRAFFIC = 0.5 * (782e6 + 728e6)  # one pass, forward and backward averaged
-CHANNEL_FLUX_TRAFFIC = 3046e6                         # residual stage over all blocks
+CHANNEL_PENCIL_SWEEP_TRAFFIC = 0.5 * (787e6 + 732e6)  # one pass, forward and backward averaged
+CHANNEL_FLUX_TRAFFIC = 3042e6                         # residual stage over all blocks
 # what the occupancy and VALU counters show binds each (rocprofv3 SQ_WAVES,
 # SQ_INSTS_VALU, VALUBusy, OccupancyPercent on the same case; see
 # profiles/channel-multiblock-1M_sq_counters.md)
-PENCIL_SWEEP_LIMITER = ("dependency latency: 184 pencils of one workgroup each, 110 steps of 1.08 us (one wave's four "
-                        "5x5 products) and the handoffs between pencils; HBM about 30 %")
-FLUX_LIMITER = ("mixed: KResidual FP64-VALU issue (VALUBusy 80 %), the viscous block diagonal with the inviscid "
-                "block sum, the relax's right-hand side and the sweep's records latency (VALU 45 %, HBM 41 %), "
-                "the viscous flux the latency of its gathers (occupancy 22 %, VALU 27 %, HBM 40 %)")
+PENCIL_SWEEP_LIMITER = ("dependency latency: 184 pencils of one workgroup each, 190 hyperplanes of 1.87 us (1.09 us of "
+                        "one wave's four 5x5 products, the rest its waits for the stagers' loads and for the pencil "
+                        "upstream); HBM about 27 %")
+FLUX_LIMITER = ("mixed: KResidual FP64-VALU issue (VALUBusy 79 %), the viscous block diagonal with the inviscid "
+                "block sum, the relax's right-hand side and the sweep's records latency (VALU 38 %, HBM 42 %), "
+                "the viscous flux the latency of its gathers (occupancy 23 %, VALU 26 %, HBM 40 %)")
 
 
 def parse():

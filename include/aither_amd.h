@@ -212,7 +212,7 @@ typedef struct {
   int flux_launches;        /* residual stages timed (one per iteration) */
   double sweep_ms;          /* summed sweep passes: each forward or backward
                                LU-SGS pass (or DP-LUR sweep) over all blocks,
-                               including its one-thread prologue */
+                               with its prologues in the tiled order */
   int sweep_launches;       /* sweep kernel launches in those passes */
   int sweep_passes;
 } ath_timing;
