@@ -1327,7 +1327,7 @@ __device__ __forceinline__ void DiagCell(const DevBlock &b, const Unit &U, int t
 // (:1396-1414, 1427-1436), and finishes.  Bound by latency: two waves a SIMD (its
 // registers), VALU 38 % busy, 1.75 GB at 3.4 TB/s on the 1.03M-cell channel.
 template <int RECON, int LIM, int MODE>
-__global__ void __launch_bounds__(256, MODE == 3 && RECON < 2 ? 2 : 1) KBlockDiag(BlockMap M, Params P) {
+__global__ void __launch_bounds__(MODE == 1 ? 128 : 256, MODE == 3 && RECON < 2 ? 2 : 1) KBlockDiag(BlockMap M, Params P) {
 #pragma clang fp contract(off)
   const Unit U = MapUnit(M);
   const DevBlock &b = *U.b;

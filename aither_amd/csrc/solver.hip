@@ -136,7 +136,7 @@ struct ath_ctx {
   // unit grids of the all-block launches (ath::BlockMap), kNumMaps of them,
   // nb entries each, and each one's total unit count
   int4 *dmaps = nullptr;
-  int mapTotal[5] = {0, 0, 0, 0, 0};
+  int mapTotal[6] = {0, 0, 0, 0, 0, 0};
   // the ghost-cell task lists of every block (ath::BlockTasks), kNumTaskMaps
   // tables of nb entries, and each one's item total
   ath::BlockTasks *dbt = nullptr;
@@ -188,9 +188,11 @@ int Grid(long n, int b = kBlk) { return (int)((n + b - 1) / b); }
 
 // the unit grids of the all-block launches: 8x8x4 tiles (residual, viscous
 // flux), the block diagonal's tiles, ranges of 256 cells (matrix residual,
-// update, initialisation; the partials of the reductions are their slots), of 256 padded cells (auxiliary variables) and of 256 lanes of the
-// pencil sweep's records
-enum { kMapTile = 0, kMapDiag = 1, kMapCell256 = 2, kMapPad256 = 3, kMapPen256 = 4, kNumMaps = 5 };
+// update, initialisation; the partials of the reductions are their slots), of
+// 256 padded cells (auxiliary variables), of 256 lanes of the pencil sweep's
+// records and of 128 cells (the wall cells' block sums: most workgroups have
+// none, 1.03M-cell channel 31 us, with 256 cells 39)
+enum { kMapTile = 0, kMapDiag = 1, kMapCell256 = 2, kMapPad256 = 3, kMapPen256 = 4, kMapCell128 = 5, kNumMaps = 6 };
 // the ghost-cell task tables: boundary patches, edge lines of the inviscid
 // and of the viscous pass, no-slip wall cells
 enum { kTaskBc = 0, kTaskEdgeInv = 1, kTaskEdgeVisc = 2, kTaskWall = 3, kNumTaskMaps = 4 };
@@ -958,6 +960,7 @@ int RebuildGroup(ath_ctx *c) {
                       Grid(d.nk, ath::kDiagTile[d.dtile].n[2]), f);
       else if (q == kMapDiag || q == kMapCell256) u = make_int4(Grid(d.ncell, ath::kRedThreads), 1, 1, f);
       else if (q == kMapPad256) u = make_int4(Grid(d.npad, 256), 1, 1, f);
+      else if (q == kMapCell128) u = make_int4(Grid(d.ncell, 128), 1, 1, f);
       else u = make_int4(d.skS ? Grid((long)d.pa * d.pb * d.prec * kPenLanes, 256) : 0, 1, 1, f);
       v[(size_t)q * nb + b] = u;
       f += u.x * u.y * u.z;
@@ -1164,8 +1167,8 @@ bool ScalarPrep(const ath_ctx *c) {
 template <int RECON, int LIM, int FLUX>
 void LaunchResidualT(ath_ctx *c) {
   const ath::Params &P = c->P;
-  const ath::BlockMap mt = c->Map(kMapTile), mc = c->Map(kMapCell256), md = c->Map(kMapDiag), mp = c->Map(kMapPad256);
-  const dim3 tiles(c->mapTotal[kMapTile]), cells(c->mapTotal[kMapCell256]),
+  const ath::BlockMap mt = c->Map(kMapTile), mc = c->Map(kMapCell128), md = c->Map(kMapDiag), mp = c->Map(kMapPad256);
+  const dim3 tiles(c->mapTotal[kMapTile]), cells(c->mapTotal[kMapCell128]),
              diag(c->mapTotal[kMapDiag]);
   ath::Params PR = P;
   if (ScalarPrep(c)) {
@@ -1182,7 +1185,7 @@ void LaunchResidualT(ath_ctx *c) {
       c->rhsFormed = PD.rhsInDiag = RhsInDiag(c) ? 1 : 0;
       hipLaunchKernelGGL((ath::KBlockDiag<RECON, LIM, 0>), diag, dim3(256), 0, c->stream, md, PD);
     } else if (c->anyPark)
-      hipLaunchKernelGGL((ath::KBlockDiag<RECON, LIM, 1>), cells, dim3(256), 0, c->stream, mc, P);
+      hipLaunchKernelGGL((ath::KBlockDiag<RECON, LIM, 1>), cells, dim3(128), 0, c->stream, mc, P);
   }
   if (!P.visc.on) return;
   // viscous ghost cells, temperature and viscosity, viscous fluxes
