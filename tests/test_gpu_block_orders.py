@@ -103,3 +103,26 @@ def test_diagonal_tiles(tmp_path, dims, eq):
         path = write_plate(str(tmp_path), dims, next(d for d in (1, 2, 0) if dims[d] > 1), 1)
     print("block diagonal's tiles", dims, eq, flush=True)
     same(path, 0)
+
+
+@pytest.mark.parametrize("solver", ["lusgs", "blusgs"])
+@pytest.mark.parametrize("sweeps,precision", [(1, 0), (2, 0), (1, 1), (2, 1)])
+def test_thin_and_thick_blocks_in_one_launch(tmp_path, solver, sweeps, precision):
+    """Cases whose records hold one step, two, eight and sixty-four, side by side
+    in a server and each alone"""
+    from aither_amd import Server
+    paths = []
+    for q, (ni, nj, nk) in enumerate([(20, 19, 18), (33, 1, 40), (1, 1, 50), (4, 30, 9), (17, 2, 2)]):
+        (tmp_path / str(q)).mkdir()
+        paths.append(cases.vortex_case(str(tmp_path / str(q)), n=max(ni, nj, nk), iterations=4, ni=ni, nj=nj, nk=nk,
+                                       solver=solver, sweeps=sweeps))
+    print("thin and thick blocks", solver, sweeps, precision, flush=True)
+
+    def states(some):
+        with Server(max_slots=8, precision=precision) as srv:
+            slots = [srv.admit(p, 1e-200, 2 ** 30) for p in some]
+            srv.step(4)
+            return [srv.state(s) for s in slots]
+    alone = [states([p])[0] for p in paths]
+    assert all(np.all(np.isfinite(a)) for a in alone)
+    assert all(np.array_equal(a, b) for a, b in zip(states(paths), alone))
